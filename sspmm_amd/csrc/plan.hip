@@ -166,7 +166,9 @@ static hipError_t static_scratch(unsigned char **ptr, hipStream_t stream) {
 bool static_spmm_fits(int m_vec, int N) { return m_vec <= kStaticMaxRows && N <= kStaticMaxN; }
 
 hipError_t launch_spmm_static(const SpmmArgs &a, int V, bool out_f16, hipStream_t stream) {
-  if (!balanced_kernel_applies(a, V, out_f16)) return launch_spmm(a, V, out_f16, stream);  // (needs no scratch)
+  // (Ragged widths take launch_spmm, which needs no scratch: such calls may overlap and may be the first of a process
+  // inside a capture.)
+  if (!rows_are_whole_pieces(a, out_f16) || !balanced_kernel_applies(a, V, out_f16)) return launch_spmm(a, V, out_f16, stream);
   unsigned char *base = nullptr;
   hipError_t e = static_scratch(&base, stream);
   if (e != hipSuccess) return e;

@@ -47,6 +47,8 @@ int last_kernel();
 // Only where balanced_kernel_applies (the MFMA kernels' alignment and size conditions).
 struct ScheduleView;
 bool balanced_kernel_applies(const SpmmArgs &args, int V, bool out_f16);
+// Whether every row of B and C is a run of whole, aligned 16-byte pieces.
+bool rows_are_whole_pieces(const SpmmArgs &args, bool out_f16);
 // bundle_base >= 0: the schedule files its whole rows in bundles, units 0 .. bundle_base - 1 are the panels of cut
 // rows (one item each), unit bundle_base + b is bundle b, and n_items counts units.
 hipError_t launch_spmm_balanced(const SpmmArgs &args, int V, bool out_f16, const ScheduleView &schedule, int n_items,

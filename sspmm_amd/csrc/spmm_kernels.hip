@@ -36,6 +36,9 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t uintx2 __attribute__((ext_vector_type(2)));
+// the same as they lie in C, whose rows may begin at any element
+typedef half8 half8_u __attribute__((aligned(2)));
+typedef floatx4 floatx4_u __attribute__((aligned(4)));
 
 // Raw buffer descriptor word 3 for gfx9-family targets: 32-bit raw (untyped) buffer.
 static constexpr uint32_t kSrdWord3 = 0x00020000u;
@@ -43,6 +46,16 @@ static constexpr uint32_t kSrdWord3 = 0x00020000u;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_srd(const void *base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, (int)kSrdWord3);
 }
+
+// B and C are read and written in pieces of eight consecutive columns (16 bytes of fp16).  The piece that begins at
+// column c < N really covers columns unit_col(c, N) .. + 7: where N is no multiple of eight the last piece of a row
+// slides back so that it ends with the row, and its first columns are computed (from the same operands in the same
+// order, so to the same bits) and stored twice.  Every access then stays inside its row, whatever the width, and for
+// whole pieces nothing changes.  Rows of such widths begin at any multiple of 2 bytes: the device's unaligned access
+// mode takes 16-byte accesses there, at the price of the extra lines they straddle.
+__device__ __forceinline__ int unit_col(int c, int N) { return min(c, N - 8); }
+// the same for four columns at c, a multiple of four from the tile's first column n0
+__device__ __forceinline__ int quad_col(int n0, int c, int N) { return unit_col(n0 + (c & ~7), N) + (c & 4); }
 
 // v_perm_b32 picks each result byte from the 8 bytes {y (bytes 4-7), x (bytes 0-3)}.
 // pack_lo = low half of x | low half of y << 16; pack_hi the same with the high halves.
@@ -89,8 +102,8 @@ struct Store8<float> {
   static __device__ __forceinline__ void run(float *p, const float (&v)[8]) {
     floatx4 a = {v[0], v[1], v[2], v[3]};
     floatx4 b = {v[4], v[5], v[6], v[7]};
-    *reinterpret_cast<floatx4 *>(p) = a;
-    *reinterpret_cast<floatx4 *>(p + 4) = b;
+    *reinterpret_cast<floatx4_u *>(p) = a;
+    *reinterpret_cast<floatx4_u *>(p + 4) = b;
   }
 };
 
@@ -102,7 +115,7 @@ struct Store8<_Float16> {
     for (int i = 0; i < 8; ++i) h[i] = (_Float16)v[i];  // v_cvt_f16_f32: round to nearest even
     // (non-temporal: the rows of B the grid keeps gathering stay in the L2; measured 1-10 % on fp16 outputs.  fp32
     // tiles of 128 columns do not come through here: they go out as whole lines, see store_tile_f32_lines)
-    __builtin_nontemporal_store(h, reinterpret_cast<half8 *>(p));
+    __builtin_nontemporal_store(h, reinterpret_cast<half8_u *>(p));
   }
 };
 
@@ -115,15 +128,16 @@ struct StoreRow<OutT, 8> {
 template <>
 struct StoreRow<float, 4> {
   static __device__ __forceinline__ void run(float *p, const float (&v)[4]) {
-    *reinterpret_cast<floatx4 *>(p) = floatx4{v[0], v[1], v[2], v[3]};
+    *reinterpret_cast<floatx4_u *>(p) = floatx4{v[0], v[1], v[2], v[3]};
   }
 };
 template <>
 struct StoreRow<_Float16, 4> {
   static __device__ __forceinline__ void run(_Float16 *p, const float (&v)[4]) {
     typedef _Float16 half4v __attribute__((ext_vector_type(4)));
+    typedef half4v half4_u __attribute__((aligned(2)));
     const half4v h = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};  // round to nearest even
-    *reinterpret_cast<half4v *>(p) = h;
+    *reinterpret_cast<half4_u *>(p) = h;
   }
 };
 
@@ -284,13 +298,14 @@ __device__ __forceinline__ void store_tile_f32_lines(float (*ctile)[128 + 4], co
       *reinterpret_cast<floatx4 *>(&ctile[v][8 * m + 4]) = floatx4{acc[4][rr], acc[5][rr], acc[6][rr], acc[7][rr]};
     }
   }
-  const int c4 = (lane & 31) * 4, gcol = tile * 128 + c4;
-  if (gcol < N) {
+  const int c4 = (lane & 31) * 4;
+  if (tile * 128 + (c4 & ~7) < N) {
+    const int gcol = quad_col(tile * 128, c4, N);
 #pragma unroll
     for (int i = 0; i < V / 2; ++i) {
       const int v = 2 * i + (lane >> 5);
       const floatx4 x = *reinterpret_cast<const floatx4 *>(&ctile[v][c4]);
-      __builtin_nontemporal_store(x, reinterpret_cast<floatx4 *>(crow + (int64_t)v * N + gcol));
+      __builtin_nontemporal_store(x, reinterpret_cast<floatx4_u *>(crow + (int64_t)v * N + gcol));
     }
   }
 }
@@ -322,8 +337,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
   const __amdgpu_buffer_rsrc_t srd_vals = make_srd(vals, (uint32_t)end * (V * 2u));
   const __amdgpu_buffer_rsrc_t srd_b = make_srd(bmat, b_bytes);
 
-  const int ncol = (int)tile * (16 * CPL) + m * CPL;
-  const bool col_ok = ncol < p.N;
+  const int col = (int)tile * (16 * CPL) + m * CPL;
+  const bool col_ok = col < p.N;
+  const int ncol = min(col, p.N - CPL);  // (unit_col for pieces of CPL columns)
   // Lanes whose columns lie beyond N aim every gather at the first byte past B.
   const uint32_t lane_n2 = col_ok ? (uint32_t)p.N * 2u : 0u;
   const uint32_t lane_col_off = col_ok ? (uint32_t)ncol * 2u : b_bytes;
@@ -498,8 +514,8 @@ __global__ __launch_bounds__(64 * kSplitWaves) void spmm_gather_split_kernel(con
       end = g_end[j];
     }
   const bool is_long = end - beg > 32 * kLongRowSteps;
-  const int ncol = (int)tile * 128 + m * 8;
-  const bool col_ok = ncol < p.N;
+  const int col = (int)tile * 128 + m * 8, ncol = unit_col(col, p.N);
+  const bool col_ok = col < p.N;
   OutT *cbase = reinterpret_cast<OutT *>(p.C) + (int64_t)batch * p.stride_C;
 
   floatx4 acc[8];
@@ -743,8 +759,8 @@ struct SlabStore<V, float, NQ> {
       const int tile = h == 0 ? (m >> 3) : 1 - (m >> 3);
 #pragma unroll
       for (int qp = 0; qp < NQ / 2; ++qp) {
-        const int col = n0 + 32 * qp + 16 * tile + 4 * g;
-        voff[h][qp] = col < N ? ((uint32_t)row * (uint32_t)N + (uint32_t)col) * 4u : kSlabDropStore;
+        const int c = 32 * qp + 16 * tile + 4 * g;
+        voff[h][qp] = n0 + (c & ~7) < N ? ((uint32_t)row * (uint32_t)N + (uint32_t)quad_col(n0, c, N)) * 4u : kSlabDropStore;
       }
     }
   }
@@ -777,7 +793,7 @@ struct SlabStore<V, _Float16, 4> {
       const int row = 8 * h + (m & 7);
       const int pair = h == 0 ? (m >> 3) : 1 - (m >> 3);
       const int col = n0 + 32 * pair + 16 * (g & 1) + 8 * (g >> 1);
-      voff[h] = col < N ? ((uint32_t)row * (uint32_t)N + (uint32_t)col) * 2u : kSlabDropStore;
+      voff[h] = col < N ? ((uint32_t)row * (uint32_t)N + (uint32_t)unit_col(col, N)) * 2u : kSlabDropStore;
     }
   }
   __device__ __forceinline__ void store(const floatx4 (&acc)[4], __amdgpu_buffer_rsrc_t srd, uint32_t crow) const {
@@ -837,7 +853,7 @@ struct SlabStore<V, _Float16, 2> {
   __device__ __forceinline__ void init(int lane, int n0, int N) {
     const int m = lane & 15, g = lane >> 4;
     const int col = n0 + 16 * (g & 1) + 8 * (g >> 1);
-    voff = (m < V && col < N) ? ((uint32_t)m * (uint32_t)N + (uint32_t)col) * 2u : kSlabDropStore;
+    voff = (m < V && col < N) ? ((uint32_t)m * (uint32_t)N + (uint32_t)unit_col(col, N)) * 2u : kSlabDropStore;
   }
   __device__ __forceinline__ void store(const floatx4 (&acc)[2], __amdgpu_buffer_rsrc_t srd, uint32_t crow) const {
     uint32_t pk[2][2];
@@ -992,7 +1008,7 @@ template <int NQ>
 __device__ __forceinline__ uint32_t slab_unit_src(const SpmmArgs &p, uint32_t u, uint32_t units, uint32_t n0, uint32_t b_bytes) {
   constexpr uint32_t kPerRow = 2u * NQ;  // 16-byte units per slab row
   const uint32_t col = n0 + (u % kPerRow) * 8u;
-  return (u < units && col < (uint32_t)p.N) ? __umul24(u / kPerRow, (uint32_t)p.N * 2u) + col * 2u : b_bytes;  // b_bytes: out of bounds, reads zeros
+  return (u < units && col < (uint32_t)p.N) ? __umul24(u / kPerRow, (uint32_t)p.N * 2u) + (uint32_t)unit_col((int)col, p.N) * 2u : b_bytes;  // b_bytes: out of bounds, reads zeros
 }
 // A 16-lane group of a slab read touches four rows at the same segment; rows 256 bytes apart share banks, so the
 // segment index is XORed with the row bits above that distance: c & 7 for 256-byte rows, (c >> 1) & 3 for 128-byte
@@ -1438,8 +1454,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(V == 8 ? 5 :
   const __amdgpu_buffer_rsrc_t srd_b = make_srd(p.B + (int64_t)batch * p.stride_B, b_bytes);
 
   // Lanes whose columns lie beyond N aim every gather at the first byte past B, where loads return zero.
-  const int ncol = (int)tile * 64 + 8 * x.pc;
-  const bool col_ok = ncol < p.N;
+  const int col = (int)tile * 64 + 8 * x.pc, ncol = unit_col(col, p.N);
+  const bool col_ok = col < p.N;
   const uint32_t lane_n2 = col_ok ? (uint32_t)p.N * 2u : 0u;
   const uint32_t lane_col_off = col_ok ? (uint32_t)ncol * 2u : b_bytes;
   floatx4 acc[4];
@@ -1557,8 +1573,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
       // a bundle of rows that stay whole: one stream of steps
       const int32_t *bp = s.bundles + (unit - (uint32_t)s.bundle_base);
       const int first = __builtin_amdgcn_readfirstlane(bp[0]), last = __builtin_amdgcn_readfirstlane(bp[1]);
-      const int ncol = (int)tile * 64 + 8 * x.pc;
-      const bool col_ok = ncol < p.N;
+      const int col = (int)tile * 64 + 8 * x.pc, ncol = unit_col(col, p.N);
+      const bool col_ok = col < p.N;
       SlabStore<V, OutT, 4> out;
       out.init(lane, (int)tile * 64, p.N);
       stage_stream<V, OutT>(x, p.col_idx, p.values + (int64_t)batch * p.stride_values,
@@ -1578,8 +1594,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     const __amdgpu_buffer_rsrc_t srd_vals = make_srd(p.values + (int64_t)batch * p.stride_values, (uint32_t)kend * (V * 2u));
     const __amdgpu_buffer_rsrc_t srd_b = make_srd(p.B + (int64_t)batch * p.stride_B, b_bytes);
     // Lanes whose columns lie beyond N aim every gather at the first byte past B, where loads return zero.
-    const int ncol = (int)tile * 64 + 8 * x.pc;
-    const bool col_ok = ncol < p.N;
+    const int col = (int)tile * 64 + 8 * x.pc, ncol = unit_col(col, p.N);
+    const bool col_ok = col < p.N;
     const uint32_t lane_n2 = col_ok ? (uint32_t)p.N * 2u : 0u;
     const uint32_t lane_col_off = col_ok ? (uint32_t)ncol * 2u : b_bytes;
     floatx4 acc[4];
@@ -1621,7 +1637,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
   }
 }
 
-// Shape-agnostic kernel: any N, any alignment.  One thread per output column, scalar gathers,
+// Shape-agnostic kernel: any N (fewer than eight columns among them), any alignment.  One thread per output column, scalar gathers,
 // accumulation in ascending vector order (the order of the reference's host check loop,
 // reference SSpMM/sspmm_test.cpp:82-94).
 template <int V, typename OutT>
@@ -1640,10 +1656,24 @@ __global__ __launch_bounds__(64) void spmm_generic_kernel(const SpmmArgs p) {
 #pragma unroll
   for (int v = 0; v < V; ++v) acc[v] = 0.f;
   const int beg = p.row_offsets[row], end = p.row_offsets[row + 1];
-  for (int j = beg; j < end; ++j) {
-    const float b = (float)bmat[(int64_t)p.col_idx[j] * p.N + n];
+  // (the eight gathers of a trip are in flight together; the additions keep their order)
+  for (int j = beg; j < end; j += 8) {
+    _Float16 b[8];
 #pragma unroll
-    for (int v = 0; v < V; ++v) acc[v] += (float)vals[(int64_t)j * V + v] * b;
+    for (int u = 0; u < 8; ++u) b[u] = bmat[(int64_t)p.col_idx[min(j + u, end - 1)] * p.N + n];
+    if (j + 8 <= end) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[v] += (float)vals[(int64_t)(j + u) * V + v] * (float)b[u];
+    } else {
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (j + u < end) {
+#pragma unroll
+          for (int v = 0; v < V; ++v) acc[v] += (float)vals[(int64_t)(j + u) * V + v] * (float)b[u];
+        }
+    }
   }
   if (has_epilogue(p)) {
 #pragma unroll
@@ -1808,20 +1838,36 @@ static hipError_t launch_v(const SpmmArgs &a, int which, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// The MFMA kernels need 16-byte row segments of B and C: N % 8 == 0 and aligned bases/strides;
-// 24-bit multiplies bound K and 2N; one buffer descriptor must span B.
+// Rows of B and C that are whole 16-byte pieces: N % 8 == 0 and aligned bases/strides.
+static bool whole_pieces(const SpmmArgs &a, bool out_f16) {
+  return (a.N % 8 == 0) && (reinterpret_cast<uintptr_t>(a.B) % 16 == 0) && (reinterpret_cast<uintptr_t>(a.C) % 16 == 0) &&
+         (a.stride_B % 8 == 0) && ((a.stride_C * (out_f16 ? 2 : 4)) % 16 == 0);
+}
+// The MFMA kernels take any width from one piece (eight columns) on (see unit_col).  Against the scalar kernel, which
+// served widths that are no multiple of eight before: 1024 x 1152 at 90 %, V = 8, N = 1225, fp32: 25.6 us for the scalar
+// kernel alone, now below the 11 us of the call; 128 x 2659 at 80 %, N = 30: 86 -> 11 us a call; 512-wide encoder layer on
+// 7 x 101 tokens 238 -> 154 us.  The error against float64 is a quarter to all of the scalar kernel's on fourteen such products
+// (7e-8 to 1.7e-7 where it has 1.8e-7 to 6e-7).
+// the value vectors are fetched
+// with 8-byte (V = 8) or 16-byte (V = 16) loads per lane from aligned memory; 24-bit multiplies bound K and 2N; one
+// buffer descriptor must span B.
 static bool mfma_kernels_apply(const SpmmArgs &a, bool out_f16) {
   const uint64_t b_bytes = (uint64_t)a.K * (uint64_t)a.N * 2u;
-  const int out_size = out_f16 ? 2 : 4;
-  // The value vectors are fetched with 8-byte (V = 8) or 16-byte (V = 16) loads per lane.
-  return (a.N % 8 == 0) && (reinterpret_cast<uintptr_t>(a.B) % 16 == 0) &&
-         (reinterpret_cast<uintptr_t>(a.C) % 16 == 0) && (a.stride_B % 8 == 0) &&
+  return (a.N >= 8) && (reinterpret_cast<uintptr_t>(a.B) % 2 == 0) &&
+         (reinterpret_cast<uintptr_t>(a.C) % (out_f16 ? 2 : 4) == 0) &&
          (reinterpret_cast<uintptr_t>(a.values) % 16 == 0) && (a.stride_values % 8 == 0) &&
-         ((a.stride_C * out_size) % 16 == 0) && (a.K < (1 << 24)) && (a.N < (1 << 23)) &&
-         (b_bytes + 16 <= 0xffffffffull);
+         (a.K < (1 << 24)) && (a.N < (1 << 23)) && (b_bytes + 16 <= 0xffffffffull);
+}
+// Ragged widths of a few short vector-rows stay with the scalar kernel, whose fp32 sums are the host loop's bit for
+// bit: such a launch is at most one wave on every fourth CU, at most sixteen trips of eight gathers long, and its
+// time is the call itself.
+static bool few_short_rows(const SpmmArgs &a, bool out_f16) {
+  return !whole_pieces(a, out_f16) && a.K <= 128 && (uint64_t)a.m_vec * (uint64_t)((a.N + 63) / 64) * (uint64_t)a.batch <= 64u;
 }
 
 static uint32_t padded_tiles(uint32_t t) { return t <= 1u ? 1u : t <= 2u ? 2u : t <= 4u ? 4u : (t + 7u) & ~7u; }
+
+bool rows_are_whole_pieces(const SpmmArgs &a, bool out_f16) { return whole_pieces(a, out_f16); }
 
 bool balanced_kernel_applies(const SpmmArgs &a, int V, bool out_f16) {
   // (one batch element's C is addressed through a 32-bit buffer descriptor, and lanes that must not store carry an
@@ -1865,7 +1911,7 @@ hipError_t launch_spmm_balanced(const SpmmArgs &a, int V, bool out_f16, const Sc
 
 hipError_t launch_spmm(const SpmmArgs &a, int V, bool out_f16, hipStream_t stream) {
   const int out_size = out_f16 ? 2 : 4;
-  const bool fast = mfma_kernels_apply(a, out_f16);
+  const bool fast = mfma_kernels_apply(a, out_f16) && !few_short_rows(a, out_f16);
   int which = 1;
   if (fast) {
     // The slab kernel pays off when enough vector-rows share a slab and there are enough

@@ -551,3 +551,54 @@ def test_wide_slab_is_the_choice_for_fp16_outputs_of_large_batches(oracle, built
         want = oracle.spmm(vs.m_vec, V, N, K, vs.row_offsets, vs.col_idx, vals[b].cpu().numpy(), B[b].cpu().numpy(), threads=8)
         assert max_rel_err(out16[b].cpu().numpy(), want) <= TIGHT_F16
         assert max_rel_err(out32[b].cpu().numpy(), want) <= TIGHT_F32
+
+
+@pytest.mark.parametrize("V", [8, 16])
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("force,K,m_vec,N", [(0, 900, 37, 8), (0, 900, 37, 9), (0, 900, 37, 63), (0, 900, 37, 65), (0, 300, 90, 1225),
+                                             (0, 6000, 19, 135), (2, 900, 37, 135), (2, 900, 37, 257), (3, 500, 70, 9),
+                                             (3, 500, 70, 191), (3, 900, 70, 193), (3, 1500, 70, 71), (6, 900, 37, 130),
+                                             (9, 500, 150, 321), (7, 5000, 40, 129)])
+def test_ragged_widths_on_the_matrix_kernels(oracle, built_library, V, out_dtype, force, K, m_vec, N):
+    """Widths that are no multiple of eight: the last piece of every row slides back over the one before it.  Every
+    kernel, a batch whose elements begin at odd offsets, C between guards with a gap behind each element."""
+    from sspmm_amd import _lib
+    L = _lib.lib()
+    rng = np.random.default_rng(K + N)
+    lens = rng.integers(0, min(K, 90), m_vec)
+    lens[[0, 9, m_vec - 1]] = [0, min(K, 700), 33]
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    cols = np.concatenate([rng.permutation(K)[:n] for n in lens]).astype(np.int32)
+    batch, M, guard = 3, m_vec * V, 1023
+    vals = (rng.standard_normal((batch, cols.size * V)) * 0.1).astype(np.float16)
+    B = rng.standard_normal((batch, K, N)).astype(np.float16)
+    stride_c = M * N + 5
+    buf = torch.full((guard + batch * stride_c + guard,), 12345.0, dtype=out_dtype, device="cuda")
+    ro, ci, dv, dB = dev(off), dev(cols), dev(vals), dev(B)
+    plan = sspmm_amd.Plan(ro, V, K, max_N=N, max_batch=batch, panel_steps=2) if force == 7 else None
+    print("ragged V=%d force=%d K=%d m_vec=%d N=%d %s" % (V, force, K, m_vec, N, out_dtype), flush=True)
+    L.sspmm_select_kernel(force)
+    try:
+        tail = (ro.data_ptr(), ci.data_ptr(), dv.data_ptr(), cols.size * V, dB.data_ptr(), K * N,
+                buf.data_ptr() + guard * buf.element_size(), stride_c, torch.cuda.current_stream().cuda_stream)
+        if plan is not None:
+            fn = L.sspmm_plan_batched_f16_f32 if out_dtype == torch.float32 else L.sspmm_plan_batched_f16_f16
+            rc = fn(plan.handle, batch, N, *tail)
+        else:
+            fn = L.sspmm_batched_f16_f32 if out_dtype == torch.float32 else L.sspmm_batched_f16_f16
+            rc = fn(batch, m_vec, V, N, K, None, *tail)
+        torch.cuda.synchronize()
+        ran = L.sspmm_last_kernel()
+    finally:
+        L.sspmm_select_kernel(0)
+    assert rc == 0 and ran != 1
+    if force:
+        assert ran == (5 if (force, K) == (3, 1500) else force)
+    got = buf.cpu().numpy()
+    assert np.all(got[:guard] == 12345.0) and np.all(got[guard + batch * stride_c:] == 12345.0)
+    tol = TIGHT_F32 if out_dtype == torch.float32 else TIGHT_F16
+    for b in range(batch):
+        lo = guard + b * stride_c
+        assert np.all(got[lo + M * N:lo + stride_c] == 12345.0), b
+        want = oracle.spmm(m_vec, V, N, K, off, cols, vals[b], B[b], threads=8)
+        assert max_rel_err(got[lo:lo + M * N].reshape(M, N), want) <= tol, b
