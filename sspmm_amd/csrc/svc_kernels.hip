@@ -172,6 +172,24 @@ __device__ __forceinline__ uint32_t resized_slots(uint32_t fill) {
   return s;
 }
 
+// Slots of the table that CPython keeps n keys in once a construction has inserted them all.
+__device__ __forceinline__ uint32_t final_slots(int n) {
+  uint32_t slots = 8;
+  for (;;) {
+    const uint32_t thr = resize_threshold(slots);
+    if (n < (int)thr) return slots;
+    slots = resized_slots(thr);
+  }
+}
+// A group whose columns are all below final_slots(number of columns) needs no replay: in the table of its last
+// construction every key sits in the slot of its own number, whatever went before, so the order is the ascending
+// one.  Dense groups of moderately wide matrices are like this, and most groups of a pruned-weight dataset: twenty matrices
+// of 512 and 2048 columns at 50 to 98 % sparsity spend 55 + 108 us in the two merge launches where the replay of every
+// group spent 464 + 163; what is left of the 108 is the replay of the 98 % matrices.  svc_count marks such groups with this bit, on the group's count until the prefix sum and in its class list
+// from then on.
+static constexpr int kAscending = (int)0x80000000u;
+static constexpr int kGroupBits = 0x7fffffff;
+
 // Writes the keys of table[0..slots) to list[0..) in slot order; when `final` also replaces each
 // entry's insertion index by its position in that order.
 template <int THREADS>
@@ -271,14 +289,24 @@ __global__ __launch_bounds__(THREADS) void svc_count_distinct_kernel(const SvcAr
   for (int w = threadIdx.x; w < words; w += THREADS) bits[w] = 0;
   __syncthreads();
   // a thread counts the bits it is the first to set: no second pass over the bitmap
-  int mine = 0;
+  int mine = 0, last = -1;
   for (int idx = e0 + (int)threadIdx.x; idx < e1; idx += THREADS) {
     const uint32_t c = (uint32_t)a.col_ind[idx], bit = 1u << (c & 31u);
-    if (c < (uint32_t)a.K) mine += (atomicOr(&bits[c >> 5], bit) & bit) ? 0 : 1;  // (a column outside [0, K) is ignored)
+    if (c < (uint32_t)a.K) {  // (a column outside [0, K) is ignored)
+      mine += (atomicOr(&bits[c >> 5], bit) & bit) ? 0 : 1;
+      last = max(last, (int)c);
+    }
   }
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) last = max(last, __shfl_xor(last, d, 64));
+  if ((threadIdx.x & 63) == 0) scratch[16 + (threadIdx.x >> 6)] = last;
   int total;
-  block_exclusive_scan<THREADS>(mine, &total, scratch);
-  if (threadIdx.x == 0) a.vec_row_ptr[grp + 1] = total;
+  block_exclusive_scan<THREADS>(mine, &total, scratch);  // (THREADS / 64 words of scratch; its barriers cover the maxima)
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int w = 0; w < THREADS / 64; ++w) last = max(last, scratch[16 + w]);
+    a.vec_row_ptr[grp + 1] = total | (total > 0 && (uint32_t)last < final_slots(total) ? kAscending : 0);
+  }
 }
 
 // The first entries of a group's member rows, fetched once: lane j of every wave holds the start of member row j
@@ -341,6 +369,95 @@ __device__ __forceinline__ void write_group_output(const SvcArgs &a, int grp, co
   }
 }
 
+// Direct mode: a group marked kAscending.  Its columns come out of a bitmap of final_slots(n) bits with a running
+// count per word; every entry of the group is read once (groups of up to 8 x THREADS entries keep theirs in
+// registers between the two passes) and the value vectors are put together in LDS where they fit and leave in whole
+// 16-byte pieces.  `lds` is the class's LDS for tables and lists, at least final_slots(n) / 4 bytes of it.
+template <int THREADS>
+__device__ __forceinline__ void write_ascending_group(const SvcArgs &a, int grp, const RowBounds &rows, int n, unsigned char *lds,
+                                                      uint32_t lds_bytes, int *scratch) {
+  const int tid = threadIdx.x;
+  const uint32_t slots = final_slots(n), words = (slots + 31u) / 32u;
+  uint32_t *bits = reinterpret_cast<uint32_t *>(lds);
+  int *prefix = reinterpret_cast<int *>(lds) + words;
+  const uint32_t tile_off = (words * 8u + 15u) & ~15u;
+  uint16_t *tile = reinterpret_cast<uint16_t *>(lds + tile_off);
+  const int v0 = a.scanned[grp];
+  const int64_t halfs = (int64_t)n * a.V;
+  const bool in_tile = (a.V & 7) == 0 && (reinterpret_cast<uintptr_t>(a.vec_val) & 15) == 0 &&
+                       (int64_t)tile_off + halfs * 2 <= (int64_t)lds_bytes;
+  const bool aligned4 = (a.V & 1) == 0 && (reinterpret_cast<uintptr_t>(a.vec_val) & 3) == 0;
+  uint16_t *out = a.vec_val ? a.vec_val + (int64_t)v0 * a.V : nullptr;
+  constexpr int kHeld = 8;
+  const int e0 = rows.start(0), e1 = rows.start(rows.count);
+  const bool held = e1 - e0 <= kHeld * THREADS;
+  uint32_t col[kHeld];
+  uint16_t val[kHeld];
+#pragma unroll
+  for (int u = 0; u < kHeld; ++u) {
+    const int idx = e0 + u * THREADS + tid;
+    col[u] = held && idx < e1 ? (uint32_t)a.col_ind[idx] : 0xffffffffu;
+    val[u] = held && idx < e1 && out ? a.csr_val[idx] : 0;
+  }
+  for (uint32_t w = tid; w < words; w += THREADS) bits[w] = 0;
+  if (out) {
+    if (in_tile) {
+      for (int64_t t = tid; t < halfs / 8; t += THREADS) reinterpret_cast<uint4 *>(tile)[t] = uint4{0u, 0u, 0u, 0u};
+    } else if (aligned4) {
+      for (int64_t t = tid; t < halfs / 2; t += THREADS) reinterpret_cast<uint32_t *>(out)[t] = 0u;
+    } else {
+      for (int64_t t = tid; t < halfs; t += THREADS) out[t] = 0;
+    }
+  }
+  __syncthreads();
+  if (held) {
+#pragma unroll
+    for (int u = 0; u < kHeld; ++u)
+      if (col[u] < slots && col[u] < (uint32_t)a.K) atomicOr(&bits[col[u] >> 5], 1u << (col[u] & 31u));
+  } else {
+    for (int idx = e0 + tid; idx < e1; idx += THREADS) {
+      const uint32_t c = (uint32_t)a.col_ind[idx];
+      if (c < slots && c < (uint32_t)a.K) atomicOr(&bits[c >> 5], 1u << (c & 31u));
+    }
+  }
+  __syncthreads();
+  const uint32_t per = (words + THREADS - 1) / THREADS;
+  const uint32_t lo = min(words, (uint32_t)tid * per), hi = min(words, lo + per);
+  int mine = 0;
+  for (uint32_t w = lo; w < hi; ++w) mine += __popc(bits[w]);
+  int total;
+  int at = block_exclusive_scan<THREADS>(mine, &total, scratch);
+  for (uint32_t w = lo; w < hi; ++w) {
+    prefix[w] = at;
+    at += __popc(bits[w]);
+  }
+  __syncthreads();
+  if (a.vec_col)
+    for (uint32_t s = tid; s < slots; s += THREADS) {
+      const uint32_t x = bits[s >> 5], bit = 1u << (s & 31u);
+      if (x & bit) a.vec_col[v0 + prefix[s >> 5] + __popc(x & (bit - 1u))] = (int)s;
+    }
+  if (!out) return;
+  uint16_t *dst = in_tile ? tile : out;
+  const auto put = [&](int idx, uint32_t c, uint16_t value) {
+    if (c >= slots || c >= (uint32_t)a.K) return;
+    const int p = prefix[c >> 5] + __popc(bits[c >> 5] & ((1u << (c & 31u)) - 1u));
+    dst[(int64_t)p * a.V + rows.row_of(idx)] = value;
+  };
+  if (held) {
+#pragma unroll
+    for (int u = 0; u < kHeld; ++u) {
+      if (e0 + u * THREADS >= e1) break;  // (uniform)
+      put(min(e0 + u * THREADS + tid, e1 - 1), col[u], val[u]);
+    }
+  } else {
+    for (int idx = e0 + tid; idx < e1; idx += THREADS) put(idx, (uint32_t)a.col_ind[idx], a.csr_val[idx]);
+  }
+  if (!in_tile) return;
+  __syncthreads();
+  for (int64_t t = tid; t < halfs / 8; t += THREADS) reinterpret_cast<uint4 *>(out)[t] = reinterpret_cast<const uint4 *>(tile)[t];
+}
+
 template <int THREADS, bool IN_LDS>
 __global__ __launch_bounds__(THREADS) void svc_merge_cpython_kernel(const SvcArgs a, int class_lo, int class_hi,
                                                                     int list_cap) {
@@ -350,7 +467,7 @@ __global__ __launch_bounds__(THREADS) void svc_merge_cpython_kernel(const SvcArg
   const bool listed = a.scanned != nullptr;
   const int n_groups = listed ? a.class_counts[kClassBeyond] : (a.group_rows ? a.groups : (a.M + a.V - 1) / a.V);
   for (int li = blockIdx.x; li < n_groups; li += gridDim.x) {
-  const int grp = listed ? a.class_lists[(int64_t)kClassBeyond * a.list_stride + li] : li;
+  const int grp = listed ? a.class_lists[(int64_t)kClassBeyond * a.list_stride + li] & kGroupBits : li;
   const int r0 = group_first_row(a, grp), r1 = group_first_row(a, grp + 1);
   const int e0 = a.row_ptr[r0], e1 = a.row_ptr[r1];
   const int bound = listed ? a.scanned[grp + 1] - a.scanned[grp] : min(e1 - e0, a.K);
@@ -798,7 +915,7 @@ __global__ __launch_bounds__(THREADS) void svc_merge_fast_kernel(const SvcArgs a
   for (int li = blockIdx.x; li < n_groups; li += gridDim.x) {
   int c = cls, at = li;
   while (at >= a.class_counts[c]) at -= a.class_counts[c--];
-  const int grp = a.class_lists[(int64_t)c * a.list_stride + at];
+  const int filed = a.class_lists[(int64_t)c * a.list_stride + at], grp = filed & kGroupBits;
   const int r0 = group_first_row(a, grp), r1 = group_first_row(a, grp + 1);
   const int count = a.scanned[grp + 1] - a.scanned[grp];
   const int e0 = a.row_ptr[r0];
@@ -820,6 +937,12 @@ __global__ __launch_bounds__(THREADS) void svc_merge_fast_kernel(const SvcArgs a
   int n = 0;
   uint32_t slots = 0;
   const RowBounds rows(a, r0, r1);
+  if (filed & kAscending) {
+    write_ascending_group<THREADS>(a, grp, rows, count, smem + 128,
+                                   (max_slots + small_slots) * 4u + (LIST_IN_LDS ? (uint32_t)list_cap * 8u : 0u), scratch);
+    __syncthreads();  // the next group reuses the LDS
+    continue;
+  }
   // CPython rebuilds the set for every member row, also for one that brings nothing new (an empty row, a row of
   // known columns); the order may still change then, because the keys go in in the previous table's slot order.
   // Two cases need no construction.  period == 1: the latest construction returned its keys in the order it got
@@ -953,7 +1076,7 @@ __global__ __launch_bounds__(1024) void svc_scan_classify_kernel(int m_vec, int3
   const int lane = threadIdx.x & 63;
   for (int base = 0; base < m_vec; base += 1024) {
     const int i = base + (int)threadIdx.x;
-    const int x = i < m_vec ? vec_row_ptr[i + 1] : 0;
+    const int counted = i < m_vec ? vec_row_ptr[i + 1] : 0, x = counted & kGroupBits;
     int total;
     const int ex = block_exclusive_scan<1024>(x, &total, scratch);  // (its barriers also cover filed[]'s set-up)
     if (i < m_vec) vec_row_ptr[i + 1] = carry + ex + x;
@@ -966,7 +1089,7 @@ __global__ __launch_bounds__(1024) void svc_scan_classify_kernel(int m_vec, int3
       int at = 0;
       if (lane == 0) at = atomicAdd(&filed[c], __popcll(members));
       at = __builtin_amdgcn_readfirstlane(at);
-      if (cls == c) class_lists[(int64_t)c * list_stride + at + __popcll(members & ((1ull << lane) - 1ull))] = i;
+      if (cls == c) class_lists[(int64_t)c * list_stride + at + __popcll(members & ((1ull << lane) - 1ull))] = i | (counted & kAscending);
     }
   }
   __syncthreads();

@@ -367,3 +367,30 @@ def test_wide_matrices_and_giant_groups_take_the_64_bit_tables(oracle, built_lib
     K2 = 100000
     cols2 = np.concatenate([np.sort(rng.choice(K2, n, replace=False)) for n in lens]).astype(np.int32)
     _compare_with_oracle(oracle, synth.Csr(24, K2, ptr, cols2, csr.values), 8)
+
+
+@pytest.mark.parametrize("V", [1, 3, 8, 16, 64])
+@pytest.mark.parametrize("slots,counts", [(8, (1, 4)), (32, (5, 19)), (128, (20, 76)), (512, (77, 306)), (2048, (308, 1228)),
+                                          (8192, (1229, 4914)), (32768, (4915, 9000))])
+def test_groups_whose_columns_all_fit_their_last_table(oracle, built_library, V, slots, counts):
+    """Groups whose columns are below the size of the table that holds them come out ascending without a replay: at
+    the ends of every table size's range of columns, with the largest column the table's last slot (ascending) and the
+    one behind it (replayed), next to each other; shuffled rows, empty rows, columns shared between the rows."""
+    rng = np.random.default_rng(slots + V)
+    K = slots + 8
+    rows = []
+    for n in counts + (counts[0],):
+        for top in (slots - 1, slots, K - 1):
+            cols = np.append(rng.permutation(min(top, slots))[:n - 1], top)
+            owner = rng.integers(0, V, n)
+            extra = rng.integers(0, V, n)
+            for r in range(V):
+                rows.append(rng.permutation(cols[(owner == r) | ((extra == r) & (r % 3 == 1))]))
+    lens = np.array([len(r) for r in rows])
+    csr = synth.Csr(len(rows), K, np.concatenate([[0], np.cumsum(lens)]).astype(np.int32),
+                    np.concatenate(rows).astype(np.int32), rng.standard_normal(int(lens.sum())).astype(np.float16))
+    vrp, vcol, _ = _compare_with_oracle(oracle, csr, V)
+    first = vcol[vrp[0]:vrp[1]]
+    assert np.array_equal(first, np.sort(first))
+    r = sspmm_amd.svc(dev(csr.row_ptr), dev(csr.col_ind), None, csr.M, csr.K, V)
+    assert np.array_equal(r.vec_col.cpu().numpy(), vcol)
