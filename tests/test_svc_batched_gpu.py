@@ -122,3 +122,26 @@ def test_converter_takes_the_files_through_one_stack(built_library, tmp_path):
     assert len(stats) == len(names)
     for n in names:
         assert (tmp_path / n).read_bytes() == open(os.path.join(GOLDEN, n.replace(".smtx", ".v8.smtx")), "rb").read()
+
+
+def test_extents_follow_the_row_pointer():
+    """The extents that matrix() hands out are those of the row pointer as it is now (host tensors: no launches)."""
+    from sspmm_amd.svc import SvcBatch
+    ptr = torch.tensor([0, 2, 5, 5, 9], dtype=torch.int32)
+    groups = np.array([0, 2, 2, 4])
+    b = SvcBatch(8, np.array([16, 0, 16]), None, groups, ptr, torch.arange(9, dtype=torch.int32), None,
+                 torch.from_numpy(groups.astype(np.int32)))
+    sizes = lambda: [b.matrix(i).num_vec for i in range(3)]  # noqa: E731
+    assert sizes() == [5, 0, 4] and b.matrix(2).vec_row_ptr.tolist() == [0, 0, 4]
+    ptr[2:4] = 3
+    assert sizes() == [3, 0, 6]
+    b.vec_row_ptr = torch.tensor([0, 1, 1, 1, 8], dtype=torch.int32)
+    assert sizes() == [1, 0, 7] and b.matrix(2).vec_col.tolist() == list(range(1, 8))
+    with torch.inference_mode():
+        b.vec_row_ptr = torch.tensor([0, 1, 1, 1, 2], dtype=torch.int32)
+        assert sizes() == [1, 0, 1]
+        b.vec_row_ptr[4] = 6
+        assert sizes() == [1, 0, 5]
+    for i in (3, -1):
+        with pytest.raises(IndexError):
+            b.matrix(i)
