@@ -3,6 +3,8 @@ import ctypes
 import os
 import subprocess
 
+import torch
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB_PATH = os.path.join(_HERE, "libsspmm_amd.so")
 _lib = None
@@ -84,6 +86,21 @@ def lib():
             fn.argtypes = args
         _lib = L
     return _lib
+
+
+_current_device = torch._C._cuda_getDevice if hasattr(torch._C, "_cuda_getDevice") else None
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def call(fn, device, *args):
+    """fn(*args, stream) with `device` current and its current stream: what every launching entry point ends with.
+    The handle is asked for directly and the device is only switched when it is another one: torch's Stream object and
+    device guard are 4 us of Python per call (an 11 us call of a 3 us kernel)."""
+    i = device.index
+    if _raw_stream is not None and i is not None and i == _current_device():
+        return fn(*args, _raw_stream(i))
+    with torch.cuda.device(device):
+        return fn(*args, torch.cuda.current_stream().cuda_stream)
 
 
 def check(code, what):

@@ -8,7 +8,7 @@ softmax_kernel.cu:208-216 and 256-266), and the block that chains them
 import torch
 
 from . import _lib
-from .spmm import _check_inputs, _ptr, _stream, bspmm
+from .spmm import _check_inputs, _ptr, bspmm
 
 
 def _check_pattern(row_indices, row_offsets, column_indices, vec_length):
@@ -41,10 +41,9 @@ def bsddmm(row_indices, row_offsets, column_indices, lhs_matrix, rhs_matrix, vec
         raise ValueError("lhs_matrix must have m_vec * vec_length = %d rows, got %d" % (m_vec * vec_length, m))
     nvec = column_indices.numel()
     out = torch.empty((batch, nvec * vec_length), dtype=torch.float16, device=lhs_matrix.device)
-    with torch.cuda.device(lhs_matrix.device):
-        rc = _lib.lib().sspmm_sddmm_batched_f16(batch, m_vec, vec_length, k, n, _ptr(row_indices), _ptr(row_offsets),
-                                                _ptr(column_indices), _ptr(lhs_matrix), m * k, _ptr(rhs_matrix), n * k,
-                                                _ptr(out), nvec * vec_length, _stream())
+    rc = _lib.call(_lib.lib().sspmm_sddmm_batched_f16, lhs_matrix.device, batch, m_vec, vec_length, k, n, _ptr(row_indices),
+                   row_offsets.data_ptr(), column_indices.data_ptr(), lhs_matrix.data_ptr(), m * k, rhs_matrix.data_ptr(), n * k,
+                   out.data_ptr(), nvec * vec_length)
     _lib.check(rc, "sspmm_sddmm")
     return out
 
@@ -64,9 +63,8 @@ def bcsr_softmax(row_indices, row_offsets, values, scaler, vec_length, batch_siz
     m_vec = row_offsets.numel() - 1
     stride = values.numel() // batch_size if batch_size > 0 else 0
     out = torch.empty_like(values)
-    with torch.cuda.device(values.device):
-        rc = _lib.lib().sspmm_softmax_batched_f16(batch_size, m_vec, vec_length, _ptr(row_indices), _ptr(row_offsets),
-                                                  _ptr(values), float(scaler), _ptr(out), stride, _stream())
+    rc = _lib.call(_lib.lib().sspmm_softmax_batched_f16, values.device, batch_size, m_vec, vec_length, _ptr(row_indices),
+                   row_offsets.data_ptr(), values.data_ptr(), float(scaler), out.data_ptr(), stride)
     _lib.check(rc, "sspmm_softmax")
     return out
 
@@ -99,10 +97,9 @@ def fused_sparse_attention(row_indices, row_offsets, column_indices, q, k, v, sc
     if k.numel() != batch * n * d or v.numel() != batch * n * d:
         raise ValueError("q, k and v must have the same batch size")
     out = torch.empty(q.shape, dtype=torch.float16, device=q.device)
-    with torch.cuda.device(q.device):
-        rc = _lib.lib().sspmm_sparse_attention_f16(batch, m_vec, vec_length, d, n, _ptr(row_indices), _ptr(row_offsets),
-                                                   _ptr(column_indices), _ptr(q), m * d, _ptr(k), n * d, _ptr(v), n * d,
-                                                   float(scaling), _ptr(out), m * d, _stream())
+    rc = _lib.call(_lib.lib().sspmm_sparse_attention_f16, q.device, batch, m_vec, vec_length, d, n, _ptr(row_indices),
+                   row_offsets.data_ptr(), column_indices.data_ptr(), q.data_ptr(), m * d, k.data_ptr(), n * d, v.data_ptr(), n * d,
+                   float(scaling), out.data_ptr(), m * d)
     _lib.check(rc, "sspmm_sparse_attention")
     return out
 
@@ -130,11 +127,10 @@ def sparse_attention_packed(row_indices, row_offsets, column_indices, qkv, num_h
         raise ValueError("qkv must have m_vec * vec_length = %d rows, got %d" % (m_vec * vec_length, seq))
     out = torch.empty((seq, bsz, e), dtype=torch.float16, device=qkv.device)
     base, ld = qkv.data_ptr(), bsz * three_e
-    with torch.cuda.device(qkv.device):
-        rc = _lib.lib().sspmm_sparse_attention_heads_f16(
-            bsz, num_heads, m_vec, vec_length, d, seq, _ptr(row_indices), _ptr(row_offsets), _ptr(column_indices),
-            base, three_e, d, ld, base + 2 * e, three_e, d, ld, base + 4 * e, three_e, d, ld, float(scaling),
-            _ptr(out), e, d, bsz * e, _stream())
+    rc = _lib.call(_lib.lib().sspmm_sparse_attention_heads_f16, qkv.device, bsz, num_heads, m_vec, vec_length, d, seq,
+                   _ptr(row_indices), row_offsets.data_ptr(), column_indices.data_ptr(),
+                   base, three_e, d, ld, base + 2 * e, three_e, d, ld, base + 4 * e, three_e, d, ld, float(scaling),
+                   out.data_ptr(), e, d, bsz * e)
     _lib.check(rc, "sspmm_sparse_attention_heads")
     return out
 

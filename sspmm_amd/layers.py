@@ -153,10 +153,8 @@ def add_layernorm(x, a, ln):
         s = x if a is None else x + a
         return ln(s.t()).t().contiguous()
     out = torch.empty_like(x)
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().sspmm_add_layernorm_f16(H, T, x.data_ptr(), 0 if a is None else a.data_ptr(), ln.weight.data_ptr(),
-                                                0 if ln.bias is None else ln.bias.data_ptr(), float(ln.eps), out.data_ptr(),
-                                                torch.cuda.current_stream().cuda_stream)
+    rc = _lib.call(_lib.lib().sspmm_add_layernorm_f16, x.device, H, T, x.data_ptr(), 0 if a is None else a.data_ptr(),
+                   ln.weight.data_ptr(), 0 if ln.bias is None else ln.bias.data_ptr(), float(ln.eps), out.data_ptr())
     _lib.check(rc, "sspmm_add_layernorm_f16")
     return out
 
@@ -174,13 +172,27 @@ def attention_fm(qkv, hidden, heads, batch, seq, scale=None):
         return None
     out = torch.empty(hidden, T, dtype=torch.float16, device=qkv.device)
     esz = qkv.element_size()
-    with torch.cuda.device(qkv.device):
-        rc = _lib.lib().sspmm_attention_fm_f16(batch, heads, seq, d, qkv.data_ptr(), qkv.data_ptr() + hidden * T * esz,
-                                               qkv.data_ptr() + 2 * hidden * T * esz, T, out.data_ptr(), T,
-                                               float(1.0 / math.sqrt(d) if scale is None else scale),
-                                               torch.cuda.current_stream().cuda_stream)
+    rc = _lib.call(_lib.lib().sspmm_attention_fm_f16, qkv.device, batch, heads, seq, d, qkv.data_ptr(),
+                   qkv.data_ptr() + hidden * T * esz, qkv.data_ptr() + 2 * hidden * T * esz, T, out.data_ptr(), T,
+                   float(1.0 / math.sqrt(d) if scale is None else scale))
     _lib.check(rc, "sspmm_attention_fm_f16")
     return out
+
+
+class _WithGelu:
+    """A SparseLinear called with the GELU behind it."""
+
+    def __init__(self, layer):
+        self.layer = layer
+
+    in_features = property(lambda self: self.layer.in_features)
+    out_features = property(lambda self: self.layer.out_features)
+
+    def dense_weight(self):
+        return self.layer.dense_weight()
+
+    def __call__(self, x):
+        return self.layer(x, activation="gelu")
 
 
 class SparseEncoderLayer(torch.nn.Module):
@@ -208,16 +220,7 @@ class SparseEncoderLayer(torch.nn.Module):
     def ffn1_gelu(self):
         """The first feed-forward product with its GELU in the product's epilogue: ffn1 itself, called with the
         activation (no second module, no second copy of the arrays)."""
-        ffn1 = self.ffn1
-
-        class _WithGelu:
-            in_features, out_features = ffn1.in_features, ffn1.out_features
-            dense_weight = staticmethod(ffn1.dense_weight)
-
-            def __call__(self, x):
-                return ffn1(x, activation="gelu")
-
-        return _WithGelu()
+        return _WithGelu(self.ffn1)
 
     def _attention(self, qkv, batch, seq):
         """qkv: [3 * hidden, batch*seq] feature-major; returns the context [hidden, batch*seq].  One HIP kernel that

@@ -16,6 +16,14 @@ def _ptr(t):
 def _check_inputs(row_indices, row_offsets, column_indices, values, rhs_matrix, vec_length):
     if vec_length not in (8, 16):
         raise ValueError("vec_length must be 8 or 16, got %r" % (vec_length,))
+    i32, f16 = torch.int32, torch.float16
+    if (row_offsets.dtype is i32 and column_indices.dtype is i32 and values.dtype is f16 and rhs_matrix.dtype is f16 and
+            row_offsets.is_cuda and column_indices.is_cuda and values.is_cuda and rhs_matrix.is_cuda and
+            row_offsets.is_contiguous() and column_indices.is_contiguous() and values.is_contiguous() and
+            rhs_matrix.is_contiguous() and
+            (row_indices is None or (row_indices.dtype is i32 and row_indices.is_cuda and row_indices.is_contiguous()))):
+        return
+    # (something is wrong: name it)
     for name, t, dt in (("row_offsets", row_offsets, torch.int32), ("column_indices", column_indices, torch.int32),
                         ("values", values, torch.float16), ("rhs_matrix", rhs_matrix, torch.float16)):
         if t.dtype != dt:
@@ -31,6 +39,15 @@ def _check_inputs(row_indices, row_offsets, column_indices, values, rhs_matrix, 
 
 def _stream():
     return torch.cuda.current_stream().cuda_stream
+
+
+def _by_type(out_dtype, f16, f32):
+    """The entry point for a result type."""
+    if out_dtype is torch.float16:
+        return f16
+    if out_dtype is torch.float32:
+        return f32
+    raise KeyError(out_dtype)
 
 
 def _check_plan(plan, m_vec, vec_length, K):
@@ -55,17 +72,16 @@ def spmm(row_indices, row_offsets, column_indices, values, rhs_matrix, vec_lengt
     out = torch.empty((m_vec * vec_length, N), dtype=out_dtype, device=rhs_matrix.device)
     if plan is not None:
         _check_plan(plan, m_vec, vec_length, K)
-        fn = {torch.float16: _lib.lib().sspmm_plan_batched_f16_f16,
-              torch.float32: _lib.lib().sspmm_plan_batched_f16_f32}[out_dtype]
-        with torch.cuda.device(rhs_matrix.device):
-            rc = fn(plan.handle, 1, N, _ptr(row_offsets), _ptr(column_indices), _ptr(values), 0, _ptr(rhs_matrix), 0,
-                    _ptr(out), 0, _stream())
+        L = _lib.lib()
+        rc = _lib.call(_by_type(out_dtype, L.sspmm_plan_batched_f16_f16, L.sspmm_plan_batched_f16_f32), rhs_matrix.device,
+                       plan.handle, 1, N, row_offsets.data_ptr(), column_indices.data_ptr(), values.data_ptr(), 0,
+                       rhs_matrix.data_ptr(), 0, out.data_ptr(), 0)
         _lib.check(rc, "sspmm_plan")
         return out
-    fn = {torch.float16: _lib.lib().sspmm_f16_f16, torch.float32: _lib.lib().sspmm_f16_f32}[out_dtype]
-    with torch.cuda.device(rhs_matrix.device):
-        rc = fn(m_vec, vec_length, N, K, _ptr(row_indices), _ptr(row_offsets), _ptr(column_indices), _ptr(values),
-                _ptr(rhs_matrix), _ptr(out), _stream())
+    L = _lib.lib()
+    rc = _lib.call(_by_type(out_dtype, L.sspmm_f16_f16, L.sspmm_f16_f32), rhs_matrix.device, m_vec, vec_length, N, K,
+                   _ptr(row_indices), row_offsets.data_ptr(), column_indices.data_ptr(), values.data_ptr(), rhs_matrix.data_ptr(),
+                   out.data_ptr())
     _lib.check(rc, "sspmm")
     return out
 
@@ -89,9 +105,9 @@ def linear(row_offsets, column_indices, values, rhs_matrix, vec_length, bias=Non
                              bias.numel() != m_vec * vec_length):
         raise ValueError("bias must be a contiguous fp16 GPU tensor of m_vec * vec_length = %d elements" % (m_vec * vec_length))
     out = torch.empty((m_vec * vec_length, N), dtype=torch.float16, device=rhs_matrix.device)
-    with torch.cuda.device(rhs_matrix.device):
-        rc = _lib.lib().sspmm_linear_f16(m_vec, vec_length, N, K, _ptr(row_offsets), _ptr(column_indices), _ptr(values),
-                                         _ptr(rhs_matrix), _ptr(bias), ACTIVATIONS[activation], _ptr(out), _stream())
+    rc = _lib.call(_lib.lib().sspmm_linear_f16, rhs_matrix.device, m_vec, vec_length, N, K, row_offsets.data_ptr(),
+                   column_indices.data_ptr(), values.data_ptr(), rhs_matrix.data_ptr(), _ptr(bias), ACTIVATIONS[activation],
+                   out.data_ptr())
     _lib.check(rc, "sspmm_linear_f16")
     return out
 
@@ -112,18 +128,16 @@ def bspmm(row_indices, row_offsets, column_indices, values, rhs_matrix, vec_leng
     out = torch.empty((batch, M, N), dtype=out_dtype, device=rhs_matrix.device)
     if plan is not None:
         _check_plan(plan, m_vec, vec_length, K)
-        fn = {torch.float16: _lib.lib().sspmm_plan_batched_f16_f16,
-              torch.float32: _lib.lib().sspmm_plan_batched_f16_f32}[out_dtype]
-        with torch.cuda.device(rhs_matrix.device):
-            rc = fn(plan.handle, batch, N, _ptr(row_offsets), _ptr(column_indices), _ptr(values), nvec * vec_length,
-                    _ptr(rhs_matrix), K * N, _ptr(out), M * N, _stream())
+        L = _lib.lib()
+        rc = _lib.call(_by_type(out_dtype, L.sspmm_plan_batched_f16_f16, L.sspmm_plan_batched_f16_f32), rhs_matrix.device,
+                       plan.handle, batch, N, row_offsets.data_ptr(), column_indices.data_ptr(), values.data_ptr(),
+                       nvec * vec_length, rhs_matrix.data_ptr(), K * N, out.data_ptr(), M * N)
         _lib.check(rc, "sspmm_plan_batched")
         return out
-    fn = {torch.float16: _lib.lib().sspmm_batched_f16_f16,
-          torch.float32: _lib.lib().sspmm_batched_f16_f32}[out_dtype]
-    with torch.cuda.device(rhs_matrix.device):
-        rc = fn(batch, m_vec, vec_length, N, K, _ptr(row_indices), _ptr(row_offsets), _ptr(column_indices),
-                _ptr(values), nvec * vec_length, _ptr(rhs_matrix), K * N, _ptr(out), M * N, _stream())
+    L = _lib.lib()
+    rc = _lib.call(_by_type(out_dtype, L.sspmm_batched_f16_f16, L.sspmm_batched_f16_f32), rhs_matrix.device, batch, m_vec,
+                   vec_length, N, K, _ptr(row_indices), row_offsets.data_ptr(), column_indices.data_ptr(), values.data_ptr(),
+                   nvec * vec_length, rhs_matrix.data_ptr(), K * N, out.data_ptr(), M * N)
     _lib.check(rc, "sspmm_batched")
     return out
 

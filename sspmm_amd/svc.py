@@ -46,7 +46,8 @@ def svc(row_ptr, col_ind, csr_val, M, K, V, order="cpython", exact_size=True):
     with torch.cuda.device(dev):
         stream = torch.cuda.current_stream().cuda_stream
         ws = torch.empty(L.svc_workspace_bytes(M, nnz, V), dtype=torch.uint8, device=dev)
-        vec_row_ptr = torch.zeros(m_vec + 1, dtype=torch.int32, device=dev)
+        # (svc_count writes every entry)
+        vec_row_ptr = (torch.empty if M > 0 else torch.zeros)(m_vec + 1, dtype=torch.int32, device=dev)
         if M == 0:
             return SvcResult(vec_row_ptr, torch.empty(0, dtype=torch.int32, device=dev),
                              None if csr_val is None else torch.empty(0, dtype=torch.float16, device=dev), 0)
@@ -170,7 +171,7 @@ def svc_batched(mat_rows, K_max, row_ptr, col_ind, csr_val, V, order="cpython", 
         d_rows = torch.from_numpy(mat_rows.astype(np.int32)).to(dev)
         d_groups = torch.empty(count + 1, dtype=torch.int32, device=dev)
         ws = torch.empty(L.svc_batched_workspace_bytes(count, M_total, nnz, V), dtype=torch.uint8, device=dev)
-        vec_row_ptr = torch.zeros(groups + 1, dtype=torch.int32, device=dev)
+        vec_row_ptr = (torch.empty if groups > 0 else torch.zeros)(groups + 1, dtype=torch.int32, device=dev)
         vec_col = torch.empty(nnz, dtype=torch.int32, device=dev)
         vec_val = None if csr_val is None else torch.empty(nnz * V, dtype=torch.float16, device=dev)
         if groups > 0:
