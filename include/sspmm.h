@@ -368,6 +368,16 @@ int svc_permute_csr(int M, const int32_t *perm, const int32_t *row_ptr, const in
 int sspmm_add_layernorm_f16(int H, int T, const sspmm_half_t *x, const sspmm_half_t *a, const sspmm_half_t *gamma,
                             const sspmm_half_t *beta, float eps, sspmm_half_t *out, void *hip_stream);
 
+/*
+ * The same on token-major rows of E features (E = 64, 128, 256, 512, 1024 or 2048), outer x inner of them:
+ * out = LayerNorm(s), s = fp16(a + x), and s itself into `sum` unless that is NULL.  Row (i, j) of x is
+ * at x + i * x_outer + j * x_inner elements (multiples of 8); a (nullable), sum and out are dense.
+ * gamma and beta may be NULL; 16-byte aligned pointers.
+ */
+int sspmm_add_layernorm_rows_f16(int outer, int inner, int E, const sspmm_half_t *x, int64_t x_outer, int64_t x_inner,
+                                 const sspmm_half_t *a, const sspmm_half_t *gamma, const sspmm_half_t *beta, float eps,
+                                 sspmm_half_t *sum, sspmm_half_t *out, void *hip_stream);
+
 /* ------------------------------------------------------------------------------------------
  * Dense attention on feature-major activations: out = softmax(Q^T K * scale) V per (batch element,
  * head), the dense attention of the reference's comparison block (reference

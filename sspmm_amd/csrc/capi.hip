@@ -489,6 +489,30 @@ int sspmm_add_layernorm_f16(int H, int T, const sspmm_half_t *x, const sspmm_hal
   return (int)sspmm::launch_add_layernorm(H, T, x, a, gamma, beta, eps, out, static_cast<hipStream_t>(hip_stream));
 }
 
+int sspmm_add_layernorm_rows_f16(int outer, int inner, int E, const sspmm_half_t *x, int64_t x_outer, int64_t x_inner,
+                                 const sspmm_half_t *a, const sspmm_half_t *gamma, const sspmm_half_t *beta, float eps,
+                                 sspmm_half_t *sum, sspmm_half_t *out, void *hip_stream) {
+  if (outer < 0 || inner < 0 || (E != 64 && E != 128 && E != 256 && E != 512 && E != 1024 && E != 2048)) return kInvalid;
+  if (outer == 0 || inner == 0) return 0;
+  if (!x || !out || x_outer < 0 || x_inner < 0 || x_outer % 8 || x_inner % 8) return kInvalid;
+  const uintptr_t bits = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(gamma) |
+                         reinterpret_cast<uintptr_t>(beta) | reinterpret_cast<uintptr_t>(sum) | reinterpret_cast<uintptr_t>(out);
+  if (bits % 16) return kInvalid;
+  sspmm::AddLayerNormRows p;
+  p.rows = (long long)outer * inner;
+  p.inner = inner;
+  p.x = x;
+  p.x_outer = x_outer;
+  p.x_inner = x_inner;
+  p.a = a;
+  p.gamma = gamma;
+  p.beta = beta;
+  p.eps = eps;
+  p.sum = sum;
+  p.out = out;
+  return (int)sspmm::launch_add_layernorm_rows(E, p, static_cast<hipStream_t>(hip_stream));
+}
+
 int sspmm_attention_fm_f16(int batch, int heads, int seq, int head_dim, const sspmm_half_t *q, const sspmm_half_t *k,
                            const sspmm_half_t *v, int64_t ld, sspmm_half_t *out, int64_t ld_out, float scale, void *hip_stream) {
   if (batch < 0 || heads < 0 || seq < 0 || head_dim <= 0) return kInvalid;

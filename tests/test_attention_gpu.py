@@ -291,3 +291,56 @@ def test_sparse_attention_encoder_matches_dense_masked_attention(built_library):
     assert got.shape == (seq, 2, 16) and got.dtype == torch.float16
     assert torch.isfinite(got).all()
     assert max_rel_err(got.float().cpu().numpy(), want.float().cpu().numpy()) <= 1e-2
+
+
+@pytest.mark.parametrize("E", [64, 128, 256, 512, 1024, 2048])
+@pytest.mark.parametrize("outer,inner", [(1, 1), (3, 1), (37, 3), (130, 2)])
+def test_row_layernorm_with_residual(built_library, E, outer, inner):
+    """Every width, row counts that leave part of a workgroup without a row, x dense and as a batch-major view, with and
+    without the residual and the sum.  The sum is exact; statistics in fp32 leave the fp16 rounding of the result."""
+    from sspmm_amd.attention import add_layernorm_rows
+    g = torch.Generator("cuda").manual_seed(E + outer)
+    ln = torch.nn.LayerNorm(E).cuda().half()
+    with torch.no_grad():
+        ln.weight.copy_(torch.randn(E, device="cuda", generator=g))
+        ln.bias.copy_(torch.randn(E, device="cuda", generator=g))
+        a = torch.randn(outer, inner, E, device="cuda", generator=g).half()
+        for x in ((torch.randn(outer, inner, E, device="cuda", generator=g) * 3 + 1).half(),
+                  (torch.randn(inner, outer, E, device="cuda", generator=g) * 3 + 1).half().transpose(0, 1)):
+            for res, keep in ((None, False), (a, False), (a, True)):
+                total, got = add_layernorm_rows(x, res, ln, keep_sum=keep)
+                s = x if res is None else res + x
+                want = torch.nn.functional.layer_norm(s.double(), (E,), ln.weight.double(), ln.bias.double(), ln.eps)
+                assert got.is_contiguous() and got.shape == (outer, inner, E)
+                assert ((got.double() - want).abs() <= 2 ** -10 * want.abs() + 1e-5).all()
+                assert (total is None) if not keep else torch.equal(total, s)
+
+
+def test_encoder_with_fused_norms_matches_the_modules(built_library):
+    """The encoder's inference path against its modules called one by one, which a hook on any of them, autograd or
+    autocast still get."""
+    from sspmm_amd import attention as A
+    model = A.SparseAttentionEncoder(50, 128, 4, 0.9, 96, 192, 16, vec_length=8, layers=3, seed=2).cuda().half().eval()
+    tokens = torch.randint(0, 50, (3, 96), device="cuda", generator=torch.Generator("cuda").manual_seed(1))
+    calls = []
+    plain = A.add_layernorm_rows
+    A.add_layernorm_rows = lambda *args, **kw: (calls.append(1), plain(*args, **kw))[1]
+    try:
+        with torch.no_grad():
+            fused = model(tokens)
+            assert len(calls) == 7
+            handle = model.blocks[1].layer_norm2.register_forward_hook(lambda m, i, o: calls.append("hook"))
+            modules = model(tokens)
+            handle.remove()
+        assert calls[7:] == ["hook"]
+        with_grad = model(tokens)
+        assert with_grad.requires_grad and len(calls) == 8
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16):
+            model(tokens)
+        assert len(calls) == 8
+    finally:
+        A.add_layernorm_rows = plain
+    # (both round every activation to fp16; a LayerNorm that differs by an ulp moves the sums behind it by as much)
+    scale = modules.float().pow(2).mean().sqrt()
+    assert (fused.float() - modules.float()).abs().max() <= 1e-2 * scale
+    assert torch.equal(with_grad.detach(), modules)
