@@ -48,6 +48,9 @@ SIGNATURES = {
     "svc_count_batched": (_int, [_int, _int, _vp, _int, _int, _int, _vp, _vp, _i64, _int, _vp, _vp, _vp, _vp]),
     "svc_fill_batched": (_int, [_int, _int, _vp, _int, _int, _int, _vp, _vp, _vp, _i64, _int, _vp, _vp, _vp, _vp, _vp]),
     "sspmm_add_layernorm_f16": (_int, [_int, _int, _vp, _vp, _vp, _vp, ctypes.c_float, _vp, _vp]),
+    "sspmm_block_pack_f16": (_int, [_int, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "sspmm_block_dense_f16": (_int, [_int, _int, _int, _vp, _i64, _i64, _vp, _vp, _vp, _vp, _vp, ctypes.c_float, _int, _vp, _vp, _vp, _vp,
+                                     _vp, _vp, ctypes.c_float, _int, _vp, _vp, _vp, _vp, _vp]),
     "sspmm_add_layernorm_rows_f16": (_int, [_int, _int, _int, _vp, _i64, _i64, _vp, _vp, _vp, ctypes.c_float, _vp, _vp, _vp]),
     "sspmm_linear_f16": (_int, [_int, _int, _int, _int, _vp, _vp, _vp, _vp, _vp, _int, _vp, _vp]),
     "sspmm_attention_fm_f16": (_int, [_int, _int, _int, _int, _vp, _vp, _vp, ctypes.c_int64, _vp, ctypes.c_int64, ctypes.c_float, _vp]),

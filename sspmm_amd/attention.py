@@ -5,6 +5,8 @@ argument order, same shape inference (sddmm_kernel.cu:1169-1186 and 1236-1258,
 softmax_kernel.cu:208-216 and 256-266), and the block that chains them
 (end2end/sspmm_e2e/spattention.py:167-179).
 """
+import ctypes
+
 import torch
 
 from . import _lib
@@ -182,6 +184,53 @@ def add_layernorm_rows(x, a, ln, keep_sum=False):
     return total, out
 
 
+BLOCK_WIDTHS = (128, 256, 512)
+
+
+def pack_weights(linears, rows_per_wave):
+    """The weights of torch.nn.Linear modules in the order in which block_dense's kernel loads them, each a tensor of its
+    own out of one allocation, by one launch; rows_per_wave[i] = embed / 4 for out_proj and linear2, 64 for the others."""
+    n = len(linears)
+    shapes = [m.weight.shape for m in linears]
+    sizes = [r * c for r, c in shapes]
+    device = linears[0].weight.device
+    packed = torch.empty(sum(sizes), dtype=torch.float16, device=device)
+    ints = ctypes.c_int32 * n
+    rc = _lib.call(_lib.lib().sspmm_block_pack_f16, device, n, (ctypes.c_void_p * n)(*[m.weight.data_ptr() for m in linears]),
+                   ints(*[r for r, _ in shapes]), ints(*[c for _, c in shapes]), ints(*rows_per_wave), packed.data_ptr())
+    _lib.check(rc, "sspmm_block_pack_f16")
+    return packed.split(sizes)
+
+
+def block_dense(x, attn, block, norm, tail=None, keep_x=False, packed=None):
+    """(x', out): everything between the attention of `block` and the next one's in one launch, on token-major activations
+    [seq, batch, embed] fp16:
+        s = out_proj(attn) + x, x' = linear2(linear1(layer_norm2(s))) + x, h = norm(x'), out = tail(h) or h itself.
+    attn None: x' = x and `block` is not looked at.  x may be a view with strides of its own in the first two dimensions,
+    attn is dense, and so are the results.  x' is only returned with keep_x.  packed: pack_weights of out_proj, linear1 and
+    linear2 (where there is attn) and tail (where there is one), in this order."""
+    outer, inner, E = x.shape
+    n_out = 0 if tail is None else tail.out_features
+    out = torch.empty((outer, inner, n_out or E), dtype=torch.float16, device=x.device)
+    kept = torch.empty((outer, inner, E), dtype=torch.float16, device=x.device) if keep_x else None
+    stride = x.stride()
+    if packed is None:
+        own = [] if attn is None else [block.out_proj, block.linear1, block.linear2]
+        if own or tail is not None:
+            packed = pack_weights(own + ([] if tail is None else [tail]), [E // 4, 64, E // 4][:len(own)] + [64] * (tail is not None))
+    if attn is None:
+        own = (None, None, None, None, 0.0, 0, None, None, None, None)
+    else:
+        proj, up, down, ln = block.out_proj, block.linear1, block.linear2, block.layer_norm2
+        own = (packed[0].data_ptr(), _ptr(proj.bias), _ptr(ln.weight), _ptr(ln.bias), float(ln.eps), up.out_features,
+               packed[1].data_ptr(), _ptr(up.bias), packed[2].data_ptr(), _ptr(down.bias))
+    last = (None, None) if tail is None else (packed[-1].data_ptr(), _ptr(tail.bias))
+    rc = _lib.call(_lib.lib().sspmm_block_dense_f16, x.device, outer, inner, E, x.data_ptr(), stride[0], stride[1], _ptr(attn),
+                   *own, _ptr(norm.weight), _ptr(norm.bias), float(norm.eps), n_out, *last, _ptr(kept), out.data_ptr())
+    _lib.check(rc, "sspmm_block_dense_f16")
+    return kept, out
+
+
 def _rows_operand(t):
     return (type(t) is torch.Tensor and t.is_cuda and t.dtype == torch.float16 and t.dim() == 3 and t.numel() > 0 and t.stride(2) == 1 and
             t.stride(0) % 8 == 0 and t.stride(1) % 8 == 0 and t.data_ptr() % 16 == 0)
@@ -198,6 +247,18 @@ def _rows_norm_applies(ln, x):
     """Whether add_layernorm_rows may stand in for ln on activations like x."""
     E, w, b = x.size(-1), ln.weight, ln.bias
     return (_plain_module(ln, torch.nn.LayerNorm) and E in ROW_WIDTHS and ln.normalized_shape == (E,) and w is not None and
+            all(t is None or (type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float16 and t.device == x.device and
+                              t.is_contiguous() and t.data_ptr() % 16 == 0) for t in (w, b)))
+
+
+def _plain_linear(m, x, in_features, out_features, multiple):
+    """Whether m is a torch.nn.Linear of these sizes (out_features None: any multiple of `multiple`) whose weights a
+    kernel may read as they lie, for activations like x."""
+    if not _plain_module(m, torch.nn.Linear):
+        return False
+    w, b = m.weight, m.bias
+    return (m.in_features == in_features and m.out_features % multiple == 0 and out_features in (None, m.out_features) and
+            w.shape == (m.out_features, in_features) and (b is None or b.shape == (m.out_features,)) and
             all(t is None or (type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float16 and t.device == x.device and
                               t.is_contiguous() and t.data_ptr() % 16 == 0) for t in (w, b)))
 
@@ -236,6 +297,12 @@ class SparseAttentionBlock(torch.nn.Module):
         self.register_buffer("row_offsets", row_offsets)
         self.register_buffer("row_indices", row_indices)
 
+    def attention_on(self, qkv):
+        """The heads' attention from the fused projection, in one launch, ahead of the output projection."""
+        scaling = float(self.embed_dim // self.num_heads) ** -0.5
+        return sparse_attention_packed(self.row_indices, self.row_offsets, self.column_indices, qkv, self.num_heads, scaling,
+                                       self.vec_length)
+
     def attention(self, x, dense_mask=None):
         """x [seq, batch, embed] -> [seq, batch, embed].  With dense_mask (bool [seq, seq]) the three sparse steps
         are replaced by dense masked attention in fp32 (for checks)."""
@@ -245,8 +312,7 @@ class SparseAttentionBlock(torch.nn.Module):
         qkv = self.in_proj(x)
         if dense_mask is None and d in FUSED_HEAD_WIDTHS and qkv.dtype == torch.float16 and packed_attention_fits(seq, bsz, 3 * E):
             # the heads are read where the projection left them and written where the output projection wants them
-            return self.out_proj(sparse_attention_packed(self.row_indices, self.row_offsets, self.column_indices,
-                                                         qkv.contiguous(), h, scaling, self.vec_length))
+            return self.out_proj(self.attention_on(qkv.contiguous()))
         q, k, v = qkv.chunk(3, dim=-1)
         # [seq, batch * heads, d] -> [batch * heads, seq, d] (spattention.py:151-157)
         q, k, v = (t.contiguous().view(seq, bsz * h, d).transpose(0, 1).contiguous() for t in (q, k, v))
@@ -294,6 +360,8 @@ class SparseAttentionEncoder(torch.nn.Module):
         out = self.encoder(tokens) * (self.embed_dim ** 0.5)
         out = out.transpose(0, 1) + self.pe[:tokens.size(1)].to(out.dtype)
         if dense_masks is None and self._fused_norms_apply(out):
+            if self._fused_blocks_apply(out):
+                return self._fused_blocks(out)
             return self.linear(self._blocks_with_fused_norms(out))
         for i, blk in enumerate(self.blocks):
             out = blk(out, None if dense_masks is None else dense_masks[i])
@@ -320,3 +388,29 @@ class SparseAttentionEncoder(torch.nn.Module):
             y = blk.linear2(blk.linear1(h))
             x, h = add_norm(x, y, self.layer_norm if last else self.blocks[i + 1].layer_norm1, keep_sum=not last)
         return h
+
+    def _fused_blocks_apply(self, x):
+        """(where the fused norms do) heads that one launch of attention takes, and products that block_dense does"""
+        seq, bsz, E = x.shape
+        return E in BLOCK_WIDTHS and packed_attention_fits(seq, bsz, 3 * E) and all(
+            b.embed_dim == E and E % b.num_heads == 0 and E // b.num_heads in FUSED_HEAD_WIDTHS and
+            _plain_linear(b.in_proj, x, E, 3 * E, 64) and _plain_linear(b.out_proj, x, E, E, 64) and
+            _plain_linear(b.linear1, x, E, None, 256) and _plain_linear(b.linear2, x, b.linear1.out_features, E, 64)
+            for b in self.blocks)
+
+    def _fused_blocks(self, x):
+        """Two launches per block: its attention, and all that follows up to the next block's projection (or the head)."""
+        E, blocks = x.size(-1), list(self.blocks)
+        head = _plain_linear(self.linear, x, E, None, 64)
+        linears, rows = [blocks[0].in_proj], [64]
+        for i, blk in enumerate(blocks):
+            tail = [blocks[i + 1].in_proj] if i + 1 < len(blocks) else [self.linear] * head
+            linears += [blk.out_proj, blk.linear1, blk.linear2] + tail
+            rows += [E // 4, 64, E // 4] + [64] * len(tail)
+        packed = pack_weights(linears, rows)
+        _, qkv = block_dense(x, None, None, blocks[0].layer_norm1, blocks[0].in_proj, packed=packed[:1])
+        for i, (blk, nxt) in enumerate(zip(blocks, blocks[1:])):
+            x, qkv = block_dense(x, blk.attention_on(qkv), blk, nxt.layer_norm1, nxt.in_proj, True, packed[1 + 4 * i:5 + 4 * i])
+        out = block_dense(x, blocks[-1].attention_on(qkv), blocks[-1], self.layer_norm, self.linear if head else None,
+                          packed=packed[4 * len(blocks) - 3:])[1]
+        return out if head else self.linear(out)

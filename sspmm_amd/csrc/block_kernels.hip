@@ -1,0 +1,439 @@
+// The dense part of a sparse attention block in one launch (the reference runs it as torch modules, reference
+// end2end/sspmm_e2e/end_to_end.py:58-75: output projection, + x, LayerNorm, two linear layers, + x, and the next
+// block's LayerNorm and input projection).
+//
+// As separate launches every one of these reads and writes an activation of tokens x 256 to 1024 features, and the
+// matrix products are then bound by those bytes, not by the matrix units.  Here a workgroup keeps TM tokens from the
+// attention's output to the next block's projection: four waves split the
+// output features of every product, the activations pass between the products through LDS as fp16, and the
+// accumulators of the second linear layer stay in registers while the hidden features are made and used 256 at a time.
+//
+// Orientation: out^T[feature, token] = W (MFMA operand A, 16 features x 32 k) * act^T (operand B, 32 k x 16 tokens).
+// Both operands then are eight consecutive k per lane: W comes straight from global memory (row-major as torch keeps it;
+// a wave reads only the rows of its own features, so nothing is loaded twice by a workgroup and LDS is not involved),
+// act from LDS rows padded by 16 bytes (sixteen rows at sixteen different bank groups).  The rows of a wave's feature
+// tiles are dealt so that two tiles leave a lane eight consecutive features of one token (feature 32 (j / 2) + 8 g + 4 (j % 2)
+// + i of tile j, accumulator i, lane group g): residual loads, LDS writes and stores are 16-byte pieces, of which the
+// four lane groups make 64 consecutive bytes.
+//
+// The weights a workgroup streams from L2 are 1.6 MB at 256 features and 1024 hidden ones, 25k cycles at the 64 bytes a
+// cycle of a CU, whatever TM, and the products 384 cycles per token.  The loads of the next D units (eight 16-byte
+// loads of a wave each) are in flight throughout, also across the products' boundaries.  The matrices are packed by
+// a launch of their own first (7 us for the 6.7 MB of a model of four blocks), so that a load instruction reads 1 KB in a
+// row: from torch's layout it reads 64 bytes of each of sixteen rows, which lie 512 to 2048 bytes apart on a few of the L2's
+// channels, and 32 tokens per workgroup took 61 us instead of 27 (8192 tokens).
+//
+// 256 features, 1024 hidden, 768 out, with the LayerNorms: 8192 tokens 26 us, 32768 tokens 58 us (0.9 PFLOP/s), against
+// 104 (the host) and 121 for the four library products and two LayerNorm launches.  What is left is the chain of products
+// and LayerNorms of one workgroup (27 us with the card to itself, 64 tokens), the stream of the weights, and for the
+// large sizes the vector instructions between the products.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "block_kernels.h"
+
+namespace sspmm {
+
+namespace {
+
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
+
+constexpr int kChunk = 256;  // hidden (or output) features a workgroup makes at a time, 64 per wave
+
+// Workgroup barrier that orders LDS only: global loads in flight stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <int NJ>
+struct Unit {  // what is loaded together: NJ tiles of 16 features x K values of k
+  static constexpr int K = NJ == 8 ? 32 : 64;
+  static constexpr uint32_t kBytes = 32u * NJ * K;
+};
+
+// A wave's share of a packed weight matrix: its 16 * NJ rows, from column k0 on.  Every unit that is asked for lies inside
+// the matrix.
+struct Weights {
+  __amdgpu_buffer_rsrc_t srd;
+  uint32_t base;
+};
+template <int NJ>
+__device__ __forceinline__ Weights weights(const uint16_t *w, int rows, int cols, int row0, int k0) {
+  Weights r;
+  r.srd = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(w), 0, (int)((uint32_t)rows * (uint32_t)cols * 2u), 0x00020000);
+  r.base = (uint32_t)row0 * (uint32_t)cols * 2u + (uint32_t)(k0 / Unit<NJ>::K) * Unit<NJ>::kBytes;
+  return r;
+}
+template <int NJ>
+__device__ __forceinline__ void issue(uintx4 (&w)[8], const Weights &a, int unit) {
+  const uint32_t lane16 = (threadIdx.x & 63u) * 16u;
+#pragma unroll
+  for (int i = 0; i < (int)(Unit<NJ>::kBytes / 1024u); ++i)
+    w[i] = __builtin_bit_cast(uintx4, __builtin_amdgcn_raw_buffer_load_b128(a.srd, lane16 + (i & 3) * 1024u,
+                                                                            a.base + unit * Unit<NJ>::kBytes + (i >> 2) * 4096u, 0));
+}
+template <int NJ, int D>
+__device__ __forceinline__ void issue_first(uintx4 (&w)[D][8], const Weights &a) {
+#pragma unroll
+  for (int u = 0; u < D; ++u) issue<NJ>(w[u], a, u);
+}
+
+// acc[tile of 16 tokens][tile of 16 features] += W * act^T over K.  The first D units of `cur` are in `w` or on their way;
+// on return those of `next` (tiles of NEXT) are.  act: the lane's address in the LDS rows (row lane % 16, k = 8 (lane / 16)).
+template <int TT, int NJ, int K, int PITCH, int NEXT, int D>
+__device__ __forceinline__ void gemm(floatx4 (&acc)[TT][NJ], const unsigned char *act, const Weights &cur, const Weights &next,
+                                     uintx4 (&w)[D][8]) {
+  constexpr int KU = Unit<NJ>::K, U = K / KU;
+  static_assert(U % D == 0, "the units of a product rotate through the buffers whole");
+  constexpr int S = KU / 32;  // steps of a unit
+  half8 b[2][TT];
+#pragma unroll
+  for (int t = 0; t < TT; ++t) b[0][t] = *reinterpret_cast<const half8 *>(act + t * 16 * PITCH);
+#pragma unroll
+  for (int s = 0; s < U * S; ++s) {
+    const int u = s / S;
+    if (s + 1 < U * S) {
+#pragma unroll
+      for (int t = 0; t < TT; ++t) b[(s + 1) & 1][t] = *reinterpret_cast<const half8 *>(act + t * 16 * PITCH + (s + 1) * 64);
+    }
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        acc[t][j] =
+            __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, w[u % D][(s % S) * NJ + j]), b[s & 1][t], acc[t][j], 0, 0, 0);
+    if (s % S == S - 1) {
+      if (u + D < U)
+        issue<NJ>(w[u % D], cur, u + D);
+      else
+        issue<NEXT>(w[u % D], next, u + D - U);
+    }
+    // (left alone, the scheduler pulls the reads of many steps ahead and spills)
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// The lane's 4 * NJ values of one row (16-byte pieces, 32 features apart) as they lie in memory, and one of them widened.
+template <int NJ>
+__device__ __forceinline__ void load_row(half8 (&v)[NJ / 2], const uint16_t *p) {
+#pragma unroll
+  for (int j = 0; j < NJ / 2; ++j) v[j] = *reinterpret_cast<const half8 *>(p + 32 * j);
+}
+template <int N>
+__device__ __forceinline__ float value(const half8 (&v)[N], int j, int i) { return (float)v[j / 2][(j & 1) * 4 + i]; }
+// Per-feature values (bias, gamma, beta); `none` where there is no such vector.
+template <int NJ>
+__device__ __forceinline__ void feature_values(half8 (&v)[NJ / 2], const uint16_t *p, int first, float none) {
+  if (p) {
+    load_row<NJ>(v, p + first);
+  } else {
+#pragma unroll
+    for (int j = 0; j < NJ / 2; ++j)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[j][i] = (_Float16)none;
+  }
+}
+
+// A lane's 4 * NJ features of one token as 16-byte pieces.
+template <int NJ>
+__device__ __forceinline__ void put_row(unsigned char *p, const floatx4 (&v)[NJ]) {
+#pragma unroll
+  for (int j = 0; j < NJ; j += 2) {
+    half8 h;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      h[i] = (_Float16)v[j][i];
+      h[4 + i] = (_Float16)v[j + 1][i];
+    }
+    *reinterpret_cast<half8 *>(p + j * 32) = h;
+  }
+}
+
+// Sum over a token's features of one value per lane and token tile: over the four lane groups, then over the four
+// waves through `part` [4][TM].  One barrier; the next use of `part` needs another one in between.
+template <int TT>
+__device__ __forceinline__ void token_sums(float (&s)[TT], float *part, int wave, int lane) {
+#pragma unroll
+  for (int t = 0; t < TT; ++t) {
+    s[t] += __shfl_xor(s[t], 16, 64);
+    s[t] += __shfl_xor(s[t], 32, 64);
+    part[wave * (TT * 16) + t * 16 + (lane & 15)] = s[t];  // (the four lane groups hold the same sum)
+  }
+  lds_barrier();
+#pragma unroll
+  for (int t = 0; t < TT; ++t) {
+    const float *q = part + t * 16 + (lane & 15);
+    s[t] = (q[0] + q[TT * 16]) + (q[2 * TT * 16] + q[3 * TT * 16]);
+  }
+}
+
+// v = LayerNorm(v) over the E features of every token, statistics in fp32, mean first.
+template <int TT, int NJ, int E>
+__device__ __forceinline__ void layer_norm(floatx4 (&v)[TT][NJ], const uint16_t *gamma, const uint16_t *beta, float eps, int first,
+                                           float *part, int wave, int lane) {
+  half8 w[NJ / 2], b[NJ / 2];
+  feature_values<NJ>(w, gamma, first, 1.f);
+  feature_values<NJ>(b, beta, first, 0.f);
+  float s[TT];
+#pragma unroll
+  for (int t = 0; t < TT; ++t) {
+    s[t] = 0.f;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) s[t] += (v[t][j][0] + v[t][j][1]) + (v[t][j][2] + v[t][j][3]);
+  }
+  token_sums<TT>(s, part, wave, lane);
+#pragma unroll
+  for (int t = 0; t < TT; ++t) {
+    const float mean = s[t] * (1.0f / (float)E);
+    s[t] = 0.f;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v[t][j][i] -= mean;
+        s[t] += v[t][j][i] * v[t][j][i];
+      }
+  }
+  token_sums<TT>(s, part + 4 * TT * 16, wave, lane);
+#pragma unroll
+  for (int t = 0; t < TT; ++t) {
+    const float rstd = rsqrtf(s[t] * (1.0f / (float)E) + eps);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[t][j][i] = v[t][j][i] * rstd * value(w, j, i) + value(b, j, i);
+  }
+}
+
+constexpr int block_waves(int E, int TM) { return TM == 64 && E < 512 ? 2 : 1; }  // per SIMD
+
+template <int E, int TM, bool ATTN>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves(E, TM), block_waves(E, TM)))) void block_dense_kernel(const BlockDenseArgs p) {
+  constexpr int NT = E / 64, TT = TM / 16, D = E == 128 || block_waves(E, TM) == 2 ? 2 : 4;
+  constexpr int kPitchA = E * 2 + 16, kPitchH = kChunk * 2 + 16;
+  __shared__ __align__(16) unsigned char act[TM * kPitchA];  // attention's output, then n, then h
+  __shared__ __align__(16) unsigned char hid[TM * kPitchH];  // kChunk hidden features
+  __shared__ float part[8 * TM];
+
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int m = lane & 15, g = lane >> 4;
+  const long long t0 = (long long)blockIdx.x * TM;
+  const int left = (int)min((long long)TM, p.tokens - t0);  // >= 1: tokens beyond the last repeat it, without storing
+  const int first = wave * (16 * NT) + g * 8;  // the lane's first feature of E
+  const int chunk_first = wave * 64 + g * 8;         // and of a chunk
+  const unsigned char *const act_op = act + m * kPitchA + g * 16, *const hid_op = hid + m * kPitchH + g * 16;
+
+  uintx4 w[D][8];
+  const int t_row = p.wt && wave * 64 < p.n_out ? wave * 64 : 0;
+  // (where nothing follows, the loads ahead go to the matrix at hand once more)
+  const Weights tail = p.wt ? weights<4>(p.wt, p.n_out, E, t_row, 0) : weights<4>(p.w1, p.mlp, E, wave * 64, 0);
+  const Weights wo = weights<NT>(p.wo, E, E, wave * (16 * NT), 0);
+  if constexpr (ATTN)
+    issue_first<NT, D>(w, wo);
+  else if (p.wt)
+    issue_first<4, D>(w, tail);
+
+  // the lane's share of x, fetched once
+  half8 x[TT][NT / 2];
+  if (p.x_inner == E && p.x_outer == p.inner * E) {
+#pragma unroll
+    for (int t = 0; t < TT; ++t) load_row<NT>(x[t], p.x + (t0 + min(t * 16 + m, left - 1)) * E + first);
+  } else {
+    const long long q0 = t0 / p.inner;
+    const uint32_t r0 = (uint32_t)(t0 - q0 * p.inner);
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+      const uint32_t r = r0 + (uint32_t)min(t * 16 + m, left - 1), q = r / (uint32_t)p.inner;
+      load_row<NT>(x[t], p.x + (q0 + q) * p.x_outer + (long long)(r - q * (uint32_t)p.inner) * p.x_inner + first);
+    }
+  }
+
+  floatx4 v[TT][NT];
+  if constexpr (ATTN) {
+    const Weights w1 = weights<4>(p.w1, p.mlp, E, wave * 64, 0);
+    const Weights w2 = weights<NT>(p.w2, E, p.mlp, wave * (16 * NT), 0);
+    half8 bias[NT / 2], bias2[NT / 2];
+    feature_values<NT>(bias, p.bo, first, 0.f);
+    feature_values<NT>(bias2, p.b2, first, 0.f);
+    constexpr int kPieces = E / 8, kRows = 256 / kPieces;
+    const int piece = threadIdx.x % kPieces, row0 = threadIdx.x / kPieces;
+#pragma unroll
+    for (int r = 0; r < TM; r += kRows)
+      *reinterpret_cast<uintx4 *>(act + (r + row0) * kPitchA + piece * 16) =
+          *reinterpret_cast<const uintx4 *>(p.attn + (t0 + min(r + row0, left - 1)) * E + piece * 8);
+    lds_barrier();
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[t][j][i] = value(bias, j, i);
+    gemm<TT, NT, E, kPitchA, 4, D>(v, act_op, wo, w1, w);
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[t][j][i] += value(x[t], j, i);
+    // (or the compiler keeps the widened values for the second use, at twice the registers)
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int j = 0; j < NT / 2; ++j) asm("" : "+v"(x[t][j]));
+    layer_norm<TT, NT, E>(v, p.gamma2, p.beta2, p.eps2, first, part, wave, lane);
+    // (every wave is past its product: the sums' barriers lie in between)
+#pragma unroll
+    for (int t = 0; t < TT; ++t) put_row<NT>(act + (t * 16 + m) * kPitchA + first * 2, v[t]);
+    lds_barrier();
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[t][j][i] = value(bias2, j, i) + value(x[t], j, i);
+    for (int c = 0; c < p.mlp; c += kChunk) {
+      floatx4 h[TT][4];
+      half8 bias1[2];
+      feature_values<4>(bias1, p.b1, c + chunk_first, 0.f);
+#pragma unroll
+      for (int t = 0; t < TT; ++t)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) h[t][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+      Weights up = w1, down = w2, then = tail;
+      up.base += (uint32_t)c * (E * 2u);
+      down.base += (uint32_t)(c / Unit<NT>::K) * Unit<NT>::kBytes;
+      if (c + kChunk < p.mlp) {
+        then = up;
+        then.base += kChunk * (E * 2u);
+      }
+      gemm<TT, 4, E, kPitchA, NT, D>(h, act_op, up, down, w);
+      lds_barrier();  // the previous chunk has been read
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) h[t][j][i] += value(bias1, j, i);
+        put_row<4>(hid + (t * 16 + m) * kPitchH + chunk_first * 2, h[t]);
+      }
+      lds_barrier();
+      gemm<TT, NT, kChunk, kPitchH, 4, D>(v, hid_op, down, then, w);
+    }
+  } else {
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[t][j][i] = value(x[t], j, i);
+  }
+  // x' as it is stored is what its LayerNorm reads
+#pragma unroll
+  for (int t = 0; t < TT; ++t) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[t][j][i] = (float)(_Float16)v[t][j][i];
+    if (p.x_out && t * 16 + m < left) put_row<NT>(reinterpret_cast<unsigned char *>(p.x_out + (t0 + t * 16 + m) * E + first), v[t]);
+  }
+
+  layer_norm<TT, NT, E>(v, p.gamma_n, p.beta_n, p.eps_n, first, part, wave, lane);
+  if (!p.wt) {
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+      if (t * 16 + m < left) put_row<NT>(reinterpret_cast<unsigned char *>(p.norm_out + (t0 + t * 16 + m) * E + first), v[t]);
+    return;
+  }
+#pragma unroll
+  for (int t = 0; t < TT; ++t) put_row<NT>(act + (t * 16 + m) * kPitchA + first * 2, v[t]);
+  lds_barrier();
+  Weights cur = tail;
+  for (int c = wave * 64; c < p.n_out; c += kChunk) {  // (no barrier from here on)
+    floatx4 o[TT][4];
+    half8 bias[2];
+    feature_values<4>(bias, p.bt, c + g * 8, 0.f);
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[t][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    Weights then = cur;
+    if (c + kChunk < p.n_out) then.base += kChunk * (E * 2u);
+    gemm<TT, 4, E, kPitchA, 4, D>(o, act_op, cur, then, w);
+    cur = then;
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[t][j][i] += value(bias, j, i);
+      if (t * 16 + m < left)
+        put_row<4>(reinterpret_cast<unsigned char *>(p.out + (t0 + t * 16 + m) * p.n_out + c + g * 8), o[t]);
+    }
+  }
+}
+
+// Up to kPackMost matrices into the order in which the waves above load them: groups of 16 * NJ rows, in each units of
+// K columns, in each a 1 KB piece per step of 32 columns and tile, in that the 16 bytes of every lane.
+__global__ __launch_bounds__(256) void block_pack_kernel(const BlockPackArgs p) {
+  int i = 0;
+  while (i + 1 < p.count && blockIdx.x >= p.m[i + 1].first_block) ++i;
+  const BlockPackArgs::Matrix &a = p.m[i];
+  const uint32_t at = (blockIdx.x - a.first_block) * 256u + threadIdx.x;  // 16-byte piece of the packed matrix
+  const uint32_t cols = a.cols, nj = a.group / 16u, ku = nj == 8 ? 32u : 64u;
+  if (at >= (uint32_t)a.rows * (cols / 8u)) return;
+  const uint32_t lane = at & 63u, m = lane & 15u, g = lane >> 4, frag = at >> 6;
+  const uint32_t per_unit = nj * ku / 32u, in_unit = frag % per_unit, unit = frag / per_unit;
+  const uint32_t units = cols / ku, group = unit / units;
+  const uint32_t row = group * a.group + 32u * (in_unit % nj / 2u) + 8u * (m >> 2) + 4u * (in_unit & 1u) + (m & 3u);
+  const uint32_t k = (unit % units) * ku + (in_unit / nj) * 32u + 8u * g;
+  reinterpret_cast<uintx4 *>(a.dst)[at] = *reinterpret_cast<const uintx4 *>(a.src + (size_t)row * cols + k);
+}
+
+template <int E, int TM>
+hipError_t launch(const BlockDenseArgs &p, hipStream_t stream) {
+  const long long blocks = (p.tokens + TM - 1) / TM;
+  if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
+  if (p.attn)
+    hipLaunchKernelGGL((block_dense_kernel<E, TM, true>), dim3((unsigned)blocks), dim3(256), 0, stream, p);
+  else
+    hipLaunchKernelGGL((block_dense_kernel<E, TM, false>), dim3((unsigned)blocks), dim3(256), 0, stream, p);
+  return hipGetLastError();
+}
+
+// 64 tokens per workgroup, two workgroups per CU (where the registers of 512 features allow one): one's LayerNorms and LDS
+// passes run under the other's products.  32768 tokens of 256 features: 58 us, with one workgroup per CU 69, with one of
+// 128 tokens 64; of 128 features 32, 39 and 35.  Up to 8192 tokens those are at most 128 workgroups, and 32 tokens give every
+// CU one: 8192 tokens of 128, 256, 512 features 15, 26, 56 us against 18, 30, 73; 10000 tokens 25, 43, 101 against 18, 31, 73.
+template <int E>
+hipError_t launch_for_width(const BlockDenseArgs &p, hipStream_t stream) {
+  return p.tokens <= 256 * 32 ? launch<E, 32>(p, stream) : launch<E, 64>(p, stream);
+}
+
+}  // namespace
+
+bool block_dense_applies(int E, int mlp, int n_out) {
+  // (a weight matrix is addressed with 32-bit byte offsets)
+  return (E == 128 || E == 256 || E == 512) && mlp > 0 && mlp % kChunk == 0 && mlp <= (1 << 20) && n_out >= 0 && n_out % 64 == 0 &&
+         n_out <= (1 << 20);
+}
+
+hipError_t launch_block_pack(const BlockPackArgs &p, uint32_t blocks, hipStream_t stream) {
+  hipLaunchKernelGGL(block_pack_kernel, dim3(blocks), dim3(256), 0, stream, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_block_dense(int E, const BlockDenseArgs &p, hipStream_t stream) {
+  switch (E) {
+    case 128: return launch_for_width<128>(p, stream);
+    case 256: return launch_for_width<256>(p, stream);
+    case 512: return launch_for_width<512>(p, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace sspmm

@@ -4,6 +4,7 @@
 
 #include "../../include/sspmm.h"
 #include "attention_kernels.h"
+#include "block_kernels.h"
 #include "coo_kernels.h"
 #include "layer_kernels.h"
 #include "plan.h"
@@ -511,6 +512,70 @@ int sspmm_add_layernorm_rows_f16(int outer, int inner, int E, const sspmm_half_t
   p.sum = sum;
   p.out = out;
   return (int)sspmm::launch_add_layernorm_rows(E, p, static_cast<hipStream_t>(hip_stream));
+}
+
+int sspmm_block_pack_f16(int count, const sspmm_half_t *const *src, const int32_t *rows, const int32_t *cols, const int32_t *group,
+                         sspmm_half_t *dst, void *hip_stream) {
+  if (count < 0 || (count > 0 && (!src || !rows || !cols || !group || !dst || reinterpret_cast<uintptr_t>(dst) % 16))) return kInvalid;
+  for (int i = 0; i < count; ++i) {
+    if (!src[i] || reinterpret_cast<uintptr_t>(src[i]) % 16 || (group[i] != 32 && group[i] != 64 && group[i] != 128)) return kInvalid;
+    if (rows[i] <= 0 || rows[i] % group[i] || cols[i] <= 0 || cols[i] % 64 || (int64_t)rows[i] * cols[i] >= (1ll << 30)) return kInvalid;
+  }
+  for (int done = 0; done < count;) {
+    sspmm::BlockPackArgs p;
+    uint32_t blocks = 0;
+    for (p.count = 0; p.count < sspmm::BlockPackArgs::kMost && done < count && blocks < (1u << 30); ++p.count, ++done) {
+      p.m[p.count] = {src[done], dst, rows[done], cols[done], group[done], blocks};
+      blocks += ((uint32_t)rows[done] * (uint32_t)(cols[done] / 8) + 255u) / 256u;
+      dst += (int64_t)rows[done] * cols[done];
+    }
+    const hipError_t e = sspmm::launch_block_pack(p, blocks, static_cast<hipStream_t>(hip_stream));
+    if (e != hipSuccess) return (int)e;
+  }
+  return 0;
+}
+
+int sspmm_block_dense_f16(int outer, int inner, int E, const sspmm_half_t *x, int64_t x_outer, int64_t x_inner, const sspmm_half_t *attn,
+                          const sspmm_half_t *wo, const sspmm_half_t *bo, const sspmm_half_t *gamma2, const sspmm_half_t *beta2,
+                          float eps2, int mlp, const sspmm_half_t *w1, const sspmm_half_t *b1, const sspmm_half_t *w2,
+                          const sspmm_half_t *b2, const sspmm_half_t *gamma_n, const sspmm_half_t *beta_n, float eps_n, int n_out,
+                          const sspmm_half_t *wt, const sspmm_half_t *bt, sspmm_half_t *x_out, sspmm_half_t *out, void *hip_stream) {
+  if (outer < 0 || inner < 0 || !sspmm::block_dense_applies(E, attn ? mlp : 256, n_out)) return kInvalid;
+  if (outer == 0 || inner == 0) return 0;
+  if (!x || !out || x_outer < 0 || x_inner < 0 || x_outer % 8 || x_inner % 8 || (wt != nullptr) != (n_out > 0)) return kInvalid;
+  if (attn && (!wo || !w1 || !w2)) return kInvalid;
+  uintptr_t bits = 0;
+  for (const sspmm_half_t *q : {x, attn, wo, bo, gamma2, beta2, w1, b1, w2, b2, gamma_n, beta_n, wt, bt, (const sspmm_half_t *)x_out,
+                                (const sspmm_half_t *)out})
+    bits |= reinterpret_cast<uintptr_t>(q);
+  if (bits % 16) return kInvalid;
+  sspmm::BlockDenseArgs p;
+  p.tokens = (long long)outer * inner;
+  p.inner = inner;
+  p.x = x;
+  p.x_outer = x_outer;
+  p.x_inner = x_inner;
+  p.attn = attn;
+  p.wo = wo;
+  p.bo = bo;
+  p.gamma2 = gamma2;
+  p.beta2 = beta2;
+  p.w1 = w1;
+  p.b1 = b1;
+  p.w2 = w2;
+  p.b2 = b2;
+  p.gamma_n = gamma_n;
+  p.beta_n = beta_n;
+  p.wt = wt;
+  p.bt = bt;
+  p.eps2 = eps2;
+  p.eps_n = eps_n;
+  p.mlp = attn ? mlp : 0;
+  p.n_out = n_out;
+  p.x_out = x_out;
+  p.norm_out = wt ? nullptr : out;
+  p.out = out;
+  return (int)sspmm::launch_block_dense(E, p, static_cast<hipStream_t>(hip_stream));
 }
 
 int sspmm_attention_fm_f16(int batch, int heads, int seq, int head_dim, const sspmm_half_t *q, const sspmm_half_t *k,

@@ -344,3 +344,69 @@ def test_encoder_with_fused_norms_matches_the_modules(built_library):
     scale = modules.float().pow(2).mean().sqrt()
     assert (fused.float() - modules.float()).abs().max() <= 1e-2 * scale
     assert torch.equal(with_grad.detach(), modules)
+
+
+def _block_by_modules(x, attn, blk, norm, tail):
+    """float64, with the roundings to fp16 that an activation written to memory has: (x', out)."""
+    lin = lambda m, t: t @ m.weight.double().t() + m.bias.double()  # noqa: E731
+    ln = lambda m, t: torch.nn.functional.layer_norm(t, m.normalized_shape, m.weight.double(), m.bias.double(), m.eps)  # noqa: E731
+    r = x.double()
+    if attn is not None:
+        n = ln(blk.layer_norm2, lin(blk.out_proj, attn.double()) + r).half().double()
+        r = (lin(blk.linear2, lin(blk.linear1, n).half().double()) + r).half().double()
+    h = ln(norm, r)
+    return r, h if tail is None else lin(tail, h.half().double())
+
+
+@pytest.mark.parametrize("E,mlp,n_out", [(128, 256, 64), (128, 1024, 384), (256, 256, 320), (256, 1024, 768), (512, 512, 1536)])
+@pytest.mark.parametrize("outer,inner", [(1, 1), (33, 1), (127, 3), (2731, 3)])
+def test_block_dense_in_one_launch(built_library, E, mlp, n_out, outer, inner):
+    """Every width and tile of tokens (32, 64) with a last tile that is not full, output widths that leave waves without a
+    chunk, x dense and batch-major, with and without attention, tail and x'.  Roundings to fp16 at other places (a
+    hidden activation an ulp away, 2^-11) stay below 4 * 2^-11 of the result's size after the sums behind them."""
+    from sspmm_amd.attention import SparseAttentionBlock, block_dense
+    g = torch.Generator("cuda").manual_seed(E + outer + n_out)
+    none = torch.zeros(1, dtype=torch.int32)
+    torch.manual_seed(E + n_out)
+    blk = SparseAttentionBlock(E, mlp, E // 32, none, none, none).cuda().half()
+    norm, tail = torch.nn.LayerNorm(E).cuda().half(), torch.nn.Linear(E, n_out).cuda().half()
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g).half()  # noqa: E731
+    with torch.no_grad():
+        for m in (norm, blk.layer_norm2):
+            m.weight.copy_(1 + 0.2 * rnd(E))
+            m.bias.copy_(rnd(E))
+        attn = rnd(outer, inner, E)
+        close = lambda got, want: ((got.double() - want).abs().max() <= 4 * 2 ** -11 * want.abs().max()).item()  # noqa: E731
+        for x in (rnd(outer, inner, E) * 2 + 1, (rnd(inner, outer, E) * 2 + 1).transpose(0, 1)):
+            for a, last, keep in ((attn, tail, True), (attn, None, False), (None, tail, False), (None, None, True)):
+                kept, got = block_dense(x, a, blk, norm, last, keep_x=keep)
+                want_x, want = _block_by_modules(x, a, blk, norm, last)
+                assert got.is_contiguous() and got.shape == (outer, inner, n_out if last is not None else E)
+                assert close(got, want), (a is None, last is None, (got.double() - want).abs().max().item(), want.abs().max().item())
+                assert (kept is None) if not keep else (torch.equal(kept, x) if a is None else close(kept, want_x))
+
+
+@pytest.mark.parametrize("embed,heads,classes", [(128, 4, 64), (256, 8, 16), (512, 8, 256)])
+def test_encoder_in_two_launches_per_block_matches_the_modules(built_library, embed, heads, classes):
+    """A head of a width that the launch does not take stays a module's; a hook on a linear layer gets its module called."""
+    from sspmm_amd import attention as A
+    model = A.SparseAttentionEncoder(50, embed, heads, 0.9, 96, 256, classes, vec_length=8, layers=3, seed=2).cuda().half().eval()
+    tokens = torch.randint(0, 50, (3, 96), device="cuda", generator=torch.Generator("cuda").manual_seed(1))
+    calls = []
+    plain = A.block_dense
+    A.block_dense = lambda *args, **kw: (calls.append(1), plain(*args, **kw))[1]
+    try:
+        with torch.no_grad():
+            fused = model(tokens)
+            assert len(calls) == 4
+            handle = model.blocks[1].linear1.register_forward_hook(lambda m, i, o: calls.append("hook"))
+            norms = model(tokens)
+            handle.remove()
+        assert calls[4:] == ["hook"]
+        modules = model(tokens)
+        assert modules.requires_grad and len(calls) == 5
+    finally:
+        A.block_dense = plain
+    scale = modules.float().pow(2).mean().sqrt()  # (as above)
+    assert (fused.float() - modules.float()).abs().max() <= 1e-2 * scale
+    assert (norms.float() - modules.float()).abs().max() <= 1e-2 * scale
