@@ -50,7 +50,7 @@ SIGNATURES = {
     "sspmm_add_layernorm_f16": (_int, [_int, _int, _vp, _vp, _vp, _vp, ctypes.c_float, _vp, _vp]),
     "sspmm_block_pack_f16": (_int, [_int, _vp, _vp, _vp, _vp, _vp, _vp]),
     "sspmm_block_dense_f16": (_int, [_int, _int, _int, _vp, _i64, _i64, _vp, _vp, _vp, _vp, _vp, ctypes.c_float, _int, _vp, _vp, _vp, _vp,
-                                     _vp, _vp, ctypes.c_float, _int, _vp, _vp, _vp, _vp, _vp]),
+                                     _vp, _vp, ctypes.c_float, _int, _int, _vp, _vp, _vp, _vp, _vp]),
     "sspmm_add_layernorm_rows_f16": (_int, [_int, _int, _int, _vp, _i64, _i64, _vp, _vp, _vp, ctypes.c_float, _vp, _vp, _vp]),
     "sspmm_linear_f16": (_int, [_int, _int, _int, _int, _vp, _vp, _vp, _vp, _vp, _int, _vp, _vp]),
     "sspmm_attention_fm_f16": (_int, [_int, _int, _int, _int, _vp, _vp, _vp, ctypes.c_int64, _vp, ctypes.c_int64, ctypes.c_float, _vp]),

@@ -25,6 +25,7 @@ struct BlockDenseArgs {
   const uint16_t *wt, *bt;                   // nullable: norm_out in their place
   float eps2, eps_n;
   int mlp, n_out;
+  int head_dim;                              // out as [n_out / E, inner, E / head_dim, tokens / inner, head_dim]; 0: as [tokens, n_out]
   uint16_t *x_out;                           // nullable: x' is not needed
   uint16_t *norm_out, *out;
 };

@@ -353,6 +353,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
   for (int t = 0; t < TT; ++t) put_row<NT>(act + (t * 16 + m) * kPitchA + first * 2, v[t]);
   lds_barrier();
   Weights cur = tail;
+  const long long outer = p.tokens / p.inner, q0 = t0 / p.inner;
+  const uint32_t r0 = (uint32_t)(t0 - q0 * p.inner);
+  const int head_shift = p.head_dim ? __builtin_ctz((unsigned)p.head_dim) : 0;
   for (int c = wave * 64; c < p.n_out; c += kChunk) {  // (no barrier from here on)
     floatx4 o[TT][4];
     half8 bias[2];
@@ -371,8 +374,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[t][j][i] += value(bias, j, i);
-      if (t * 16 + m < left)
-        put_row<4>(reinterpret_cast<unsigned char *>(p.out + (t0 + t * 16 + m) * p.n_out + c + g * 8), o[t]);
+      if (t * 16 + m < left) {
+        if (p.head_dim == 0) {
+          put_row<4>(reinterpret_cast<unsigned char *>(p.out + (t0 + t * 16 + m) * p.n_out + c + g * 8), o[t]);
+        } else {  // (a head is at least as wide as the 32 features of two tiles)
+          const uint32_t r = r0 + (uint32_t)(t * 16 + m), i = r / (uint32_t)p.inner;  // token (q0 + i, r - i * inner)
+          uint16_t *const row = p.out + (r - i * (uint32_t)p.inner) * (E * outer) + (q0 + i) * p.head_dim + g * 8;
+#pragma unroll
+          for (int j = 0; j < 4; j += 2) {
+            const int f = c + 16 * j, in_part = f % E;
+            const floatx4 pair[2] = {o[t][j], o[t][j + 1]};
+            put_row<2>(reinterpret_cast<unsigned char *>(row + (f / E) * (p.inner * outer * E) + (in_part >> head_shift) * (outer * p.head_dim) +
+                                                         (in_part & (p.head_dim - 1))),
+                       pair);
+          }
+        }
+      }
     }
   }
 }

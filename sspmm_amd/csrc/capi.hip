@@ -538,12 +538,13 @@ int sspmm_block_pack_f16(int count, const sspmm_half_t *const *src, const int32_
 int sspmm_block_dense_f16(int outer, int inner, int E, const sspmm_half_t *x, int64_t x_outer, int64_t x_inner, const sspmm_half_t *attn,
                           const sspmm_half_t *wo, const sspmm_half_t *bo, const sspmm_half_t *gamma2, const sspmm_half_t *beta2,
                           float eps2, int mlp, const sspmm_half_t *w1, const sspmm_half_t *b1, const sspmm_half_t *w2,
-                          const sspmm_half_t *b2, const sspmm_half_t *gamma_n, const sspmm_half_t *beta_n, float eps_n, int n_out,
+                          const sspmm_half_t *b2, const sspmm_half_t *gamma_n, const sspmm_half_t *beta_n, float eps_n, int n_out, int head_dim,
                           const sspmm_half_t *wt, const sspmm_half_t *bt, sspmm_half_t *x_out, sspmm_half_t *out, void *hip_stream) {
   if (outer < 0 || inner < 0 || !sspmm::block_dense_applies(E, attn ? mlp : 256, n_out)) return kInvalid;
   if (outer == 0 || inner == 0) return 0;
   if (!x || !out || x_outer < 0 || x_inner < 0 || x_outer % 8 || x_inner % 8 || (wt != nullptr) != (n_out > 0)) return kInvalid;
   if (attn && (!wo || !w1 || !w2)) return kInvalid;
+  if (head_dim != 0 && ((head_dim != 32 && head_dim != 64 && head_dim != 128) || n_out % E)) return kInvalid;
   uintptr_t bits = 0;
   for (const sspmm_half_t *q : {x, attn, wo, bo, gamma2, beta2, w1, b1, w2, b2, gamma_n, beta_n, wt, bt, (const sspmm_half_t *)x_out,
                                 (const sspmm_half_t *)out})
@@ -572,6 +573,7 @@ int sspmm_block_dense_f16(int outer, int inner, int E, const sspmm_half_t *x, in
   p.eps_n = eps_n;
   p.mlp = attn ? mlp : 0;
   p.n_out = n_out;
+  p.head_dim = head_dim;
   p.x_out = x_out;
   p.norm_out = wt ? nullptr : out;
   p.out = out;

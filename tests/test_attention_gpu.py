@@ -382,8 +382,26 @@ def test_block_dense_in_one_launch(built_library, E, mlp, n_out, outer, inner):
                 kept, got = block_dense(x, a, blk, norm, last, keep_x=keep)
                 want_x, want = _block_by_modules(x, a, blk, norm, last)
                 assert got.is_contiguous() and got.shape == (outer, inner, n_out if last is not None else E)
+                if last is not None and n_out % E == 0:  # the same split into heads
+                    for d in (32, 64, 128):
+                        split = block_dense(x, a, blk, norm, last, head_dim=d)[1]
+                        assert torch.equal(split, got.view(outer, inner, n_out // E, E // d, d).permute(2, 1, 3, 0, 4))
                 assert close(got, want), (a is None, last is None, (got.double() - want).abs().max().item(), want.abs().max().item())
                 assert (kept is None) if not keep else (torch.equal(kept, x) if a is None else close(kept, want_x))
+
+
+@pytest.mark.parametrize("d,heads", [(32, 4), (64, 3), (128, 2)])
+@pytest.mark.parametrize("V", [8, 16])
+def test_attention_on_split_heads_is_the_packed_one(built_library, V, d, heads):
+    """The same launch on other strides: bit for bit, with and without a permutation of the rows."""
+    seq, bsz = 208, 3
+    vs = _pattern(seq // V, seq, V, 0.8, seed=d)
+    qkv = torch.randn(seq, bsz, 3 * heads * d, device="cuda", generator=torch.Generator("cuda").manual_seed(d)).half()
+    split = qkv.view(seq, bsz, 3, heads, d).permute(2, 1, 3, 0, 4).contiguous()
+    off, col = dev(vs.row_offsets), dev(vs.col_idx)
+    want = sspmm_amd.attention.sparse_attention_packed(None, off, col, qkv, heads, 0.2, V)
+    for rows in (None, torch.randperm(seq // V, device="cuda").int()):
+        assert torch.equal(sspmm_amd.attention.sparse_attention_split(rows, off, col, split, 0.2, V), want)
 
 
 @pytest.mark.parametrize("embed,heads,classes", [(128, 4, 64), (256, 8, 16), (512, 8, 256)])
