@@ -331,6 +331,13 @@ int svc_fill_batched(int count, int groups, const int32_t *mat_rows, int M_total
                      const int32_t *vec_row_ptr, void *workspace, int32_t *vec_col, sspmm_half_t *vec_val,
                      void *hip_stream);
 
+/*
+ * The stack's row pointer cut into the matrices' own, all in one launch: matrix i's entries, from zero, at out_ptr +
+ * mat_groups[i] + i (groups + count entries in all), and bounds[count + 1], the first vector of every matrix and the end.
+ */
+int svc_split_row_ptr(int count, int groups, const int32_t *mat_groups, const int32_t *vec_row_ptr, int32_t *out_ptr, int32_t *bounds,
+                      void *hip_stream);
+
 /* ------------------------------------------------------------------------------------------
  * Row reordering ahead of the SVC: the step the reference runs as `python row_merge_reorder.py`
  * (reference README.md:36) to write its dataset-v8 / dataset-v16 folders, which the harness

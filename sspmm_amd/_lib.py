@@ -45,6 +45,7 @@ SIGNATURES = {
     "svc_count": (_int, [_int, _int, _int, _vp, _vp, _i64, _int, _vp, _vp, _vp]),
     "svc_fill": (_int, [_int, _int, _int, _vp, _vp, _vp, _i64, _int, _vp, _vp, _vp, _vp, _vp]),
     "svc_batched_workspace_bytes": (ctypes.c_size_t, [_int, _int, _i64, _int]),
+    "svc_split_row_ptr": (_int, [_int, _int, _vp, _vp, _vp, _vp, _vp]),
     "svc_count_batched": (_int, [_int, _int, _vp, _int, _int, _int, _vp, _vp, _i64, _int, _vp, _vp, _vp, _vp]),
     "svc_fill_batched": (_int, [_int, _int, _vp, _int, _int, _int, _vp, _vp, _vp, _i64, _int, _vp, _vp, _vp, _vp, _vp]),
     "sspmm_add_layernorm_f16": (_int, [_int, _int, _vp, _vp, _vp, _vp, ctypes.c_float, _vp, _vp]),
@@ -94,6 +95,13 @@ def lib():
 
 _current_device = torch._C._cuda_getDevice if hasattr(torch._C, "_cuda_getDevice") else None
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def stream_of(device):
+    """The handle of `device`'s current stream."""
+    if _raw_stream is not None and device.index is not None:
+        return _raw_stream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 def call(fn, device, *args):

@@ -591,6 +591,14 @@ int sspmm_attention_fm_f16(int batch, int heads, int seq, int head_dim, const ss
   return (int)sspmm::launch_attention_fm(batch, heads, seq, q, k, v, ld, out, ld_out, scale, static_cast<hipStream_t>(hip_stream));
 }
 
+int svc_split_row_ptr(int count, int groups, const int32_t *mat_groups, const int32_t *vec_row_ptr, int32_t *out_ptr, int32_t *bounds,
+                      void *hip_stream) {
+  if (count < 0 || groups < 0 || (int64_t)count + groups >= (1ll << 31) - 512) return kInvalid;
+  if (count == 0) return 0;
+  if (!mat_groups || !vec_row_ptr || !out_ptr || !bounds) return kInvalid;
+  return (int)sspmm::launch_svc_split_row_ptr(count, groups, mat_groups, vec_row_ptr, out_ptr, bounds, static_cast<hipStream_t>(hip_stream));
+}
+
 size_t svc_coo_workspace_bytes(int64_t n) { return sspmm::coo_workspace_bytes(n); }
 
 int svc_coo_to_csr(int M, int K, int64_t n, const int32_t *coo_row, const int32_t *coo_col, int32_t *row_ptr,

@@ -39,6 +39,10 @@ bool svc_direct(int order, int K);
 // Total workspace bytes; optional byte offsets of the pos, table and class-list views.
 size_t svc_workspace_layout(int64_t nnz, int m_vec, size_t *off_pos, size_t *off_tables, size_t *off_lists);
 
+// The row pointer of a stack cut into the matrices' own (see the kernel).
+hipError_t launch_svc_split_row_ptr(int count, int groups, const int32_t *mat_groups, const int32_t *vec_row_ptr, int32_t *out_ptr,
+                                    int32_t *bounds, hipStream_t stream);
+
 // group_rows[groups + 1] and mat_groups[count + 1] of a stack of matrices from mat_rows[count + 1] (device arrays).
 hipError_t launch_svc_group_rows(int count, int V, int groups, const int32_t *mat_rows, int32_t *group_rows,
                                  int32_t *mat_groups, hipStream_t stream);

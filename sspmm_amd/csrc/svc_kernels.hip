@@ -275,6 +275,29 @@ __global__ __launch_bounds__(1024) void svc_group_rows_kernel(int count, int V, 
   }
 }
 
+// The row pointer of a stack cut into the matrices' own: out_ptr[mat_groups[i] + i + j] = entry j of matrix i's, from zero, and
+// bounds[i] = its first vector (bounds[count] the end).  One thread per entry; the matrix by bisection (a few steps).
+__global__ __launch_bounds__(256) void svc_split_row_ptr_kernel(int count, int groups, const int32_t *mat_groups, const int32_t *vec_row_ptr,
+                                                                int32_t *out_ptr, int32_t *bounds) {
+  const int at = blockIdx.x * 256 + threadIdx.x;
+  if (at <= count) bounds[at] = vec_row_ptr[mat_groups[at]];
+  if (at >= groups + count) return;
+  int lo = 0, hi = count - 1;  // the last matrix i with mat_groups[i] + i <= at
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (mat_groups[mid] + mid <= at) lo = mid;
+    else hi = mid - 1;
+  }
+  out_ptr[at] = vec_row_ptr[at - lo] - vec_row_ptr[mat_groups[lo]];
+}
+
+hipError_t launch_svc_split_row_ptr(int count, int groups, const int32_t *mat_groups, const int32_t *vec_row_ptr, int32_t *out_ptr,
+                                    int32_t *bounds, hipStream_t stream) {
+  hipLaunchKernelGGL(svc_split_row_ptr_kernel, dim3((groups + count + 1 + 255) / 256), dim3(256), 0, stream, count, groups, mat_groups,
+                     vec_row_ptr, out_ptr, bounds);
+  return hipGetLastError();
+}
+
 // Class of a vector-row group by its key bound: which kernel instance handles it.
 __device__ __forceinline__ bool in_class(int bound, int lo, int hi) { return bound > lo && bound <= hi; }
 

@@ -77,31 +77,44 @@ class SvcBatch:
         self.V, self.rows, self.cols = V, rows, cols
         self._groups = groups_of            # host: first group of every matrix, [count + 1]
         self._mat_groups = mat_groups       # the same on the device, or None
-        self._bounds = None                 # (vec_row_ptr, its version, first vector of every matrix and the end)
+        self._split = None                  # (vec_row_ptr, its version, first vector of every matrix and the end, row pointers)
         self.vec_row_ptr, self.vec_col, self.vec_val = vec_row_ptr, vec_col, vec_val
 
     def __len__(self):
         return len(self.rows)
 
-    def _extent(self, i, ptr):
-        # One read-back brings the extents of all matrices: a gather, a copy and a wait per matrix made up two thirds of a
-        # pass over twenty (1.2 ms, 0.45 ms with one).  They are read again whenever the row pointer is another tensor
-        # or has been written since; a tensor that does not record writes has them read for every matrix.
+    def _taken(self, i, g0, g1):
+        # (row pointer from zero, first vector, end) of matrix i, whose groups are g0 .. g1 - 1.  One launch rebases
+        # the row pointers of all matrices and one read-back brings their extents: twenty matrices one by one took a
+        # launch each (0.4 ms a pass, 0.3 ms like this), and with a read-back each 1.2 ms.  Both are done again whenever the
+        # row pointer is another tensor or has been written since.  A row pointer is handed out once (what a caller
+        # writes into it is not in the next one), and on the stream that it was allocated on.  Host tensors and ones that
+        # do not record writes go one by one.
         whole = self.vec_row_ptr
-        if self._mat_groups is None or whole.is_inference():
-            return (int(x) for x in ptr[[0, -1]].tolist())
-        if self._bounds is None or self._bounds[0] is not whole or self._bounds[1] != whole._version:
-            self._bounds = (whole, whole._version, whole.index_select(0, self._mat_groups).tolist())
-        return self._bounds[2][i], self._bounds[2][i + 1]
+        if self._mat_groups is None or whole.is_inference() or not whole.is_cuda:
+            ptr = whole[g0:g1 + 1]
+            lo, hi = (int(x) for x in ptr[[0, -1]].tolist())
+            return ptr - lo, lo, hi
+        stream = _lib.stream_of(whole.device)
+        if self._split is None or self._split[0] is not whole or self._split[1] != whole._version:
+            count, groups = len(self), int(self._groups[-1])
+            own = torch.empty(groups + count, dtype=torch.int32, device=whole.device)
+            bounds = torch.empty(count + 1, dtype=torch.int32, device=whole.device)
+            _lib.check(_lib.call(_lib.lib().svc_split_row_ptr, whole.device, count, groups, self._mat_groups.data_ptr(), whole.data_ptr(),
+                                 own.data_ptr(), bounds.data_ptr()), "svc_split_row_ptr")
+            sizes = [int(self._groups[j + 1] - self._groups[j]) + 1 for j in range(count)]
+            self._split = (whole, whole._version, bounds.tolist(), dict(enumerate(own.split(sizes))), stream)
+        _, _, bounds, own, own_stream = self._split
+        lo, hi = bounds[i], bounds[i + 1]
+        mine = own.pop(i, None) if stream == own_stream else None
+        return (whole[g0:g1 + 1] - lo if mine is None else mine), lo, hi
 
     def matrix(self, i):
         g0, g1 = int(self._groups[i]), int(self._groups[i + 1])
         if g1 < g0:
             raise IndexError("matrix %d of %d" % (i, len(self)))
-        ptr = self.vec_row_ptr[g0:g1 + 1]
-        lo, hi = self._extent(i, ptr)   # (the views need their extent on the host)
-        return SvcResult(ptr - lo, self.vec_col[lo:hi], None if self.vec_val is None else self.vec_val[lo * self.V:hi * self.V],
-                         hi - lo)
+        ptr, lo, hi = self._taken(i, g0, g1)   # (the views need their extent on the host)
+        return SvcResult(ptr, self.vec_col[lo:hi], None if self.vec_val is None else self.vec_val[lo * self.V:hi * self.V], hi - lo)
 
     def to_host(self):
         ptr = self.vec_row_ptr.cpu().numpy()

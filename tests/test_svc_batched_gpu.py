@@ -145,3 +145,25 @@ def test_extents_follow_the_row_pointer():
     for i in (3, -1):
         with pytest.raises(IndexError):
             b.matrix(i)
+
+
+@pytest.mark.parametrize("rows", [[16], [0, 0], [0, 24, 0, 0, 7, 300, 0], [8] * 70])
+def test_row_pointers_of_a_stack_are_each_matrix_s_own(built_library, rows):
+    """Empty matrices at either end and in a row, more matrices than a wave has lanes; a second call and one on another
+    stream get arrays of their own, and what a caller writes stays with that caller."""
+    rng = np.random.default_rng(len(rows))
+    mats = []
+    for M in rows:
+        ptr = np.concatenate([[0], np.cumsum(rng.integers(0, 9, M))]).astype(np.int32)
+        mats.append((M, 512, ptr, np.concatenate([np.sort(rng.choice(512, n, replace=False)) for n in np.diff(ptr)] + [np.zeros(0)])
+                     .astype(np.int32), None))
+    at, K, ptr, col, _ = sspmm_amd.stack_csr(mats)
+    batch = sspmm_amd.svc_batched(at, K, torch.from_numpy(ptr).cuda(), torch.from_numpy(col).cuda(), None, 8)
+    want = [p for p, _, _ in batch.to_host()]
+    first = [batch.matrix(i).vec_row_ptr for i in range(len(rows))]
+    for got, w in zip(first, want):
+        assert got.cpu().tolist() == w.tolist()
+        got.fill_(-1)
+    with torch.cuda.stream(torch.cuda.Stream()):
+        other = [batch.matrix(i).vec_row_ptr.cpu().tolist() for i in range(len(rows))]
+    assert other == [w.tolist() for w in want] == [batch.matrix(i).vec_row_ptr.cpu().tolist() for i in range(len(rows))]
