@@ -21,8 +21,8 @@
 // (insertion index << 32 | key): a later key that is displaced by an earlier one resumes its own
 // probe sequence behind that slot.  So one thread per key inserts a whole phase at once.
 //
-// One workgroup owns one vector-row group.  The list and the table live in LDS (64-thread groups
-// for up to 306 keys, 256 threads up to 1228, 1024 threads up to 4914) or, beyond that, in the
+// One workgroup owns one vector-row group.  The list and the table live in LDS (64 threads,
+// or 256 beside wider groups, for up to 306 keys, 1024 threads up to 4914) or, beyond that, in the
 // caller's workspace.
 //
 // Which phase does what.  The caller sizes the outputs from svc_count's row pointer, so the count
@@ -1412,7 +1412,7 @@ hipError_t launch_svc_fill(const SvcArgs &args, int order, const uint16_t *csr_v
     // Everything on the caller's stream: either no group can be larger than the small class, or the matrix has so
     // few groups that each gets a CU of its own in one launch of the wide workgroups (which then also take the
     // small groups); a fork and a join of a helper stream would cost more than they hide.
-    if (!medium)
+    if (!medium)  // (one wave per group: 16384 x 290, 8 a row, 81 us; with four 84)
       e = launch_fast_class<64, true>(a, min(m_vec, 32 * cus), 0, 0, kSmallKeys, 512, key_bits, stream);
     else
       e = launch_fast_class<1024, true>(a, m_vec, large ? 2 : 1, 0, kLargeKeys, 8192, key_bits, stream, 81 * 1024);
@@ -1428,7 +1428,10 @@ hipError_t launch_svc_fill(const SvcArgs &args, int order, const uint16_t *csr_v
   if ((e = fork_streams(ss, stream, st, 1)) != hipSuccess) return e;
   // (from here on the helper is joined back into the caller's stream whatever happens)
   e = launch_fast_class<1024, true>(a, min(m_vec, cus), large ? 2 : 1, 1, kLargeKeys, 8192, key_bits, st[0], 81 * 1024);
-  if (e == hipSuccess) e = launch_fast_class<64, true>(a, min(m_vec, 32 * cus), 0, 0, kSmallKeys, 512, key_bits, st[1]);
+  // (four waves per small group where there are wider ones too: groups of 64 to 306 keys, whose phases are chains of
+  // placements, halve their chain and those of a few keys lose little.  Power-law matrices, 64 / 256 / 512 threads:
+  // 4096 x 4096, 16 a row, 155 / 137 / 142 us; 16384 x 1024, 32 a row, 154 / 139 / 198; 16384 x 16384 level)
+  if (e == hipSuccess) e = launch_fast_class<256, true>(a, min(m_vec, 8 * cus), 0, 0, kSmallKeys, 512, key_bits, st[1]);
   rare_classes(st[1]);
   const hipError_t ej = join_streams(ss, stream, 1);
   return e != hipSuccess ? e : ej;

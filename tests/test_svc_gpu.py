@@ -394,3 +394,21 @@ def test_groups_whose_columns_all_fit_their_last_table(oracle, built_library, V,
     assert np.array_equal(first, np.sort(first))
     r = sspmm_amd.svc(dev(csr.row_ptr), dev(csr.col_ind), None, csr.M, csr.K, V)
     assert np.array_equal(r.vec_col.cpu().numpy(), vcol)
+
+
+@pytest.mark.parametrize("V", [8, 16])
+def test_small_groups_beside_wide_ones(oracle, built_library, V):
+    """Groups of 0 to 306 columns (around the sizes of a wave, of the table sizes and of the class) among hundreds, with a few
+    of more: the small class then runs with four waves per group on a stream of its own."""
+    rng = np.random.default_rng(V)
+    sizes = np.resize([0, 1, 4, 5, 19, 20, 63, 64, 65, 76, 77, 127, 128, 255, 256, 257, 305, 306, 307, 400], 320)
+    ptr, cols = [0], []
+    for n in sizes:
+        names = rng.choice(40000, n, replace=False)
+        for part in np.array_split(names, V):
+            row = np.unique(np.concatenate([part, rng.choice(names, min(n, 3))]) if n else part)
+            cols.append(row)
+            ptr.append(ptr[-1] + row.size)
+    cols = np.concatenate(cols).astype(np.int32)
+    csr = synth.Csr(sizes.size * V, 40000, np.array(ptr, np.int32), cols, rng.standard_normal(cols.size).astype(np.float16))
+    _compare_with_oracle(oracle, csr, V)
