@@ -428,3 +428,25 @@ def test_encoder_in_two_launches_per_block_matches_the_modules(built_library, em
     scale = modules.float().pow(2).mean().sqrt()  # (as above)
     assert (fused.float() - modules.float()).abs().max() <= 1e-2 * scale
     assert (norms.float() - modules.float()).abs().max() <= 1e-2 * scale
+
+
+@pytest.mark.parametrize("V", [8, 16])
+@pytest.mark.parametrize("scaler", [0.3, -0.7])
+def test_softmax_with_masked_entries(built_library, V, scaler):
+    """Entries that a mask of the far infinity (or of the type's far end) takes out, in rows around what a wave keeps in registers
+    (256 and 512 vectors), some of which keep one entry: against float64, half an fp16 ulp of a result up to 1 and what
+    the base-2 exponential adds in fp32 (2^-20 relative)."""
+    rng = np.random.default_rng(V)
+    lens = np.array([1, 2, 63, 64, 65, 255, 256, 257, 511, 512, 513, 700])
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    x = (rng.standard_normal((off[-1], V)) * 5).astype(np.float16)
+    masked = rng.random(x.shape) < 0.5
+    masked[off[:-1]] = False
+    far = -np.sign(scaler) * np.where(rng.random(x.shape) < 0.5, np.inf, 65504)
+    x = np.where(masked, far, x).astype(np.float16)
+    got = sspmm_amd.csr_softmax(None, dev(off), dev(x.reshape(-1)), scaler, V).cpu().numpy().reshape(-1, V).astype(np.float64)
+    for i in range(len(lens)):
+        z = x[off[i]:off[i + 1]].astype(np.float64) * scaler
+        e = np.exp(z - z.max(axis=0))
+        want = e / e.sum(axis=0)
+        assert (np.abs(got[off[i]:off[i + 1]] - want) <= want * (2.0 ** -11 + 2.0 ** -20) + 2.0 ** -24).all()
