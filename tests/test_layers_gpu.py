@@ -82,6 +82,12 @@ def test_feature_major_add_layernorm_matches_torch(built_library, H, T, residual
         assert (odd.float() - want[:, :T - 1]).abs().max().item() <= 4e-3 * max(1.0, want.abs().max().item())
 
 
+@pytest.mark.parametrize("H", [127, 128, 129, 512, 513, 640, 769, 1023, 1025])
+@pytest.mark.parametrize("T", [4, 76])
+def test_feature_major_add_layernorm_at_the_edges_of_its_kernels(built_library, H, T):
+    test_feature_major_add_layernorm_matches_torch(built_library, H, T, True)
+
+
 def _attention_reference(q, k, v, batch, heads, seq, scale):
     """fp32 attention of feature-major [heads * d, batch * seq] operands, written out with plain matmuls."""
     d = q.shape[0] // heads
