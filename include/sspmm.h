@@ -390,14 +390,15 @@ int sspmm_add_layernorm_rows_f16(int outer, int inner, int E, const sspmm_half_t
  *   s  = attn Wo^T + bo + x            n = LayerNorm2(s)
  *   x' = (n W1^T + b1) W2^T + b2 + x   h = LayerNormN(x')      (the next block's first, or the model's last)
  * out = h Wt^T + bt (n_out features; the next block's input projection, or the head), or h itself where wt is NULL, and
- * x' into x_out unless that is NULL.  attn NULL: x' = x, and what only leads to it (wo .. b2, eps2, mlp) is not
+ * x' into x_out unless that is NULL.  With pos [outer, E] x is an embedding and fp16(x * x_scale) + pos, rounded to fp16
+ * again, stands in its place.  attn NULL: x' = x, and what only leads to it (wo .. b2, eps2, mlp) is not
  * looked at.  out is [outer, inner, n_out], or with head_dim = 32, 64 or 128 (n_out then a multiple of E) split into heads as
  * sspmm_sparse_attention_heads_f16 reads them best: [n_out / E, inner, E / head_dim, outer, head_dim].  n and the hidden features are rounded to fp16, sums are fp32.  The weight matrices are packed (below): wo
  * [E, E] and w2 [E, mlp] in groups of E / 4 rows, w1 [mlp, E] and wt [n_out, E] of 64; biases, gammas and betas may be NULL.  Row (i, j) of x is at x + i * x_outer + j * x_inner elements (multiples
  * of 8), everything else is dense; 16-byte aligned pointers.  E = 128, 256 or 512, mlp a multiple of 256, n_out of 64.
  */
-int sspmm_block_dense_f16(int outer, int inner, int E, const sspmm_half_t *x, int64_t x_outer, int64_t x_inner, const sspmm_half_t *attn,
-                          const sspmm_half_t *wo, const sspmm_half_t *bo, const sspmm_half_t *gamma2, const sspmm_half_t *beta2,
+int sspmm_block_dense_f16(int outer, int inner, int E, const sspmm_half_t *x, int64_t x_outer, int64_t x_inner, const sspmm_half_t *pos,
+                          float x_scale, const sspmm_half_t *attn, const sspmm_half_t *wo, const sspmm_half_t *bo, const sspmm_half_t *gamma2, const sspmm_half_t *beta2,
                           float eps2, int mlp, const sspmm_half_t *w1, const sspmm_half_t *b1, const sspmm_half_t *w2,
                           const sspmm_half_t *b2, const sspmm_half_t *gamma_n, const sspmm_half_t *beta_n, float eps_n, int n_out, int head_dim,
                           const sspmm_half_t *wt, const sspmm_half_t *bt, sspmm_half_t *x_out, sspmm_half_t *out, void *hip_stream);

@@ -224,14 +224,15 @@ def pack_weights(linears, rows_per_wave):
     return packed.split(sizes)
 
 
-def block_dense(x, attn, block, norm, tail=None, keep_x=False, packed=None, head_dim=0):
+def block_dense(x, attn, block, norm, tail=None, keep_x=False, packed=None, head_dim=0, pos=None, scale=1.0):
     """(x', out): everything between the attention of `block` and the next one's in one launch, on token-major activations
     [seq, batch, embed] fp16:
         s = out_proj(attn) + x, x' = linear2(linear1(layer_norm2(s))) + x, h = norm(x'), out = tail(h) or h itself.
     attn None: x' = x and `block` is not looked at.  x may be a view with strides of its own in the first two dimensions,
     attn is dense, and so are the results.  x' is only returned with keep_x.  packed: pack_weights of out_proj, linear1 and
     linear2 (where there is attn) and tail (where there is one), in this order.  head_dim: out as
-    [tail.out_features / embed, batch, embed / head_dim, seq, head_dim], for sparse_attention_split."""
+    [tail.out_features / embed, batch, embed / head_dim, seq, head_dim], for sparse_attention_split.  pos
+    [seq, embed]: x is an embedding, and (x * scale) + pos stands in its place, each rounded to fp16."""
     outer, inner, E = x.shape
     n_out = 0 if tail is None else tail.out_features
     shape = (n_out // E, inner, E // head_dim, outer, head_dim) if head_dim else (outer, inner, n_out or E)
@@ -249,8 +250,8 @@ def block_dense(x, attn, block, norm, tail=None, keep_x=False, packed=None, head
         own = (packed[0].data_ptr(), _ptr(proj.bias), _ptr(ln.weight), _ptr(ln.bias), float(ln.eps), up.out_features,
                packed[1].data_ptr(), _ptr(up.bias), packed[2].data_ptr(), _ptr(down.bias))
     last = (None, None) if tail is None else (packed[-1].data_ptr(), _ptr(tail.bias))
-    rc = _lib.call(_lib.lib().sspmm_block_dense_f16, x.device, outer, inner, E, x.data_ptr(), stride[0], stride[1], _ptr(attn),
-                   *own, _ptr(norm.weight), _ptr(norm.bias), float(norm.eps), n_out, head_dim, *last, _ptr(kept), out.data_ptr())
+    rc = _lib.call(_lib.lib().sspmm_block_dense_f16, x.device, outer, inner, E, x.data_ptr(), stride[0], stride[1], _ptr(pos), float(scale),
+                   _ptr(attn), *own, _ptr(norm.weight), _ptr(norm.bias), float(norm.eps), n_out, head_dim, *last, _ptr(kept), out.data_ptr())
     _lib.check(rc, "sspmm_block_dense_f16")
     return kept, out
 
@@ -376,11 +377,15 @@ class SparseAttentionEncoder(torch.nn.Module):
 
     def forward(self, tokens, dense_masks=None):
         """tokens: int [batch, seq] -> [seq, batch, num_class]."""
-        out = self.encoder(tokens) * (self.embed_dim ** 0.5)
+        out, scale = self.encoder(tokens), self.embed_dim ** 0.5
+        if dense_masks is None and out.dim() == 3:
+            x, pe = out.transpose(0, 1), self.pe[:tokens.size(1)].to(out.dtype)
+            if pe.shape == (x.size(0), 1, x.size(2)) and _rows_operand(pe) and pe.is_contiguous() and pe.device == x.device and \
+                    self._fused_norms_apply(x) and self._fused_blocks_apply(x):
+                return self._fused_blocks(x, pe, scale)
+        out = out * scale
         out = out.transpose(0, 1) + self.pe[:tokens.size(1)].to(out.dtype)
         if dense_masks is None and self._fused_norms_apply(out):
-            if self._fused_blocks_apply(out):
-                return self._fused_blocks(out)
             return self.linear(self._blocks_with_fused_norms(out))
         for i, blk in enumerate(self.blocks):
             out = blk(out, None if dense_masks is None else dense_masks[i])
@@ -417,8 +422,8 @@ class SparseAttentionEncoder(torch.nn.Module):
             _plain_linear(b.linear1, x, E, None, 256) and _plain_linear(b.linear2, x, b.linear1.out_features, E, 64)
             for b in self.blocks)
 
-    def _fused_blocks(self, x):
-        """Two launches per block: its attention, and all that follows up to the next block's projection (or the head)."""
+    def _fused_blocks(self, x, pe, scale):
+        """(x * scale) + pe through the blocks and the head.  Two launches per block: its attention, and all that follows up to the next block's projection (or the head)."""
         E, blocks = x.size(-1), list(self.blocks)
         head = _plain_linear(self.linear, x, E, None, 64)
         linears, rows = [blocks[0].in_proj], [64]
@@ -432,7 +437,7 @@ class SparseAttentionEncoder(torch.nn.Module):
             # (in the pattern's own order: the longest rows last, which row_indices asks for, cost 1 to 4 %)
             return sparse_attention_split(None, blk.row_offsets, blk.column_indices, qkv, float(qkv.size(-1)) ** -0.5, blk.vec_length)
 
-        _, qkv = block_dense(x, None, None, blocks[0].layer_norm1, blocks[0].in_proj, packed=packed[:1], head_dim=E // blocks[0].num_heads)
+        x, qkv = block_dense(x, None, None, blocks[0].layer_norm1, blocks[0].in_proj, True, packed[:1], E // blocks[0].num_heads, pe, scale)
         for i, (blk, nxt) in enumerate(zip(blocks, blocks[1:])):
             x, qkv = block_dense(x, attention(blk, qkv), blk, nxt.layer_norm1, nxt.in_proj, True, packed[1 + 4 * i:5 + 4 * i],
                                  E // nxt.num_heads)

@@ -18,6 +18,8 @@ struct BlockDenseArgs {
   long long tokens, inner;
   const uint16_t *x;
   long long x_outer, x_inner;
+  const uint16_t *pos;                       // nullable: x is an embedding, fp16(x * x_scale) + pos[token / inner] in its place
+  float x_scale;
   const uint16_t *attn;                      // nullable, and the next two lines with it
   const uint16_t *wo, *bo, *gamma2, *beta2;
   const uint16_t *w1, *b1, *w2, *b2;

@@ -240,7 +240,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
 
   // the lane's share of x, fetched once
   half8 x[TT][NT / 2];
-  if (p.x_inner == E && p.x_outer == p.inner * E) {
+  if (p.x_inner == E && p.x_outer == p.inner * E && !p.pos) {
 #pragma unroll
     for (int t = 0; t < TT; ++t) load_row<NT>(x[t], p.x + (t0 + min(t * 16 + m, left - 1)) * E + first);
   } else {
@@ -250,6 +250,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
     for (int t = 0; t < TT; ++t) {
       const uint32_t r = r0 + (uint32_t)min(t * 16 + m, left - 1), q = r / (uint32_t)p.inner;
       load_row<NT>(x[t], p.x + (q0 + q) * p.x_outer + (long long)(r - q * (uint32_t)p.inner) * p.x_inner + first);
+      if (p.pos) {  // (uniform) fp16(x * scale) + pos, rounded as an activation in between
+        half8 at[NT / 2];
+        load_row<NT>(at, p.pos + (q0 + q) * E + first);
+#pragma unroll
+        for (int j = 0; j < NT / 2; ++j) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) x[t][j][i] = (_Float16)((float)x[t][j][i] * p.x_scale);
+          x[t][j] += at[j];
+        }
+      }
     }
   }
 

@@ -535,8 +535,8 @@ int sspmm_block_pack_f16(int count, const sspmm_half_t *const *src, const int32_
   return 0;
 }
 
-int sspmm_block_dense_f16(int outer, int inner, int E, const sspmm_half_t *x, int64_t x_outer, int64_t x_inner, const sspmm_half_t *attn,
-                          const sspmm_half_t *wo, const sspmm_half_t *bo, const sspmm_half_t *gamma2, const sspmm_half_t *beta2,
+int sspmm_block_dense_f16(int outer, int inner, int E, const sspmm_half_t *x, int64_t x_outer, int64_t x_inner, const sspmm_half_t *pos,
+                          float x_scale, const sspmm_half_t *attn, const sspmm_half_t *wo, const sspmm_half_t *bo, const sspmm_half_t *gamma2, const sspmm_half_t *beta2,
                           float eps2, int mlp, const sspmm_half_t *w1, const sspmm_half_t *b1, const sspmm_half_t *w2,
                           const sspmm_half_t *b2, const sspmm_half_t *gamma_n, const sspmm_half_t *beta_n, float eps_n, int n_out, int head_dim,
                           const sspmm_half_t *wt, const sspmm_half_t *bt, sspmm_half_t *x_out, sspmm_half_t *out, void *hip_stream) {
@@ -546,7 +546,7 @@ int sspmm_block_dense_f16(int outer, int inner, int E, const sspmm_half_t *x, in
   if (attn && (!wo || !w1 || !w2)) return kInvalid;
   if (head_dim != 0 && ((head_dim != 32 && head_dim != 64 && head_dim != 128) || n_out % E)) return kInvalid;
   uintptr_t bits = 0;
-  for (const sspmm_half_t *q : {x, attn, wo, bo, gamma2, beta2, w1, b1, w2, b2, gamma_n, beta_n, wt, bt, (const sspmm_half_t *)x_out,
+  for (const sspmm_half_t *q : {x, pos, attn, wo, bo, gamma2, beta2, w1, b1, w2, b2, gamma_n, beta_n, wt, bt, (const sspmm_half_t *)x_out,
                                 (const sspmm_half_t *)out})
     bits |= reinterpret_cast<uintptr_t>(q);
   if (bits % 16) return kInvalid;
@@ -556,6 +556,8 @@ int sspmm_block_dense_f16(int outer, int inner, int E, const sspmm_half_t *x, in
   p.x = x;
   p.x_outer = x_outer;
   p.x_inner = x_inner;
+  p.pos = pos;
+  p.x_scale = x_scale;
   p.attn = attn;
   p.wo = wo;
   p.bo = bo;

@@ -382,6 +382,14 @@ def test_block_dense_in_one_launch(built_library, E, mlp, n_out, outer, inner):
                 kept, got = block_dense(x, a, blk, norm, last, keep_x=keep)
                 want_x, want = _block_by_modules(x, a, blk, norm, last)
                 assert got.is_contiguous() and got.shape == (outer, inner, n_out if last is not None else E)
+                if a is None:  # an embedding in the place of x: the same values as torch makes of it
+                    pos = rnd(outer, 1, E)
+                    embedded = x * 16.0 + pos
+                    made, from_table = block_dense(x, a, blk, norm, last, keep_x=True, pos=pos, scale=16.0)
+                    assert torch.equal(made, embedded) and torch.equal(from_table, block_dense(embedded, a, blk, norm, last)[1])
+                    # (torch rounds the scaled product to fp16 once, the kernel to fp32 first: an ulp of it apart at a tie)
+                    other = block_dense(x, a, blk, norm, last, keep_x=True, pos=pos, scale=11.3)[0]
+                    assert ((other.float() - (x * 11.3 + pos).float()).abs() <= 2 ** -10 * (x.float() * 11.3).abs() + 2 ** -10 * other.float().abs()).all()
                 if last is not None and n_out % E == 0:  # the same split into heads
                     for d in (32, 64, 128):
                         split = block_dense(x, a, blk, norm, last, head_dim=d)[1]
