@@ -17,13 +17,14 @@
 // four lane groups make 64 consecutive bytes.
 //
 // The weights a workgroup streams from L2 are 1.6 MB at 256 features and 1024 hidden ones, 25k cycles at the 64 bytes a
-// cycle of a CU, whatever TM, and the products 384 cycles per token.  The loads of the next D units (eight 16-byte
-// loads of a wave each) are in flight throughout, also across the products' boundaries.  The matrices are packed by
+// cycle of a CU, whatever TM, and the products 384 cycles per token.  The loads of the next two units (eight 16-byte
+// loads of a wave each) are in flight throughout, also across the products' boundaries; four units, at 64 registers more, were
+// level at best and slower where they make the compiler spill (512 features, 32768 tokens: 164 us, with two 149).  The matrices are packed by
 // a launch of their own first (7 us for the 6.7 MB of a model of four blocks), so that a load instruction reads 1 KB in a
 // row: from torch's layout it reads 64 bytes of each of sixteen rows, which lie 512 to 2048 bytes apart on a few of the L2's
 // channels, and 32 tokens per workgroup took 61 us instead of 27 (8192 tokens).
 //
-// 256 features, 1024 hidden, 768 out, with the LayerNorms: 8192 tokens 26 us, 32768 tokens 58 us (0.9 PFLOP/s), against
+// 256 features, 1024 hidden, 768 out, with the LayerNorms: 8192 tokens 24 us, 32768 tokens 59 us (0.9 PFLOP/s), against
 // 104 (the host) and 121 for the four library products and two LayerNorm launches.  What is left is the chain of products
 // and LayerNorms of one workgroup (27 us with the card to itself, 64 tokens), the stream of the weights, and for the
 // large sizes the vector instructions between the products.
@@ -210,11 +211,11 @@ __device__ __forceinline__ void layer_norm(floatx4 (&v)[TT][NJ], const uint16_t 
   }
 }
 
-constexpr int block_waves(int E, int TM) { return TM == 64 && E < 512 ? 2 : 1; }  // per SIMD
+constexpr int block_waves(int E, int TM) { return TM == 16 || (TM == 64 && E < 512) ? 2 : 1; }  // per SIMD
 
 template <int E, int TM, bool ATTN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves(E, TM), block_waves(E, TM)))) void block_dense_kernel(const BlockDenseArgs p) {
-  constexpr int NT = E / 64, TT = TM / 16, D = E == 128 || block_waves(E, TM) == 2 ? 2 : 4;
+  constexpr int NT = E / 64, TT = TM / 16, D = 2;
   constexpr int kPitchA = E * 2 + 16, kPitchH = kChunk * 2 + 16;
   __shared__ __align__(16) unsigned char act[TM * kPitchA];  // attention's output, then n, then h
   __shared__ __align__(16) unsigned char hid[TM * kPitchH];  // kChunk hidden features
@@ -436,8 +437,12 @@ hipError_t launch(const BlockDenseArgs &p, hipStream_t stream) {
 // passes run under the other's products.  32768 tokens of 256 features: 58 us, with one workgroup per CU 69, with one of
 // 128 tokens 64; of 128 features 32, 39 and 35.  Up to 8192 tokens those are at most 128 workgroups, and 32 tokens give every
 // CU one: 8192 tokens of 128, 256, 512 features 15, 26, 56 us against 18, 30, 73; 10000 tokens 25, 43, 101 against 18, 31, 73.
+// Up to 4096 tokens 16 do the same, and a workgroup's chain of products and LayerNorms is shorter: 2048 tokens 10.0, 17.5, 43 us
+// against 12.3, 20.1, 48 with 32 (without attention 4.6, 7.4, 17 against 5.6, 9.2, 20), 4096 tokens 10.9, 19.3, 46 against 12.6, 21.2,
+// 49; 8192 tokens without attention 7.6, 14.2, 36 against 6.6, 11.1, 25.
 template <int E>
 hipError_t launch_for_width(const BlockDenseArgs &p, hipStream_t stream) {
+  if (p.tokens <= 256 * 16) return launch<E, 16>(p, stream);
   return p.tokens <= 256 * 32 ? launch<E, 32>(p, stream) : launch<E, 64>(p, stream);
 }
 

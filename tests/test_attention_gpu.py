@@ -359,9 +359,9 @@ def _block_by_modules(x, attn, blk, norm, tail):
 
 
 @pytest.mark.parametrize("E,mlp,n_out", [(128, 256, 64), (128, 1024, 384), (256, 256, 320), (256, 1024, 768), (512, 512, 1536)])
-@pytest.mark.parametrize("outer,inner", [(1, 1), (33, 1), (127, 3), (2731, 3)])
+@pytest.mark.parametrize("outer,inner", [(1, 1), (33, 1), (127, 3), (4096, 1), (4097, 1), (2731, 3)])
 def test_block_dense_in_one_launch(built_library, E, mlp, n_out, outer, inner):
-    """Every width and tile of tokens (32, 64) with a last tile that is not full, output widths that leave waves without a
+    """Every width and tile of tokens (16, 32, 64) with a last tile that is not full, output widths that leave waves without a
     chunk, x dense and batch-major, with and without attention, tail and x'.  Roundings to fp16 at other places (a
     hidden activation an ulp away, 2^-11) stay below 4 * 2^-11 of the result's size after the sums behind them."""
     from sspmm_amd.attention import SparseAttentionBlock, block_dense
