@@ -64,6 +64,14 @@ def svc(row_ptr, col_ind, csr_val, M, K, V, order="cpython", exact_size=True):
     return SvcResult(vec_row_ptr, vec_col, vec_val, nvec)
 
 
+class _RowPointer:
+    """The row pointer of a stack and what matrix() may keep of it: as long as it is `alone`, nobody but the batch (and
+    its shallow copies, which share this object) has the tensor, so nobody can have written it."""
+
+    def __init__(self, whole):
+        self.whole, self.alone, self.split = whole, False, None
+
+
 class SvcBatch:
     """The SVC of a stack of matrices (svc_batched): device arrays over the whole stack and views per matrix.
 
@@ -71,42 +79,55 @@ class SvcBatch:
     after the other and are sized for the bound nvec <= nnz (what lies behind vec_row_ptr[-1] vectors is
     unspecified).  `matrix(i)` returns matrix i's SvcResult as device views (its row pointer rebased to zero);
     `to_host()` brings everything over in one go and returns one (vec_row_ptr, vec_col, vec_val) numpy triple per
-    matrix."""
+    matrix.  Both go by the row pointer as it is at the call, whoever wrote it and however: once `vec_row_ptr` has been
+    read or assigned, matrix(i) reads its extent back every time."""
 
     def __init__(self, V, rows, cols, groups_of, vec_row_ptr, vec_col, vec_val, mat_groups=None):
         self.V, self.rows, self.cols = V, rows, cols
         self._groups = groups_of            # host: first group of every matrix, [count + 1]
         self._mat_groups = mat_groups       # the same on the device, or None
-        self._split = None                  # (vec_row_ptr, its version, first vector of every matrix and the end, row pointers)
-        self.vec_row_ptr, self.vec_col, self.vec_val = vec_row_ptr, vec_col, vec_val
+        self._row_ptr = _RowPointer(vec_row_ptr)
+        self.vec_col, self.vec_val = vec_col, vec_val
+
+    @property
+    def vec_row_ptr(self):
+        p = self._row_ptr
+        p.alone, p.split = False, None
+        return p.whole
+
+    @vec_row_ptr.setter
+    def vec_row_ptr(self, whole):
+        self._row_ptr = _RowPointer(whole)
 
     def __len__(self):
         return len(self.rows)
 
     def _taken(self, i, g0, g1):
-        # (row pointer from zero, first vector, end) of matrix i, whose groups are g0 .. g1 - 1.  One launch rebases
-        # the row pointers of all matrices and one read-back brings their extents: twenty matrices one by one took a
-        # launch each (0.4 ms a pass, 0.3 ms like this), and with a read-back each 1.2 ms.  Both are done again whenever the
-        # row pointer is another tensor or has been written since.  A row pointer is handed out once (what a caller
-        # writes into it is not in the next one), and on the stream that it was allocated on.  Host tensors and ones that
-        # do not record writes go one by one.
-        whole = self.vec_row_ptr
-        if self._mat_groups is None or whole.is_inference() or not whole.is_cuda:
+        # (row pointer from zero, first vector, end) of matrix i, whose groups are g0 .. g1 - 1.  Of a row pointer that
+        # svc_batched made and nobody else has seen, one launch rebases all matrices' and one read-back brings their
+        # extents: twenty matrices one by one took a launch each (0.4 ms a pass, 0.3 ms like this), and with a
+        # read-back each 1.2 ms.  Any other one is a caller's tensor (of any type, stride, length and device), written in
+        # ways that leave no trace on the host: those go one by one.  A piece of the split is handed out once (what a
+        # caller writes into it is not in the next one), on the stream that it was allocated on, and in the
+        # inference mode that it was made in.
+        p = self._row_ptr
+        whole = p.whole
+        if not p.alone:
             ptr = whole[g0:g1 + 1]
             lo, hi = (int(x) for x in ptr[[0, -1]].tolist())
             return ptr - lo, lo, hi
-        stream = _lib.stream_of(whole.device)
-        if self._split is None or self._split[0] is not whole or self._split[1] != whole._version:
+        stream, split = _lib.stream_of(whole.device), p.split
+        if split is None:
             count, groups = len(self), int(self._groups[-1])
             own = torch.empty(groups + count, dtype=torch.int32, device=whole.device)
             bounds = torch.empty(count + 1, dtype=torch.int32, device=whole.device)
             _lib.check(_lib.call(_lib.lib().svc_split_row_ptr, whole.device, count, groups, self._mat_groups.data_ptr(), whole.data_ptr(),
                                  own.data_ptr(), bounds.data_ptr()), "svc_split_row_ptr")
             sizes = [int(self._groups[j + 1] - self._groups[j]) + 1 for j in range(count)]
-            self._split = (whole, whole._version, bounds.tolist(), dict(enumerate(own.split(sizes))), stream)
-        _, _, bounds, own, own_stream = self._split
+            p.split = split = (bounds.tolist(), dict(enumerate(own.split(sizes))), stream, own.is_inference())
+        bounds, own, own_stream, inference = split
         lo, hi = bounds[i], bounds[i + 1]
-        mine = own.pop(i, None) if stream == own_stream else None
+        mine = own.pop(i, None) if stream == own_stream and inference == torch.is_inference_mode_enabled() else None
         return (whole[g0:g1 + 1] - lo if mine is None else mine), lo, hi
 
     def matrix(self, i):
@@ -117,7 +138,7 @@ class SvcBatch:
         return SvcResult(ptr, self.vec_col[lo:hi], None if self.vec_val is None else self.vec_val[lo * self.V:hi * self.V], hi - lo)
 
     def to_host(self):
-        ptr = self.vec_row_ptr.cpu().numpy()
+        ptr = self._row_ptr.whole.cpu().numpy()
         n = int(ptr[-1])
         col = self.vec_col[:n].cpu().numpy()
         val = None if self.vec_val is None else self.vec_val[:n * self.V].cpu().numpy()
@@ -195,4 +216,6 @@ def svc_batched(mat_rows, K_max, row_ptr, col_ind, csr_val, V, order="cpython", 
                                           col_ind.data_ptr(), 0 if csr_val is None else csr_val.data_ptr(), nnz,
                                           _ORDERS[order], vec_row_ptr.data_ptr(), ws.data_ptr(), vec_col.data_ptr(),
                                           0 if vec_val is None else vec_val.data_ptr(), stream), "svc_fill_batched")
-    return SvcBatch(V, np.diff(mat_rows), cols, groups_of, vec_row_ptr, vec_col, vec_val, d_groups if groups > 0 else None)
+    batch = SvcBatch(V, np.diff(mat_rows), cols, groups_of, vec_row_ptr, vec_col, vec_val, d_groups if groups > 0 else None)
+    batch._row_ptr.alone = groups > 0
+    return batch

@@ -167,3 +167,84 @@ def test_row_pointers_of_a_stack_are_each_matrix_s_own(built_library, rows):
     with torch.cuda.stream(torch.cuda.Stream()):
         other = [batch.matrix(i).vec_row_ptr.cpu().tolist() for i in range(len(rows))]
     assert other == [w.tolist() for w in want] == [batch.matrix(i).vec_row_ptr.cpu().tolist() for i in range(len(rows))]
+
+
+def _stacked(rng, rows, V=8):
+    """(batch, its row pointer as a list, first group of every matrix) of random matrices of these row counts."""
+    mats = []
+    for M in rows:
+        ptr = np.concatenate([[0], np.cumsum(rng.integers(1, 9, M))]).astype(np.int32)
+        mats.append((M, 512, ptr, np.concatenate([np.sort(rng.choice(512, n, replace=False)) for n in np.diff(ptr)]).astype(np.int32), None))
+    at, K, ptr, col, _ = sspmm_amd.stack_csr(mats)
+    batch = sspmm_amd.svc_batched(at, K, torch.from_numpy(ptr).cuda(), torch.from_numpy(col).cuda(), None, V)
+    want = np.concatenate([[0], np.cumsum(np.concatenate([np.diff(p) for p, _, _ in batch.to_host()]))]).tolist()
+    return batch, want, np.concatenate([[0], np.cumsum([(M + V - 1) // V for M in rows])]).tolist()
+
+
+def _check_matrices(batch, ptr, groups, matrices):
+    for i in matrices:
+        own = ptr[groups[i]:groups[i + 1] + 1]
+        r = batch.matrix(i)
+        assert r.num_vec == own[-1] - own[0], i
+        assert r.vec_row_ptr.cpu().tolist() == [p - own[0] for p in own], i
+        assert torch.equal(r.vec_col, batch.vec_col[own[0]:own[-1]]), i
+
+
+@pytest.mark.parametrize("how", ["in place", "data", "raw pointer", "graph", "shallow copy", "int64", "strided", "host", "inference"])
+@pytest.mark.parametrize("taken", [0, 2, 4])
+def test_matrices_follow_a_row_pointer_on_the_device(built_library, how, taken):
+    """Extents and row pointers are those of vec_row_ptr as it is, after a caller wrote or replaced it, whether or not some
+    matrices had been taken before.  (Written: entries kept in order and inside vec_col, as a merge leaves them.)"""
+    import copy
+    from sspmm_amd import _lib
+    batch, ptr, groups = _stacked(np.random.default_rng(taken), [40, 8, 100, 33])
+    assert batch.matrix(1).num_vec == ptr[groups[2]] - ptr[groups[1]]
+    _check_matrices(batch, ptr, groups, range(taken))
+    other = [p - (i % 3 if 0 < i else 0) for i, p in enumerate(ptr)]
+    there = torch.tensor(other, dtype=torch.int32, device="cuda")
+    if how == "in place":
+        batch.vec_row_ptr.copy_(there)
+    elif how == "data":
+        batch.vec_row_ptr.data.copy_(there)
+    elif how == "raw pointer":  # (this entry of the library writes groups + 1 entries of one matrix)
+        one, bounds = torch.tensor([0, groups[-1]], dtype=torch.int32, device="cuda"), torch.empty(2, dtype=torch.int32, device="cuda")
+        assert _lib.lib().svc_split_row_ptr(1, groups[-1], one.data_ptr(), there.data_ptr(), batch.vec_row_ptr.data_ptr(), bounds.data_ptr(),
+                                            torch.cuda.current_stream().cuda_stream) == 0
+    elif how == "graph":
+        whole, graph = batch.vec_row_ptr, torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            whole.copy_(there)
+        for _ in range(2):
+            _check_matrices(batch, ptr, groups, range(4))
+        graph.replay()
+    elif how == "shallow copy":
+        copy.copy(batch).vec_row_ptr.copy_(there)
+    elif how == "int64":
+        batch.vec_row_ptr = there.long()
+    elif how == "strided":
+        batch.vec_row_ptr = torch.stack([there, there + 1], dim=1)[:, 0]
+    elif how == "host":
+        batch.vec_row_ptr = there.cpu()
+    else:
+        with torch.inference_mode():
+            batch.vec_row_ptr = there.clone()
+            _check_matrices(batch, other, groups, range(4))
+    _check_matrices(batch, other, groups, range(4))
+    _check_matrices(batch, other, groups, range(4))
+
+
+def test_a_shorter_row_pointer_is_not_read_past_its_end(built_library):
+    batch, ptr, groups = _stacked(np.random.default_rng(5), [40, 8, 100, 33])
+    batch.vec_row_ptr = batch.vec_row_ptr[:groups[2] + 1].clone()
+    _check_matrices(batch, ptr, groups, [0, 1])
+
+
+def test_row_pointers_taken_in_inference_mode_stay_there(built_library):
+    """A row pointer is an inference tensor only for the caller who took it in inference mode."""
+    batch, ptr, groups = _stacked(np.random.default_rng(6), [40, 8, 100])
+    with torch.inference_mode():
+        assert batch.matrix(0).vec_row_ptr.is_inference()
+    got = batch.matrix(1).vec_row_ptr
+    assert not got.is_inference()
+    got.add_(1)
+    _check_matrices(batch, ptr, groups, range(3))
