@@ -280,7 +280,8 @@ __global__ __launch_bounds__(1024) void svc_group_rows_kernel(int count, int V, 
 __global__ __launch_bounds__(256) void svc_split_row_ptr_kernel(int count, int groups, const int32_t *mat_groups, const int32_t *vec_row_ptr,
                                                                 int32_t *out_ptr, int32_t *bounds) {
   const int at = blockIdx.x * 256 + threadIdx.x;
-  if (at <= count) bounds[at] = vec_row_ptr[mat_groups[at]];
+  // (a stack whose caller miscounted its groups has entries beyond `groups` in mat_groups: nothing past the arrays is read)
+  if (at <= count) bounds[at] = vec_row_ptr[min(max(mat_groups[at], 0), groups)];
   if (at >= groups + count) return;
   int lo = 0, hi = count - 1;  // the last matrix i with mat_groups[i] + i <= at
   while (lo < hi) {
@@ -288,7 +289,7 @@ __global__ __launch_bounds__(256) void svc_split_row_ptr_kernel(int count, int g
     if (mat_groups[mid] + mid <= at) lo = mid;
     else hi = mid - 1;
   }
-  out_ptr[at] = vec_row_ptr[at - lo] - vec_row_ptr[mat_groups[lo]];
+  out_ptr[at] = vec_row_ptr[min(at - lo, groups)] - vec_row_ptr[min(max(mat_groups[lo], 0), groups)];
 }
 
 hipError_t launch_svc_split_row_ptr(int count, int groups, const int32_t *mat_groups, const int32_t *vec_row_ptr, int32_t *out_ptr,

@@ -248,3 +248,33 @@ def test_row_pointers_taken_in_inference_mode_stay_there(built_library):
     assert not got.is_inference()
     got.add_(1)
     _check_matrices(batch, ptr, groups, range(3))
+
+
+@pytest.mark.parametrize("mat_groups", [[0, 3, 7, 5], [0, 40, 50, 60], [-4, 2, 3, 5], [9, 9, 9, 9]])
+def test_split_of_a_miscounted_stack_stays_inside_its_arrays(built_library, mat_groups):
+    """svc_split_row_ptr with first groups beyond `groups` or out of order, as a stack with a wrong group count leaves
+    them: entries come out of the row pointer's own groups + 1 (here all below 100), and nothing else is written."""
+    from sspmm_amd import _lib
+    groups, count = 5, 3
+    buf = torch.full((64 + groups + 1 + 64,), 10 ** 6, dtype=torch.int32, device="cuda")
+    whole = buf[64:64 + groups + 1]
+    whole.copy_(torch.tensor([0, 3, 9, 9, 20, 31], device="cuda"))
+    out = torch.full((groups + count + 8,), -7, dtype=torch.int32, device="cuda")
+    bounds = torch.full((count + 1 + 8,), -7, dtype=torch.int32, device="cuda")
+    at = dev(np.array(mat_groups, np.int32))
+    assert _lib.lib().svc_split_row_ptr(count, groups, at.data_ptr(), whole.data_ptr(), out.data_ptr(), bounds.data_ptr(),
+                                        torch.cuda.current_stream().cuda_stream) == 0
+    out, bounds = out.cpu(), bounds.cpu()
+    assert (out[:groups + count].abs() < 100).all() and (bounds[:count + 1].abs() < 100).all()
+    assert (out[groups + count:] == -7).all() and (bounds[count + 1:] == -7).all()
+
+
+def test_split_rejects_what_it_cannot_do(built_library):
+    """(valid device pointers throughout: nothing is launched for a rejected call)"""
+    from sspmm_amd import _lib
+    L, p = _lib.lib(), torch.zeros(64, dtype=torch.int32, device="cuda").data_ptr()
+    assert L.svc_split_row_ptr(-1, 4, p, p, p, p, None) == 1 and L.svc_split_row_ptr(1, -1, p, p, p, p, None) == 1
+    assert L.svc_split_row_ptr(2 ** 30, 2 ** 30, p, p, p, p, None) == 1
+    for args in ((None, p, p, p), (p, None, p, p), (p, p, None, p), (p, p, p, None)):
+        assert L.svc_split_row_ptr(1, 4, *args, None) == 1
+    assert L.svc_split_row_ptr(0, 0, None, None, None, None, None) == 0
