@@ -276,13 +276,17 @@ def _rows_norm_applies(ln, x):
                               t.is_contiguous() and t.data_ptr() % 16 == 0) for t in (w, b)))
 
 
+BLOCK_FEATURES = 1 << 20  # hidden or output features that block_dense takes at most
+
+
 def _plain_linear(m, x, in_features, out_features, multiple):
-    """Whether m is a torch.nn.Linear of these sizes (out_features None: any multiple of `multiple`) whose weights a
-    kernel may read as they lie, for activations like x."""
+    """Whether m is a torch.nn.Linear of these sizes (out_features None: any multiple of `multiple` up to BLOCK_FEATURES)
+    whose weights a kernel may read as they lie, for activations like x."""
     if not _plain_module(m, torch.nn.Linear):
         return False
     w, b = m.weight, m.bias
-    return (m.in_features == in_features and m.out_features % multiple == 0 and out_features in (None, m.out_features) and
+    return (m.in_features == in_features and m.out_features % multiple == 0 and m.out_features <= BLOCK_FEATURES and
+            out_features in (None, m.out_features) and
             w.shape == (m.out_features, in_features) and (b is None or b.shape == (m.out_features,)) and
             all(t is None or (type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float16 and t.device == x.device and
                               t.is_contiguous() and t.data_ptr() % 16 == 0) for t in (w, b)))

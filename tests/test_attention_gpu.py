@@ -458,3 +458,17 @@ def test_softmax_with_masked_entries(built_library, V, scaler):
         e = np.exp(z - z.max(axis=0))
         want = e / e.sum(axis=0)
         assert (np.abs(got[off[i]:off[i + 1]] - want) <= want * (2.0 ** -11 + 2.0 ** -20) + 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("mlp,classes", [(256, 2 ** 20 + 64), (2 ** 20 + 256, 64)])
+def test_encoder_with_more_features_than_the_dense_launch_takes(built_library, mlp, classes):
+    """A head or a hidden layer of more than 2^20 features runs on the modules, as wide ones of any other size do."""
+    from sspmm_amd import attention as A
+    model = A.SparseAttentionEncoder(10, 128, 4, 0.5, 16, mlp, classes, vec_length=8, layers=1, seed=2).cuda().half().eval()
+    tokens = torch.randint(0, 10, (1, 16), device="cuda", generator=torch.Generator("cuda").manual_seed(1))
+    with torch.no_grad():
+        got = model(tokens)
+    want = model(tokens).detach()  # (with gradients: the modules one by one)
+    assert got.shape == (16, 1, classes)
+    scale = want.float().pow(2).mean().sqrt()
+    assert (got.float() - want.float()).abs().max() <= 1e-2 * scale
