@@ -22,7 +22,7 @@
 // probe sequence behind that slot.  So one thread per key inserts a whole phase at once.
 //
 // One workgroup owns one vector-row group.  The list and the table live in LDS (64 threads,
-// or 256 beside wider groups, for up to 306 keys, 1024 threads up to 4914) or, beyond that, in the
+// or 256 where there are few groups and wider ones among them, for up to 306 keys, 1024 threads up to 4914) or, beyond that, in the
 // caller's workspace.
 //
 // Which phase does what.  The caller sizes the outputs from svc_count's row pointer, so the count
@@ -1429,10 +1429,14 @@ hipError_t launch_svc_fill(const SvcArgs &args, int order, const uint16_t *csr_v
   if ((e = fork_streams(ss, stream, st, 1)) != hipSuccess) return e;
   // (from here on the helper is joined back into the caller's stream whatever happens)
   e = launch_fast_class<1024, true>(a, min(m_vec, cus), large ? 2 : 1, 1, kLargeKeys, 8192, key_bits, st[0], 81 * 1024);
-  // (four waves per small group where there are wider ones too: groups of 64 to 306 keys, whose phases are chains of
-  // placements, halve their chain and those of a few keys lose little.  Power-law matrices, 64 / 256 / 512 threads:
-  // 4096 x 4096, 16 a row, 155 / 137 / 142 us; 16384 x 1024, 32 a row, 154 / 139 / 198; 16384 x 16384 level)
-  if (e == hipSuccess) e = launch_fast_class<256, true>(a, min(m_vec, 8 * cus), 0, 0, kSmallKeys, 512, key_bits, st[1]);
+  // Four waves per small group as long as the chip holds all groups at once that way (the registers leave four such
+  // workgroups on a CU): a group's chain of placements is then what is waited for, and four waves shorten it.  Uneven (power-law)
+  // matrices, one wave / four: 8192 x 2000, 8 a row (1024 groups) 163 / 126 us; 1024 groups of 280 columns 186 / 169, of 8 to
+  // 128 level, of 32 out of 1024 columns 10 % slower.  With more groups than that they queue, four times as many of them at a time with one
+  // wave each: 2048 groups of 128 columns 155 / 191 us, 4096 168 / 315, 8192 229 / 553; 2^20 x 65536, 3 a row, 1.4 / 4.6 ms.
+  if (e == hipSuccess)
+    e = m_vec <= 4 * cus ? launch_fast_class<256, true>(a, m_vec, 0, 0, kSmallKeys, 512, key_bits, st[1])
+                         : launch_fast_class<64, true>(a, min(m_vec, 32 * cus), 0, 0, kSmallKeys, 512, key_bits, st[1]);
   rare_classes(st[1]);
   const hipError_t ej = join_streams(ss, stream, 1);
   return e != hipSuccess ? e : ej;
