@@ -278,3 +278,24 @@ def test_split_rejects_what_it_cannot_do(built_library):
     for args in ((None, p, p, p), (p, None, p, p), (p, p, None, p), (p, p, p, None)):
         assert L.svc_split_row_ptr(1, 4, *args, None) == 1
     assert L.svc_split_row_ptr(0, 0, None, None, None, None, None) == 0
+
+
+@pytest.mark.parametrize("most", [1, 64, 65, 300])
+def test_group_table_of_more_matrices_than_a_workgroup_has_threads(built_library, most):
+    """2100 matrices (three tiles of 1024 in the launch that makes the table) of 0 up to `most` groups, few of them large: either
+    way in which that launch writes a tile's groups."""
+    V = 8
+    rng = np.random.default_rng(most)
+    per = rng.integers(0, 3, 2100)
+    per[rng.choice(2100, 3, replace=False)] = most
+    rows = np.maximum(per * V - rng.integers(0, V, 2100) * (per > 0), 0)
+    at = np.concatenate([[0], np.cumsum(rows)]).astype(np.int64)
+    lens = rng.integers(0, 4, at[-1])
+    ptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    col = np.concatenate([np.sort(rng.choice(64, n, replace=False)) for n in lens]).astype(np.int32)
+    batch = sspmm_amd.svc_batched(at, 64, dev(ptr), dev(col), None, V, order="sorted")
+    got = batch.vec_row_ptr.cpu().numpy()
+    starts = np.concatenate([np.arange(a, b, V) for a, b in zip(at[:-1], at[1:])] + [at[-1:]])
+    ends = np.concatenate([np.minimum(np.arange(a, b, V) + V, b) for a, b in zip(at[:-1], at[1:])])
+    want = np.concatenate([[0], np.cumsum([np.unique(col[ptr[a]:ptr[b]]).size for a, b in zip(starts, ends)])])
+    assert np.array_equal(got, want)
