@@ -277,6 +277,17 @@ def _rows_norm_applies(ln, x):
 
 
 BLOCK_FEATURES = 1 << 20  # hidden or output features that block_dense takes at most
+# Every workgroup of block_dense streams the weights whole, 64 bytes a cycle of a CU (256 features, 4096 hidden ones: 66 us a
+# block), where a library product spreads them over the chip.  Up to this many weights in a matrix the one launch is ahead all the
+# same, by what the separate launches cost the host: forward pass of one block at 64 to 4096 tokens, E x hidden features, in one launch /
+# as modules / modules with the norms fused, us: 256 x 4096 108 / 215 / 230, 512 x 4096 121-137 / 220 / 217, 256 x 8192
+# 109-121 / 225 / 230; twice as many 180-195 / 220 / 219 and 193-215 / 220 / 218, level for one block and behind once the
+# device is what is waited for (four blocks: 190 us of the device a block against 150 of the host).  From 8192 tokens
+# on there are workgroups for every CU and the one launch is ahead whatever the sizes: 512 x 16384, 8192 tokens 396 / 494 / 443 us,
+# 32768 tokens 1054 / 1449 / 1295; at 6144 tokens 365 / 406 / 359.  A head is level with the library's product at best when it is
+# that large and behind beyond, with many tokens too: outputs in the launch / as a module, us of the device, 512 x 4096, 64 and
+# 32768 tokens 90 / 54 and 351 / 374, 512 x 8192 134 / 54 and 573 / 559, 256 x 65536 413 / 35 at 64 tokens and 814 / 487 at 8192.
+BLOCK_WEIGHTS = 1 << 21
 
 
 def _plain_linear(m, x, in_features, out_features, multiple):
@@ -418,18 +429,20 @@ class SparseAttentionEncoder(torch.nn.Module):
         return h
 
     def _fused_blocks_apply(self, x):
-        """(where the fused norms do) heads that one launch of attention takes, and products that block_dense does"""
+        """(where the fused norms do) heads that one launch of attention takes, and products that block_dense does and is
+        ahead with (see BLOCK_WEIGHTS)"""
         seq, bsz, E = x.shape
         return E in BLOCK_WIDTHS and packed_attention_fits(seq, bsz, 3 * E) and all(
             b.embed_dim == E and E % b.num_heads == 0 and E // b.num_heads in FUSED_HEAD_WIDTHS and
             _plain_linear(b.in_proj, x, E, 3 * E, 64) and _plain_linear(b.out_proj, x, E, E, 64) and
-            _plain_linear(b.linear1, x, E, None, 256) and _plain_linear(b.linear2, x, b.linear1.out_features, E, 64)
+            _plain_linear(b.linear1, x, E, None, 256) and _plain_linear(b.linear2, x, b.linear1.out_features, E, 64) and
+            (E * b.linear1.out_features <= BLOCK_WEIGHTS or seq * bsz > 4096)
             for b in self.blocks)
 
     def _fused_blocks(self, x, pe, scale):
         """(x * scale) + pe through the blocks and the head.  Two launches per block: its attention, and all that follows up to the next block's projection (or the head)."""
         E, blocks = x.size(-1), list(self.blocks)
-        head = _plain_linear(self.linear, x, E, None, 64)
+        head = _plain_linear(self.linear, x, E, None, 64) and E * self.linear.out_features <= BLOCK_WEIGHTS
         linears, rows = [blocks[0].in_proj], [64]
         for i, blk in enumerate(blocks):
             tail = [blocks[i + 1].in_proj] if i + 1 < len(blocks) else [self.linear] * head

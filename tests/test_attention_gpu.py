@@ -472,3 +472,26 @@ def test_encoder_with_more_features_than_the_dense_launch_takes(built_library, m
     assert got.shape == (16, 1, classes)
     scale = want.float().pow(2).mean().sqrt()
     assert (got.float() - want.float()).abs().max() <= 1e-2 * scale
+
+
+@pytest.mark.parametrize("embed,mlp,classes,batch,launches,with_head", [(512, 4096, 4096, 1, 3, True), (512, 4352, 64, 1, 0, None), (512, 4352, 64, 43, 3, True),
+                                                                        (256, 512, 8192, 1, 3, True), (256, 512, 8256, 1, 3, False),
+                                                                        (128, 16384, 64, 1, 3, True), (128, 16640, 64, 1, 0, None)])
+def test_wide_hidden_layers_and_heads_go_to_the_library(built_library, embed, mlp, classes, batch, launches, with_head):
+    """Either side of the sizes up to which one launch per block beats the products one by one (hidden layers: of up to 4096
+    tokens; 43 x 96 are more), with the results of the modules."""
+    from sspmm_amd import attention as A
+    model = A.SparseAttentionEncoder(50, embed, 4, 0.9, 96, mlp, classes, vec_length=8, layers=2, seed=2).cuda().half().eval()
+    tokens = torch.randint(0, 50, (batch, 96), device="cuda", generator=torch.Generator("cuda").manual_seed(1))
+    tails = []
+    plain = A.block_dense
+    A.block_dense = lambda x, attn, block, norm, tail=None, *args, **kw: (tails.append(tail), plain(x, attn, block, norm, tail, *args, **kw))[1]
+    try:
+        with torch.no_grad():
+            got = model(tokens)
+    finally:
+        A.block_dense = plain
+    assert len(tails) == launches and (not tails or (tails[-1] is not None) == with_head)
+    want = model(tokens).detach()  # (with gradients: the modules one by one)
+    scale = want.float().pow(2).mean().sqrt()
+    assert (got.float() - want.float()).abs().max() <= 1e-2 * scale
