@@ -272,10 +272,12 @@ struct Halfs {
 // result).  The first kSoftmaxCached vectors of every lane (512 / 256 vectors of the row for V = 8 / 16) are
 // loaded once, all loads in flight together, and stay in registers; only the rest of a longer row is read again (from
 // the caches).  As much of the time goes into vector instructions as into memory, so there are few per value: the
-// extreme of a row is taken on packed halves (x * scaler is monotonic: the maximum for a scaler >= 0, the minimum for
-// a negative one), exp(x * s - max) is one multiply-add of x by s * log2(e) and the base-2 exponential, and the exponentials
-// of the second pass are kept for the third.  48 heads, 4096 keys, 90 % masked: 62 us with the three passes on
-// floats, 54 with the exponentials kept, 50 so; 16 heads, 2000 keys 9.3, 8.3, 8.1.
+// extreme of a row is taken on packed halves (x * scaler is monotonic: the maximum of x for a scaler >= 0, of -x, by its
+// sign bit, for a negative one), exp(x * s - max) is one multiply-add of x by s * log2(e) and the base-2 exponential, the exponentials
+// of the second pass are kept for the third, and what a short row leaves empty is passed by.  48 heads, 4096 keys, 90 % masked:
+// 62 us with the three passes on floats, 54 with the exponentials kept, 48 so; 16 heads, 2000 keys 9.3, 8.3, 7.2.  48 heads
+// of 512 rows of 60 vectors 22.5 us on floats, 25.3 with a branch on the scaler's sign at every step and the empty slots
+// gone through, 20.7 so.
 template <int V>
 struct SoftmaxCached {
   static constexpr int value = V == 8 ? 8 : 4;
@@ -296,28 +298,34 @@ __global__ __launch_bounds__(64) void softmax_kernel(const SoftmaxArgs p) {
   uint16_t *out = p.out + (int64_t)batch * p.stride;
   const float s2 = p.scaler * 1.4426950408889634f;
   const bool falling = p.scaler < 0.f;
+  const uint32_t sign = falling ? 0x80008000u : 0u;
   const int tail = beg + lane + 64 * KC;  // the lane's first vector that is not held in registers
 
+  // (a lane past the row's end in a slot that other lanes need: a value that changes no extreme; its exponentials are
+  // skipped below)
   Halfs<V> cached[KC];
 #pragma unroll
   for (int i = 0; i < KC; ++i) {
     const int j = beg + lane + 64 * i;
-    cached[i] = j < end ? Halfs<V>::load(in + (int64_t)j * V) : Halfs<V>::all(falling ? INFINITY : -INFINITY);
+    if (beg + 64 * i < end) cached[i] = j < end ? Halfs<V>::load(in + (int64_t)j * V) : Halfs<V>::all(falling ? INFINITY : -INFINITY);
   }
-  // (a slot past the row changes no extreme; its exponentials are skipped below)
-  Halfs<V> top = cached[0];
+  Halfs<V> top = Halfs<V>::all(-INFINITY);
   const auto fold = [&](const Halfs<V> &x) {
 #pragma unroll
-    for (int i = 0; i < V / 8; ++i) top.h[i] = falling ? __builtin_elementwise_min(top.h[i], x.h[i]) : __builtin_elementwise_max(top.h[i], x.h[i]);
+    for (int i = 0; i < V / 8; ++i) {
+      const uintx4 y = __builtin_bit_cast(uintx4, x.h[i]) ^ uintx4{sign, sign, sign, sign};
+      top.h[i] = __builtin_elementwise_max(top.h[i], __builtin_bit_cast(half8, y));
+    }
   };
 #pragma unroll
-  for (int i = 1; i < KC; ++i) fold(cached[i]);
+  for (int i = 0; i < KC; ++i)
+    if (beg + 64 * i < end) fold(cached[i]);
   for (int j = tail; j < end; j += 64) fold(Halfs<V>::load(in + (int64_t)j * V));
 
   float mx[V], sum[V];
 #pragma unroll
   for (int v = 0; v < V; ++v) {
-    mx[v] = (falling ? -wave_max(-top.at(v)) : wave_max(top.at(v))) * s2;
+    mx[v] = wave_max(top.at(v)) * (falling ? -s2 : s2);
     sum[v] = 0.f;
   }
   const auto exponentials = [&](const Halfs<V> &x, float (&e)[V]) {
@@ -352,13 +360,121 @@ __global__ __launch_bounds__(64) void softmax_kernel(const SoftmaxArgs p) {
   }
 }
 
+// Long rows of 16-row vectors: the three passes on floats, the exponentials made again in the third.  Such rows' values outgrow the
+// L2 between the passes, and this kernel, whose registers are as many, gets more of them from the memory behind it: 512
+// rows x 8 heads of 256 vectors 16.0 us against 23.2 with the kernel above, 409 24.6 against 30.2, 600 34.9 against 40.8,
+// 1500 109 against 113 (200: 14.7 against 14.0, 100: 10.7 against 10.1).
+struct WideVec {
+  static __device__ __forceinline__ void load(const uint16_t *p, _Float16 (&x)[16]) {
+    const half8 lo = *reinterpret_cast<const half8 *>(p), hi = *reinterpret_cast<const half8 *>(p + 8);
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      x[v] = lo[v];
+      x[8 + v] = hi[v];
+    }
+  }
+  static __device__ __forceinline__ void store(uint16_t *p, const _Float16 (&x)[16]) {
+    half8 lo, hi;
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      lo[v] = x[v];
+      hi[v] = x[8 + v];
+    }
+    __builtin_nontemporal_store(lo, reinterpret_cast<half8 *>(p));
+    __builtin_nontemporal_store(hi, reinterpret_cast<half8 *>(p + 8));
+  }
+};
+__global__ __launch_bounds__(64) void softmax_long_kernel(const SoftmaxArgs p) {
+  constexpr int V = 16, KC = SoftmaxCached<V>::value;
+  const uint32_t w = xcd_work_index(p.per_xcd);
+  if (w >= p.total_work) return;
+  const uint32_t r = w % (uint32_t)p.m_vec;
+  const uint32_t batch = w / (uint32_t)p.m_vec;
+  const int row = p.row_indices ? p.row_indices[r] : (int)r;
+  const int beg = p.row_offsets[row], end = p.row_offsets[row + 1];
+  if (beg == end) return;
+  const int lane = threadIdx.x;
+  const uint16_t *in = p.values + (int64_t)batch * p.stride;
+  uint16_t *out = p.out + (int64_t)batch * p.stride;
+  const float s = p.scaler;
+  const int tail = beg + lane + 64 * KC;
+
+  _Float16 cached[KC][V];
+#pragma unroll
+  for (int i = 0; i < KC; ++i) {
+    const int j = beg + lane + 64 * i;
+    if (j < end) {
+      WideVec::load(in + (int64_t)j * V, cached[i]);
+    } else {
+#pragma unroll
+      for (int v = 0; v < V; ++v) cached[i][v] = (_Float16)0;  // never used: the passes below skip these slots
+    }
+  }
+
+  float mx[V], sum[V];
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+    mx[v] = -INFINITY;
+    sum[v] = 0.f;
+  }
+#pragma unroll
+  for (int i = 0; i < KC; ++i)
+    if (beg + lane + 64 * i < end) {
+#pragma unroll
+      for (int v = 0; v < V; ++v) mx[v] = fmaxf(mx[v], (float)cached[i][v] * s);
+    }
+  for (int j = tail; j < end; j += 64) {
+    _Float16 x[V];
+    WideVec::load(in + (int64_t)j * V, x);
+#pragma unroll
+    for (int v = 0; v < V; ++v) mx[v] = fmaxf(mx[v], (float)x[v] * s);
+  }
+#pragma unroll
+  for (int v = 0; v < V; ++v) mx[v] = wave_max(mx[v]);
+#pragma unroll
+  for (int i = 0; i < KC; ++i)
+    if (beg + lane + 64 * i < end) {
+#pragma unroll
+      for (int v = 0; v < V; ++v) sum[v] += __expf((float)cached[i][v] * s - mx[v]);
+    }
+  for (int j = tail; j < end; j += 64) {
+    _Float16 x[V];
+    WideVec::load(in + (int64_t)j * V, x);
+#pragma unroll
+    for (int v = 0; v < V; ++v) sum[v] += __expf((float)x[v] * s - mx[v]);
+  }
+#pragma unroll
+  for (int v = 0; v < V; ++v) sum[v] = 1.0f / wave_sum(sum[v]);
+#pragma unroll
+  for (int i = 0; i < KC; ++i) {
+    const int j = beg + lane + 64 * i;
+    if (j < end) {
+      _Float16 y[V];
+#pragma unroll
+      for (int v = 0; v < V; ++v) y[v] = (_Float16)(__expf((float)cached[i][v] * s - mx[v]) * sum[v]);
+      WideVec::store(out + (int64_t)j * V, y);
+    }
+  }
+  for (int j = tail; j < end; j += 64) {
+    _Float16 x[V], y[V];
+    WideVec::load(in + (int64_t)j * V, x);
+#pragma unroll
+    for (int v = 0; v < V; ++v) y[v] = (_Float16)(__expf((float)x[v] * s - mx[v]) * sum[v]);
+    WideVec::store(out + (int64_t)j * V, y);
+  }
+}
+
 hipError_t launch_softmax(const SoftmaxArgs &a, int V, hipStream_t stream) {
   SoftmaxArgs p = a;
   p.total_work = (uint32_t)a.m_vec * (uint32_t)a.batch;
   p.per_xcd = (p.total_work + 7u) / 8u;
   if (p.total_work == 0) return hipSuccess;
+  // (the batch stride is the number of stored values, so it tells a row's mean length; 0, of a single product, does not)
+  const bool long_rows = V == 16 && (a.stride <= 0 || a.stride > (int64_t)a.m_vec * (16 * 208));
   if (V == 8)
     hipLaunchKernelGGL(softmax_kernel<8>, dim3(p.per_xcd * 8u), dim3(64), 0, stream, p);
+  else if (long_rows)
+    hipLaunchKernelGGL(softmax_long_kernel, dim3(p.per_xcd * 8u), dim3(64), 0, stream, p);
   else
     hipLaunchKernelGGL(softmax_kernel<16>, dim3(p.per_xcd * 8u), dim3(64), 0, stream, p);
   return hipGetLastError();

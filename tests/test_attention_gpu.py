@@ -495,3 +495,29 @@ def test_wide_hidden_layers_and_heads_go_to_the_library(built_library, embed, ml
     want = model(tokens).detach()  # (with gradients: the modules one by one)
     scale = want.float().pow(2).mean().sqrt()
     assert (got.float() - want.float()).abs().max() <= 1e-2 * scale
+
+
+@pytest.mark.parametrize("V", [8, 16])
+@pytest.mark.parametrize("batch,lens", [(3, [1, 63, 64, 65, 0, 128, 129, 191]), (2, [207, 208, 209, 208]), (2, [209, 208, 209, 210]),
+                                        (2, [255, 256, 257, 300]), (1, [511, 512, 513, 1100, 0, 3])])
+@pytest.mark.parametrize("scaler", [0.3, -0.7, 0.0])
+def test_softmax_either_side_of_its_kernels(built_library, V, batch, lens, scaler):
+    """Rows up to and beyond what a wave's slots hold, mean lengths either side of 208 (where 16-row vectors change kernels), a scaler
+    of either sign and none: against float64, half an fp16 ulp of a result up to 1 and 2^-20 for the exponential.  In place
+    and without a stride (the single product) the same bits as that."""
+    from sspmm_amd import _lib
+    rng = np.random.default_rng(len(lens) + V)
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    x = (rng.standard_normal((batch, off[-1], V)) * 4).astype(np.float16)
+    got = sspmm_amd.bcsr_softmax(None, dev(off), dev(x.reshape(batch, -1)), scaler, V, batch).cpu().numpy().reshape(batch, -1, V).astype(np.float64)
+    for i in range(len(lens)):
+        z = x[:, off[i]:off[i + 1]].astype(np.float64) * scaler
+        if lens[i] == 0:
+            continue
+        e = np.exp(z - z.max(axis=1, keepdims=True))
+        want = e / e.sum(axis=1, keepdims=True)
+        assert (np.abs(got[:, off[i]:off[i + 1]] - want) <= want * (2.0 ** -11 + 2.0 ** -20) + 2.0 ** -24).all()
+    one = dev(x[0].reshape(-1))
+    assert _lib.lib().sspmm_softmax_f16(len(lens), V, None, dev(off).data_ptr(), one.data_ptr(), scaler, one.data_ptr(),
+                                        torch.cuda.current_stream().cuda_stream) == 0
+    assert np.abs(one.cpu().numpy().reshape(-1, V).astype(np.float64) - got[0]).max() <= 2.0 ** -11
