@@ -99,6 +99,7 @@ struct Store8;
 
 template <>
 struct Store8<float> {
+  template <bool RAGGED>
   static __device__ __forceinline__ void run(float *p, const float (&v)[8]) {
     floatx4 a = {v[0], v[1], v[2], v[3]};
     floatx4 b = {v[4], v[5], v[6], v[7]};
@@ -109,13 +110,18 @@ struct Store8<float> {
 
 template <>
 struct Store8<_Float16> {
+  template <bool RAGGED>
   static __device__ __forceinline__ void run(_Float16 *p, const float (&v)[8]) {
     half8 h;
 #pragma unroll
     for (int i = 0; i < 8; ++i) h[i] = (_Float16)v[i];  // v_cvt_f16_f32: round to nearest even
     // (non-temporal: the rows of B the grid keeps gathering stay in the L2; measured 1-10 % on fp16 outputs.  fp32
-    // tiles of 128 columns do not come through here: they go out as whole lines, see store_tile_f32_lines)
-    __builtin_nontemporal_store(h, reinterpret_cast<half8_u *>(p));
+    // tiles of 128 columns do not come through here: they go out as whole lines, see
+    // store_tile_f32_lines.  Ragged rows: see stores_ragged)
+    if constexpr (RAGGED)
+      *reinterpret_cast<half8_u *>(p) = h;
+    else
+      __builtin_nontemporal_store(h, reinterpret_cast<half8_u *>(p));
   }
 };
 
@@ -123,16 +129,19 @@ template <typename OutT, int CPL>
 struct StoreRow;
 template <typename OutT>
 struct StoreRow<OutT, 8> {
-  static __device__ __forceinline__ void run(OutT *p, const float (&v)[8]) { Store8<OutT>::run(p, v); }
+  template <bool RAGGED>
+  static __device__ __forceinline__ void run(OutT *p, const float (&v)[8]) { Store8<OutT>::template run<RAGGED>(p, v); }
 };
 template <>
 struct StoreRow<float, 4> {
+  template <bool RAGGED>
   static __device__ __forceinline__ void run(float *p, const float (&v)[4]) {
     *reinterpret_cast<floatx4_u *>(p) = floatx4{v[0], v[1], v[2], v[3]};
   }
 };
 template <>
 struct StoreRow<_Float16, 4> {
+  template <bool RAGGED>
   static __device__ __forceinline__ void run(_Float16 *p, const float (&v)[4]) {
     typedef _Float16 half4v __attribute__((ext_vector_type(4)));
     typedef half4v half4_u __attribute__((aligned(2)));
@@ -286,7 +295,7 @@ __device__ __forceinline__ void mac_chunk(const Chunk<CPL> &c, floatx4 (&acc)[CP
 // bytes per instruction, non-temporal.  Launches of few vectors per row are mostly these stores: measured up to
 // 2.2x at 95-98 % sparsity, 0.85-0.9x the time over a sweep of shapes at 90 %.
 // acc[q][rr] = C[row 4g + rr][column 8m + q] of the tile; crow = the tile's first row of C, at column 0.
-template <int V>
+template <int V, bool RAGGED>
 __device__ __forceinline__ void store_tile_f32_lines(float (*ctile)[128 + 4], const floatx4 (&acc)[8], int lane, float *crow,
                                                      int N, int tile) {
   const int m = lane & 15, g = lane >> 4;
@@ -305,7 +314,11 @@ __device__ __forceinline__ void store_tile_f32_lines(float (*ctile)[128 + 4], co
     for (int i = 0; i < V / 2; ++i) {
       const int v = 2 * i + (lane >> 5);
       const floatx4 x = *reinterpret_cast<const floatx4 *>(&ctile[v][c4]);
-      __builtin_nontemporal_store(x, reinterpret_cast<floatx4_u *>(crow + (int64_t)v * N + gcol));
+      floatx4_u *const out = reinterpret_cast<floatx4_u *>(crow + (int64_t)v * N + gcol);
+      if constexpr (RAGGED)
+        *out = x;
+      else
+        __builtin_nontemporal_store(x, out);
     }
   }
 }
@@ -314,7 +327,7 @@ __device__ __forceinline__ void store_tile_f32_lines(float (*ctile)[128 + 4], co
 // spilling; a launch with more waves than two per SIMD can hold at once runs 6-8 % faster that way (more gathers in
 // flight per CU), one that fits anyway runs level or a few per cent slower, so the launcher picks by the grid.
 // (Three chunk buffers in rotation, two chunks of gathers in flight per wave, were measured as well: 15-30 % slower.)
-template <int V, typename OutT, int CPL, int WPE = 2>
+template <int V, typename OutT, int CPL, int WPE = 2, bool RAGGED = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void spmm_gather_kernel(const SpmmArgs p) {
   __shared__ __align__(16) unsigned char val_tiles[2][val_tile_bytes(V)];  // the value tiles of two chunks in turn
   const uint32_t id = blockIdx.x;
@@ -398,7 +411,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
   }
   if constexpr (std::is_same<OutT, float>::value && CPL == 8) {
     __shared__ __align__(16) float ctile[V][128 + 4];
-    store_tile_f32_lines<V>(ctile, acc, lane, reinterpret_cast<float *>(p.C) + (int64_t)batch * p.stride_C + (int64_t)row * V * p.N,
+    store_tile_f32_lines<V, RAGGED>(ctile, acc, lane, reinterpret_cast<float *>(p.C) + (int64_t)batch * p.stride_C + (int64_t)row * V * p.N,
                             p.N, (int)tile);
   } else if (col_ok) {
     OutT *cbase = reinterpret_cast<OutT *>(p.C) + (int64_t)batch * p.stride_C;
@@ -409,7 +422,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
         float o[CPL];
 #pragma unroll
         for (int q = 0; q < CPL; ++q) o[q] = acc[q][rr];
-        StoreRow<OutT, CPL>::run(cbase + ((int64_t)row * V + v) * p.N + ncol, o);
+        StoreRow<OutT, CPL>::template run<RAGGED>(cbase + ((int64_t)row * V + v) * p.N + ncol, o);
       }
     }
   }
@@ -523,7 +536,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void spmm_gather_split_kernel(con
     gather_accumulate<V>(acc, p, batch, beg, end, end, lane, ncol, col_ok, val_tiles_all[wave]);
     if constexpr (std::is_same<OutT, float>::value) {
       __shared__ __align__(16) float ctile_all[kSplitWaves][V][128 + 4];
-      store_tile_f32_lines<V>(ctile_all[wave], acc, lane, reinterpret_cast<float *>(cbase) + (int64_t)row * V * p.N, p.N, (int)tile);
+      store_tile_f32_lines<V, false>(ctile_all[wave], acc, lane, reinterpret_cast<float *>(cbase) + (int64_t)row * V * p.N, p.N, (int)tile);
     } else if (col_ok) {
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) {
@@ -532,7 +545,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void spmm_gather_split_kernel(con
           float o[8];
 #pragma unroll
           for (int q = 0; q < 8; ++q) o[q] = acc[q][rr];
-          Store8<OutT>::run(cbase + ((int64_t)row * V + v) * p.N + ncol, o);
+          Store8<OutT>::template run<false>(cbase + ((int64_t)row * V + v) * p.N + ncol, o);
         }
       }
     }
@@ -569,7 +582,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void spmm_gather_split_kernel(con
       if (v < V) {
         const floatx4 lo = part[wave][0][lane], hi = part[wave][1][lane];
         const float o[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        Store8<OutT>::run(cbase + ((int64_t)lrow * V + v) * p.N + ncol, o);
+        Store8<OutT>::template run<false>(cbase + ((int64_t)lrow * V + v) * p.N + ncol, o);
       }
     }
     __syncthreads();  // part is rewritten for the next long row
@@ -719,8 +732,12 @@ __device__ __forceinline__ void slab_issue(SlabLoads<V> &r, int row, int kc, int
 // return in order among themselves, so while an awaited load is outstanding so are its n younger
 // loads, and the wait cannot pass early whatever the stores do; stores in flight only make it
 // pass later.  The trailing s_nop covers the cycles in which the store still reads its data registers.
+template <bool RAGGED>
 __device__ __forceinline__ void slab_store_line(uintx4 line, __amdgpu_buffer_rsrc_t srd, uint32_t voff, uint32_t soff) {
-  asm volatile("buffer_store_dwordx4 %0, %1, %2, %3 offen nt\n\ts_nop 1" ::"v"(line), "v"(voff), "s"(srd), "s"(soff));
+  if constexpr (RAGGED)  // (see stores_ragged)
+    asm volatile("buffer_store_dwordx4 %0, %1, %2, %3 offen\n\ts_nop 1" ::"v"(line), "v"(voff), "s"(srd), "s"(soff));
+  else
+    asm volatile("buffer_store_dwordx4 %0, %1, %2, %3 offen nt\n\ts_nop 1" ::"v"(line), "v"(voff), "s"(srd), "s"(soff));
 }
 
 // Writing a finished V x 64 tile of C.  The MFMAs run with the slab as their first operand, so
@@ -764,6 +781,7 @@ struct SlabStore<V, float, NQ> {
       }
     }
   }
+  template <bool RAGGED>
   __device__ __forceinline__ void store(const floatx4 (&acc)[NQ], __amdgpu_buffer_rsrc_t srd, uint32_t crow) const {
 #pragma unroll
     for (int qp = 0; qp < NQ / 2; ++qp) {
@@ -777,7 +795,7 @@ struct SlabStore<V, float, NQ> {
           const uint32_t x = __builtin_bit_cast(uint32_t, fx), y = __builtin_bit_cast(uint32_t, fy);
           line[r] = h == 0 ? dpp_from_m_minus_8(x, y) : dpp_from_m_plus_8(x, y);
         }
-        slab_store_line(line, srd, voff[h][qp], crow);
+        slab_store_line<RAGGED>(line, srd, voff[h][qp], crow);
       }
     }
   }
@@ -796,6 +814,7 @@ struct SlabStore<V, _Float16, 4> {
       voff[h] = col < N ? ((uint32_t)row * (uint32_t)N + (uint32_t)unit_col(col, N)) * 2u : kSlabDropStore;
     }
   }
+  template <bool RAGGED>
   __device__ __forceinline__ void store(const floatx4 (&acc)[4], __amdgpu_buffer_rsrc_t srd, uint32_t crow) const {
     // pr[pair][0..3]: after the swaps, lane (m, g) holds columns 8 * (g >> 1) .. + 7 of tile
     // 2 * pair + (g & 1), row m
@@ -825,7 +844,7 @@ struct SlabStore<V, _Float16, 4> {
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         line[r] = h == 0 ? dpp_from_m_minus_8(pr[0][r], pr[1][r]) : dpp_from_m_plus_8(pr[0][r], pr[1][r]);
-      slab_store_line(line, srd, voff[h], crow);
+      slab_store_line<RAGGED>(line, srd, voff[h], crow);
     }
   }
 };
@@ -838,10 +857,11 @@ struct SlabStore<V, _Float16, 8> {
     half_lo.init(lane, n0, N);
     half_hi.init(lane, n0 + 64, N);
   }
+  template <bool RAGGED>
   __device__ __forceinline__ void store(const floatx4 (&acc)[8], __amdgpu_buffer_rsrc_t srd, uint32_t crow) const {
     const floatx4 a[4] = {acc[0], acc[1], acc[2], acc[3]}, b[4] = {acc[4], acc[5], acc[6], acc[7]};
-    half_lo.store(a, srd, crow);
-    half_hi.store(b, srd, crow);
+    half_lo.template store<RAGGED>(a, srd, crow);
+    half_hi.template store<RAGGED>(b, srd, crow);
   }
 };
 
@@ -855,6 +875,7 @@ struct SlabStore<V, _Float16, 2> {
     const int col = n0 + 16 * (g & 1) + 8 * (g >> 1);
     voff = (m < V && col < N) ? ((uint32_t)m * (uint32_t)N + (uint32_t)unit_col(col, N)) * 2u : kSlabDropStore;
   }
+  template <bool RAGGED>
   __device__ __forceinline__ void store(const floatx4 (&acc)[2], __amdgpu_buffer_rsrc_t srd, uint32_t crow) const {
     uint32_t pk[2][2];
 #pragma unroll
@@ -872,7 +893,7 @@ struct SlabStore<V, _Float16, 2> {
       line[w] = sw[0];
       line[2 + w] = sw[1];
     }
-    slab_store_line(line, srd, voff, crow);
+    slab_store_line<RAGGED>(line, srd, voff, crow);
   }
 };
 
@@ -888,7 +909,7 @@ struct SlabCtx {
 
 // One wave's share of a work item: the vector-rows it claims from the item's row table,
 // against the slab at byte offset slab_base of LDS.
-template <int V, typename OutT, int NQ, int L>
+template <int V, typename OutT, int NQ, int L, bool RAGGED>
 __device__ __forceinline__ void slab_process_item(const SlabCtx<V, OutT> &x, unsigned char *lds, uint32_t slab_base,
                                                   const SlabRows &rows, const uint16_t *vals,
                                                   __amdgpu_buffer_rsrc_t srd_c, const SlabStore<V, OutT, NQ> &out) {
@@ -962,7 +983,7 @@ __device__ __forceinline__ void slab_process_item(const SlabCtx<V, OutT> &x, uns
 #pragma unroll
       for (int q = 0; q < NQ; ++q) acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[q].h, a.h, acc[q], 0, 0, 0);
       if (left <= 32) {  // last step of the vector-row: write its V x 64 tile of C and start over from zero
-        out.store(acc, srd_c, (uint32_t)ld[cur].row * x.c_vrow_bytes);
+        out.template store<RAGGED>(acc, srd_c, (uint32_t)ld[cur].row * x.c_vrow_bytes);
 #pragma unroll
         for (int q = 0; q < NQ; ++q) acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(zero_op.h, zero_op.h, zero_c, 0, 0, 0);
       }
@@ -1036,7 +1057,7 @@ __device__ __forceinline__ intx4 slab_table_fetch(const SpmmArgs &p, const int32
   return e;
 }
 
-template <int V, typename OutT, int L, int NQ>
+template <int V, typename OutT, int L, int NQ, bool RAGGED>
 __global__ __launch_bounds__(kSlabThreads) void spmm_slab_kernel(const SpmmArgs p,
                                                                  const int32_t *__restrict__ row_offsets,
                                                                  const int32_t *__restrict__ row_indices) {
@@ -1141,7 +1162,7 @@ __global__ __launch_bounds__(kSlabThreads) void spmm_slab_kernel(const SpmmArgs 
       // One buffer descriptor spans this batch element's C (the launcher checks it is at most 2 GiB).
       const __amdgpu_buffer_rsrc_t srd_c = make_srd(reinterpret_cast<OutT *>(p.C) + (int64_t)cur.batch * p.stride_C,
                                                     (uint32_t)p.m_vec * x.c_vrow_bytes);
-      slab_process_item<V, OutT, NQ, L>(x, lds, layout_buffer_off(L, NQ, zero_row + 1u, slab_sel), rows, p.values + (int64_t)cur.batch * p.stride_values,
+      slab_process_item<V, OutT, NQ, L, RAGGED>(x, lds, layout_buffer_off(L, NQ, zero_row + 1u, slab_sel), rows, p.values + (int64_t)cur.batch * p.stride_values,
                                  srd_c, out);
     }
     if (!has_next) break;
@@ -1392,7 +1413,7 @@ __device__ __forceinline__ void stage_stream(const StageLane<V> &x, const int32_
       acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b.h, a.h, acc[q], 0, 0, 0);
     }
     if (d.kc + 32 >= d.end) {  // the row's last step: its tile of C, and the next row starts from zero
-      out.store(acc, srd_c, (uint32_t)d.row * c_vrow_bytes);
+      out.template store<false>(acc, srd_c, (uint32_t)d.row * c_vrow_bytes);
 #pragma unroll
       for (int q = 0; q < 4; ++q) acc[q] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
@@ -1477,7 +1498,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(V == 8 ? 5 :
   // One buffer descriptor spans this batch element's C (the launcher checks it is at most 2 GiB).
   const __amdgpu_buffer_rsrc_t srd_c = make_srd(reinterpret_cast<OutT *>(p.C) + (int64_t)batch * p.stride_C,
                                                 (uint32_t)p.m_vec * c_vrow_bytes);
-  out.store(acc, srd_c, (uint32_t)row * c_vrow_bytes);
+  out.template store<false>(acc, srd_c, (uint32_t)row * c_vrow_bytes);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1633,7 +1654,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     // One buffer descriptor spans this batch element's C (the launcher checks it is at most 2 GiB).
     const __amdgpu_buffer_rsrc_t srd_c = make_srd(reinterpret_cast<OutT *>(p.C) + (int64_t)batch * p.stride_C,
                                                   (uint32_t)p.m_vec * c_vrow_bytes);
-    out.store(acc, srd_c, (uint32_t)row * c_vrow_bytes);
+    out.template store<false>(acc, srd_c, (uint32_t)row * c_vrow_bytes);
   }
 }
 
@@ -1732,9 +1753,9 @@ static uint32_t device_cus() {  // of the current device
   return cus[dev];
 }
 
-template <int V, typename OutT, int L, int NQ>
+template <int V, typename OutT, int L, int NQ, bool RAGGED>
 static hipError_t launch_slab_kernel(const SpmmArgs &p, uint32_t grid, uint32_t lds, hipStream_t stream) {
-  auto kern = spmm_slab_kernel<V, OutT, L, NQ>;
+  auto kern = spmm_slab_kernel<V, OutT, L, NQ, RAGGED>;
   static bool raised[kMaxDevices] = {};  // per instantiation and device
   const int dev = current_device();
   if (!raised[dev]) {
@@ -1746,7 +1767,7 @@ static hipError_t launch_slab_kernel(const SpmmArgs &p, uint32_t grid, uint32_t 
   return hipGetLastError();
 }
 
-template <int V, typename OutT, int NQ>
+template <int V, typename OutT, int NQ, bool RAGGED>
 static hipError_t launch_slab(const SpmmArgs &a, hipStream_t stream) {
   SpmmArgs p = a;
   p.n_tiles = (uint32_t)((a.N + 16 * NQ - 1) / (16 * NQ));
@@ -1776,20 +1797,20 @@ static hipError_t launch_slab(const SpmmArgs &a, hipStream_t stream) {
   const uint32_t lds = slab_lds_bytes(a.K, V, rows, layout, NQ);
   const uint32_t grid = 8u * wgs_per_xcd;
   if (NQ == 4) {
-    if (layout == kPadDouble) return launch_slab_kernel<V, OutT, kPadDouble, 4>(p, grid, lds, stream);
-    if (layout == kPadSingle) return launch_slab_kernel<V, OutT, kPadSingle, 4>(p, grid, lds, stream);
+    if (layout == kPadDouble) return launch_slab_kernel<V, OutT, kPadDouble, 4, RAGGED>(p, grid, lds, stream);
+    if (layout == kPadSingle) return launch_slab_kernel<V, OutT, kPadSingle, 4, RAGGED>(p, grid, lds, stream);
   }
-  if (NQ == 8) return launch_slab_kernel<V, OutT, kXorSingle, NQ>(p, grid, lds, stream);  // (128-column slabs: one buffer)
-  return layout == kXorDouble ? launch_slab_kernel<V, OutT, kXorDouble, NQ == 8 ? 4 : NQ>(p, grid, lds, stream)
-                              : launch_slab_kernel<V, OutT, kXorSingle, NQ>(p, grid, lds, stream);
+  if (NQ == 8) return launch_slab_kernel<V, OutT, kXorSingle, NQ, RAGGED>(p, grid, lds, stream);  // (128-column slabs: one buffer)
+  return layout == kXorDouble ? launch_slab_kernel<V, OutT, kXorDouble, NQ == 8 ? 4 : NQ, RAGGED>(p, grid, lds, stream)
+                              : launch_slab_kernel<V, OutT, kXorSingle, NQ, RAGGED>(p, grid, lds, stream);
 }
 
 template <int V, typename OutT>
-static hipError_t launch_v(const SpmmArgs &a, int which, hipStream_t stream) {
+static hipError_t launch_v(const SpmmArgs &a, int which, bool ragged, hipStream_t stream) {
   SpmmArgs p = a;
-  if (which == 3) return launch_slab<V, OutT, 4>(a, stream);
-  if (which == 5) return launch_slab<V, OutT, 2>(a, stream);
-  if (which == 9) return launch_slab<V, OutT, 8>(a, stream);
+  if (which == 3) return ragged ? launch_slab<V, OutT, 4, true>(a, stream) : launch_slab<V, OutT, 4, false>(a, stream);
+  if (which == 5) return ragged ? launch_slab<V, OutT, 2, true>(a, stream) : launch_slab<V, OutT, 2, false>(a, stream);
+  if (which == 9) return ragged ? launch_slab<V, OutT, 8, true>(a, stream) : launch_slab<V, OutT, 8, false>(a, stream);
   if (which == 2) {
     p.n_tiles = (uint32_t)((a.N + 127) / 128);
     p.total_work = (uint32_t)a.m_vec * p.n_tiles * (uint32_t)a.batch;
@@ -1803,6 +1824,10 @@ static hipError_t launch_v(const SpmmArgs &a, int which, hipStream_t stream) {
     // (Not for K above 3072: where such a matrix is denser than 90 % its long rows cost the staged form 1.5x.)
     const bool few_waves = a.K <= 3072 && p.total_work <= 2u * device_cus();
     const bool epilogue = a.bias != nullptr || a.act != 0;  // (the split-row kernel does not apply one)
+    // Ordinary stores take room in the L2 from the rows of B: the gather keeps to non-temporal ones for matrices so tall that
+    // even at 90 % their rows have more than a hundred vectors (24576 x 1152, V = 16, N = 257, 15.7 us against 18.2 with
+    // ordinary ones; 24576 x 576 at N = 1225 47.3 against 30.8).
+    const bool gather_plain = ragged && a.K <= 1024;
     if ((g_kernel_override == 6 || a.N <= 64 || (few_waves && g_kernel_override == 0)) && c_ok) {
       p.n_tiles = (uint32_t)((a.N + 63) / 64);
       p.total_work = (uint32_t)a.m_vec * p.n_tiles * (uint32_t)a.batch;
@@ -1828,9 +1853,11 @@ static hipError_t launch_v(const SpmmArgs &a, int which, hipStream_t stream) {
     } else if (p.total_work > 8u * device_cus()) {
       // more waves than the chip holds at two per SIMD: three per SIMD (the first feed-forward product of the encoder
       // layer, 3072 x 768 at N = 4096, 10.6 -> 9.9 us)
-      hipLaunchKernelGGL((spmm_gather_kernel<V, OutT, 8, 3>), dim3(p.per_xcd * 8u), dim3(64), 0, stream, p);
+      if (gather_plain) hipLaunchKernelGGL((spmm_gather_kernel<V, OutT, 8, 3, true>), dim3(p.per_xcd * 8u), dim3(64), 0, stream, p);
+      else hipLaunchKernelGGL((spmm_gather_kernel<V, OutT, 8, 3>), dim3(p.per_xcd * 8u), dim3(64), 0, stream, p);
     } else {
-      hipLaunchKernelGGL((spmm_gather_kernel<V, OutT, 8>), dim3(p.per_xcd * 8u), dim3(64), 0, stream, p);
+      if (gather_plain) hipLaunchKernelGGL((spmm_gather_kernel<V, OutT, 8, 2, true>), dim3(p.per_xcd * 8u), dim3(64), 0, stream, p);
+      else hipLaunchKernelGGL((spmm_gather_kernel<V, OutT, 8>), dim3(p.per_xcd * 8u), dim3(64), 0, stream, p);
     }
   } else {
     p.n_tiles = (uint32_t)((a.N + 63) / 64);
@@ -1860,6 +1887,13 @@ static bool mfma_kernels_apply(const SpmmArgs &a, bool out_f16) {
          (reinterpret_cast<uintptr_t>(a.C) % (out_f16 ? 2 : 4) == 0) &&
          (reinterpret_cast<uintptr_t>(a.values) % 16 == 0) && (a.stride_values % 8 == 0) &&
          (a.K < (1 << 24)) && (a.N < (1 << 23)) && (b_bytes + 16 <= 0xffffffffull);
+}
+// Whether rows of C begin at any element, so that the pieces of a tile cover parts of lines whose rest another wave writes.
+// Stored non-temporally, as whole pieces are, such parts go out to memory one by one; ordinary stores meet in the L2.
+// 12288 x 256 at 90 %, N = 3137, V = 8, fp32 / fp16: 58.7 / 40.6 us non-temporal, 36.8 / 34.1 so (one column less,
+// rows of whole lines: 29 / 17; the scalar kernel 87 / 82); 12288 x 576 at 70 %: 118 / 81 (slab kernels) and 81 / 75.
+static bool stores_ragged(const SpmmArgs &a, bool out_f16) {
+  return a.N % 8 != 0 || reinterpret_cast<uintptr_t>(a.C) % 16 != 0 || (a.stride_C * (out_f16 ? 2 : 4)) % 16 != 0;
 }
 // Ragged widths of a few short vector-rows stay with the scalar kernel, whose fp32 sums are the host loop's bit for
 // bit: such a launch is at most one wave on every fourth CU, at most sixteen trips of eight gathers long, and its
@@ -1913,6 +1947,7 @@ hipError_t launch_spmm_balanced(const SpmmArgs &a, int V, bool out_f16, const Sc
 }
 
 hipError_t launch_spmm(const SpmmArgs &a, int V, bool out_f16, hipStream_t stream) {
+  const bool ragged = stores_ragged(a, out_f16);
   const int out_size = out_f16 ? 2 : 4;
   const bool fast = mfma_kernels_apply(a, out_f16) && !few_short_rows(a, out_f16);
   int which = 1;
@@ -1962,6 +1997,11 @@ hipError_t launch_spmm(const SpmmArgs &a, int V, bool out_f16, hipStream_t strea
     const bool wide_ok = which == 3 && slab_fits(a.K, V, 8) && a.N >= 192;
     const bool dense_known = a.mean_row_vectors > 0 && (int64_t)a.mean_row_vectors * 5 >= (int64_t)a.K;  // 20 % and denser
     if (wide_ok && (out_f16 || dense_known)) which = 9;
+    // Ragged rows of C leave a slab tile in pieces of 64 to 256 bytes, a gather tile in rows of 512, so short vector-rows are
+    // quicker gathered: N = 3137, V = 8, fp32 / fp16, 3072 x 256 at 90 % 17.3 / 23.7 us with slabs, 13.1 / 11.8 gathered
+    // (at 98 % 17.1 / 23.7 and 11.6 / 9.8), 12288 x 256 at 90 % 47 / 56 and 37 / 34, at 70 % 56 / 62 and 72 / 71, 12288 x 576 at 70 % 81 / 80
+    // and 138 / 137.  The line is at about 50 vectors a row, 90 % of the columns left out where the length is not known.
+    if (ragged && (a.mean_row_vectors > 0 ? a.mean_row_vectors <= 64 : a.K <= 512)) which = 2;
     if (g_kernel_override == 2 || g_kernel_override == 6) which = 2;
     if (g_kernel_override == 3 && slab_ok) which = 3;
     if (g_kernel_override == 9 && slab_fits(a.K, V, 8) && c_ok && a.m_vec >= 64) which = 9;
@@ -1970,8 +2010,8 @@ hipError_t launch_spmm(const SpmmArgs &a, int V, bool out_f16, hipStream_t strea
   }
   if (g_kernel_override == 1) which = 1;
   g_last_kernel = which;
-  if (V == 8) return out_f16 ? launch_v<8, _Float16>(a, which, stream) : launch_v<8, float>(a, which, stream);
-  return out_f16 ? launch_v<16, _Float16>(a, which, stream) : launch_v<16, float>(a, which, stream);
+  if (V == 8) return out_f16 ? launch_v<8, _Float16>(a, which, ragged, stream) : launch_v<8, float>(a, which, ragged, stream);
+  return out_f16 ? launch_v<16, _Float16>(a, which, ragged, stream) : launch_v<16, float>(a, which, ragged, stream);
 }
 
 }  // namespace sspmm

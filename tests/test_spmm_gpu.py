@@ -602,3 +602,41 @@ def test_ragged_widths_on_the_matrix_kernels(oracle, built_library, V, out_dtype
         assert np.all(got[lo + M * N:lo + stride_c] == 12345.0), b
         want = oracle.spmm(m_vec, V, N, K, off, cols, vals[b], B[b], threads=8)
         assert max_rel_err(got[lo:lo + M * N].reshape(M, N), want) <= tol, b
+
+
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("K,want", [(512, 2), (520, None)])
+def test_ragged_widths_of_short_rows_are_gathered(oracle, built_library, K, want, out_dtype):
+    """Where whole widths take the slab kernels, ragged ones do from K > 512 on, and gather below."""
+    from sspmm_amd import _lib
+    vs = synth.vector_sparse(8 * 512, K, 8, 0.95, seed=K)
+    check(oracle, vs, synth.dense_rhs(K, 2048, seed=1), out_dtype)
+    whole = _lib.lib().sspmm_last_kernel()
+    assert whole in (3, 9)
+    check(oracle, vs, synth.dense_rhs(K, 2047, seed=2), out_dtype)
+    assert _lib.lib().sspmm_last_kernel() == (want or whole)
+
+
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.float16])
+def test_one_column_more_costs_little(built_library, out_dtype):
+    """Rows of C that begin anywhere: the parts of lines at the ends of a tile meet in the L2.  (12288 x 256, 90 %: measured
+    1.2 and 1.9 times the time of N = 3136; with non-temporal stores 3.9 and 3.8 times.)"""
+    rng = np.random.default_rng(0)
+    off = torch.arange(1537, dtype=torch.int32, device="cuda") * 26
+    cols = torch.from_numpy(np.concatenate([np.sort(rng.permutation(256)[:26]) for _ in range(1536)]).astype(np.int32)).cuda()
+    vals = torch.randn(cols.numel() * 8, device="cuda").half()
+    times = []
+    for N in (3136, 3137):
+        B = torch.randn(256, N, device="cuda").half()
+        best = 1e9
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(20):
+                sspmm_amd.spmm(None, off, cols, vals, B, 8, out_dtype=out_dtype)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        times.append(best)
+    print("ms of 20 products, N = 3136 and 3137:", times, flush=True)
+    assert times[1] <= 2.6 * times[0], times
