@@ -62,6 +62,9 @@ const char *sspmm_error_string(int code);
  *   B and C are row-major and dense; C is fully overwritten, all-zero vector-rows included;
  *   K*N and nvec*V must be below 2^31.  row_indices may be NULL (natural order); results do
  *   not depend on it.
+ *   Which kernel runs, and with it the order of the fp32 sums, follows from the sizes.  The order of a plain host
+ *   loop over the vectors is the scalar kernel's, which takes N < 8, values that are not 16-byte aligned, and,
+ *   where rows of B or C are not whole 16-byte pieces, small products: K <= 128 and m_vec * ceil(N / 64) * batch <= 64.
  */
 int sspmm_f16_f32(int m_vec, int V, int N, int K, const int32_t *row_indices, const int32_t *row_offsets,
                   const int32_t *col_idx, const sspmm_half_t *values, const sspmm_half_t *B, float *C,

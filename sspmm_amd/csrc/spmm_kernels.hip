@@ -1875,12 +1875,11 @@ static bool whole_pieces(const SpmmArgs &a, bool out_f16) {
 }
 // The MFMA kernels take any width from one piece (eight columns) on (see unit_col).  Against the scalar kernel, which
 // served widths that are no multiple of eight before: 1024 x 1152 at 90 %, V = 8, N = 1225, fp32: 25.6 us for the scalar
-// kernel alone, now below the 11 us of the call; 128 x 2659 at 80 %, N = 30: 86 -> 11 us a call; 512-wide encoder layer on
+// kernel alone, now below the 6.9 us of the call; 128 x 2659 at 80 %, N = 30: 86 -> 11 us a call; 512-wide encoder layer on
 // 7 x 101 tokens 238 -> 154 us.  The error against float64 is a quarter to all of the scalar kernel's on fourteen such products
 // (7e-8 to 1.7e-7 where it has 1.8e-7 to 6e-7).
-// the value vectors are fetched
-// with 8-byte (V = 8) or 16-byte (V = 16) loads per lane from aligned memory; 24-bit multiplies bound K and 2N; one
-// buffer descriptor must span B.
+// The value vectors are fetched with 8-byte (V = 8) or 16-byte (V = 16) loads per lane from aligned memory; 24-bit
+// multiplies bound K and 2N; one buffer descriptor must span B.
 static bool mfma_kernels_apply(const SpmmArgs &a, bool out_f16) {
   const uint64_t b_bytes = (uint64_t)a.K * (uint64_t)a.N * 2u;
   return (a.N >= 8) && (reinterpret_cast<uintptr_t>(a.B) % 2 == 0) &&
@@ -1895,9 +1894,12 @@ static bool mfma_kernels_apply(const SpmmArgs &a, bool out_f16) {
 static bool stores_ragged(const SpmmArgs &a, bool out_f16) {
   return a.N % 8 != 0 || reinterpret_cast<uintptr_t>(a.C) % 16 != 0 || (a.stride_C * (out_f16 ? 2 : 4)) % 16 != 0;
 }
-// Ragged widths of a few short vector-rows stay with the scalar kernel, whose fp32 sums are the host loop's bit for
-// bit: such a launch is at most one wave on every fourth CU, at most sixteen trips of eight gathers long, and its
-// time is the call itself.
+// Ragged widths of a few short vector-rows stay with the scalar kernel where no kernel is forced: K <= 128 and at most 64 of its
+// waves.  Not for speed but for its sums, which are the host loop's bit for bit, as all ragged widths' once were: callers that
+// compare small products with that loop keep their bits, and beyond the line (at K = 129, at the 65th wave, as where any other
+// two kernels meet) the order of the sums changes.  What it costs, the kernel alone, five vector-rows, V = 8, N = 130, scalar / matrix kernel: rows
+// of 3 vectors 2.6 / 2.9 us, of 12 3.2 / 2.9, of 38 4.9 / 3.2, of 76 (K = 128 at 40 %) 7.4 / 3.3 (V = 16 15.8 / 3.4), in a call
+// of 6.9.
 static bool few_short_rows(const SpmmArgs &a, bool out_f16) {
   return !whole_pieces(a, out_f16) && a.K <= 128 && (uint64_t)a.m_vec * (uint64_t)((a.N + 63) / 64) * (uint64_t)a.batch <= 64u;
 }
@@ -1949,7 +1951,8 @@ hipError_t launch_spmm_balanced(const SpmmArgs &a, int V, bool out_f16, const Sc
 hipError_t launch_spmm(const SpmmArgs &a, int V, bool out_f16, hipStream_t stream) {
   const bool ragged = stores_ragged(a, out_f16);
   const int out_size = out_f16 ? 2 : 4;
-  const bool fast = mfma_kernels_apply(a, out_f16) && !few_short_rows(a, out_f16);
+  const bool forced = g_kernel_override == 2 || g_kernel_override == 3 || g_kernel_override == 6 || g_kernel_override == 9;
+  const bool fast = mfma_kernels_apply(a, out_f16) && (forced || !few_short_rows(a, out_f16));
   int which = 1;
   if (fast) {
     // The slab kernel pays off when enough vector-rows share a slab and there are enough

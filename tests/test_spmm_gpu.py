@@ -168,7 +168,8 @@ def test_narrow_right_hand_side_on_a_wide_matrix(oracle, built_library, V, out_d
 @pytest.mark.parametrize("V", [8, 16])
 @pytest.mark.parametrize("N", [1, 3, 17, 66, 130])
 def test_odd_widths_take_the_generic_kernel_and_match_the_oracle_bit_for_bit(oracle, built_library, V, N):
-    """N % 8 != 0 runs the scalar kernel, which adds in the oracle's order: fp32 results are identical."""
+    """N % 8 != 0 runs the scalar kernel on products as small as these, which adds in the oracle's order: fp32 results are
+    identical."""
     vs = synth.vector_sparse(5 * V, 70, V, 0.5, seed=40 + N)
     got, want = check(oracle, vs, synth.dense_rhs(70, N, seed=N))
     assert np.array_equal(got, want)
@@ -640,3 +641,35 @@ def test_one_column_more_costs_little(built_library, out_dtype):
         times.append(best)
     print("ms of 20 products, N = 3136 and 3137:", times, flush=True)
     assert times[1] <= 2.6 * times[0], times
+
+
+@pytest.mark.parametrize("V", [8, 16])
+@pytest.mark.parametrize("m_vec,K,N,batch,scalar", [(5, 128, 130, 1, True), (5, 129, 130, 1, False), (64, 128, 63, 1, True), (65, 128, 63, 1, False),
+                                                    (16, 100, 66, 2, True), (16, 100, 66, 3, False), (5, 70, 128, 1, False), (5, 70, 7, 1, True)])
+def test_small_ragged_products_are_the_host_loops_bit_for_bit(oracle, built_library, V, m_vec, K, N, batch, scalar):
+    """Widths that are no multiple of eight stay with the scalar kernel up to K = 128 and 64 of its waves, whose sums are the
+    oracle's bit for bit; beyond, and for whole widths, they run on the matrix kernels.  A kernel that is forced runs in
+    either case."""
+    from sspmm_amd import _lib
+    L = _lib.lib()
+    vs = synth.vector_sparse(m_vec * V, K, V, 0.5, seed=K + N)
+    vals = np.stack([vs.values] * batch)
+    B = np.stack([synth.dense_rhs(K, N, seed=b) for b in range(batch)])
+    product = lambda: sspmm_amd.bspmm(None, dev(vs.row_offsets), dev(vs.col_idx), dev(vals), dev(B), V, out_dtype=torch.float32).cpu().numpy()  # noqa: E731
+    got = product()
+    assert (L.sspmm_last_kernel() == 1) == scalar
+    want = [oracle.spmm(vs.m_vec, V, N, K, vs.row_offsets, vs.col_idx, vs.values, B[b]) for b in range(batch)]
+    for b in range(batch):
+        if scalar:
+            assert np.array_equal(got[b], want[b])
+        assert max_rel_err(got[b], want[b]) <= TIGHT_F32
+    for force in (1, 2, 6):
+        L.sspmm_select_kernel(force)
+        try:
+            got = product()
+            ran = L.sspmm_last_kernel()
+        finally:
+            L.sspmm_select_kernel(0)
+        assert ran == (1 if N < 8 else 6 if (force, N <= 64) == (2, True) else force)
+        for b in range(batch):
+            assert max_rel_err(got[b], want[b]) <= TIGHT_F32
