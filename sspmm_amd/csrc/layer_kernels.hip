@@ -250,10 +250,17 @@ hipError_t launch_add_layernorm(int H, int T, const uint16_t *x, const uint16_t 
                                 const uint16_t *beta, float eps, uint16_t *out, hipStream_t stream) {
   // 16 tokens and eight waves per workgroup, six rows per thread in flight (measured on 768 x 4096 against 32 and 64
   // tokens, 4 to 16 waves, 3 to 12 rows: 8.5 us against 9-15); up to 1024 features the sums fit the registers of that shape,
-  // beyond they take the pass over LDS
-  if (H <= 512) return launch_ln_held<4>(H, T, x, a, gamma, beta, eps, out, stream);
-  if (H <= 768) return launch_ln_held<6>(H, T, x, a, gamma, beta, eps, out, stream);
-  if (H <= 1024) return launch_ln_held<8>(H, T, x, a, gamma, beta, eps, out, stream);
+  // beyond they take the pass over LDS.  So do most calls of 40 MiB and more, which is more than the L2 holds: the held sums'
+  // registers leave fewer workgroups on a CU (three instead of four up to 512 features, two beyond; held to fewer they spill,
+  // 512 x 8192 8.0 -> 8.8 us).  Held / over LDS, with a residual: 256 x 32768 23.7 / 20.5 us, 320 x 24576 21.6 / 19.8, 512 x 16384 21.5 /
+  // 19.3, 512 x 65536 96 / 94, 448 x 24576 30.2 / 31.5; without: 384 x 32768 25.2 / 22.3, 512 x 32768 32.7 / 29.0, 640 x 32768 39.7 / 36.1,
+  // 1024 x 16384 31.1 / 24.8.  On the other side: 384 x 16384 12.4 / 13.9, 512 x 8192 8.0 / 9.6, 128 x 65536 23.9 / 25.4 and, without,
+  // 160 x 131072 41.4 / 47.0; more than 512 features with a residual, 640 x 32768 55.0 / 58.5, 1024 x 32768 84.9 / 91.2.
+  const bool large = (int64_t)H * T * (a ? 6 : 4) >= (40 << 20);
+  const bool held = H <= 1024 && !(large && H >= 256 && (H <= 512 || !a));
+  if (held && H <= 512) return launch_ln_held<4>(H, T, x, a, gamma, beta, eps, out, stream);
+  if (held && H <= 768) return launch_ln_held<6>(H, T, x, a, gamma, beta, eps, out, stream);
+  if (held) return launch_ln_held<8>(H, T, x, a, gamma, beta, eps, out, stream);
   return launch_ln<16, 512, 6>(H, T, x, a, gamma, beta, eps, out, stream);
 }
 

@@ -243,3 +243,10 @@ def test_sparse_linear_fuses_bias_and_activation(built_library):
     from sspmm_amd import _lib
     L = _lib.lib()
     assert L.sspmm_linear_f16(1, 16, 8, 8, 0, 0, 0, 0, 0, 2, 0, 0) == 1  # unknown activation
+
+
+@pytest.mark.parametrize("H,T,residual", [(255, 27416, True), (256, 27304, True), (256, 27308, True), (512, 20476, False), (512, 20480, False),
+                                         (513, 20440, False), (1024, 10236, False), (1024, 10240, False), (1024, 10240, True)])
+def test_feature_major_add_layernorm_of_more_than_the_caches_hold(built_library, H, T, residual):
+    """Either side of 40 MiB of operands, from where most widths go through LDS."""
+    test_feature_major_add_layernorm_matches_torch(built_library, H, T, residual)
