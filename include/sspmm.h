@@ -174,10 +174,13 @@ int sspmm_plan_batched_f16_f16(const sspmm_plan_t *plan, int batch, int N, const
  *   All calls on one GPU share the array: two calls that overlap on a GPU (different streams,
  *   or threads) race and give wrong results; calls on one stream are safe.
  *   The first call on a device looks the array's address up and must come before any capture:
- *   made on a capturing stream it returns hipErrorInvalidValue and records nothing.  Patterns that
- *   the load-balanced kernel does not cover (N not a multiple of 8, unaligned pointers) take the
- *   kernels of sspmm_f16_f32 and use no scratch.  Same results as sspmm_plan_batched_f16_f32 with a plan of the same pattern, bit
- *   for bit, as long as the plan's panels also fit 8 MB of partial tiles.
+ *   made on a capturing stream it returns hipErrorInvalidValue and records nothing.
+ *   Same results as sspmm_plan_batched_f16_f32 with a plan of the same pattern, bit for bit, as long
+ *   as the plan's panels also fit 8 MB of partial tiles and rows of B and C are whole 16-byte
+ *   pieces (N a multiple of 8, 16-byte aligned pointers).  Products of other widths or alignments
+ *   run on the kernels of sspmm_f16_f32 and give its results, bit for bit: they use no scratch and build no
+ *   schedule, so they may overlap and may be the first call, inside a capture too.  (A plan cuts long
+ *   vector-rows at every width from 8 on and adds the panels' fp32 sums in another order.)
  */
 #define SSPMM_ERROR_STATIC_SCRATCH_TOO_SMALL 9001
 int sspmm_noalloc_f16_f32(int m_vec, int V, int N, int K, const int32_t *row_offsets, const int32_t *col_idx,

@@ -147,3 +147,42 @@ def test_two_patterns_recorded_into_one_graph(built_library):
         torch.cuda.synchronize()
         assert torch.equal(outs[0], eager[0]), replay
         assert torch.equal(outs[1], eager[1]), replay
+
+
+@pytest.mark.parametrize("V", [8, 16])
+@pytest.mark.parametrize("N", [9, 63, 130, 257])
+def test_ragged_widths_give_the_plain_products_bits_and_the_plans_within_rounding(oracle, built_library, V, N):
+    """N that is no multiple of eight, on a skewed pattern: the allocation-free entry is sspmm_f16_f32 bit for bit, the plan
+    cuts the long rows and differs by the order of its fp32 sums."""
+    L = _lib.lib()
+    vs = _pattern(300, 6000, V, seed=V, long_rows=24)
+    B = synth.dense_rhs(6000, N, seed=N)
+    got, planned, cut = _both(L, vs, B, N)
+    assert cut > 0 and L.sspmm_last_kernel() == 7
+    plain = torch.empty_like(got)
+    ro, ci, vv, dB = dev(vs.row_offsets), dev(vs.col_idx), dev(vs.values), dev(B)
+    assert L.sspmm_f16_f32(vs.m_vec, V, N, vs.K, None, ro.data_ptr(), ci.data_ptr(), vv.data_ptr(), dB.data_ptr(), plain.data_ptr(),
+                           torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(got, plain)
+    ref = oracle.spmm(vs.m_vec, V, N, 6000, vs.row_offsets, vs.col_idx, vs.values, B, threads=8)
+    for out in (got, planned):
+        assert max_rel_err(out.cpu().numpy(), ref) <= TIGHT_F32
+
+
+def test_ragged_widths_may_overlap(oracle, built_library):
+    """Two streams at once: such products use no scratch.  (Enough work on each that they do run side by side.)"""
+    L = _lib.lib()
+    streams, jobs = [torch.cuda.Stream(), torch.cuda.Stream()], []
+    for k in range(2):
+        vs = _pattern(2000, 6000, 8, seed=50 + k, long_rows=40)
+        B = synth.dense_rhs(6000, 129, seed=k)
+        jobs.append((vs, B, [dev(a) for a in (vs.row_offsets, vs.col_idx, vs.values, B)], torch.zeros(vs.m_vec * 8, 129, device="cuda")))
+    torch.cuda.synchronize()
+    for _ in range(20):
+        for s, (vs, _, (ro, ci, vv, dB), out) in zip(streams, jobs):
+            assert L.sspmm_noalloc_f16_f32(vs.m_vec, 8, 129, 6000, ro.data_ptr(), ci.data_ptr(), vv.data_ptr(), dB.data_ptr(), out.data_ptr(),
+                                           s.cuda_stream) == 0
+    torch.cuda.synchronize()
+    for vs, B, _, out in jobs:
+        ref = oracle.spmm(vs.m_vec, 8, 129, 6000, vs.row_offsets, vs.col_idx, vs.values, B, threads=8)
+        assert max_rel_err(out.cpu().numpy(), ref) <= TIGHT_F32
