@@ -4,9 +4,8 @@
 //
 // As separate launches every one of these reads and writes an activation of tokens x 256 to 1024 features, and the
 // matrix products are then bound by those bytes, not by the matrix units.  Here a workgroup keeps TM tokens from the
-// attention's output to the next block's projection: four waves split the
-// output features of every product, the activations pass between the products through LDS as fp16, and the
-// accumulators of the second linear layer stay in registers while the hidden features are made and used 256 at a time.
+// attention's output to the next block's projection: four waves split the output features of every product, the
+// activations pass between the products through LDS as fp16, and the accumulators of the second linear layer stay in registers while the hidden features are made and used 256 at a time.
 //
 // Orientation: out^T[feature, token] = W (MFMA operand A, 16 features x 32 k) * act^T (operand B, 32 k x 16 tokens).
 // Both operands then are eight consecutive k per lane: W comes straight from global memory (row-major as torch keeps it;
@@ -37,7 +36,6 @@ namespace sspmm {
 
 namespace {
 
-typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
@@ -405,7 +403,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
   }
 }
 
-// Up to kPackMost matrices into the order in which the waves above load them: groups of 16 * NJ rows, in each units of
+// Up to BlockPackArgs::kMost matrices into the order in which the waves above load them: groups of 16 * NJ rows, in each units of
 // K columns, in each a 1 KB piece per step of 32 columns and tile, in that the 16 bytes of every lane.
 __global__ __launch_bounds__(256) void block_pack_kernel(const BlockPackArgs p) {
   int i = 0;

@@ -85,6 +85,46 @@ def test_argument_errors_without_device_work(built_library):
     assert L.sspmm_error_string(0) == b"success"
 
 
+def test_argument_errors_of_the_dense_block_entries(built_library):
+    """Widths, alignments, missing operands and sizes beyond what the kernels address, all rejected on the host."""
+    import ctypes as C
+    from sspmm_amd import _lib
+    L = _lib.lib()
+    p = 4096  # a 16-byte aligned pointer value; rejected calls never dereference it
+
+    def rows(outer=2, inner=3, E=64, x=p, x_outer=192, x_inner=64, a=p, gamma=p, beta=p, total=p, out=p):
+        return L.sspmm_add_layernorm_rows_f16(outer, inner, E, x, x_outer, x_inner, a, gamma, beta, 1e-5, total, out, None)
+
+    for bad in (dict(outer=-1), dict(inner=-1), dict(E=96), dict(E=0), dict(x=None), dict(out=None), dict(x_outer=-8), dict(x_outer=4),
+                dict(x_inner=12), dict(x=p + 2), dict(a=p + 8), dict(gamma=p + 4), dict(beta=p + 2), dict(total=p + 8), dict(out=p + 8)):
+        assert rows(**bad) == 1, bad
+    assert rows(outer=0) == 0 and rows(inner=0, x=None) == 0
+
+    def dense(outer=2, inner=3, E=128, x=p, x_outer=384, x_inner=128, pos=None, attn=p, wo=p, mlp=256, w1=p, w2=p, n_out=128, head_dim=0, wt=p,
+              bt=p, x_out=p, out=p):
+        return L.sspmm_block_dense_f16(outer, inner, E, x, x_outer, x_inner, pos, 1.0, attn, wo, p, p, p, 1e-5, mlp, w1, p, w2, p, p, p, 1e-5,
+                                       n_out, head_dim, wt, bt, x_out, out, None)
+
+    for bad in (dict(outer=-1), dict(inner=-1), dict(E=64), dict(E=192), dict(E=1024), dict(mlp=0), dict(mlp=128), dict(mlp=-256),
+                dict(mlp=(1 << 20) + 256), dict(n_out=96), dict(n_out=-64), dict(n_out=(1 << 20) + 64), dict(n_out=0), dict(wt=None), dict(x=None),
+                dict(out=None), dict(wo=None), dict(w1=None), dict(w2=None), dict(x_outer=4), dict(x_inner=-8), dict(head_dim=16),
+                dict(head_dim=64, n_out=192), dict(x=p + 2), dict(pos=p + 8), dict(attn=p + 2), dict(bt=p + 8), dict(x_out=p + 4), dict(out=p + 2)):
+        assert dense(**bad) == 1, bad
+    assert dense(outer=0) == 0 and dense(inner=0, x=None) == 0
+
+    def pack(src=p, rows=256, cols=128, group=32, dst=p, count=1):
+        return L.sspmm_block_pack_f16(count, (C.c_void_p * 1)(src), (C.c_int32 * 1)(rows), (C.c_int32 * 1)(cols), (C.c_int32 * 1)(group), dst, None)
+
+    for bad in (dict(count=-1), dict(src=None), dict(src=p + 2), dict(dst=None), dict(dst=p + 8), dict(group=16), dict(group=48), dict(rows=240),
+                dict(rows=0), dict(cols=96), dict(cols=0), dict(rows=1 << 20, cols=1 << 10)):
+        assert pack(**bad) == 1, bad
+    assert L.sspmm_block_pack_f16(1, None, None, None, None, p, None) == 1
+    assert L.sspmm_block_pack_f16(0, None, None, None, None, None, None) == 0
+
+    assert L.svc_split_row_ptr(-1, 4, p, p, p, p, None) == 1 and L.svc_split_row_ptr(1, 4, p, None, p, p, None) == 1
+    assert L.svc_split_row_ptr(0, 0, None, None, None, None, None) == 0
+
+
 def test_python_operator_rejects_bad_arguments(built_library):
     import torch
     import sspmm_amd
