@@ -341,8 +341,8 @@ int svc_fill_batched(int count, int groups, const int32_t *mat_rows, int M_total
  * The stack's row pointer cut into the matrices' own, all in one launch: matrix i's entries, from zero, at out_ptr +
  * mat_groups[i] + i (groups + count entries in all), and bounds[count + 1], the first vector of every matrix and the end.
  */
-int svc_split_row_ptr(int count, int groups, const int32_t *mat_groups, const int32_t *vec_row_ptr, int32_t *out_ptr, int32_t *bounds,
-                      void *hip_stream);
+int svc_split_row_ptr(int count, int groups, const int32_t *mat_groups, const int32_t *vec_row_ptr, int32_t *out_ptr,
+                      int32_t *bounds, void *hip_stream);
 
 /* ------------------------------------------------------------------------------------------
  * Row reordering ahead of the SVC: the step the reference runs as `python row_merge_reorder.py`
@@ -395,28 +395,33 @@ int sspmm_add_layernorm_rows_f16(int outer, int inner, int E, const sspmm_half_t
  * The dense part of a sparse attention block in one launch, on outer x inner token-major rows of E features:
  *   s  = attn Wo^T + bo + x            n = LayerNorm2(s)
  *   x' = (n W1^T + b1) W2^T + b2 + x   h = LayerNormN(x')      (the next block's first, or the model's last)
- * out = h Wt^T + bt (n_out features; the next block's input projection, or the head), or h itself where wt is NULL, and
- * x' into x_out unless that is NULL.  With pos [outer, E] x is an embedding and fp16(x * x_scale) + pos, rounded to fp16
- * again, stands in its place.  attn NULL: x' = x, and what only leads to it (wo .. b2, eps2, mlp) is not
- * looked at.  out is [outer, inner, n_out], or with head_dim = 32, 64 or 128 (n_out then a multiple of E) split into heads as
- * sspmm_sparse_attention_heads_f16 reads them best: [n_out / E, inner, E / head_dim, outer, head_dim].  n and the hidden features are rounded to fp16, sums are fp32.  The weight matrices are packed (below): wo
- * [E, E] and w2 [E, mlp] in groups of E / 4 rows, w1 [mlp, E] and wt [n_out, E] of 64; biases, gammas and betas may be NULL.  Row (i, j) of x is at x + i * x_outer + j * x_inner elements (multiples
- * of 8), everything else is dense; 16-byte aligned pointers.  E = 128, 256 or 512, mlp a multiple of 256, n_out of 64.
+ * out = h Wt^T + bt (n_out features; the next block's input projection, or the head), or h itself where wt
+ * is NULL, and x' into x_out unless that is NULL.  With pos [outer, E] x is an embedding and
+ * fp16(x * x_scale) + pos, rounded to fp16 again, stands in its place.  attn NULL: x' = x, and what only
+ * leads to it (wo .. b2, eps2, mlp) is not looked at.  out is [outer, inner, n_out], or with head_dim = 32, 64
+ * or 128 (n_out then a multiple of E) split into heads as sspmm_sparse_attention_heads_f16 reads them best:
+ * [n_out / E, inner, E / head_dim, outer, head_dim].  n and the hidden features are rounded to fp16, sums are
+ * fp32.  The weight matrices are packed (below): wo [E, E] and w2 [E, mlp] in groups of E / 4 rows, w1
+ * [mlp, E] and wt [n_out, E] of 64; biases, gammas and betas may be NULL.  Row (i, j) of x is at
+ * x + i * x_outer + j * x_inner elements (multiples of 8), everything else is dense; 16-byte aligned pointers.
+ * E = 128, 256 or 512, mlp a multiple of 256, n_out of 64, both up to 2^20.
  */
-int sspmm_block_dense_f16(int outer, int inner, int E, const sspmm_half_t *x, int64_t x_outer, int64_t x_inner, const sspmm_half_t *pos,
-                          float x_scale, const sspmm_half_t *attn, const sspmm_half_t *wo, const sspmm_half_t *bo, const sspmm_half_t *gamma2, const sspmm_half_t *beta2,
-                          float eps2, int mlp, const sspmm_half_t *w1, const sspmm_half_t *b1, const sspmm_half_t *w2,
-                          const sspmm_half_t *b2, const sspmm_half_t *gamma_n, const sspmm_half_t *beta_n, float eps_n, int n_out, int head_dim,
-                          const sspmm_half_t *wt, const sspmm_half_t *bt, sspmm_half_t *x_out, sspmm_half_t *out, void *hip_stream);
+int sspmm_block_dense_f16(int outer, int inner, int E, const sspmm_half_t *x, int64_t x_outer, int64_t x_inner,
+                          const sspmm_half_t *pos, float x_scale, const sspmm_half_t *attn, const sspmm_half_t *wo,
+                          const sspmm_half_t *bo, const sspmm_half_t *gamma2, const sspmm_half_t *beta2, float eps2,
+                          int mlp, const sspmm_half_t *w1, const sspmm_half_t *b1, const sspmm_half_t *w2,
+                          const sspmm_half_t *b2, const sspmm_half_t *gamma_n, const sspmm_half_t *beta_n, float eps_n,
+                          int n_out, int head_dim, const sspmm_half_t *wt, const sspmm_half_t *bt, sspmm_half_t *x_out,
+                          sspmm_half_t *out, void *hip_stream);
 
 /*
  * Weight matrices [rows, cols] (row-major, 16-byte aligned) into the order in which sspmm_block_dense_f16 loads them,
- * one after the other into dst: the same elements, fragment by fragment of a matrix instruction.  group[i] = 32, 64 or 128
- * rows belong to one wave; rows[i] a multiple of it, cols[i] of 64.  The four arrays are host memory and are read before
- * the call returns.
+ * one after the other into dst: the same elements, fragment by fragment of a matrix instruction.  group[i] =
+ * 32, 64 or 128 rows belong to one wave; rows[i] a multiple of it, cols[i] of 64.  The four arrays are host
+ * memory and are read before the call returns.
  */
-int sspmm_block_pack_f16(int count, const sspmm_half_t *const *src, const int32_t *rows, const int32_t *cols, const int32_t *group,
-                         sspmm_half_t *dst, void *hip_stream);
+int sspmm_block_pack_f16(int count, const sspmm_half_t *const *src, const int32_t *rows, const int32_t *cols,
+                         const int32_t *group, sspmm_half_t *dst, void *hip_stream);
 
 /* ------------------------------------------------------------------------------------------
  * Dense attention on feature-major activations: out = softmax(Q^T K * scale) V per (batch element,

@@ -5,7 +5,8 @@
 // As separate launches every one of these reads and writes an activation of tokens x 256 to 1024 features, and the
 // matrix products are then bound by those bytes, not by the matrix units.  Here a workgroup keeps TM tokens from the
 // attention's output to the next block's projection: four waves split the output features of every product, the
-// activations pass between the products through LDS as fp16, and the accumulators of the second linear layer stay in registers while the hidden features are made and used 256 at a time.
+// activations pass between the products through LDS as fp16, and the accumulators of the second linear layer stay in
+// registers while the hidden features are made and used 256 at a time.
 //
 // Orientation: out^T[feature, token] = W (MFMA operand A, 16 features x 32 k) * act^T (operand B, 32 k x 16 tokens).
 // Both operands then are eight consecutive k per lane: W comes straight from global memory (row-major as torch keeps it;
@@ -23,10 +24,12 @@
 // row: from torch's layout it reads 64 bytes of each of sixteen rows, which lie 512 to 2048 bytes apart on a few of the L2's
 // channels, and 32 tokens per workgroup took 61 us instead of 27 (8192 tokens).
 //
-// 256 features, 1024 hidden, 768 out, with the LayerNorms: 8192 tokens 24 us, 32768 tokens 59 us (0.9 PFLOP/s), against
-// 104 (the host) and 121 for the four library products and two LayerNorm launches.  What is left is the chain of products
-// and LayerNorms of one workgroup (27 us with the card to itself, 64 tokens), the stream of the weights, and for the
-// large sizes the vector instructions between the products.
+// 256 features, 1024 hidden, 768 out, with the LayerNorms: 8192 tokens 26 us, 32768 tokens 58 us (0.9 PFLOP/s) back to
+// back, 27 and 63 between the attention launches of a model, against 104 (the host) and 121 for the four library products
+// and two LayerNorm launches.  Counters of the launches in a model: the CU's path to its first-level cache passes 64 bytes
+// a cycle and is used for 64 % of the cycles at 8192 tokens and 73 % at 32768 (two workgroups per CU fetch the weights
+// each), nearly all of it weights; the matrix units are busy for 24 and 47 %, LDS for 15 and 29 %.  The rest at 8192 tokens
+// is waiting: a SIMD holds one wave there, and nothing covers its LayerNorms, barriers and the start of a product.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

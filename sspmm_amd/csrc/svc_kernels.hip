@@ -185,8 +185,8 @@ __device__ __forceinline__ uint32_t final_slots(int n) {
 // construction every key sits in the slot of its own number, whatever went before, so the order is the ascending
 // one.  Dense groups of moderately wide matrices are like this, and most groups of a pruned-weight dataset: twenty matrices
 // of 512 and 2048 columns at 50 to 98 % sparsity spend 55 + 108 us in the two merge launches where the replay of every
-// group spent 464 + 163; what is left of the 108 is the replay of the 98 % matrices.  svc_count marks such groups with this bit, on the group's count until the prefix sum and in its class list
-// from then on.
+// group spent 464 + 163; what is left of the 108 is the replay of the 98 % matrices.  svc_count marks such groups with this
+// bit, on the group's count until the prefix sum and in its class list from then on.
 static constexpr int kAscending = (int)0x80000000u;
 static constexpr int kGroupBits = 0x7fffffff;
 
