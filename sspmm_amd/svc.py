@@ -69,7 +69,33 @@ class _RowPointer:
     its shallow copies, which share this object) has the tensor, so nobody can have written it."""
 
     def __init__(self, whole):
-        self.whole, self.alone, self.split = whole, False, None
+        self.whole, self.alone, self.split, self.ahead = whole, False, None, None
+
+    def __getstate__(self):  # (deep copies and pickles: what is on its way to the host stays with the original)
+        return dict(self.__dict__, ahead=None)
+
+
+class _ReadBack:
+    """Device values on their way to the host: what is queued behind this runs on, and wait() lasts until the copy is done."""
+
+    def __init__(self, values):
+        self._host = torch.empty(values.shape, dtype=values.dtype, pin_memory=True)
+        self._host.copy_(values, non_blocking=True)
+        self._done = torch.cuda.Event()
+        self._done.record()
+
+    def wait(self):
+        self._done.synchronize()
+        return self._host.tolist()
+
+
+def _split_row_ptr(count, groups, mat_groups, whole):
+    """(all matrices' row pointers from zero, one after the other; the first vector of each and the end of the last)"""
+    own = torch.empty(groups + count, dtype=torch.int32, device=whole.device)
+    bounds = torch.empty(count + 1, dtype=torch.int32, device=whole.device)
+    _lib.check(_lib.call(_lib.lib().svc_split_row_ptr, whole.device, count, groups, mat_groups.data_ptr(), whole.data_ptr(),
+                         own.data_ptr(), bounds.data_ptr()), "svc_split_row_ptr")
+    return own, bounds
 
 
 class SvcBatch:
@@ -85,6 +111,7 @@ class SvcBatch:
     def __init__(self, V, rows, cols, groups_of, vec_row_ptr, vec_col, vec_val, mat_groups=None):
         self.V, self.rows, self.cols = V, rows, cols
         self._groups = groups_of            # host: first group of every matrix, [count + 1]
+        self._first = groups_of.tolist() if hasattr(groups_of, "tolist") else list(groups_of)
         self._mat_groups = mat_groups       # the same on the device, or None
         self._row_ptr = _RowPointer(vec_row_ptr)
         self.vec_col, self.vec_val = vec_col, vec_val
@@ -92,7 +119,7 @@ class SvcBatch:
     @property
     def vec_row_ptr(self):
         p = self._row_ptr
-        p.alone, p.split = False, None
+        p.alone, p.split, p.ahead = False, None, None
         return p.whole
 
     @vec_row_ptr.setter
@@ -106,10 +133,11 @@ class SvcBatch:
         # (row pointer from zero, first vector, end) of matrix i, whose groups are g0 .. g1 - 1.  Of a row pointer that
         # svc_batched made and nobody else has seen, one launch rebases all matrices' and one read-back brings their
         # extents: twenty matrices one by one took a launch each (0.4 ms a pass, 0.3 ms like this), and with a
-        # read-back each 1.2 ms.  Any other one is a caller's tensor (of any type, stride, length and device), written in
-        # ways that leave no trace on the host: those go one by one.  A piece of the split is handed out once (what a
-        # caller writes into it is not in the next one), on the stream that it was allocated on, and in the
-        # inference mode that it was made in.
+        # read-back each 1.2 ms.  svc_batched queues both between its phases (`ahead`), so that the host has the extents while
+        # the merge still runs and takes the next stack (twenty matrices 297 -> 212 us a pass).  Any other one is a caller's
+        # tensor (of any type, stride, length and device), written in ways that leave no trace on the host: those go one by
+        # one.  A piece of the split is handed out once (what a caller writes into it is not in the next one), on the stream
+        # that it was allocated on, and in the inference mode that it was made in.
         p = self._row_ptr
         whole = p.whole
         if not p.alone:
@@ -118,20 +146,21 @@ class SvcBatch:
             return ptr - lo, lo, hi
         stream, split = _lib.stream_of(whole.device), p.split
         if split is None:
-            count, groups = len(self), int(self._groups[-1])
-            own = torch.empty(groups + count, dtype=torch.int32, device=whole.device)
-            bounds = torch.empty(count + 1, dtype=torch.int32, device=whole.device)
-            _lib.check(_lib.call(_lib.lib().svc_split_row_ptr, whole.device, count, groups, self._mat_groups.data_ptr(), whole.data_ptr(),
-                                 own.data_ptr(), bounds.data_ptr()), "svc_split_row_ptr")
-            sizes = [int(self._groups[j + 1] - self._groups[j]) + 1 for j in range(count)]
-            p.split = split = (bounds.tolist(), dict(enumerate(own.split(sizes))), stream, own.is_inference())
+            count, ahead = len(self), p.__dict__.pop("ahead", None)  # (by one thread only)
+            if ahead is not None and ahead[2] == stream and ahead[0].is_inference() == torch.is_inference_mode_enabled():
+                own, bounds = ahead[0], ahead[1].wait()
+            else:
+                own, bounds = _split_row_ptr(count, self._first[-1], self._mat_groups, whole)
+                bounds = bounds.tolist()
+            sizes = [b - a + 1 for a, b in zip(self._first, self._first[1:])]
+            p.split = split = (bounds, dict(enumerate(own.split(sizes))), stream, own.is_inference())
         bounds, own, own_stream, inference = split
         lo, hi = bounds[i], bounds[i + 1]
         mine = own.pop(i, None) if stream == own_stream and inference == torch.is_inference_mode_enabled() else None
         return (whole[g0:g1 + 1] - lo if mine is None else mine), lo, hi
 
     def matrix(self, i):
-        g0, g1 = int(self._groups[i]), int(self._groups[i + 1])
+        g0, g1 = self._first[i], self._first[i + 1]
         if g1 < g0:
             raise IndexError("matrix %d of %d" % (i, len(self)))
         ptr, lo, hi = self._taken(i, g0, g1)   # (the views need their extent on the host)
@@ -180,7 +209,8 @@ def svc_batched(mat_rows, K_max, row_ptr, col_ind, csr_val, V, order="cpython", 
 
     mat_rows: host int array [count + 1], first row of every matrix in the stack (as stack_csr returns it);
     row_ptr[M_total + 1], col_ind[nnz]: int32 GPU tensors of the stacked CSR; csr_val: fp16 GPU tensor or None.
-    Nothing is read back: both phases are queued on the current stream.  Returns an SvcBatch."""
+    Nothing is waited for: both phases are queued on the current stream, between them the matrices' extents, on their way
+    to the host for matrix().  Returns an SvcBatch."""
     import numpy as np
     if order not in _ORDERS:
         raise ValueError("order must be 'cpython' or 'sorted'")
@@ -192,17 +222,21 @@ def svc_batched(mat_rows, K_max, row_ptr, col_ind, csr_val, V, order="cpython", 
         raise ValueError("row_ptr and col_ind must live on the GPU")
     mat_rows = np.asarray(mat_rows, dtype=np.int64)
     count, M_total = mat_rows.size - 1, int(mat_rows[-1])
-    if count < 0 or row_ptr.numel() != M_total + 1 or np.any(np.diff(mat_rows) < 0):
+    rows = np.diff(mat_rows)
+    if count < 0 or row_ptr.numel() != M_total + 1 or (rows < 0).any():
         raise ValueError("mat_rows must be non-decreasing with mat_rows[-1] + 1 == len(row_ptr)")
-    per = (np.diff(mat_rows) + V - 1) // V
-    groups_of = np.concatenate([[0], np.cumsum(per)]).astype(np.int64)
+    groups_of = np.zeros(count + 1, dtype=np.int64)
+    np.cumsum((rows + V - 1) // V, out=groups_of[1:])
     groups = int(groups_of[-1])
     L = _lib.lib()
     dev = row_ptr.device
     nnz = col_ind.numel()
     with torch.cuda.device(dev):
         stream = torch.cuda.current_stream().cuda_stream
-        d_rows = torch.from_numpy(mat_rows.astype(np.int32)).to(dev)
+        d_rows, capturing, ahead = torch.from_numpy(mat_rows.astype(np.int32)), torch.cuda.is_current_stream_capturing(), None
+        # (from pinned memory the copy waits for nothing; a stream that is captured refuses the other one, as it has to: a replay
+        # would read the numbers from memory that has gone to others)
+        d_rows = d_rows.to(dev) if capturing else d_rows.pin_memory().to(dev, non_blocking=True)
         d_groups = torch.empty(count + 1, dtype=torch.int32, device=dev)
         ws = torch.empty(L.svc_batched_workspace_bytes(count, M_total, nnz, V), dtype=torch.uint8, device=dev)
         vec_row_ptr = (torch.empty if groups > 0 else torch.zeros)(groups + 1, dtype=torch.int32, device=dev)
@@ -212,10 +246,13 @@ def svc_batched(mat_rows, K_max, row_ptr, col_ind, csr_val, V, order="cpython", 
             _lib.check(L.svc_count_batched(count, groups, d_rows.data_ptr(), M_total, K_max, V, row_ptr.data_ptr(),
                                            col_ind.data_ptr(), nnz, _ORDERS[order], d_groups.data_ptr(),
                                            vec_row_ptr.data_ptr(), ws.data_ptr(), stream), "svc_count_batched")
+            if not capturing:
+                own, bounds = _split_row_ptr(count, groups, d_groups, vec_row_ptr)
+                ahead = (own, _ReadBack(bounds), stream)
             _lib.check(L.svc_fill_batched(count, groups, d_rows.data_ptr(), M_total, K_max, V, row_ptr.data_ptr(),
                                           col_ind.data_ptr(), 0 if csr_val is None else csr_val.data_ptr(), nnz,
                                           _ORDERS[order], vec_row_ptr.data_ptr(), ws.data_ptr(), vec_col.data_ptr(),
                                           0 if vec_val is None else vec_val.data_ptr(), stream), "svc_fill_batched")
-    batch = SvcBatch(V, np.diff(mat_rows), cols, groups_of, vec_row_ptr, vec_col, vec_val, d_groups if groups > 0 else None)
-    batch._row_ptr.alone = groups > 0
+    batch = SvcBatch(V, rows, cols, groups_of, vec_row_ptr, vec_col, vec_val, d_groups if groups > 0 else None)
+    batch._row_ptr.alone, batch._row_ptr.ahead = groups > 0, ahead
     return batch

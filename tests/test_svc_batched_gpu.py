@@ -181,6 +181,29 @@ def _stacked(rng, rows, V=8):
     return batch, want, np.concatenate([[0], np.cumsum([(M + V - 1) // V for M in rows])]).tolist()
 
 
+@pytest.mark.parametrize("how", ["deep copy", "pickle", "other stream first", "dropped"])
+def test_extents_on_their_way_to_the_host_stay_with_their_batch(built_library, how):
+    """What svc_batched sends ahead for matrix() is not part of a copy, serves its own stream only, and may be dropped unread."""
+    import copy
+    import io
+    batch, ptr, groups = _stacked(np.random.default_rng(9), [40, 3, 8, 100])
+    if how == "deep copy":
+        _check_matrices(copy.deepcopy(batch), ptr, groups, range(4))
+    elif how == "pickle":
+        f = io.BytesIO()
+        torch.save(batch, f)
+        f.seek(0)
+        _check_matrices(torch.load(f, weights_only=False), ptr, groups, range(4))
+    elif how == "other stream first":
+        torch.cuda.synchronize()
+        with torch.cuda.stream(torch.cuda.Stream()):
+            _check_matrices(batch, ptr, groups, range(4))
+    else:
+        for seed in range(20):
+            _stacked(np.random.default_rng(seed), [8] * (seed + 1))
+    _check_matrices(batch, ptr, groups, range(4))
+
+
 def _check_matrices(batch, ptr, groups, matrices):
     for i in matrices:
         own = ptr[groups[i]:groups[i + 1] + 1]
