@@ -48,6 +48,7 @@
 namespace sspmm {
 
 typedef unsigned long long u64;
+typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 static constexpr u64 kEmpty = ~0ull;
 
 // Size classes by a group's number of columns: the largest sets CPython keeps in tables of 512, 2048, 8192 and
@@ -147,20 +148,14 @@ __device__ __forceinline__ int block_rank_of_flag(bool flag, int *total, int *sc
     *total = (int)__popcll(m);
     return in_wave;
   }
-  const int wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   int *mine = scratch + (turn & 1) * WAVES;
   ++turn;
-  if ((threadIdx.x & 63) == 0) mine[wave] = (int)__popcll(m);
+  if (lane == 0) mine[wave] = (int)__popcll(m);
   __syncthreads();
-  int base = 0, sum = 0;
-#pragma unroll
-  for (int wv = 0; wv < WAVES; ++wv) {
-    const int t = mine[wv];
-    if (wv < wave) base += t;
-    sum += t;
-  }
-  *total = sum;
-  return base + in_wave;
+  const int c = lane < WAVES ? mine[lane] : 0, incl = (int)wave_inclusive_sum((uint32_t)c);
+  *total = __builtin_amdgcn_readlane(incl, WAVES - 1);
+  return __builtin_amdgcn_readlane(incl - c, wave) + in_wave;
 }
 
 __device__ __forceinline__ uint32_t resize_threshold(uint32_t slots) { return (3u * (slots - 1u) + 4u) / 5u; }
@@ -173,8 +168,11 @@ __device__ __forceinline__ uint32_t resized_slots(uint32_t fill) {
 }
 
 // Slots of the table that CPython keeps n keys in once a construction has inserted them all.
+// (A table of less than 50 000 keys grows fourfold, so its thresholds are known; the loop costs a lone wave 2000 cycles, and
+// every construction asks.)
 __device__ __forceinline__ uint32_t final_slots(int n) {
-  uint32_t slots = 8;
+  if (n < 4915) return n < 77 ? (n < 5 ? 8u : n < 19 ? 32u : 128u) : n < 307 ? 512u : n < 1229 ? 2048u : 8192u;
+  uint32_t slots = 32768;
   for (;;) {
     const uint32_t thr = resize_threshold(slots);
     if (n < (int)thr) return slots;
@@ -374,6 +372,17 @@ template <int THREADS, typename PositionOf>
 __device__ __forceinline__ void write_group_output(const SvcArgs &a, int grp, const RowBounds &rows, const int *list, int n,
                                                    PositionOf position_of) {
   const int v0 = a.scanned[grp], n_out = a.scanned[grp + 1] - v0;
+  // (the first entries of the group are on their way while the columns and the zeros leave)
+  constexpr int kHeld = 4;
+  const int e0 = rows.start(0), e_end = rows.start(rows.count);
+  uint32_t col[kHeld];
+  uint16_t val[kHeld];
+#pragma unroll
+  for (int u = 0; u < kHeld; ++u) {
+    const int idx = e0 + u * THREADS + (int)threadIdx.x;
+    col[u] = idx < e_end ? (uint32_t)a.col_ind[idx] : 0xffffffffu;
+    val[u] = idx < e_end && a.vec_val ? a.csr_val[idx] : 0;
+  }
   if (a.vec_col)
     for (int p = threadIdx.x; p < n_out; p += THREADS) a.vec_col[v0 + p] = p < n ? list[p] : 0;
   if (!a.vec_val) return;
@@ -394,14 +403,17 @@ __device__ __forceinline__ void write_group_output(const SvcArgs &a, int grp, co
   if (n == 0) return;
   // the member rows' entries are one contiguous run of the CSR arrays: one pass over it, the row found from the
   // boundaries in registers, so that no load waits for another
-  const int e_end = rows.start(rows.count);
-  for (int idx = rows.start(0) + (int)threadIdx.x; idx < e_end; idx += THREADS) {
-    const uint32_t c = (uint32_t)a.col_ind[idx];
-    const uint16_t value = a.csr_val[idx];
+  const auto put = [&](int idx, uint32_t c, uint16_t value) {
     const int r = rows.row_of(idx);
     const int p = c < (uint32_t)a.K ? position_of(c) : -1;
     if (p >= 0 && p < n_out) out[(int64_t)p * a.V + r] = value;
+  };
+#pragma unroll
+  for (int u = 0; u < kHeld; ++u) {
+    const int idx = e0 + u * THREADS + (int)threadIdx.x;
+    if (idx < e_end) put(idx, col[u], val[u]);
   }
+  for (int idx = e0 + kHeld * THREADS + (int)threadIdx.x; idx < e_end; idx += THREADS) put(idx, (uint32_t)a.col_ind[idx], a.csr_val[idx]);
 }
 
 // Direct mode: a group marked kAscending.  Its columns come out of a bitmap of final_slots(n) bits with a running
@@ -473,11 +485,12 @@ __device__ __forceinline__ void write_ascending_group(const SvcArgs &a, int grp,
       if (x & bit) a.vec_col[v0 + prefix[s >> 5] + __popc(x & (bit - 1u))] = (int)s;
     }
   if (!out) return;
-  uint16_t *dst = in_tile ? tile : out;
   const auto put = [&](int idx, uint32_t c, uint16_t value) {
     if (c >= slots || c >= (uint32_t)a.K) return;
     const int p = prefix[c >> 5] + __popc(bits[c >> 5] & ((1u << (c & 31u)) - 1u));
-    dst[(int64_t)p * a.V + rows.row_of(idx)] = value;
+    const int64_t at = (int64_t)p * a.V + rows.row_of(idx);
+    if (in_tile) tile[at] = value;  // (a pointer that may be either makes it a flat store)
+    else out[at] = value;
   };
   if (held) {
 #pragma unroll
@@ -583,14 +596,32 @@ struct Table32 {
   uint32_t key_bits, key_mask;
 };
 
+// Slot that holds `key`, or -1.  Four slots of the window at a time: a probe of one is an LDS round trip.
 __device__ __forceinline__ int find_slot32(const Table32 &t, uint32_t mask, uint32_t key) {
   uint32_t i, perturb, lin;
   probe_start(key, mask, i, perturb, lin);
   for (;;) {
-    const uint32_t x = t.slots[i + lin];
-    if (x == kEmpty32) return -1;
-    if ((x & t.key_mask) == key) return (int)(i + lin);
-    probe_next(mask, i, perturb, lin);
+    const uint32_t s0 = i + lin;
+    const bool window = i + 9u <= mask;
+    const uint32_t valid = window ? min(10u - lin, 4u) : 1u;
+    uint32_t x[4];
+    // (slots behind the table's end are read and not used: every table is followed by other LDS of the group)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = t.slots[s0 + j];
+    uint32_t found = 4u, free = 4u;
+#pragma unroll
+    for (int j = 3; j >= 0; --j) {
+      found = (x[j] & t.key_mask) == key ? (uint32_t)j : found;
+      free = x[j] == kEmpty32 ? (uint32_t)j : free;
+    }
+    // (an empty slot's low bits may look like the key)
+    if (found < min(free, valid)) return (int)(s0 + found);
+    if (free < valid) return -1;
+    const bool more = window & (lin + 4u <= 9u);
+    const uint32_t shifted = perturb >> 5, jumped = (i * 5u + 1u + shifted) & mask;
+    lin = more ? lin + 4u : 0u;
+    perturb = more ? perturb : shifted;
+    i = more ? i : jumped;
   }
 }
 
@@ -632,8 +663,9 @@ __device__ __forceinline__ void place32(const Table32 &t, uint32_t mask, uint32_
 // Together with its attempt on a slot a key reads the three slots behind it: an entry only ever gets smaller
 // (atomic min), so a slot that holds an earlier key now is lost to this key for good and can be passed without an
 // atomic; if the attempt fails, the next one goes to the first of the three that is free or holds a later key, or to
-// the slot behind them.  The reads are in flight with the atomic and add nothing to the round trip; rounds, and
-// with them the wave-rounds a phase costs, come down to about half.  Passing over slots unseen would also pass
+// the slot behind them.  Rounds, and with them the wave-rounds a phase costs, come down to about half.  (The compiler
+// issues the reads behind the attempt, where a failed one wants them.  Held in flight with it, so that a round is one round
+// trip, every successful attempt pays for them too: phases of a 2500-column group 5 to 15 % longer.)  Passing over slots unseen would also pass
 // over an earlier copy of the same key, which only a row that repeats a column (invalid input) can bring:
 // `safe` = true switches the passing off and the test for the same key on (the caller falls back to it when a
 // group turns out to hold more keys than distinct columns).
@@ -684,18 +716,16 @@ __device__ __forceinline__ void list_store(int *list, int idx, int v) {
 // Writes the keys of a table to list[] in slot order and returns their number; with `final`, the
 // table entries are rewritten as (rank, key).  wcount: one word of LDS per wave.  Contains
 // barriers; the table must be complete (a barrier behind the last insert) on entry.
-// check (optional): compares the new order with the list as it was (the construction's input) and with the input
-// of the construction before (check->before, if kept), and leaves the old list there for the next comparison.
+// check (optional): compares the new order with the list as it was (the construction's input).
 struct OrderCheck {
   bool on;            // off: nothing is compared or kept (both answers "no")
-  int *before;        // LDS copy of the previous construction's input, or null
-  int *wave_words;    // LDS, one int per wave, free between the barriers inside a compaction
   bool same_as_input;   // out: every key landed on the list entry that already held it
-  bool same_as_before;  // out: ... on the entry of `before` that held it (meaningful when `before` was that input)
+  bool same_as_before;  // out: ... on the entry that held it in the input of the construction before (where that is kept)
 };
-template <int THREADS, bool LIST_IN_LDS>
+// (the list in the workspace; wave_words: LDS, one int per wave)
+template <int THREADS>
 __device__ __forceinline__ int compact_table32(const Table32 &t, uint32_t slots, uint32_t *wcount, int *list, bool final,
-                                               OrderCheck *check = nullptr) {
+                                               int *wave_words = nullptr, OrderCheck *check = nullptr) {
   constexpr int WAVES = THREADS / 64;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -728,7 +758,7 @@ __device__ __forceinline__ int compact_table32(const Table32 &t, uint32_t slots,
       kept_u += c;
     }
   }
-  int moved = 0, moved_before = 0;
+  int moved = 0;
   for (uint32_t w0 = w_beg; w0 < w_end; w0 += 4) {
     uint32_t x[4];
 #pragma unroll
@@ -744,34 +774,101 @@ __device__ __forceinline__ int compact_table32(const Table32 &t, uint32_t slots,
       const uint32_t rank = running + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
       running += (uint32_t)__popcll(m);
       if (occ) {
-        // (entry `rank` of either list is written by this thread alone, so what it reads here is the old content)
-        if (check) {
-          const int key = (int)(x[j] & t.key_mask), was = list_load<LIST_IN_LDS>(list, (int)rank);
-          moved |= was != key;
-          if (check->before) {
-            moved_before |= check->before[rank] != key;
-            check->before[rank] = was;
-          }
-        }
-        list_store<LIST_IN_LDS>(list, (int)rank, (int)(x[j] & t.key_mask));
+        // (entry `rank` is written by this thread alone, so what it reads here is the old content)
+        if (check) moved |= list_load<false>(list, (int)rank) != (int)(x[j] & t.key_mask);
+        list_store<false>(list, (int)rank, (int)(x[j] & t.key_mask));
         if (final) t.slots[s] = (rank << t.key_bits) | (x[j] & t.key_mask);
       }
     }
   }
   const int kept = (int)kept_u;
   if (check) {
-    // both answers through one word per wave (the library's workgroup-wide "or" is three barriers per answer)
-    const int mine = (__ballot(moved) != 0 ? 1 : 0) | (__ballot(moved_before) != 0 ? 2 : 0);
-    if (lane == 0) check->wave_words[wave] = mine;
+    const bool any = __ballot(moved) != 0;
+    if (lane == 0) wave_words[wave] = any ? 1 : 0;
     __syncthreads();
-    int any = 0;
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) any |= check->wave_words[w];
-    check->same_as_input = (any & 1) == 0;
-    check->same_as_before = check->before != nullptr && (any & 2) == 0;
+    const int of_wave = lane < WAVES ? wave_words[lane] : 0;
+    check->same_as_input = __ballot(of_wave) == 0;
+    check->same_as_before = false;
   }
   __syncthreads();  // (also: the wave words may be written again)
   return kept;
+}
+
+// The same where the list is in LDS and the table is a construction's last: a wave has at most eight words, which stay in
+// registers between the count and the result, and the lists' entries are all read before any is written, so that the pass
+// is four LDS round trips instead of one or two per word.  `words`: 2 * WAVES ints that nothing else uses.
+template <int THREADS>
+__device__ __forceinline__ int compact_in_lds(const Table32 &t, uint32_t slots, int *words, int *list, int *before, OrderCheck &check) {
+  constexpr int WAVES = THREADS / 64, MOST = 8;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const uint32_t n_words = slots >= 64u ? slots / 64u : 1u;
+  const uint32_t per_wave = (n_words + WAVES - 1u) / WAVES;  // <= MOST: 512 slots a wave, 8192 sixteen
+  const uint32_t w_beg = min(n_words, (uint32_t)wave * per_wave), mine = min(n_words, w_beg + per_wave) - w_beg;
+  uint32_t x[MOST], rank[MOST];
+#pragma unroll
+  for (int j = 0; j < MOST; ++j) {
+    const uint32_t at = (w_beg + j) * 64u + lane;
+    x[j] = kEmpty32;
+    if ((uint32_t)j < mine && at < slots) x[j] = t.slots[at];
+  }
+  uint32_t in_wave = 0;
+#pragma unroll
+  for (int j = 0; j < MOST; ++j) {
+    const unsigned long long m = __ballot(x[j] != kEmpty32);
+    rank[j] = in_wave + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+    in_wave += (uint32_t)__popcll(m);
+  }
+  uint32_t before_wave = 0, kept = in_wave;
+  if (WAVES > 1) {
+    if (lane == 0) words[wave] = (int)in_wave;
+    __syncthreads();
+    // (a lane per wave: sixteen waves that each go through sixteen counts keep the CU's scalar unit busy for 1000 cycles)
+    const uint32_t c = lane < WAVES ? (uint32_t)words[lane] : 0u, incl = wave_inclusive_sum(c);
+    before_wave = (uint32_t)__builtin_amdgcn_readlane((int)(incl - c), wave);
+    kept = (uint32_t)__builtin_amdgcn_readlane((int)incl, WAVES - 1);
+  }
+  int moved = 0, moved_before = 0;
+  if (check.on) {
+    int was[MOST], prior[MOST];
+    // (entry `rank` of either list is written by this lane alone, so what it reads here is the old content)
+#pragma unroll
+    for (int j = 0; j < MOST; ++j) {
+      was[j] = prior[j] = 0;
+      if (x[j] != kEmpty32) {
+        was[j] = list[before_wave + rank[j]];
+        prior[j] = before[before_wave + rank[j]];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < MOST; ++j)
+      if (x[j] != kEmpty32) {
+        const int key = (int)(x[j] & t.key_mask);
+        moved |= was[j] != key;
+        moved_before |= prior[j] != key;
+        before[before_wave + rank[j]] = was[j];
+      }
+  }
+#pragma unroll
+  for (int j = 0; j < MOST; ++j)
+    if (x[j] != kEmpty32) {
+      const uint32_t r = before_wave + rank[j], key = x[j] & t.key_mask;
+      list[r] = (int)key;
+      t.slots[(w_beg + j) * 64u + lane] = (r << t.key_bits) | key;
+    }
+  check.same_as_input = check.same_as_before = false;
+  if (check.on) {
+    // both answers through one word per wave (the library's workgroup-wide "or" is three barriers per answer)
+    const int answer = (__ballot(moved) != 0 ? 1 : 0) | (__ballot(moved_before) != 0 ? 2 : 0);
+    if (lane == 0) words[WAVES + wave] = answer;
+    __syncthreads();
+    const int of_wave = lane < WAVES ? words[WAVES + lane] : 0;
+    check.same_as_input = __ballot(of_wave & 1) == 0;
+    check.same_as_before = __ballot(of_wave & 2) == 0;
+  } else {
+    __syncthreads();
+  }
+  return (int)kept;
 }
 
 // The two table regions of a group: consecutive phases of a construction alternate between them,
@@ -785,27 +882,24 @@ struct TableRegions {
 // list[0 .. cnt) (insertion index = list index), or the previous table's keys, indexed by their
 // slot, and the list keys [prev_cnt, cnt) behind them.  A thread inserts its keys in order
 // (me, me + STRIDE, ...), so the threads work through the keys in chunks and a later key rarely
-// arrives before an earlier one; keys are fetched eight at a time ahead of the inserts.
-template <int STRIDE, bool LIST_IN_LDS>
-__device__ __forceinline__ void phase_insert(const Table32 &t, uint32_t mask, const int *list, int cnt, const uint32_t *old_table,
-                                             uint32_t old_slots, int prev_cnt, int me, bool safe) {
-  if (LIST_IN_LDS) {
-    // every key comes from LDS: nothing to fetch ahead, and two inlined placements instead of sixteen calls
-    uint32_t first = 0;
-    if (old_table != nullptr) {
-      first = old_slots;
+// arrives before an earlier one; from the workspace keys are fetched eight at a time ahead of the inserts.
+template <int STRIDE>
+__device__ __forceinline__ void phase_insert_lds(const Table32 &t, uint32_t mask, const int *list, int cnt, const uint32_t *old_table,
+                                                 uint32_t old_slots, int prev_cnt, int me, bool safe) {
+  // every key comes from LDS: nothing to fetch ahead, and two inlined placements instead of sixteen calls
 #pragma unroll 1
-      for (uint32_t s = me; s < old_slots; s += STRIDE) {
-        const uint32_t x = old_table[s];
-        if (x != kEmpty32) place32_inline(t, mask, x & t.key_mask, s, safe);
-      }
-    }
-    me = (me + STRIDE - (int)(first % (uint32_t)STRIDE)) % STRIDE;
-#pragma unroll 1
-    for (int idx = prev_cnt + me; idx < cnt; idx += STRIDE)
-      place32_inline(t, mask, (uint32_t)list[idx], first + (uint32_t)(idx - prev_cnt), safe);
-    return;
+  for (uint32_t s = me; s < old_slots; s += STRIDE) {
+    const uint32_t x = old_table[s];
+    if (x != kEmpty32) place32_inline(t, mask, x & t.key_mask, s, safe);
   }
+  me = (me + STRIDE - (int)(old_slots % (uint32_t)STRIDE)) % STRIDE;
+#pragma unroll 1
+  for (int idx = prev_cnt + me; idx < cnt; idx += STRIDE)
+    place32_inline(t, mask, (uint32_t)list[idx], old_slots + (uint32_t)(idx - prev_cnt), safe);
+}
+template <int STRIDE>
+__device__ __forceinline__ void phase_insert(const Table32 &t, uint32_t mask, const int *list, int cnt, const uint32_t *old_table,
+                                             uint32_t old_slots, int prev_cnt, int me) {
   if (old_table != nullptr) {
     for (uint32_t base = me; base < old_slots; base += 8 * STRIDE) {
       uint32_t x8[8];
@@ -828,7 +922,7 @@ __device__ __forceinline__ void phase_insert(const Table32 &t, uint32_t mask, co
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int idx = base + j * STRIDE;
-      k8[j] = idx < cnt ? list_load<LIST_IN_LDS>(list, idx) : 0;
+      k8[j] = idx < cnt ? list_load<false>(list, idx) : 0;
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -867,11 +961,10 @@ __device__ __forceinline__ void phase_insert_solo(const Table32 &t, uint32_t mas
 // is the old table first compacted into the list.  The phases of the smallest tables (a few dozen
 // keys) are run by the first wave alone, without workgroup barriers.
 static constexpr uint32_t kSoloSlots = 128;
-// check: see compact_table32; both answers are "no" when the list was rewritten between phases, and
-// check.before is then cleared (what it would receive is not the input).
-template <int THREADS, bool LIST_IN_LDS>
-__device__ __forceinline__ uint32_t rebuild_set32(Table32 &t, const TableRegions &reg, int *list, int &n, OrderCheck &check,
-                                                  bool safe) {
+// check: see compact_table32; the answer is "no" when the list was rewritten between phases.
+template <int THREADS>
+__device__ __forceinline__ uint32_t rebuild_set32(Table32 &t, const TableRegions &reg, int *wave_words, int *list, int &n,
+                                                  OrderCheck &check, bool safe) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   uint32_t slots = 8, old_slots = 0;
@@ -900,7 +993,7 @@ __device__ __forceinline__ uint32_t rebuild_set32(Table32 &t, const TableRegions
       old.slots = cur;
       prev_cnt = 0;
       list_rewritten = true;
-      compact_table32<THREADS, LIST_IN_LDS>(old, old_slots, nt, list, false);
+      compact_table32<THREADS>(old, old_slots, nt, list, false);
       nt = cur;
       cur = nullptr;
     }
@@ -911,7 +1004,7 @@ __device__ __forceinline__ uint32_t rebuild_set32(Table32 &t, const TableRegions
         for (uint32_t s = lane; s < slots; s += 64) nt[s] = kEmpty32;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");  // the wave's LDS operations execute in order
         __builtin_amdgcn_wave_barrier();
-        phase_insert_solo<LIST_IN_LDS>(t, mask, list, cnt, cur, old_slots, prev_cnt, lane, safe);
+        phase_insert_solo<false>(t, mask, list, cnt, cur, old_slots, prev_cnt, lane, safe);
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
         __builtin_amdgcn_wave_barrier();
       }
@@ -919,13 +1012,12 @@ __device__ __forceinline__ uint32_t rebuild_set32(Table32 &t, const TableRegions
     } else {
       for (uint32_t s = tid; s < slots; s += THREADS) nt[s] = kEmpty32;
       __syncthreads();
-      phase_insert<THREADS, LIST_IN_LDS>(t, mask, list, cnt, cur, old_slots, prev_cnt, tid, safe);
+      phase_insert<THREADS>(t, mask, list, cnt, cur, old_slots, prev_cnt, tid);
       __syncthreads();
     }
     if (n < (int)thr) {
       if (solo_pending) __syncthreads();
-      if (list_rewritten || !check.on) check.before = nullptr;
-      n = compact_table32<THREADS, LIST_IN_LDS>(t, slots, other, list, true, check.on ? &check : nullptr);
+      n = compact_table32<THREADS>(t, slots, other, list, true, wave_words, check.on ? &check : nullptr);
       if (list_rewritten || !check.on) check.same_as_input = check.same_as_before = false;
       return slots;
     }
@@ -935,6 +1027,72 @@ __device__ __forceinline__ uint32_t rebuild_set32(Table32 &t, const TableRegions
     next_in_a = nt != reg.a;
     slots = resized_slots(thr);
   }
+}
+
+// The same with the key list in LDS.  There every table of a construction has a place of its own (the one of S slots
+// behind the (S - 8) / 3 slots of the smaller ones), so all of them are cleared at once, by the waves that have nothing to do
+// while the first one runs the smallest phases.
+// A construction is a chain of LDS round trips and barriers, and what every wave of sixteen does for itself counts sixteen
+// times.  2494 columns (16384 columns, power-law rows), cycles: phases of 8, 32 and 128 slots 980, 2340 and 3680, of 512, 2048
+// and 8192 slots 6000, 10600 and 5700, compaction 5600, between two constructions 2000; with tables cleared phase by phase,
+// a compaction that reads the table twice and the tables' sizes found by a loop it was 46 000 together, now 37 000.  Twenty
+// dataset matrices: the launches of the small and the wide groups 106 and 56 -> 86 and 48 us; 16384 power-law rows 161 -> 146
+// us.  Taken back: the phases of 8 and 32 slots key after key with the table in a register (24 keys cost 4000 cycles,
+// as before), the phases from 512 slots on by 8 or 4 waves instead of 16 (2048 slots: 12 900 and 18 100 cycles against 10 300).
+__host__ __device__ constexpr uint32_t table_offset(uint32_t slots) { return (slots - 8u) / 3u; }
+static constexpr int kFastHeader = 256;  // bytes of LDS in front of the tables: 32 ints of the scans, 32 of the compaction
+template <int THREADS>
+__device__ __forceinline__ uint32_t rebuild_in_lds(Table32 &t, uint32_t *tables, int *words, int *list, int *before, int &n, OrderCheck &check,
+                                                   bool safe) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t last = final_slots(n);
+  // (16 bytes at a time: every table begins and ends at a multiple of 32)
+  const uintx4 empty = {kEmpty32, kEmpty32, kEmpty32, kEmpty32};
+  uint32_t slots = 8, old_slots = 0;
+  uint32_t *cur = nullptr;
+  int prev_cnt = 0;
+  const auto advance = [&]() {
+    cur = tables + table_offset(slots);
+    old_slots = slots;
+    prev_cnt = (int)resize_threshold(slots);
+    slots *= 4u;  // (the smallest power of two above four times the threshold)
+  };
+  if (THREADS == 64 || wave == 0) {
+    const uint32_t stop = table_offset(4u * (THREADS == 64 ? last : min(last, kSoloSlots)));
+    for (uint32_t s = 4u * lane; s < stop; s += 256u) *reinterpret_cast<uintx4 *>(tables + s) = empty;
+    for (;;) {
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");  // the wave's LDS operations execute in order
+      __builtin_amdgcn_wave_barrier();
+      t.slots = tables + table_offset(slots);
+      phase_insert_solo<true>(t, slots - 1u, list, min(n, (int)resize_threshold(slots)), cur, old_slots, prev_cnt, lane, safe);
+      if (slots == last || (THREADS > 64 && slots == kSoloSlots)) break;
+      advance();
+    }
+  } else if (last > kSoloSlots) {
+    const uint32_t stop = table_offset(4u * last);
+    for (uint32_t s = table_offset(4u * kSoloSlots) + 4u * (uint32_t)(tid - 64); s < stop; s += 4u * (THREADS - 64))
+      *reinterpret_cast<uintx4 *>(tables + s) = empty;
+  }
+  if (THREADS > 64) {
+    __syncthreads();
+    if (last > kSoloSlots) {
+      slots = kSoloSlots;
+      for (;;) {
+        advance();
+        t.slots = tables + table_offset(slots);
+        phase_insert_lds<THREADS>(t, slots - 1u, list, min(n, (int)resize_threshold(slots)), cur, old_slots, prev_cnt, tid, safe);
+        __syncthreads();
+        if (slots == last) break;
+      }
+    }
+  } else {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+  }
+  t.slots = tables + table_offset(last);
+  n = compact_in_lds<THREADS>(t, last, words, list, before, check);
+  return last;
 }
 
 template <int THREADS, bool LIST_IN_LDS>
@@ -955,9 +1113,9 @@ __global__ __launch_bounds__(THREADS) void svc_merge_fast_kernel(const SvcArgs a
   const int count = a.scanned[grp + 1] - a.scanned[grp];
   const int e0 = a.row_ptr[r0];
 
-  int *scratch = reinterpret_cast<int *>(smem);  // 32 ints
+  int *scratch = reinterpret_cast<int *>(smem);  // 64 ints
   Table32 t;
-  t.slots = reinterpret_cast<uint32_t *>(smem + 128);
+  t.slots = reinterpret_cast<uint32_t *>(smem + kFastHeader);
   t.key_bits = key_bits;
   t.key_mask = (1u << key_bits) - 1u;
   TableRegions reg;
@@ -965,7 +1123,7 @@ __global__ __launch_bounds__(THREADS) void svc_merge_fast_kernel(const SvcArgs a
   reg.cap_a = max_slots;
   reg.b = t.slots + max_slots;
   reg.cap_b = small_slots;
-  int *list = LIST_IN_LDS ? reinterpret_cast<int *>(smem + 128 + ((size_t)max_slots + small_slots) * 4) : a.tmp_cols + e0;
+  int *list = LIST_IN_LDS ? reinterpret_cast<int *>(smem + kFastHeader + ((size_t)max_slots + small_slots) * 4) : a.tmp_cols + e0;
   int *const list_before = LIST_IN_LDS ? list + list_cap : nullptr;  // the input of the latest construction
   const int cap = count;
 
@@ -973,7 +1131,7 @@ __global__ __launch_bounds__(THREADS) void svc_merge_fast_kernel(const SvcArgs a
   uint32_t slots = 0;
   const RowBounds rows(a, r0, r1);
   if (filed & kAscending) {
-    write_ascending_group<THREADS>(a, grp, rows, count, smem + 128,
+    write_ascending_group<THREADS>(a, grp, rows, count, smem + kFastHeader,
                                    (max_slots + small_slots) * 4u + (LIST_IN_LDS ? (uint32_t)list_cap * 8u : 0u), scratch);
     __syncthreads();  // the next group reuses the LDS
     continue;
@@ -993,14 +1151,15 @@ __global__ __launch_bounds__(THREADS) void svc_merge_fast_kernel(const SvcArgs a
   // later (`cap`, counted beforehand): the group is then done again with the placements that look.
   bool safe = false;
   OrderCheck check;
-  check.wave_words = scratch;
   auto construct = [&](bool without_new_keys, bool compare) {
     const bool had_input = before_is_input;
     check.on = compare;
-    check.before = list_before;
-    slots = rebuild_set32<THREADS, LIST_IN_LDS>(t, reg, list, n, check, safe);
+    if constexpr (LIST_IN_LDS)
+      slots = rebuild_in_lds<THREADS>(t, reg.a, scratch + 32, list, list_before, n, check, safe);
+    else
+      slots = rebuild_set32<THREADS>(t, reg, scratch + 32, list, n, check, safe);
     period = check.same_as_input ? 1 : (without_new_keys && had_input && check.same_as_before) ? 2 : 0;
-    before_is_input = check.before != nullptr;
+    before_is_input = LIST_IN_LDS && compare;
   };
   for (;;) {
   bool overfull = false;
@@ -1008,47 +1167,60 @@ __global__ __launch_bounds__(THREADS) void svc_merge_fast_kernel(const SvcArgs a
   slots = 0;
   period = owed = 0;
   before_is_input = false;
-  for (int row = r0; row < r1; ++row) {
-    const int b = rows.start(row - r0), e = rows.start(row - r0 + 1);
-    // acc + row: append the row's columns that are not in acc yet, in row order
+  // (a row's first columns are fetched while the row before it is put into its set)
+  const auto first_column = [&](int row) {
+    const int idx = rows.start(row - r0) + tid;
+    return row < r1 && idx < rows.start(min(row - r0 + 1, r1 - r0)) ? (uint32_t)a.col_ind[idx] : 0u;
+  };
+  uint32_t ahead = first_column(r0);
+  // (one place for every construction, the one that is still owed behind the last row included: inlined several times
+  // they fill the instruction cache)
+  for (int row = r0; row < r1 || owed; ++row) {
+    const bool behind = row >= r1;
     int appended = 0;
-    for (int base = b; base < e; base += THREADS) {
-      const int idx = base + tid;
-      bool is_new = false;
-      uint32_t k = 0;
-      if (idx < e) {
-        k = (uint32_t)a.col_ind[idx];
-        is_new = k < (uint32_t)a.K && ((slots == 0) || find_slot32(t, slots - 1u, k) < 0);
+    if (!behind) {
+      const int b = rows.start(row - r0), e = rows.start(row - r0 + 1);
+      const uint32_t first = ahead;
+      ahead = first_column(row + 1);
+      // acc + row: append the row's columns that are not in acc yet, in row order
+      for (int base = b; base < e; base += THREADS) {
+        const int idx = base + tid;
+        bool is_new = false;
+        uint32_t k = 0;
+        if (idx < e) {
+          k = base == b ? first : (uint32_t)a.col_ind[idx];
+          is_new = k < (uint32_t)a.K && ((slots == 0) || find_slot32(t, slots - 1u, k) < 0);
+        }
+        int total;
+        const int rank = block_rank_of_flag<THREADS>(is_new, &total, scratch, scan_turn);
+        if (is_new && n + appended + rank < cap) list_store<LIST_IN_LDS>(list, n + appended + rank, (int)k);
+        appended += total;
       }
-      int total;
-      const int rank = block_rank_of_flag<THREADS>(is_new, &total, scratch, scan_turn);
-      if (is_new && n + appended + rank < cap) list_store<LIST_IN_LDS>(list, n + appended + rank, (int)k);
-      appended += total;
+      overfull = appended > cap - n;
+      appended = min(appended, cap - n);  // the cap only bites for invalid input (a row that repeats a column)
+      __syncthreads();
+      if (overfull && !safe) break;
     }
-    overfull = appended > cap - n;
-    appended = min(appended, cap - n);  // the cap only bites for invalid input (a row that repeats a column)
-    __syncthreads();
-    if (overfull && !safe) break;
-    if (appended == 0 && slots != 0) {
+    const bool nothing_new = appended == 0 && slots != 0;
+    if (nothing_new && !behind) {
       if (period == 1) continue;
       if (period == 2) {
         owed ^= 1;
         continue;
       }
-      construct(true, true);
-      continue;
     }
-    if (owed) {  // the order the new keys go behind is the other one of the pair (the new keys wait behind list[n])
-      construct(true, false);
+    // what is owed comes first: the order the new keys go behind is the other one of the pair (they wait behind list[n])
+    for (bool first_owed = owed != 0;; first_owed = false) {
       owed = 0;
+      if (!first_owed) n += appended;
+      construct(first_owed || nothing_new,
+                !first_owed && (nothing_new || (row + 1 < r1 && rows.start(row - r0 + 1) == rows.start(row - r0 + 2))));
+      if (!first_owed || behind) break;
     }
-    n += appended;
-    construct(false, row + 1 < r1 && rows.start(row - r0 + 1) == rows.start(row - r0 + 2));
   }
   if (!overfull || safe) break;
   safe = true;
   }
-  if (owed) construct(true, false);
 
   write_group_output<THREADS>(a, grp, rows, list, n, [&](uint32_t key) {
     const int sl = find_slot32(t, slots - 1u, key);
@@ -1230,14 +1402,15 @@ static hipError_t launch_fast_class(const SvcArgs &a, int grid, int cls, int cls
                                     uint32_t key_bits, hipStream_t stream, size_t min_lds = 0) {
   // second table region: a quarter of the first (what the phase before the largest needs), less where LDS is short;
   // it also serves as the running-count array of the compaction of a table in the first region (slots / 64 + 1 words)
-  uint32_t small_slots = slots / 4u;
+  // (with the key list in LDS: the places of all smaller tables)
+  uint32_t small_slots = LIST_IN_LDS ? table_offset(slots) : slots / 4u;
   // (a key list in LDS has a second copy behind it: the input of the latest construction)
   const size_t list_bytes = LIST_IN_LDS ? (size_t)hi * 8 : 0;
   // (16 bytes behind everything: a placement reads up to three slots past the end of its table)
   constexpr size_t kTail = 16;
-  while (128 + ((size_t)slots + small_slots) * 4 + list_bytes + kTail > 160 * 1024) small_slots /= 4u;
+  while (!LIST_IN_LDS && kFastHeader + ((size_t)slots + small_slots) * 4 + list_bytes + kTail > 160 * 1024) small_slots /= 4u;
   if (small_slots < slots / 64u + 1u) return hipErrorInvalidValue;
-  size_t lds = 128 + ((size_t)slots + small_slots) * 4 + list_bytes + kTail;
+  size_t lds = kFastHeader + ((size_t)slots + small_slots) * 4 + list_bytes + kTail;
   if (lds < min_lds) lds = min_lds;  // asking for more than half of a CU's LDS keeps a workgroup alone on its CU
   auto kern = svc_merge_fast_kernel<THREADS, LIST_IN_LDS>;
   if (lds > 64 * 1024) {

@@ -114,6 +114,29 @@ def test_a_groups_class_comes_from_its_distinct_columns(oracle, built_library, d
     assert vrp[2] - vrp[1] == distinct
 
 
+@pytest.mark.parametrize("keys", [4, 5, 18, 19, 76, 77, 306, 307, 1228, 1229, 4914])
+def test_either_side_of_every_table_size(oracle, built_library, keys):
+    """Groups whose last construction, or one in the middle, is the largest of a table size or the smallest of the next,
+    whose columns are wider than the table (no ascending order), alone and with an empty row behind; beside a wide group and
+    without one, so that the small ones run with a wave and with more."""
+    rng = np.random.default_rng(keys)
+    V, K = 8, 100000
+    for wide in (0, 2000):
+        rows = []
+        for layout in ([keys, 0, 0, 0, 0, 0, 0, 0], [keys - 1, 1, 0, 3, 0, 0, 1, 0], [1] * 7 + [max(keys - 7, 1)], [wide] + [0] * 7):
+            cols = rng.permutation(K)[:sum(layout)]
+            cols[:1] = K - 1
+            cols = np.unique(cols)
+            for n in layout:
+                pick = rng.permutation(cols.size)[:n]
+                rows.append(np.sort(cols[pick]))
+                cols = np.delete(cols, pick)
+        ptr = np.concatenate([[0], np.cumsum([r.size for r in rows])]).astype(np.int32)
+        flat = np.concatenate(rows).astype(np.int32)
+        csr = synth.Csr(len(rows), K, ptr, flat, rng.standard_normal(flat.size).astype(np.float16))
+        _compare_with_oracle(oracle, csr, V)
+
+
 @pytest.mark.parametrize("keys", [5, 40, 200, 700, 2500, 4000])
 def test_member_rows_that_bring_nothing_new(oracle, built_library, keys):
     """CPython rebuilds the set for every member row, also for an empty row and for a row whose columns are all
