@@ -114,6 +114,29 @@ int sspmm_linear_f16(int m_vec, int V, int N, int K, const int32_t *row_offsets,
                      sspmm_half_t *C, void *hip_stream);
 
 /* ------------------------------------------------------------------------------------------
+ * What follows the attention in a post-LayerNorm encoder layer with vector-sparse weights, in one
+ * launch (the reference's comparison block runs it as torch modules, reference
+ * end2end/sspmm_e2e/end_to_end.py:55-75): with x, context and out feature-major [hidden, tokens],
+ *   s  = x + (Wo context + bo)                     n   = LayerNorm1(s)
+ *   s' = n + (W2 gelu(W1 n + b1) + b2)             out = LayerNorm2(s')
+ * Wo is [hidden, hidden], W1 [ffn, hidden], W2 [hidden, ffn], each row offsets, column indices and
+ * values as for sspmm_linear_f16, biases and beta or NULL.  Every activation is rounded to fp16, sums
+ * and statistics are fp32.  out may be neither x nor context.
+ * tokens a multiple of 4, hidden up to 1024, hidden and ffn multiples of V and together up to about
+ * 4300 (they share a CU's LDS); values 16-byte, activations 8-byte aligned.  Other sizes: error.
+ * ---------------------------------------------------------------------------------------- */
+int sspmm_encoder_tail_fits(int hidden, int ffn, int tokens, int V); /* 1 where the launch takes these sizes, else 0 */
+int sspmm_encoder_tail_f16(int hidden, int ffn, int tokens, int V, const sspmm_half_t *x,
+                           const sspmm_half_t *context, const int32_t *o_offsets, const int32_t *o_cols,
+                           const sspmm_half_t *o_values, const sspmm_half_t *o_bias,
+                           const sspmm_half_t *gamma1, const sspmm_half_t *beta1, float eps1,
+                           const int32_t *f1_offsets, const int32_t *f1_cols, const sspmm_half_t *f1_values,
+                           const sspmm_half_t *f1_bias, const int32_t *f2_offsets, const int32_t *f2_cols,
+                           const sspmm_half_t *f2_values, const sspmm_half_t *f2_bias,
+                           const sspmm_half_t *gamma2, const sspmm_half_t *beta2, float eps2,
+                           sspmm_half_t *out, void *hip_stream);
+
+/* ------------------------------------------------------------------------------------------
  * Plans: what the library can know about a sparsity pattern before its first product.
  *
  * The reference starts one thread block per vector-row whatever its length (reference

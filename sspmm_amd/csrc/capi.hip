@@ -103,6 +103,44 @@ int sspmm_linear_f16(int m_vec, int V, int N, int K, const int32_t *row_offsets,
                     activation);
 }
 
+int sspmm_encoder_tail_fits(int hidden, int ffn, int tokens, int V) { return sspmm::encoder_tail_applies(V, hidden, ffn, tokens) ? 1 : 0; }
+
+int sspmm_encoder_tail_f16(int hidden, int ffn, int tokens, int V, const sspmm_half_t *x, const sspmm_half_t *context,
+                           const int32_t *o_offsets, const int32_t *o_cols, const sspmm_half_t *o_values, const sspmm_half_t *o_bias,
+                           const sspmm_half_t *gamma1, const sspmm_half_t *beta1, float eps1, const int32_t *f1_offsets,
+                           const int32_t *f1_cols, const sspmm_half_t *f1_values, const sspmm_half_t *f1_bias,
+                           const int32_t *f2_offsets, const int32_t *f2_cols, const sspmm_half_t *f2_values,
+                           const sspmm_half_t *f2_bias, const sspmm_half_t *gamma2, const sspmm_half_t *beta2, float eps2,
+                           sspmm_half_t *out, void *hip_stream) {
+  if (hidden < 0 || ffn < 0 || tokens < 0) return kInvalid;
+  if (tokens == 0) return 0;
+  if (!sspmm::encoder_tail_applies(V, hidden, ffn, tokens)) return kInvalid;
+  if (!x || !context || !out || !gamma1 || !gamma2 || !o_offsets || !f1_offsets || !f2_offsets) return kInvalid;
+  // (a weight without a stored vector may come with null arrays)
+  uintptr_t values = 0, rows = 0, ints = 0;
+  for (const sspmm_half_t *q : {o_values, f1_values, f2_values}) values |= reinterpret_cast<uintptr_t>(q);
+  for (const sspmm_half_t *q : {x, context, (const sspmm_half_t *)out}) rows |= reinterpret_cast<uintptr_t>(q);
+  for (const int32_t *q : {o_offsets, o_cols, f1_offsets, f1_cols, f2_offsets, f2_cols}) ints |= reinterpret_cast<uintptr_t>(q);
+  if (values % 16 || rows % 8 || ints % 4) return kInvalid;
+  sspmm::EncoderTailArgs p;
+  p.hidden = hidden;
+  p.ffn = ffn;
+  p.tokens = tokens;
+  p.x = x;
+  p.context = context;
+  p.w[0] = {o_offsets, o_cols, o_values, o_bias};
+  p.w[1] = {f1_offsets, f1_cols, f1_values, f1_bias};
+  p.w[2] = {f2_offsets, f2_cols, f2_values, f2_bias};
+  p.gamma1 = gamma1;
+  p.beta1 = beta1;
+  p.gamma2 = gamma2;
+  p.beta2 = beta2;
+  p.eps1 = eps1;
+  p.eps2 = eps2;
+  p.out = out;
+  return (int)sspmm::launch_encoder_tail(p, V, static_cast<hipStream_t>(hip_stream));
+}
+
 int sspmm_batched_f16_f16(int batch, int m_vec, int V, int N, int K, const int32_t *row_indices,
                           const int32_t *row_offsets, const int32_t *col_idx, const sspmm_half_t *values,
                           int64_t stride_values, const sspmm_half_t *B, int64_t stride_B, sspmm_half_t *C,

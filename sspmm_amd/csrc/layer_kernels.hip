@@ -15,6 +15,7 @@
 
 #include <mutex>
 
+#include "lane_ops.h"
 #include "layer_kernels.h"
 
 namespace sspmm {
@@ -126,14 +127,6 @@ __global__ __launch_bounds__(THREADS) void add_layernorm_kernel(int H, int T, co
 // The same for up to 128 * TRIP features with the sums kept in registers: no pass over LDS, two barriers (one per
 // reduction) and the reductions on lane moves of the vector unit.  A workgroup's loads, gamma and beta among them, are all
 // in flight together.  768 x 4096: 7.2 us against 8.7, 512 x 4096 5.6 against 6.9, 1024 x 8192 18.3 against 19.7.
-__device__ __forceinline__ float sum_over_row_groups(float v) {  // over the lanes of a wave with the same lane % 4
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, false));  // rotated by 8 in each 16
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xf, 0xf, false));  // and by 4
-  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
 template <int TRIP>
 __global__ __launch_bounds__(512) void add_layernorm_held_kernel(int H, int T, const _Float16 *__restrict__ x, const _Float16 *__restrict__ a,
                                                                  const _Float16 *__restrict__ gamma, const _Float16 *__restrict__ beta,
@@ -175,7 +168,7 @@ __global__ __launch_bounds__(512) void add_layernorm_held_kernel(int H, int T, c
 #pragma unroll
   for (int pass = 0; pass < 2; ++pass) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] = sum_over_row_groups(acc[i]);
+    for (int i = 0; i < 4; ++i) acc[i] = sum_over_quads(acc[i]);
     if (lane < S::kLanes) red[pass][wave][tl] = acc;
     __syncthreads();
     floatx4 sum = {0.f, 0.f, 0.f, 0.f};

@@ -34,6 +34,23 @@ struct SpmmArgs {
 // the gather kernel otherwise.
 hipError_t launch_spmm(const SpmmArgs &args, int V, bool out_f16, hipStream_t stream);
 
+// What follows the attention in an encoder layer, on feature-major activations of `tokens` columns:
+//   s = x + (Wo context + bo)      n = LayerNorm1(s)      s' = n + (W2 gelu(W1 n + b1) + b2)      out = LayerNorm2(s')
+// w: Wo [hidden, hidden], W1 [ffn, hidden], W2 [hidden, ffn], vector-sparse; every activation rounded to fp16.
+struct EncoderTailArgs {
+  int hidden, ffn, tokens;
+  const uint16_t *x, *context;
+  struct Weight {
+    const int32_t *row_offsets, *col_idx;
+    const uint16_t *values, *bias;  // bias nullable
+  } w[3];
+  const uint16_t *gamma1, *beta1, *gamma2, *beta2;  // beta nullable
+  float eps1, eps2;
+  uint16_t *out;
+};
+bool encoder_tail_applies(int V, int hidden, int ffn, int tokens);
+hipError_t launch_encoder_tail(const EncoderTailArgs &args, int V, hipStream_t stream);
+
 // Forces a kernel where its preconditions hold: 0 automatic, 1 scalar, 2 gather, 3 LDS slab, 6 staged gather,
 // 7 load-balanced gather (calls with a plan only), 9 LDS slab 128 columns wide.
 // Per host thread: meant for tests and tuning.  Returns the previous value.

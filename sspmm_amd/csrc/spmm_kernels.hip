@@ -27,12 +27,14 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "lane_ops.h"
 #include "schedule.h"
 #include "spmm_kernels.h"
 
 namespace sspmm {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t uintx2 __attribute__((ext_vector_type(2)));
@@ -909,10 +911,10 @@ struct SlabCtx {
 
 // One wave's share of a work item: the vector-rows it claims from the item's row table,
 // against the slab at byte offset slab_base of LDS.
-template <int V, typename OutT, int NQ, int L, bool RAGGED>
+template <int V, typename OutT, int NQ, int L, bool RAGGED, typename Out>
 __device__ __forceinline__ void slab_process_item(const SlabCtx<V, OutT> &x, unsigned char *lds, uint32_t slab_base,
                                                   const SlabRows &rows, const uint16_t *vals,
-                                                  __amdgpu_buffer_rsrc_t srd_c, const SlabStore<V, OutT, NQ> &out) {
+                                                  __amdgpu_buffer_rsrc_t srd_c, const Out &out) {
   SlabCursor head;  // issues loads
   head.claim = cursor_claim(rows, 0);
   cursor_prefetch(head, rows);
@@ -966,6 +968,7 @@ __device__ __forceinline__ void slab_process_item(const SlabCtx<V, OutT> &x, uns
         addr[h] = layout_pad(L) ? __umul24(c, layout_row_bytes(L, NQ)) + lane_base
                   : NQ == 8     ? (((c << 8) + lane_base) | ((c << 5) & 0xe0u))
                   : NQ == 4     ? (((c << 7) + lane_base) | ((c << 4) & 0x60u))
+                  : NQ == 1     ? (c << 5) + lane_base
                                 : (((c << 6) + lane_base) | ((c << 3) & 0x20u));
       }
       Half8Bits b[NQ];
@@ -1211,6 +1214,221 @@ __global__ __launch_bounds__(kSlabThreads) void spmm_slab_kernel(const SpmmArgs 
     cur = nxt;
     ++it;
   }
+}
+
+// ------------------------------------------------------------------------------------------
+// What follows the attention in an encoder layer, in one launch (the reference's comparison block runs it as torch modules,
+// reference end2end/sspmm_e2e/end_to_end.py:55-75, on dense weights): output projection, + x, LayerNorm, the two
+// feed-forward products with the GELU between them, + x, LayerNorm, on feature-major activations [features, tokens].
+//
+// As five launches every step waits for the slowest workgroup of the one before, starts on cold caches and moves its
+// activations through memory.  Here a workgroup of 16 waves keeps 16 tokens from the context to the result: the activations
+// lie in LDS as [feature][16 tokens], rows of 32 bytes, and every product is the slab kernel's loop on a slab of one
+// column tile, whose rows are the features of the step before; its tiles go back to LDS through the epilogue.  Every
+// activation is rounded to fp16 where the separate launches round it.
+//   LDS: x (then x + a, then its LayerNorm, then that + y): hidden rows; the context, then the hidden features: ffn rows; a zero
+//   row behind either; value tiles, row tables of the three products, biases.  The workgroups of 64 consecutive tokens share
+//   an XCD (ids 8 apart), so that a line of x, context or result crosses the fabric once.
+// 768 features, 3072 hidden, V = 16 at 90 %, 4096 tokens (a workgroup per CU): 43 us, where the five launches took 5, 11, 15, 14
+// and 11; the layer 82 -> 63 us.  1200 steps of 32 vectors a workgroup: bound by the step's chain (value tile to LDS and
+// back, rows of the slab, MFMA) on four waves per SIMD, 29 ns a step and CU as in the slab kernel, and by the 7 us of vector
+// instructions of 49 000 GELUs.
+struct SlabTailStore {
+  unsigned char *rows;   // LDS: row r of the product at rows + 32 r
+  const _Float16 *bias;  // LDS
+  int act, lane, last;   // last: lanes m beyond it hold no row
+  bool add;              // to what lies there
+  template <bool RAGGED>
+  __device__ __forceinline__ void store(const floatx4 (&acc)[1], __amdgpu_buffer_rsrc_t, uint32_t crow) const {
+    const int m = lane & 15, g = lane >> 4;
+    if (m > last) return;
+    half4 *const at = reinterpret_cast<half4 *>(rows + crow + (uint32_t)m * 32u + (uint32_t)g * 8u);
+    const float b = (float)bias[(crow >> 5) + (uint32_t)m];
+    half4 h;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) h[i] = (_Float16)epilogue_value(acc[0][i], b, act);
+    if (add) h = *at + h;
+    *at = h;
+  }
+};
+
+// LayerNorm of the 16 tokens over H rows (16 waves; H <= 1024), statistics in fp32, mean first.  dst: the rows' own place, or
+// memory with `pitch` elements between rows.  Contains barriers; every thread must call it.
+template <bool TO_MEMORY>
+__device__ __forceinline__ void slab_tail_norm(unsigned char *rows, int H, const _Float16 *gamma, const _Float16 *beta, float eps,
+                                               floatx4 (*red)[kSlabWaves][4], _Float16 *dst, int64_t pitch, bool live) {
+  constexpr int TRIP = 4, kGroups = kSlabThreads / 4;
+  const int tid = threadIdx.x, tl = tid & 3, rg = tid >> 2, lane = tid & 63, wave = tid >> 6;
+  half4 s[TRIP];
+  float w[TRIP], b[TRIP];
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < TRIP; ++u) {
+    const int h = rg + u * kGroups;
+    s[u] = half4{0, 0, 0, 0};
+    w[u] = 1.0f;
+    b[u] = 0.0f;
+    if (h < H) {
+      s[u] = *reinterpret_cast<const half4 *>(rows + h * 32 + tl * 8);
+      w[u] = (float)gamma[h];
+      if (beta) b[u] = (float)beta[h];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] += (float)s[u][i];
+  }
+  floatx4 stat[2];  // mean, 1 / deviation
+#pragma unroll
+  for (int pass = 0; pass < 2; ++pass) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = sum_over_quads(acc[i]);
+    if (lane < 4) red[pass][wave][tl] = acc;
+    __syncthreads();
+    floatx4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int v = 0; v < kSlabWaves; ++v) sum += red[pass][v][tl];
+    stat[pass] = sum;
+    if (pass == 0) {
+      stat[0] *= 1.0f / (float)H;
+      acc = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int u = 0; u < TRIP; ++u)
+        if (rg + u * kGroups < H) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float d = (float)s[u][i] - stat[0][i];
+            acc[i] += d * d;
+          }
+        }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) stat[1][i] = rsqrtf(stat[1][i] / (float)H + eps);
+#pragma unroll
+  for (int u = 0; u < TRIP; ++u) {
+    const int h = rg + u * kGroups;
+    if (h >= H) break;
+    half4 o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = (_Float16)(((float)s[u][i] - stat[0][i]) * stat[1][i] * w[u] + b[u]);
+    if (!TO_MEMORY) *reinterpret_cast<half4 *>(rows + h * 32 + tl * 8) = o;
+    else if (live) *reinterpret_cast<half4 *>(dst + (int64_t)h * pitch + 4 * tl) = o;
+  }
+}
+
+struct SlabTailLds {  // byte offsets
+  uint32_t wide, tiles, tables[3], bias[3], red, total;
+};
+__host__ __device__ inline SlabTailLds slab_tail_lds(int V, int hidden, int ffn) {
+  SlabTailLds o;
+  const uint32_t h = (uint32_t)hidden, f = (uint32_t)ffn, rows[3] = {h, f, h};
+  o.wide = (h + 1u) * 32u;
+  uint32_t at = o.wide + ((f > h ? f : h) + 1u) * 32u;
+  o.tiles = at;
+  at += kSlabWaves * (uint32_t)wave_lds_bytes(V);
+  for (int i = 0; i < 3; ++i) {
+    o.tables[i] = at;
+    at += (rows[i] / (uint32_t)V + 2u) * 16u;
+  }
+  o.red = at;
+  at += 2u * kSlabWaves * 4u * 16u;
+  for (int i = 0; i < 3; ++i) {
+    o.bias[i] = at;
+    at += rows[i] * 2u;
+  }
+  o.total = at;
+  return o;
+}
+
+template <int V>
+__global__ __launch_bounds__(kSlabThreads) void encoder_tail_kernel(const EncoderTailArgs p) {
+  extern __shared__ __align__(256) unsigned char lds[];
+  const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
+  const int first = (((idx / 4) * 8 + xcd) * 4 + (idx % 4)) * 16;
+  if (first >= p.tokens) return;  // (the whole workgroup: the grid is padded to eight groups of 64 tokens)
+  const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int H = p.hidden, F = p.ffn;
+  const SlabTailLds at = slab_tail_lds(V, H, F);
+  const bool live = first + 4 * (tid & 3) < p.tokens;  // (tokens is a multiple of 4)
+
+  const _Float16 *const xg = reinterpret_cast<const _Float16 *>(p.x) + first, *const cg = reinterpret_cast<const _Float16 *>(p.context) + first;
+  half4 xs[4], cs[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int h = (tid >> 2) + u * (kSlabThreads / 4);
+    xs[u] = cs[u] = half4{0, 0, 0, 0};
+    if (live && h < H) {
+      cs[u] = *reinterpret_cast<const half4 *>(cg + (int64_t)h * p.tokens + 4 * (tid & 3));
+      xs[u] = *reinterpret_cast<const half4 *>(xg + (int64_t)h * p.tokens + 4 * (tid & 3));
+    }
+  }
+  const int out_rows[3] = {H, F, H};
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const int n = out_rows[i] / V;
+    intx4 *const table = reinterpret_cast<intx4 *>(lds + at.tables[i]);
+    for (int r = tid; r < n + 2; r += kSlabThreads) {
+      intx4 e = {0, 0, 0, 0};
+      if (r < n) e = intx4{r, p.w[i].row_offsets[r], p.w[i].row_offsets[r + 1], 1};
+      table[r] = e;
+    }
+    _Float16 *const bias = reinterpret_cast<_Float16 *>(lds + at.bias[i]);
+    for (int r = tid; r < out_rows[i]; r += kSlabThreads)
+      bias[r] = p.w[i].bias ? reinterpret_cast<const _Float16 *>(p.w[i].bias)[r] : (_Float16)0;
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int h = (tid >> 2) + u * (kSlabThreads / 4);
+    if (h < H) {
+      *reinterpret_cast<half4 *>(lds + h * 32 + (tid & 3) * 8) = xs[u];
+      *reinterpret_cast<half4 *>(lds + at.wide + h * 32 + (tid & 3) * 8) = cs[u];
+    }
+  }
+  if (tid < 8) {  // the zero rows behind x and the context
+    *reinterpret_cast<half4 *>(lds + (tid < 4 ? 0u : at.wide) + H * 32 + (tid & 3) * 8) = half4{0, 0, 0, 0};
+  }
+  __syncthreads();
+
+  SlabCtx<V, _Float16> x;
+  x.lane = lane;
+  x.val_tile = lds + at.tiles + wave * wave_lds_bytes(V);
+  x.val_dst = x.val_tile + lane * (V * 2u * 32u / 64u);
+  x.a_off = (uint32_t)(8 * g + (m >> 2)) * (V * 2u) + (uint32_t)(m & 3) * 8u;
+  x.slot0 = (uint32_t)(8 * g + (m >> 2));
+  x.b_lane_off = (uint32_t)(m & 3) * 8u;
+  x.c_vrow_bytes = V * 32u;
+  floatx4(*const red)[kSlabWaves][4] = reinterpret_cast<floatx4(*)[kSlabWaves][4]>(lds + at.red);
+  SlabTailStore out;
+  out.lane = lane;
+  out.last = V - 1;
+  // (unrolled: what differs between the products is known to the compiler)
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const int n = (i == 1 ? F : H) / V;
+    const uint32_t table = at.tables[i];
+    SlabRows rows;
+    rows.table = reinterpret_cast<const intx4 *>(lds + table);
+    rows.n_rows = n;
+    rows.counter = reinterpret_cast<int *>(lds + table + (n + 1) * 16);
+    rows.lane = lane;
+    x.zero_row = (uint32_t)(i == 2 ? F : H);
+    // (in scalar registers, or every load of column indices becomes a loop over the lanes' descriptors)
+    x.srd_cols = make_srd(p.w[i].col_idx, (uint32_t)__builtin_amdgcn_readfirstlane(p.w[i].row_offsets[n]) * 4u);
+    out.rows = lds + (i == 1 ? at.wide : 0u);
+    out.bias = reinterpret_cast<const _Float16 *>(lds + at.bias[i]);
+    out.act = i == 1 ? 1 : 0;
+    out.add = i != 1;
+    slab_process_item<V, _Float16, 1, kXorSingle, false>(x, lds, i == 1 ? 0u : at.wide, rows, p.w[i].values, x.srd_cols, out);
+    __syncthreads();
+    if (i == 0) {
+      if (tid < 4) *reinterpret_cast<half4 *>(lds + at.wide + F * 32 + tid * 8) = half4{0, 0, 0, 0};  // (the context has been read)
+      slab_tail_norm<false>(lds, H, reinterpret_cast<const _Float16 *>(p.gamma1), reinterpret_cast<const _Float16 *>(p.beta1), p.eps1, red,
+                            nullptr, 0, live);
+      __syncthreads();
+    }
+  }
+  slab_tail_norm<true>(lds, H, reinterpret_cast<const _Float16 *>(p.gamma2), reinterpret_cast<const _Float16 *>(p.beta2), p.eps2, red,
+                       reinterpret_cast<_Float16 *>(p.out) + first, p.tokens, live);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1765,6 +1983,31 @@ static hipError_t launch_slab_kernel(const SpmmArgs &p, uint32_t grid, uint32_t 
   }
   hipLaunchKernelGGL(kern, dim3(grid), dim3(kSlabThreads), lds, stream, p, p.row_offsets, p.row_indices);
   return hipGetLastError();
+}
+
+bool encoder_tail_applies(int V, int hidden, int ffn, int tokens) {
+  return (V == 8 || V == 16) && hidden > 0 && ffn > 0 && hidden <= 1024 && hidden % V == 0 && ffn % V == 0 && ffn <= 8192 && tokens > 0 &&
+         tokens % 4 == 0 && tokens <= (1 << 24) && slab_tail_lds(V, hidden, ffn).total <= kSlabLds;
+}
+
+template <int V>
+static hipError_t launch_encoder_tail_v(const EncoderTailArgs &p, hipStream_t stream) {
+  auto kern = encoder_tail_kernel<V>;
+  static bool raised[kMaxDevices] = {};  // per instantiation and device
+  const int dev = current_device();
+  if (!raised[dev]) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSlabLds);
+    if (e != hipSuccess) return e;
+    raised[dev] = true;
+  }
+  const uint32_t line_groups = ((uint32_t)p.tokens + 63u) / 64u, grid = (line_groups + 7u) / 8u * 32u;
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(kSlabThreads), slab_tail_lds(V, p.hidden, p.ffn).total, stream, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_encoder_tail(const EncoderTailArgs &p, int V, hipStream_t stream) {
+  if (!encoder_tail_applies(V, p.hidden, p.ffn, p.tokens)) return hipErrorInvalidValue;
+  return V == 8 ? launch_encoder_tail_v<8>(p, stream) : launch_encoder_tail_v<16>(p, stream);
 }
 
 template <int V, typename OutT, int NQ, bool RAGGED>

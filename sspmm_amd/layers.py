@@ -18,6 +18,7 @@ import math
 import numpy as np
 import torch
 
+from .attention import _eager_inference, _plain_module
 from .spmm import linear as linear_op, spmm
 from .svc import svc
 
@@ -179,6 +180,84 @@ def attention_fm(qkv, hidden, heads, batch, seq, scale=None):
     return out
 
 
+# LDS of a workgroup of the launch below, which holds 16 tokens' activations of both widths, value tiles, row tables and biases
+_TAIL_LDS = 160 * 1024
+
+
+def encoder_tail_fits(hidden, ffn, tokens, V):
+    """Whether sspmm_encoder_tail_f16 takes these sizes."""
+    lds = 32 * (hidden + 1 + max(hidden, ffn) + 1) + 16 * (528 if V == 8 else 1024) + 16 * ((2 * hidden + ffn) // V + 6) + 2048 + 2 * (2 * hidden + ffn)
+    return V in (8, 16) and 0 < hidden <= 1024 and 0 < ffn <= 8192 and hidden % V == 0 and ffn % V == 0 and 0 < tokens <= 1 << 24 and \
+        tokens % 4 == 0 and lds <= _TAIL_LDS
+
+
+def encoder_tail_pays(hidden, tokens, vectors, cus):
+    """Whether the one launch is ahead of the five it replaces; `vectors`: stored vectors of its three weights.  A workgroup of
+    16 tokens, one per CU, takes as long however few of them there are: some 28 us and 0.45 us per thousand vectors, where the
+    separate launches' time follows the tokens.  Layer with 768 features (replayed, so that the host plays no part), separate / one
+    launch, us: V = 16 at 90 % (33 000 vectors) 512 tokens 47 / 55, 1024 57 / 57, 4096 89 / 69; V = 8 at 90 % (66 000) 1024
+    60 / 74, 2048 76 / 80, 3072 96 / 86, 4096 107 / 88; V = 8 at 50 % (330 000) 1536 117 / 180, 4096 210 / 205.  Beyond one
+    workgroup per CU a nearly empty last round costs a whole one: 8192 tokens 144 / 123, 7168 137 / 120, and narrow or dense weights
+    are level there (256 features V = 8 at 50 % 90 / 92, 512 at 50 % 203 / 210)."""
+    if vectors > 100000 or tokens < max(1024, vectors // 30):
+        return False
+    per_round = 16 * cus
+    rounds = -(-tokens // per_round)
+    return rounds == 1 or (hidden >= 512 and 20 * tokens >= 17 * rounds * per_round)
+
+
+_CUS = {}
+
+
+def _cus(device):
+    n = _CUS.get(device)
+    if n is None:
+        n = _CUS[device] = torch.cuda.get_device_properties(device).multi_processor_count
+    return n
+
+
+def _tail_weight(m, in_features, out_features, V, dev):
+    """(row offsets, columns, values, bias) of a SparseLinear of these sizes that does nothing but its product, without a plan,
+    on the current GPU, as the launch takes them; None otherwise."""
+    if not (_plain_module(m, SparseLinear) and m.in_features == in_features and m.out_features == out_features and m.vec_length == V and
+            m.out_dtype == torch.float16 and m.__dict__.get("plan") is None):
+        return None
+    own = m._buffers
+    off, col, val, bias = own.get("row_offsets"), own.get("column_indices"), own.get("values"), own.get("bias")
+    if not (_plain_tensor(off, torch.int32, dev) and _plain_tensor(col, torch.int32, dev) and _plain_tensor(val, torch.float16, dev) and
+            off.numel() == out_features // V + 1 and val.numel() >= col.numel() * V and
+            (bias is None or (_plain_tensor(bias, torch.float16, dev) and bias.numel() == out_features))):
+        return None
+    at = val.data_ptr()
+    return None if at % 16 else (off.data_ptr(), col.data_ptr(), at, None if bias is None else bias.data_ptr())
+
+
+def _plain_tensor(t, dtype, dev):
+    return type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == dtype and t.get_device() == dev and t.is_contiguous()
+
+
+def _tail_norm(ln, features, dev):
+    """(weight, bias, eps) of a plain LayerNorm over `features`, or None."""
+    if not (_plain_module(ln, torch.nn.LayerNorm) and ln.normalized_shape == (features,)):
+        return None
+    own = ln._parameters
+    w, b = own.get("weight"), own.get("bias")
+    if not (_plain_tensor(w, torch.float16, dev) and (b is None or _plain_tensor(b, torch.float16, dev))):
+        return None
+    return w.data_ptr(), None if b is None else b.data_ptr(), float(ln.eps)
+
+
+def encoder_tail(x, context, ffn, V, o, norm1, ffn1, ffn2, norm2):
+    """LayerNorm2(n + ffn2(gelu(ffn1(n)))) with n = LayerNorm1(x + o(context)) on feature-major activations
+    [hidden, tokens] fp16 in one launch; the weights and norms as _tail_weight and _tail_norm give them."""
+    from . import _lib
+    out = torch.empty_like(x)
+    rc = _lib.call(_lib.lib().sspmm_encoder_tail_f16, x.device, x.size(0), ffn, x.size(1), V, x.data_ptr(),
+                   context.data_ptr(), *o, *norm1, *ffn1, *ffn2, *norm2, out.data_ptr())
+    _lib.check(rc, "sspmm_encoder_tail_f16")
+    return out
+
+
 class _WithGelu:
     """A SparseLinear called with the GELU behind it."""
 
@@ -236,12 +315,42 @@ class SparseEncoderLayer(torch.nn.Module):
         ctx = torch.nn.functional.scaled_dot_product_attention(c[0], c[1], c[2], scale=1.0 / math.sqrt(d))
         return ctx.permute(1, 3, 0, 2).reshape(self.hidden, batch * seq)
 
+    def _one_launch_tail(self, x):
+        """What encoder_tail takes besides the activations, where everything behind the attention may run in that one launch
+        and is ahead so: nothing but the values is wanted, plain layers and norms, sizes that a workgroup's LDS holds."""
+        H = self.hidden
+        if not (type(self) is SparseEncoderLayer and type(x) is torch.Tensor and x.is_cuda and x.dtype == torch.float16 and x.dim() == 2 and
+                x.is_contiguous() and x.size(0) == H and x.data_ptr() % 8 == 0):
+            return None
+        own = self._modules
+        o, ffn1, ffn2 = own.get("o"), own.get("ffn1"), own.get("ffn2")
+        if not (type(o) is SparseLinear and type(ffn1) is SparseLinear and type(ffn2) is SparseLinear and o.activation is None and
+                ffn2.activation is None):
+            return None
+        V, F, T = o.vec_length, ffn1.out_features, x.size(1)
+        vectors = sum(m._buffers["column_indices"].numel() for m in (o, ffn1, ffn2))
+        if not (encoder_tail_fits(H, F, T, V) and encoder_tail_pays(H, T, vectors, _cus(x.device)) and _eager_inference()):
+            return None
+        dev = x.get_device()
+        parts = (_tail_weight(o, H, H, V, dev), _tail_norm(own.get("ln1"), H, dev), _tail_weight(ffn1, H, F, V, dev),
+                 _tail_weight(ffn2, F, H, V, dev), _tail_norm(own.get("ln2"), H, dev))
+        return None if None in parts else (F, V) + parts
+
     def forward(self, x, batch, seq, linear=None):
         """x: [hidden, batch*seq] fp16.  `linear(name, layer, x)` may replace how a projection ("qkv", "o",
         "ffn1_gelu", "ffn2"; "ffn1_gelu" is the first feed-forward product with the GELU behind it) is evaluated
         (the benchmark passes a dense matmul there to time the same layer without sparsity)."""
         f = linear or (lambda name, layer, t: layer(t))
-        a = f("o", self.o, self._attention(f("qkv", self.qkv, x), batch, seq))
+        tail = self._one_launch_tail(x) if linear is None else None
+        if tail is not None:
+            context = self._attention(self.qkv(x), batch, seq)
+            if context.shape == x.shape and context.dtype == x.dtype and context.device == x.device:
+                return encoder_tail(x, context.contiguous(), *tail)
+            return self._tail(f, x, context)
+        return self._tail(f, x, self._attention(f("qkv", self.qkv, x), batch, seq))
+
+    def _tail(self, f, x, context):
+        a = f("o", self.o, context)
         x = add_layernorm(x, a, self.ln1)
         y = f("ffn2", self.ffn2, f("ffn1_gelu", self.ffn1_gelu, x))
         return add_layernorm(x, y, self.ln2)

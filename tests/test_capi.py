@@ -125,6 +125,29 @@ def test_argument_errors_of_the_dense_block_entries(built_library):
     assert L.svc_split_row_ptr(0, 0, None, None, None, None, None) == 0
 
 
+def test_argument_errors_of_the_encoder_tail(built_library):
+    """Sizes that a workgroup's LDS does not hold, token counts, alignments and missing operands, rejected on the host; the
+    sizes that Python takes for the launch are those that the entry takes."""
+    from sspmm_amd import _lib
+    from sspmm_amd.layers import encoder_tail_fits
+    L = _lib.lib()
+    p = 4096
+
+    def tail(hidden=768, ffn=3072, tokens=64, V=16, x=p, context=p, offsets=p, cols=p, values=p, bias=p, gamma=p, beta=p, out=p):
+        w = (offsets, cols, values, bias)
+        return L.sspmm_encoder_tail_f16(hidden, ffn, tokens, V, x, context, *w, gamma, beta, 1e-5, *w, *w, gamma, beta, 1e-5, out, None)
+
+    for bad in (dict(hidden=-16), dict(ffn=-1), dict(tokens=-4), dict(tokens=66), dict(V=4), dict(V=32), dict(hidden=776), dict(ffn=3080),
+                dict(hidden=1040), dict(hidden=1024, ffn=4096), dict(hidden=0), dict(ffn=0), dict(x=None), dict(context=None), dict(out=None),
+                dict(offsets=None), dict(gamma=None), dict(x=p + 4), dict(context=p + 2), dict(out=p + 4), dict(values=p + 8), dict(cols=p + 2)):
+        assert tail(**bad) == 1, bad
+    assert tail(tokens=0) == 0
+    for V in (8, 16):
+        for hidden in range(V, 1100, 3 * V):
+            for ffn in range(V, 5000, 7 * V):
+                assert encoder_tail_fits(hidden, ffn, 64, V) == (L.sspmm_encoder_tail_fits(hidden, ffn, 64, V) == 1), (hidden, ffn, V)
+
+
 def test_python_operator_rejects_bad_arguments(built_library):
     import torch
     import sspmm_amd

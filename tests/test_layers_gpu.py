@@ -250,3 +250,49 @@ def test_sparse_linear_fuses_bias_and_activation(built_library):
 def test_feature_major_add_layernorm_of_more_than_the_caches_hold(built_library, H, T, residual):
     """Either side of 40 MiB of operands, from where most widths go through LDS."""
     test_feature_major_add_layernorm_matches_torch(built_library, H, T, residual)
+
+
+@pytest.mark.parametrize("V", [8, 16])
+@pytest.mark.parametrize("hidden,ffn,batch,seq", [(64, 64, 1, 4), (64, 256, 1, 20), (128, 64, 3, 64), (320, 1280, 1, 132), (512, 2048, 2, 68),
+                                                  (768, 3072, 3, 100), (768, 3072, 8, 512), (1024, 1024, 1, 1100)])
+def test_encoder_layers_tail_in_one_launch_matches_the_separate_launches(built_library, V, hidden, ffn, batch, seq):
+    """Output projection, norms and feed-forward products in one launch against the same layer step by step: token counts
+    around the 16 and 64 of a workgroup and its lines, rows of 0 to a few hundred vectors, with and without biases.
+    The steps round the same values to fp16 at the same places; their sums run in another order, so an activation may
+    land on the fp16 next to it (2^-11 relative), which the two norms and products behind it carry on: 2^-8 of the largest."""
+    import sspmm_amd.layers as layers_mod
+    heads = hidden // 64
+    g = torch.Generator("cuda").manual_seed(hidden + seq)
+    calls, kernel, pays = [], layers_mod.encoder_tail, layers_mod.encoder_tail_pays
+
+    def sparse(o, i, seed, bias):
+        keep = torch.rand(o // V, i, device="cuda", generator=g) < 0.1
+        keep[0] = False                            # a vector-row without vectors
+        keep[-1] = torch.arange(i, device="cuda") < 40
+        offsets = torch.zeros(o // V + 1, dtype=torch.int32, device="cuda")
+        offsets[1:] = keep.sum(1).cumsum(0).int()
+        cols = keep.nonzero()[:, 1].int().contiguous()
+        values = (torch.randn(cols.numel() * V, device="cuda", generator=g) * 0.1).half()
+        return SparseLinear.from_cvse(i, V, offsets, cols, values, torch.randn(o, device="cuda", generator=g).half() if bias else None)
+
+    for bias in (True, False):
+        layer = SparseEncoderLayer(hidden, heads, ffn, *(sparse(hidden, hidden, s, True) for s in range(3)), sparse(hidden, hidden, 4, bias),
+                                   sparse(ffn, hidden, 5, bias), sparse(hidden, ffn, 6, bias)).cuda().half().eval()
+        with torch.no_grad():
+            for ln in (layer.ln1, layer.ln2):
+                ln.weight.copy_(1 + 0.1 * torch.randn(hidden, device="cuda", generator=g))
+                ln.bias.copy_(0.1 * torch.randn(hidden, device="cuda", generator=g))
+            x = torch.randn(hidden, batch * seq, device="cuda", generator=g).half()
+            want = layer(x, batch, seq, linear=lambda name, lin, t: lin(t))
+            layers_mod.encoder_tail = lambda *a: (calls.append(1), kernel(*a))[1]
+            layers_mod.encoder_tail_pays = lambda *a: True
+            try:
+                got = layer(x, batch, seq)
+                hook = layer.o.register_forward_hook(lambda *a: None)  # (whoever watches a layer gets it called)
+                hooked = layer(x, batch, seq)
+                hook.remove()
+            finally:
+                layers_mod.encoder_tail, layers_mod.encoder_tail_pays = kernel, pays
+        assert max_rel_err(got.float().cpu().numpy(), want.float().cpu().numpy()) <= 2.0 ** -8
+        assert torch.equal(hooked, want)
+    assert len(calls) == 2
