@@ -461,6 +461,11 @@ int sspmm_block_pack_f16(int count, const sspmm_half_t *const *src, const int32_
  * ---------------------------------------------------------------------------------------- */
 int sspmm_attention_fm_f16(int batch, int heads, int seq, int head_dim, const sspmm_half_t *q, const sspmm_half_t *k,
                            const sspmm_half_t *v, int64_t ld, sspmm_half_t *out, int64_t ld_out, float scale, void *hip_stream);
+/* The same for sequences of any length up to 16384, any ld and ld_out of at least batch * seq, and rows that begin
+ * at any element.  Whole tiles of 64 aligned tokens run the same kernel as above. */
+int sspmm_attention_fm_ragged_f16(int batch, int heads, int seq, int head_dim, const sspmm_half_t *q, const sspmm_half_t *k,
+                                  const sspmm_half_t *v, int64_t ld, sspmm_half_t *out, int64_t ld_out, float scale,
+                                  void *hip_stream);
 
 /* ------------------------------------------------------------------------------------------
  * Coordinate list -> CSR, the step between a Matrix Market file and the RowMerge in the

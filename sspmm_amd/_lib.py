@@ -57,6 +57,7 @@ SIGNATURES = {
     "sspmm_encoder_tail_f16": (_int, [_int] * 4 + [_vp] * 8 + [ctypes.c_float] + [_vp] * 10 + [ctypes.c_float, _vp, _vp]),
     "sspmm_linear_f16": (_int, [_int, _int, _int, _int, _vp, _vp, _vp, _vp, _vp, _int, _vp, _vp]),
     "sspmm_attention_fm_f16": (_int, [_int, _int, _int, _int, _vp, _vp, _vp, ctypes.c_int64, _vp, ctypes.c_int64, ctypes.c_float, _vp]),
+    "sspmm_attention_fm_ragged_f16": (_int, [_int, _int, _int, _int, _vp, _vp, _vp, ctypes.c_int64, _vp, ctypes.c_int64, ctypes.c_float, _vp]),
     "svc_coo_workspace_bytes": (ctypes.c_size_t, [_i64]),
     "svc_coo_to_csr": (_int, [_int, _int, _i64, _vp, _vp, _vp, _vp, _vp, ctypes.c_size_t, _vp]),
     "svc_reorder_workspace_bytes": (ctypes.c_size_t, [_int]),

@@ -33,6 +33,8 @@ hipError_t launch_add_layernorm_rows(int E, const AddLayerNormRows &args, hipStr
 // size of 64, seq a multiple of 64 up to 16384, ld and ld_out multiples of 8 and 16-byte aligned pointers.
 bool attention_fm_applies(int batch, int heads, int seq, int head_dim, const void *q, const void *k, const void *v,
                           long long ld, const void *out, long long ld_out);
+// The same for sequences of any length up to 16384 and rows at any element.
+bool attention_fm_ragged_applies(int batch, int heads, int seq, int head_dim, const void *q, const void *k, const void *v, const void *out);
 hipError_t launch_attention_fm(int batch, int heads, int seq, const uint16_t *q, const uint16_t *k, const uint16_t *v,
                                long long ld, uint16_t *out, long long ld_out, float scale, hipStream_t stream);
 

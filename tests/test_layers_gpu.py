@@ -122,6 +122,36 @@ def test_feature_major_attention_matches_fp32_attention(built_library, batch, he
     assert torch.all(out[:, T:] == 7.0)
 
 
+@pytest.mark.parametrize("batch,heads,seq", [(1, 1, 1), (1, 2, 7), (3, 1, 24), (2, 2, 32), (2, 3, 33), (1, 1, 63), (5, 2, 65), (1, 4, 100), (3, 2, 127),
+                                             (2, 1, 160), (1, 1, 191), (8, 12, 500), (1, 2, 1000), (3, 1, 64)])
+def test_feature_major_attention_on_ragged_sequences(built_library, batch, heads, seq):
+    """Lengths either side of the 32 keys of a wave, the 64 of a block and the eight tokens of a piece, rows at odd elements: the
+    context against fp32 attention (same bound as for whole blocks), nothing written beside it, and what surrounds the
+    operands (NaN) not let in."""
+    from sspmm_amd import _lib
+    from sspmm_amd.layers import attention_fm
+    hidden, T = heads * 64, batch * seq
+    g = torch.Generator("cuda").manual_seed(seq + heads)
+    qkv = torch.randn(3 * hidden, T, device="cuda", generator=g).half()
+    got = attention_fm(qkv, hidden, heads, batch, seq)
+    want = _attention_reference(qkv[:hidden], qkv[hidden:2 * hidden], qkv[2 * hidden:], batch, heads, seq, 0.125)
+    assert got.shape == want.shape and (got.float() - want).abs().max().item() <= 2e-3 * max(1.0, want.abs().max().item())
+    for scale, lead in ((0.125, 3), (2.0, 1)):
+        ld, ld_out = T + 5, T + 3
+        q, k, v = (torch.full((hidden * ld + 16,), float("nan"), dtype=torch.float16, device="cuda") for _ in range(3))
+        views = [t[lead:lead + hidden * ld].view(hidden, ld) for t in (q, k, v)]
+        for t in views:
+            t[:, :T] = (torch.randn(hidden, T, device="cuda", generator=g) * (0.25 if scale > 1 else 1)).half()
+        out = torch.full((hidden * ld_out + 16,), 7.0, dtype=torch.float16, device="cuda")
+        o = out[lead:lead + hidden * ld_out].view(hidden, ld_out)
+        rc = _lib.lib().sspmm_attention_fm_ragged_f16(batch, heads, seq, 64, *(t.data_ptr() for t in views), ld, o.data_ptr(), ld_out, scale,
+                                                      torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        want = _attention_reference(*(t[:, :T] for t in views), batch, heads, seq, scale)
+        assert (o[:, :T].float() - want).abs().max().item() <= 2e-3 * max(1.0, want.abs().max().item())
+        assert torch.all(o[:, T:] == 7.0) and torch.all(out[:lead] == 7.0) and torch.all(out[lead + hidden * ld_out:] == 7.0)
+
+
 def test_feature_major_attention_with_maxima_that_keep_growing(built_library):
     """Keys whose norm grows along the sequence: the running maximum of a query's scores rises by many units from one
     block of keys to the next, so the kernel moves the reference point of its exponentials again and again (it
