@@ -122,8 +122,8 @@ int sspmm_linear_f16(int m_vec, int V, int N, int K, const int32_t *row_offsets,
  * Wo is [hidden, hidden], W1 [ffn, hidden], W2 [hidden, ffn], each row offsets, column indices and
  * values as for sspmm_linear_f16, biases and beta or NULL.  Every activation is rounded to fp16, sums
  * and statistics are fp32.  out may be neither x nor context.
- * tokens a multiple of 4, hidden up to 1024, hidden and ffn multiples of V and together up to about
- * 4300 (they share a CU's LDS); values 16-byte, activations 8-byte aligned.  Other sizes: error.
+ * Hidden up to 1024, hidden and ffn multiples of V and together up to about 4300 (they share a CU's LDS);
+ * values 16-byte aligned, activations at any element, any number of tokens.  Other sizes: error.
  * ---------------------------------------------------------------------------------------- */
 int sspmm_encoder_tail_fits(int hidden, int ffn, int tokens, int V); /* 1 where the launch takes these sizes, else 0 */
 int sspmm_encoder_tail_f16(int hidden, int ffn, int tokens, int V, const sspmm_half_t *x,
@@ -403,6 +403,10 @@ int svc_permute_csr(int M, const int32_t *perm, const int32_t *row_ptr, const in
  * ---------------------------------------------------------------------------------------- */
 int sspmm_add_layernorm_f16(int H, int T, const sspmm_half_t *x, const sspmm_half_t *a, const sspmm_half_t *gamma,
                             const sspmm_half_t *beta, float eps, sspmm_half_t *out, void *hip_stream);
+/* The same for any T and rows that begin at any element. */
+int sspmm_add_layernorm_ragged_f16(int H, int T, const sspmm_half_t *x, const sspmm_half_t *a, const sspmm_half_t *gamma,
+                                   const sspmm_half_t *beta, float eps, sspmm_half_t *out, void *hip_stream);
+
 
 /*
  * The same on token-major rows of E features (E = 64, 128, 256, 512, 1024 or 2048), outer x inner of them:

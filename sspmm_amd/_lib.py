@@ -49,6 +49,7 @@ SIGNATURES = {
     "svc_count_batched": (_int, [_int, _int, _vp, _int, _int, _int, _vp, _vp, _i64, _int, _vp, _vp, _vp, _vp]),
     "svc_fill_batched": (_int, [_int, _int, _vp, _int, _int, _int, _vp, _vp, _vp, _i64, _int, _vp, _vp, _vp, _vp, _vp]),
     "sspmm_add_layernorm_f16": (_int, [_int, _int, _vp, _vp, _vp, _vp, ctypes.c_float, _vp, _vp]),
+    "sspmm_add_layernorm_ragged_f16": (_int, [_int, _int, _vp, _vp, _vp, _vp, ctypes.c_float, _vp, _vp]),
     "sspmm_block_pack_f16": (_int, [_int, _vp, _vp, _vp, _vp, _vp, _vp]),
     "sspmm_block_dense_f16": (_int, [_int, _int, _int, _vp, _i64, _i64, _vp, ctypes.c_float, _vp, _vp, _vp, _vp, _vp, ctypes.c_float, _int, _vp, _vp, _vp, _vp,
                                      _vp, _vp, ctypes.c_float, _int, _int, _vp, _vp, _vp, _vp, _vp]),

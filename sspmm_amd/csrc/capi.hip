@@ -121,7 +121,7 @@ int sspmm_encoder_tail_f16(int hidden, int ffn, int tokens, int V, const sspmm_h
   for (const sspmm_half_t *q : {o_values, f1_values, f2_values}) values |= reinterpret_cast<uintptr_t>(q);
   for (const sspmm_half_t *q : {x, context, (const sspmm_half_t *)out}) rows |= reinterpret_cast<uintptr_t>(q);
   for (const int32_t *q : {o_offsets, o_cols, f1_offsets, f1_cols, f2_offsets, f2_cols}) ints |= reinterpret_cast<uintptr_t>(q);
-  if (values % 16 || rows % 8 || ints % 4) return kInvalid;
+  if (values % 16 || rows % 2 || ints % 4) return kInvalid;
   sspmm::EncoderTailArgs p;
   p.hidden = hidden;
   p.ffn = ffn;
@@ -525,6 +525,15 @@ int sspmm_add_layernorm_f16(int H, int T, const sspmm_half_t *x, const sspmm_hal
   if (!x || !out) return kInvalid;
   if (reinterpret_cast<uintptr_t>(x) % 8 || reinterpret_cast<uintptr_t>(a) % 8 || reinterpret_cast<uintptr_t>(out) % 8)
     return kInvalid;
+  return (int)sspmm::launch_add_layernorm(H, T, x, a, gamma, beta, eps, out, static_cast<hipStream_t>(hip_stream));
+}
+
+int sspmm_add_layernorm_ragged_f16(int H, int T, const sspmm_half_t *x, const sspmm_half_t *a, const sspmm_half_t *gamma,
+                                   const sspmm_half_t *beta, float eps, sspmm_half_t *out, void *hip_stream) {
+  if (H < 0 || T < 0 || H > 4096 || T > (1 << 30)) return kInvalid;
+  if (H == 0 || T == 0) return 0;
+  if (!x || !out) return kInvalid;
+  if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(out)) % 2) return kInvalid;
   return (int)sspmm::launch_add_layernorm(H, T, x, a, gamma, beta, eps, out, static_cast<hipStream_t>(hip_stream));
 }
 

@@ -76,6 +76,40 @@ __device__ __forceinline__ float wave_sum_all(float x) {
 // The value lane 63 holds, in every lane.
 __device__ __forceinline__ uint32_t from_last_lane(uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, 63); }
 
+// Four consecutive fp16 values of a row of which `left` exist.  RAGGED: the row begins at any element, and what lies behind its
+// end is neither read nor written.
+typedef _Float16 four_halfs __attribute__((ext_vector_type(4)));
+typedef _Float16 four_halfs_any __attribute__((ext_vector_type(4), aligned(2)));
+template <bool RAGGED, bool NT = false>
+__device__ __forceinline__ four_halfs load_four(const _Float16 *p, int left) {
+  if constexpr (RAGGED) {
+    if (left >= 4) return *reinterpret_cast<const four_halfs_any *>(p);
+    four_halfs v = {0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      if (i < left) v[i] = p[i];
+    return v;
+  } else if constexpr (NT) {
+    return __builtin_nontemporal_load(reinterpret_cast<const four_halfs *>(p));
+  } else {
+    return *reinterpret_cast<const four_halfs *>(p);
+  }
+}
+template <bool RAGGED>
+__device__ __forceinline__ void store_four(_Float16 *p, four_halfs v, int left) {
+  if constexpr (RAGGED) {
+    if (left >= 4) {
+      *reinterpret_cast<four_halfs_any *>(p) = v;
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      if (i < left) p[i] = v[i];
+  } else {
+    *reinterpret_cast<four_halfs *>(p) = v;
+  }
+}
+
 // Sum of v over the lanes of the wave with the same lane % 4, in each of them.
 __device__ __forceinline__ float sum_over_quads(float v) {
   v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, false));  // rotated by 8 in each 16

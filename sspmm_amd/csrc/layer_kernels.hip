@@ -51,7 +51,9 @@ __device__ __forceinline__ floatx4 block_sum_per_token(floatx4 v, floatx4 *red, 
   return s;
 }
 
-template <int TOK, int THREADS, int TRIP, bool NT = true>
+// RAGGED: T any number of tokens, rows at any element (such calls had torch's LayerNorm between two transposed copies: 768 x 4000
+// 46 us a call where this takes 9, 768 x 1665 29 and 12, of which the host is most).
+template <int TOK, int THREADS, int TRIP, bool RAGGED>
 __global__ __launch_bounds__(THREADS) void add_layernorm_kernel(int H, int T, const _Float16 *__restrict__ x,
                                                                  const _Float16 *__restrict__ a,
                                                                  const _Float16 *__restrict__ gamma,
@@ -68,7 +70,8 @@ __global__ __launch_bounds__(THREADS) void add_layernorm_kernel(int H, int T, co
   const int first = (((idx / S::kParts) * 8 + xcd) * S::kParts + (idx % S::kParts)) * TOK;
   if (first >= T) return;  // (the whole workgroup: the grid is padded to eight line groups)
   const int t0 = first + 4 * tl;
-  const bool live = t0 < T;  // (T is a multiple of 4: a group of four tokens is inside or outside as a whole)
+  const bool live = t0 < T;
+  const int left = T - t0;  // (at least 4 where T is a multiple of it)
   floatx4 acc = {0.f, 0.f, 0.f, 0.f};
   // (the loads of TRIP rows are issued together: the kernel is bound by how many bytes its workgroups keep in flight)
   for (int h0 = rg; h0 < H; h0 += S::kRowGroups * TRIP) {
@@ -79,13 +82,8 @@ __global__ __launch_bounds__(THREADS) void add_layernorm_kernel(int H, int T, co
       xs[u] = half4{0, 0, 0, 0};
       as[u] = half4{0, 0, 0, 0};
       if (live && h < H) {
-        if (NT) {
-          xs[u] = __builtin_nontemporal_load(reinterpret_cast<const half4 *>(x + (size_t)h * T + t0));
-          if (a) as[u] = __builtin_nontemporal_load(reinterpret_cast<const half4 *>(a + (size_t)h * T + t0));
-        } else {
-          xs[u] = *reinterpret_cast<const half4 *>(x + (size_t)h * T + t0);
-          if (a) as[u] = *reinterpret_cast<const half4 *>(a + (size_t)h * T + t0);
-        }
+        xs[u] = load_four<RAGGED, true>(x + (size_t)h * T + t0, left);
+        if (a) as[u] = load_four<RAGGED, true>(a + (size_t)h * T + t0, left);
       }
     }
 #pragma unroll
@@ -120,14 +118,14 @@ __global__ __launch_bounds__(THREADS) void add_layernorm_kernel(int H, int T, co
     half4 o;
 #pragma unroll
     for (int i = 0; i < 4; ++i) o[i] = (_Float16)(((float)s[i] - mean[i]) * rstd[i] * w + b);
-    *reinterpret_cast<half4 *>(out + (size_t)h * T + t0) = o;
+    store_four<RAGGED>(out + (size_t)h * T + t0, o, left);
   }
 }
 
 // The same for up to 128 * TRIP features with the sums kept in registers: no pass over LDS, two barriers (one per
 // reduction) and the reductions on lane moves of the vector unit.  A workgroup's loads, gamma and beta among them, are all
 // in flight together.  768 x 4096: 7.2 us against 8.7, 512 x 4096 5.6 against 6.9, 1024 x 8192 18.3 against 19.7.
-template <int TRIP>
+template <int TRIP, bool RAGGED>
 __global__ __launch_bounds__(512) void add_layernorm_held_kernel(int H, int T, const _Float16 *__restrict__ x, const _Float16 *__restrict__ a,
                                                                  const _Float16 *__restrict__ gamma, const _Float16 *__restrict__ beta,
                                                                  float eps, _Float16 *__restrict__ out) {
@@ -139,6 +137,7 @@ __global__ __launch_bounds__(512) void add_layernorm_held_kernel(int H, int T, c
   if (first >= T) return;
   const int t0 = first + 4 * tl;
   const bool live = t0 < T;
+  const int left = T - t0;
   half4 s[TRIP], r[TRIP];
   float w[TRIP], b[TRIP];
 #pragma unroll
@@ -147,8 +146,8 @@ __global__ __launch_bounds__(512) void add_layernorm_held_kernel(int H, int T, c
     s[u] = half4{0, 0, 0, 0};
     r[u] = half4{0, 0, 0, 0};
     if (live && h < H) {
-      s[u] = __builtin_nontemporal_load(reinterpret_cast<const half4 *>(x + (size_t)h * T + t0));
-      if (a) r[u] = __builtin_nontemporal_load(reinterpret_cast<const half4 *>(a + (size_t)h * T + t0));
+      s[u] = load_four<RAGGED, true>(x + (size_t)h * T + t0, left);
+      if (a) r[u] = load_four<RAGGED, true>(a + (size_t)h * T + t0, left);
     }
   }
 #pragma unroll
@@ -200,24 +199,24 @@ __global__ __launch_bounds__(512) void add_layernorm_held_kernel(int H, int T, c
     half4 o;
 #pragma unroll
     for (int i = 0; i < 4; ++i) o[i] = (_Float16)(((float)s[u][i] - stat[0][i]) * stat[1][i] * w[u] + b[u]);
-    *reinterpret_cast<half4 *>(out + (size_t)h * T + t0) = o;
+    store_four<RAGGED>(out + (size_t)h * T + t0, o, left);
   }
 }
-template <int TRIP>
+template <int TRIP, bool RAGGED>
 static hipError_t launch_ln_held(int H, int T, const uint16_t *x, const uint16_t *a, const uint16_t *gamma, const uint16_t *beta, float eps,
                                  uint16_t *out, hipStream_t stream) {
   const int line_groups = (T + 63) / 64, blocks = ((line_groups + 7) / 8) * 8 * 4;
-  hipLaunchKernelGGL((add_layernorm_held_kernel<TRIP>), dim3(blocks), dim3(512), 0, stream, H, T, reinterpret_cast<const _Float16 *>(x),
+  hipLaunchKernelGGL((add_layernorm_held_kernel<TRIP, RAGGED>), dim3(blocks), dim3(512), 0, stream, H, T, reinterpret_cast<const _Float16 *>(x),
                      reinterpret_cast<const _Float16 *>(a), reinterpret_cast<const _Float16 *>(gamma),
                      reinterpret_cast<const _Float16 *>(beta), eps, reinterpret_cast<_Float16 *>(out));
   return hipGetLastError();
 }
 
-template <int TOK, int THREADS, int TRIP, bool NT = true>
+template <int TOK, int THREADS, int TRIP, bool RAGGED>
 static hipError_t launch_ln(int H, int T, const uint16_t *x, const uint16_t *a, const uint16_t *gamma, const uint16_t *beta,
                             float eps, uint16_t *out, hipStream_t stream) {
   const size_t lds = (size_t)H * TOK * 2 + (size_t)(THREADS / 64) * (TOK / 4) * 16;
-  auto kern = add_layernorm_kernel<TOK, THREADS, TRIP, NT>;
+  auto kern = add_layernorm_kernel<TOK, THREADS, TRIP, RAGGED>;
   if (lds > 64 * 1024) {
     // the runtime is told once per device and size
     static int raised[16] = {};
@@ -239,7 +238,8 @@ static hipError_t launch_ln(int H, int T, const uint16_t *x, const uint16_t *a, 
   return hipGetLastError();
 }
 
-hipError_t launch_add_layernorm(int H, int T, const uint16_t *x, const uint16_t *a, const uint16_t *gamma,
+template <bool RAGGED>
+static hipError_t launch_ln_any(int H, int T, const uint16_t *x, const uint16_t *a, const uint16_t *gamma,
                                 const uint16_t *beta, float eps, uint16_t *out, hipStream_t stream) {
   // 16 tokens and eight waves per workgroup, six rows per thread in flight (measured on 768 x 4096 against 32 and 64
   // tokens, 4 to 16 waves, 3 to 12 rows: 8.5 us against 9-15); up to 1024 features the sums fit the registers of that shape,
@@ -251,10 +251,16 @@ hipError_t launch_add_layernorm(int H, int T, const uint16_t *x, const uint16_t 
   // 160 x 131072 41.4 / 47.0; more than 512 features with a residual, 640 x 32768 55.0 / 58.5, 1024 x 32768 84.9 / 91.2.
   const bool large = (int64_t)H * T * (a ? 6 : 4) >= (40 << 20);
   const bool held = H <= 1024 && !(large && H >= 256 && (H <= 512 || !a));
-  if (held && H <= 512) return launch_ln_held<4>(H, T, x, a, gamma, beta, eps, out, stream);
-  if (held && H <= 768) return launch_ln_held<6>(H, T, x, a, gamma, beta, eps, out, stream);
-  if (held) return launch_ln_held<8>(H, T, x, a, gamma, beta, eps, out, stream);
-  return launch_ln<16, 512, 6>(H, T, x, a, gamma, beta, eps, out, stream);
+  if (held && H <= 512) return launch_ln_held<4, RAGGED>(H, T, x, a, gamma, beta, eps, out, stream);
+  if (held && H <= 768) return launch_ln_held<6, RAGGED>(H, T, x, a, gamma, beta, eps, out, stream);
+  if (held) return launch_ln_held<8, RAGGED>(H, T, x, a, gamma, beta, eps, out, stream);
+  return launch_ln<16, 512, 6, RAGGED>(H, T, x, a, gamma, beta, eps, out, stream);
+}
+// (T a multiple of 4 with rows at multiples of 8 bytes keeps the kernels without the tests for a row's end)
+hipError_t launch_add_layernorm(int H, int T, const uint16_t *x, const uint16_t *a, const uint16_t *gamma,
+                                const uint16_t *beta, float eps, uint16_t *out, hipStream_t stream) {
+  const bool whole = T % 4 == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(out)) & 7u) == 0;
+  return whole ? launch_ln_any<false>(H, T, x, a, gamma, beta, eps, out, stream) : launch_ln_any<true>(H, T, x, a, gamma, beta, eps, out, stream);
 }
 
 // ------------------------------------------------------------------------------------------

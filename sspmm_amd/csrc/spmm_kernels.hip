@@ -1253,10 +1253,10 @@ struct SlabTailStore {
 };
 
 // LayerNorm of the 16 tokens over H rows (16 waves; H <= 1024), statistics in fp32, mean first.  dst: the rows' own place, or
-// memory with `pitch` elements between rows.  Contains barriers; every thread must call it.
-template <bool TO_MEMORY>
+// memory with `pitch` elements between rows, `left` of the thread's four tokens.  Contains barriers; every thread must call it.
+template <bool TO_MEMORY, bool RAGGED>
 __device__ __forceinline__ void slab_tail_norm(unsigned char *rows, int H, const _Float16 *gamma, const _Float16 *beta, float eps,
-                                               floatx4 (*red)[kSlabWaves][4], _Float16 *dst, int64_t pitch, bool live) {
+                                               floatx4 (*red)[kSlabWaves][4], _Float16 *dst, int64_t pitch, int left) {
   constexpr int TRIP = 4, kGroups = kSlabThreads / 4;
   const int tid = threadIdx.x, tl = tid & 3, rg = tid >> 2, lane = tid & 63, wave = tid >> 6;
   half4 s[TRIP];
@@ -1311,7 +1311,7 @@ __device__ __forceinline__ void slab_tail_norm(unsigned char *rows, int H, const
 #pragma unroll
     for (int i = 0; i < 4; ++i) o[i] = (_Float16)(((float)s[u][i] - stat[0][i]) * stat[1][i] * w[u] + b[u]);
     if (!TO_MEMORY) *reinterpret_cast<half4 *>(rows + h * 32 + tl * 8) = o;
-    else if (live) *reinterpret_cast<half4 *>(dst + (int64_t)h * pitch + 4 * tl) = o;
+    else if (left > 0) store_four<RAGGED>(dst + (int64_t)h * pitch + 4 * tl, o, left);
   }
 }
 
@@ -1339,7 +1339,7 @@ __host__ __device__ inline SlabTailLds slab_tail_lds(int V, int hidden, int ffn)
   return o;
 }
 
-template <int V>
+template <int V, bool RAGGED>
 __global__ __launch_bounds__(kSlabThreads) void encoder_tail_kernel(const EncoderTailArgs p) {
   extern __shared__ __align__(256) unsigned char lds[];
   const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
@@ -1349,7 +1349,7 @@ __global__ __launch_bounds__(kSlabThreads) void encoder_tail_kernel(const Encode
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int H = p.hidden, F = p.ffn;
   const SlabTailLds at = slab_tail_lds(V, H, F);
-  const bool live = first + 4 * (tid & 3) < p.tokens;  // (tokens is a multiple of 4)
+  const int left = p.tokens - first - 4 * (tid & 3);  // tokens from the thread's four on
 
   const _Float16 *const xg = reinterpret_cast<const _Float16 *>(p.x) + first, *const cg = reinterpret_cast<const _Float16 *>(p.context) + first;
   half4 xs[4], cs[4];
@@ -1357,9 +1357,9 @@ __global__ __launch_bounds__(kSlabThreads) void encoder_tail_kernel(const Encode
   for (int u = 0; u < 4; ++u) {
     const int h = (tid >> 2) + u * (kSlabThreads / 4);
     xs[u] = cs[u] = half4{0, 0, 0, 0};
-    if (live && h < H) {
-      cs[u] = *reinterpret_cast<const half4 *>(cg + (int64_t)h * p.tokens + 4 * (tid & 3));
-      xs[u] = *reinterpret_cast<const half4 *>(xg + (int64_t)h * p.tokens + 4 * (tid & 3));
+    if (left > 0 && h < H) {
+      cs[u] = load_four<RAGGED>(cg + (int64_t)h * p.tokens + 4 * (tid & 3), left);
+      xs[u] = load_four<RAGGED>(xg + (int64_t)h * p.tokens + 4 * (tid & 3), left);
     }
   }
   const int out_rows[3] = {H, F, H};
@@ -1422,13 +1422,13 @@ __global__ __launch_bounds__(kSlabThreads) void encoder_tail_kernel(const Encode
     __syncthreads();
     if (i == 0) {
       if (tid < 4) *reinterpret_cast<half4 *>(lds + at.wide + F * 32 + tid * 8) = half4{0, 0, 0, 0};  // (the context has been read)
-      slab_tail_norm<false>(lds, H, reinterpret_cast<const _Float16 *>(p.gamma1), reinterpret_cast<const _Float16 *>(p.beta1), p.eps1, red,
-                            nullptr, 0, live);
+      slab_tail_norm<false, RAGGED>(lds, H, reinterpret_cast<const _Float16 *>(p.gamma1), reinterpret_cast<const _Float16 *>(p.beta1), p.eps1, red,
+                                    nullptr, 0, left);
       __syncthreads();
     }
   }
-  slab_tail_norm<true>(lds, H, reinterpret_cast<const _Float16 *>(p.gamma2), reinterpret_cast<const _Float16 *>(p.beta2), p.eps2, red,
-                       reinterpret_cast<_Float16 *>(p.out) + first, p.tokens, live);
+  slab_tail_norm<true, RAGGED>(lds, H, reinterpret_cast<const _Float16 *>(p.gamma2), reinterpret_cast<const _Float16 *>(p.beta2), p.eps2, red,
+                               reinterpret_cast<_Float16 *>(p.out) + first, p.tokens, left);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1987,12 +1987,12 @@ static hipError_t launch_slab_kernel(const SpmmArgs &p, uint32_t grid, uint32_t 
 
 bool encoder_tail_applies(int V, int hidden, int ffn, int tokens) {
   return (V == 8 || V == 16) && hidden > 0 && ffn > 0 && hidden <= 1024 && hidden % V == 0 && ffn % V == 0 && ffn <= 8192 && tokens > 0 &&
-         tokens % 4 == 0 && tokens <= (1 << 24) && slab_tail_lds(V, hidden, ffn).total <= kSlabLds;
+         tokens <= (1 << 24) && slab_tail_lds(V, hidden, ffn).total <= kSlabLds;
 }
 
-template <int V>
+template <int V, bool RAGGED>
 static hipError_t launch_encoder_tail_v(const EncoderTailArgs &p, hipStream_t stream) {
-  auto kern = encoder_tail_kernel<V>;
+  auto kern = encoder_tail_kernel<V, RAGGED>;
   static bool raised[kMaxDevices] = {};  // per instantiation and device
   const int dev = current_device();
   if (!raised[dev]) {
@@ -2007,7 +2007,9 @@ static hipError_t launch_encoder_tail_v(const EncoderTailArgs &p, hipStream_t st
 
 hipError_t launch_encoder_tail(const EncoderTailArgs &p, int V, hipStream_t stream) {
   if (!encoder_tail_applies(V, p.hidden, p.ffn, p.tokens)) return hipErrorInvalidValue;
-  return V == 8 ? launch_encoder_tail_v<8>(p, stream) : launch_encoder_tail_v<16>(p, stream);
+  const bool whole = p.tokens % 4 == 0 && ((reinterpret_cast<uintptr_t>(p.x) | reinterpret_cast<uintptr_t>(p.context) | reinterpret_cast<uintptr_t>(p.out)) & 7u) == 0;
+  if (V == 8) return whole ? launch_encoder_tail_v<8, false>(p, stream) : launch_encoder_tail_v<8, true>(p, stream);
+  return whole ? launch_encoder_tail_v<16, false>(p, stream) : launch_encoder_tail_v<16, true>(p, stream);
 }
 
 template <int V, typename OutT, int NQ, bool RAGGED>

@@ -147,15 +147,24 @@ def add_layernorm(x, a, ln):
     where its shape limits hold, torch on transposed copies otherwise."""
     from . import _lib
     H, T = x.shape
-    ok = (x.dtype == torch.float16 and x.is_cuda and x.is_contiguous() and T % 4 == 0 and H <= 4096 and
+    w, b = ln.weight, ln.bias
+    whole = T % 4 == 0
+    ok = (x.dtype == torch.float16 and x.is_cuda and x.is_contiguous() and H <= 4096 and
           (a is None or (a.dtype == torch.float16 and a.is_contiguous() and a.shape == x.shape)) and
-          ln.weight is not None and ln.weight.dtype == torch.float16 and tuple(ln.normalized_shape) == (H,))
+          w is not None and w.dtype == torch.float16 and tuple(ln.normalized_shape) == (H,))
+    if ok and not whole:
+        # (tokens that are no multiple of 4 had torch's module, which whoever wants gradients or watches it still gets)
+        dev = x.get_device()
+        ok = (0 < T <= 1 << 30 and _plain_module(ln, torch.nn.LayerNorm) and _eager_inference() and type(x) is torch.Tensor and
+              (a is None or (type(a) is torch.Tensor and a.get_device() == dev)) and _plain_tensor(w, torch.float16, dev) and
+              (b is None or _plain_tensor(b, torch.float16, dev)))
     if not ok:
         s = x if a is None else x + a
         return ln(s.t()).t().contiguous()
     out = torch.empty_like(x)
-    rc = _lib.call(_lib.lib().sspmm_add_layernorm_f16, x.device, H, T, x.data_ptr(), 0 if a is None else a.data_ptr(),
-                   ln.weight.data_ptr(), 0 if ln.bias is None else ln.bias.data_ptr(), float(ln.eps), out.data_ptr())
+    L = _lib.lib()
+    rc = _lib.call(L.sspmm_add_layernorm_f16 if whole else L.sspmm_add_layernorm_ragged_f16, x.device, H, T, x.data_ptr(),
+                   0 if a is None else a.data_ptr(), w.data_ptr(), 0 if b is None else b.data_ptr(), float(ln.eps), out.data_ptr())
     _lib.check(rc, "sspmm_add_layernorm_f16")
     return out
 
@@ -195,7 +204,10 @@ def encoder_tail_fits(hidden, ffn, tokens, V):
     """Whether sspmm_encoder_tail_f16 takes these sizes."""
     lds = 32 * (hidden + 1 + max(hidden, ffn) + 1) + 16 * (528 if V == 8 else 1024) + 16 * ((2 * hidden + ffn) // V + 6) + 2048 + 2 * (2 * hidden + ffn)
     return V in (8, 16) and 0 < hidden <= 1024 and 0 < ffn <= 8192 and hidden % V == 0 and ffn % V == 0 and 0 < tokens <= 1 << 24 and \
-        tokens % 4 == 0 and lds <= _TAIL_LDS
+        lds <= _TAIL_LDS
+
+
+TAIL_TOKENS = 1024
 
 
 def encoder_tail_pays(hidden, tokens, vectors, cus):
@@ -206,7 +218,7 @@ def encoder_tail_pays(hidden, tokens, vectors, cus):
     60 / 74, 2048 76 / 80, 3072 96 / 86, 4096 107 / 88; V = 8 at 50 % (330 000) 1536 117 / 180, 4096 210 / 205.  Beyond one
     workgroup per CU a nearly empty last round costs a whole one: 8192 tokens 144 / 123, 7168 137 / 120, and narrow or dense weights
     are level there (256 features V = 8 at 50 % 90 / 92, 512 at 50 % 203 / 210)."""
-    if vectors > 100000 or tokens < max(1024, vectors // 30):
+    if vectors > 100000 or tokens < max(TAIL_TOKENS, vectors // 30):
         return False
     per_round = 16 * cus
     rounds = -(-tokens // per_round)
@@ -325,9 +337,10 @@ class SparseEncoderLayer(torch.nn.Module):
     def _one_launch_tail(self, x):
         """What encoder_tail takes besides the activations, where everything behind the attention may run in that one launch
         and is ahead so: nothing but the values is wanted, plain layers and norms, sizes that a workgroup's LDS holds."""
+        if type(x) is not torch.Tensor or x.dim() != 2 or x.size(1) < TAIL_TOKENS:  # (small calls are not kept waiting by the rest)
+            return None
         H = self.hidden
-        if not (type(self) is SparseEncoderLayer and type(x) is torch.Tensor and x.is_cuda and x.dtype == torch.float16 and x.dim() == 2 and
-                x.is_contiguous() and x.size(0) == H and x.data_ptr() % 8 == 0):
+        if not (type(self) is SparseEncoderLayer and x.is_cuda and x.dtype == torch.float16 and x.is_contiguous() and x.size(0) == H):
             return None
         own = self._modules
         o, ffn1, ffn2 = own.get("o"), own.get("ffn1"), own.get("ffn2")

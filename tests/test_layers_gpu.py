@@ -284,16 +284,17 @@ def test_feature_major_add_layernorm_of_more_than_the_caches_hold(built_library,
 
 @pytest.mark.parametrize("V", [8, 16])
 @pytest.mark.parametrize("hidden,ffn,batch,seq", [(64, 64, 1, 4), (64, 256, 1, 20), (128, 64, 3, 64), (320, 1280, 1, 132), (512, 2048, 2, 68),
-                                                  (768, 3072, 3, 100), (768, 3072, 8, 512), (1024, 1024, 1, 1100)])
+                                                  (768, 3072, 3, 100), (768, 3072, 8, 512), (1024, 1024, 1, 1100),
+                                                  (64, 128, 1, 1), (128, 128, 1, 15), (256, 64, 1, 18), (512, 2048, 3, 37), (768, 3072, 5, 333)])
 def test_encoder_layers_tail_in_one_launch_matches_the_separate_launches(built_library, V, hidden, ffn, batch, seq):
     """Output projection, norms and feed-forward products in one launch against the same layer step by step: token counts
-    around the 16 and 64 of a workgroup and its lines, rows of 0 to a few hundred vectors, with and without biases.
+    around the 16 and 64 of a workgroup and its lines and no multiple of the 4 of a thread, rows of 0 to a few hundred vectors, with and without biases.
     The steps round the same values to fp16 at the same places; their sums run in another order, so an activation may
     land on the fp16 next to it (2^-11 relative), which the two norms and products behind it carry on: 2^-8 of the largest."""
     import sspmm_amd.layers as layers_mod
     heads = hidden // 64
     g = torch.Generator("cuda").manual_seed(hidden + seq)
-    calls, kernel, pays = [], layers_mod.encoder_tail, layers_mod.encoder_tail_pays
+    calls, kernel, pays, least = [], layers_mod.encoder_tail, layers_mod.encoder_tail_pays, layers_mod.TAIL_TOKENS
 
     def sparse(o, i, seed, bias):
         keep = torch.rand(o // V, i, device="cuda", generator=g) < 0.1
@@ -315,14 +316,43 @@ def test_encoder_layers_tail_in_one_launch_matches_the_separate_launches(built_l
             x = torch.randn(hidden, batch * seq, device="cuda", generator=g).half()
             want = layer(x, batch, seq, linear=lambda name, lin, t: lin(t))
             layers_mod.encoder_tail = lambda *a: (calls.append(1), kernel(*a))[1]
-            layers_mod.encoder_tail_pays = lambda *a: True
+            layers_mod.encoder_tail_pays, layers_mod.TAIL_TOKENS = lambda *a: True, 1
             try:
                 got = layer(x, batch, seq)
                 hook = layer.o.register_forward_hook(lambda *a: None)  # (whoever watches a layer gets it called)
                 hooked = layer(x, batch, seq)
                 hook.remove()
             finally:
-                layers_mod.encoder_tail, layers_mod.encoder_tail_pays = kernel, pays
+                layers_mod.encoder_tail, layers_mod.encoder_tail_pays, layers_mod.TAIL_TOKENS = kernel, pays, least
         assert max_rel_err(got.float().cpu().numpy(), want.float().cpu().numpy()) <= 2.0 ** -8
         assert torch.equal(hooked, want)
     assert len(calls) == 2
+
+
+@pytest.mark.parametrize("H", [40, 200, 512, 768, 1000, 1100])
+@pytest.mark.parametrize("T", [1, 2, 3, 5, 15, 18, 63, 65, 130, 1021])
+def test_feature_major_add_layernorm_on_any_number_of_tokens(built_library, H, T):
+    """The kernels on rows at odd elements against the same kernels on the same tokens padded to a multiple of four (the same
+    operations on every token: the same bits), with what surrounds the operands (NaN) not let in and nothing written beside
+    the result; and the module once more for whoever wants gradients."""
+    from sspmm_amd import _lib
+    from sspmm_amd.layers import add_layernorm
+    g = torch.Generator("cuda").manual_seed(H + T)
+    wide = (T + 3) // 4 * 4
+    ln = torch.nn.LayerNorm(H).cuda().half()
+    xs, rs = (torch.randn(H, wide, device="cuda", generator=g).half() for _ in range(2))
+    with torch.no_grad():
+        ln.weight.copy_(1 + 0.1 * torch.randn(H, device="cuda", generator=g))
+        ln.bias.copy_(0.1 * torch.randn(H, device="cuda", generator=g))
+        want = add_layernorm(xs, rs, ln)[:, :T]
+        x, r = xs[:, :T].contiguous(), rs[:, :T].contiguous()
+        assert torch.equal(add_layernorm(x, r, ln), want)
+        assert torch.equal(add_layernorm(x, None, ln), add_layernorm(xs, None, ln)[:, :T])
+        x_in, r_in = (torch.full((H * T + 8,), float("nan"), dtype=torch.float16, device="cuda") for _ in range(2))
+        out = torch.full((H * T + 8,), 7.0, dtype=torch.float16, device="cuda")
+        x_in[3:3 + H * T], r_in[1:1 + H * T] = x.flatten(), r.flatten()
+        rc = _lib.lib().sspmm_add_layernorm_ragged_f16(H, T, x_in[3:].data_ptr(), r_in[1:].data_ptr(), ln.weight.data_ptr(), ln.bias.data_ptr(),
+                                                       ln.eps, out[1:].data_ptr(), torch.cuda.current_stream().cuda_stream)
+        assert rc == 0 and torch.equal(out[1:1 + H * T].view(H, T), want)
+        assert out[0] == 7.0 and torch.all(out[1 + H * T:] == 7.0)
+    assert add_layernorm(x, r, ln).requires_grad == (T % 4 != 0)
