@@ -648,10 +648,13 @@ static constexpr int wave_lds_bytes(int V) { return val_tile_bytes(V); }
 
 // steps whose loads are in flight or waiting in registers (bounded by the 128 registers a lane has
 // with 16 waves per CU)
-static constexpr int slab_ring(int V) { return V == 8 ? 6 : 5; }
+// One column tile (the encoder layer's tail): three.  A wave has 3 to 36 steps a product there, and a step is long beside the
+// L2's answer (sixteen waves share the CU), so filling a deeper ring only delays the first one.  Layer of 768 features, 8 x 512
+// tokens, V = 16 / 8 at 90 %: 69.3 / 97.9 us with two, 63.3 / 84.0 with three, 65.0 / 84.9 with five.
+static constexpr int slab_ring(int V, int NQ) { return NQ == 1 ? 3 : V == 8 ? 6 : 5; }
 
 template <int V>
-struct SlabLoads {    // what the head records for a step; the step consumes it slab_ring(V) - 1 steps later
+struct SlabLoads {    // what the head records for a step; the step consumes it slab_ring(V, NQ) - 1 steps later
   uint32_t col[2];    // column index of k slots 8g + m/4 and 8g + 4 + m/4
   typename SlabVals<V>::type vraw;
   int row, left;      // (wave-uniform) vector-row and its vectors from this step on
@@ -665,7 +668,7 @@ struct SlabLoads {    // what the head records for a step; the step consumes it 
 // fixed share of rows a third sooner than the younger ones), so a fixed deal of rows would leave
 // the fast waves idle at the end of every item.  A vector-row of n vectors is ceil(n / 32) steps,
 // and an empty vector-row is one step without vectors (its zeros still have to be written).  The
-// cursor runs slab_ring(V) - 1 steps ahead of the arithmetic: it issues the loads of a step and
+// cursor runs slab_ring(V, NQ) - 1 steps ahead of the arithmetic: it issues the loads of a step and
 // records the step's vector-row and length in the ring slot that receives them.  Both LDS round
 // trips behind a new row are off the critical path: the claim of a position is issued two rows
 // ahead and the read of its table entry one row ahead.
@@ -921,7 +924,7 @@ __device__ __forceinline__ void slab_process_item(const SlabCtx<V, OutT> &x, uns
   cursor_take_next(head, rows);
   if (!head.valid) return;
 
-  constexpr int R = slab_ring(V);
+  constexpr int R = slab_ring(V, NQ);
   SlabLoads<V> ld[R];
 #pragma unroll
   for (int i = 0; i < R - 1; ++i) {
@@ -1229,8 +1232,8 @@ __global__ __launch_bounds__(kSlabThreads) void spmm_slab_kernel(const SpmmArgs 
 //   LDS: x (then x + a, then its LayerNorm, then that + y): hidden rows; the context, then the hidden features: ffn rows; a zero
 //   row behind either; value tiles, row tables of the three products, biases.  The workgroups of 64 consecutive tokens share
 //   an XCD (ids 8 apart), so that a line of x, context or result crosses the fabric once.
-// 768 features, 3072 hidden, V = 16 at 90 %, 4096 tokens (a workgroup per CU): 43 us, where the five launches took 5, 11, 15, 14
-// and 11; the layer 82 -> 63 us.  1200 steps of 32 vectors a workgroup: bound by the step's chain (value tile to LDS and
+// 768 features, 3072 hidden, V = 16 at 90 %, 4096 tokens (a workgroup per CU): 42 us, where the five launches took 5, 11, 15, 14
+// and 11; the layer 82 -> 62 us.  1200 steps of 32 vectors a workgroup: bound by the step's chain (value tile to LDS and
 // back, rows of the slab, MFMA) on four waves per SIMD, 29 ns a step and CU as in the slab kernel, and by the 7 us of vector
 // instructions of 49 000 GELUs.
 struct SlabTailStore {
