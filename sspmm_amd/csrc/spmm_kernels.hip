@@ -646,15 +646,18 @@ static constexpr uint32_t layout_buffer_off(int L, int NQ, uint32_t rows, uint32
 // bytes past its 512).
 static constexpr int wave_lds_bytes(int V) { return val_tile_bytes(V); }
 
-// steps whose loads are in flight or waiting in registers (bounded by the 128 registers a lane has
-// with 16 waves per CU)
-// One column tile (the encoder layer's tail): three.  A wave has 3 to 36 steps a product there, and a step is long beside the
-// L2's answer (sixteen waves share the CU), so filling a deeper ring only delays the first one.  Layer of 768 features, 8 x 512
-// tokens, V = 16 / 8 at 90 %: 69.3 / 97.9 us with two, 63.3 / 84.0 with three, 65.0 / 84.9 with five.
-static constexpr int slab_ring(int V, int NQ) { return NQ == 1 ? 3 : V == 8 ? 6 : 5; }
+// Ring slots: steps whose loads are in flight or waiting in registers.  A step is long beside the L2's answer (sixteen waves
+// share the CU), so two steps ahead, three with slabs of two column tiles, whose steps are the shortest, cover it; a deeper
+// ring delays the first step of every item and keeps more loads in a memory pipeline that the stores of C need.
+// Six slots (V = 8; five for V = 16) / three: A 2048 x 512 at 90 %, N = 256, batch 128, fp32 C 56.2 / 53.6 us, at 70 %, batch 64
+// 45.4 / 43.6, 1536 x 1024 at 80 %, N = 500, batch 32 44.6 / 43.1, V = 16 level; two tiles, 2048 x 2048 at 80 %, N = 512, batch 16,
+// fp16 C six 60.3, five 60.1, four 60.1, three 61.2, at 90 %, N = 256, fp32 23.0, 22.7, 22.2, 22.4.  One tile (the encoder layer's
+// tail, 3 to 36 steps a wave and product): layer of 768 features, 8 x 512 tokens, V = 16 / 8 at 90 % two slots 69.3 / 97.9, three
+// 63.3 / 84.0, five 65.0 / 84.9.
+static constexpr int slab_ring(int NQ) { return NQ == 2 ? 4 : 3; }
 
 template <int V>
-struct SlabLoads {    // what the head records for a step; the step consumes it slab_ring(V, NQ) - 1 steps later
+struct SlabLoads {    // what the head records for a step; the step consumes it slab_ring(NQ) - 1 steps later
   uint32_t col[2];    // column index of k slots 8g + m/4 and 8g + 4 + m/4
   typename SlabVals<V>::type vraw;
   int row, left;      // (wave-uniform) vector-row and its vectors from this step on
@@ -668,7 +671,7 @@ struct SlabLoads {    // what the head records for a step; the step consumes it 
 // fixed share of rows a third sooner than the younger ones), so a fixed deal of rows would leave
 // the fast waves idle at the end of every item.  A vector-row of n vectors is ceil(n / 32) steps,
 // and an empty vector-row is one step without vectors (its zeros still have to be written).  The
-// cursor runs slab_ring(V, NQ) - 1 steps ahead of the arithmetic: it issues the loads of a step and
+// cursor runs slab_ring(NQ) - 1 steps ahead of the arithmetic: it issues the loads of a step and
 // records the step's vector-row and length in the ring slot that receives them.  Both LDS round
 // trips behind a new row are off the critical path: the claim of a position is issued two rows
 // ahead and the read of its table entry one row ahead.
@@ -924,7 +927,7 @@ __device__ __forceinline__ void slab_process_item(const SlabCtx<V, OutT> &x, uns
   cursor_take_next(head, rows);
   if (!head.valid) return;
 
-  constexpr int R = slab_ring(V, NQ);
+  constexpr int R = slab_ring(NQ);
   SlabLoads<V> ld[R];
 #pragma unroll
   for (int i = 0; i < R - 1; ++i) {
