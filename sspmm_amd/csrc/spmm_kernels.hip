@@ -649,7 +649,8 @@ static constexpr int wave_lds_bytes(int V) { return val_tile_bytes(V); }
 // Ring slots: steps whose loads are in flight or waiting in registers.  A step is long beside the L2's answer (sixteen waves
 // share the CU), so two steps ahead, three with slabs of two column tiles, whose steps are the shortest, cover it; a deeper
 // ring delays the first step of every item and keeps more loads in a memory pipeline that the stores of C need.
-// Six slots (V = 8; five for V = 16) / three: A 2048 x 512 at 90 %, N = 256, batch 128, fp32 C 56.2 / 53.6 us, at 70 %, batch 64
+// Six slots (V = 8; five for V = 16) / three: A 2048 x 512 at 90 %, N = 256, batch 128, fp32 C 56.2 / 53.6 us (55.8 / 55.5 on another
+// card), at 70 %, batch 64
 // 45.4 / 43.6, 1536 x 1024 at 80 %, N = 500, batch 32 44.6 / 43.1, V = 16 level; two tiles, 2048 x 2048 at 80 %, N = 512, batch 16,
 // fp16 C six 60.3, five 60.1, four 60.1, three 61.2, at 90 %, N = 256, fp32 23.0, 22.7, 22.2, 22.4.  One tile (the encoder layer's
 // tail, 3 to 36 steps a wave and product): layer of 768 features, 8 x 512 tokens, V = 16 / 8 at 90 % two slots 69.3 / 97.9, three
