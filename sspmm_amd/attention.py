@@ -303,16 +303,21 @@ def _plain_linear(m, x, in_features, out_features, multiple):
                               t.is_contiguous() and t.data_ptr() % 16 == 0) for t in (w, b)))
 
 
-def _eager_inference():
-    """Nothing but the values is wanted: no gradients in either direction, no tracing or compiling, no autocast, no
-    modes or module hooks that want to see every operator."""
+def _eager():
+    """Nothing watches the operators: no forward-mode gradients, no tracing or compiling, no autocast, no modes or module hooks
+    that want to see every one of them."""
     nn_module = torch.nn.modules.module
-    return not (torch.is_grad_enabled() or torch.jit.is_tracing() or torch.compiler.is_compiling() or
+    return not (torch.jit.is_tracing() or torch.compiler.is_compiling() or
                 torch.is_autocast_enabled("cuda") or torch.autograd.forward_ad._current_level >= 0 or
                 torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack() or
                 torch._C._functorch.maybe_current_level() is not None or
                 nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks or
                 nn_module._global_backward_hooks or nn_module._global_backward_pre_hooks)
+
+
+def _eager_inference():
+    """Nothing but the values is wanted: as _eager, and no gradients."""
+    return not torch.is_grad_enabled() and _eager()
 
 
 class SparseAttentionBlock(torch.nn.Module):

@@ -18,7 +18,7 @@ import math
 import numpy as np
 import torch
 
-from .attention import _eager_inference, _plain_module
+from .attention import _eager, _eager_inference, _plain_module
 from .spmm import linear as linear_op, spmm
 from .svc import svc
 
@@ -178,7 +178,7 @@ def attention_fm(qkv, hidden, heads, batch, seq, scale=None):
     """softmax(Q^T K * scale) V per (batch element, head) on the fused feature-major projections qkv
     [3 * hidden, batch * seq] fp16 (rows 0 .. hidden-1 the queries, then keys, then values; token b * seq + s in
     column b * seq + s); returns the context [hidden, batch * seq], or None where the kernel's shape limits do not
-    hold (the caller then takes another route)."""
+    hold or, with sequences that are no multiple of 64, more than the values is wanted (the caller then takes another route)."""
     from . import _lib
     d = hidden // heads
     T = batch * seq
@@ -186,6 +186,8 @@ def attention_fm(qkv, hidden, heads, batch, seq, scale=None):
             d == 64 and hidden == heads * d and batch >= 1 and
             1 <= seq <= (16384 if seq % 64 == 0 and T % 8 == 0 else ATTENTION_FM_RAGGED)):
         return None
+    if seq % 64 and not (type(qkv) is torch.Tensor and _eager() and not (torch.is_grad_enabled() and qkv.requires_grad)):
+        return None  # (ragged lengths had torch's attention, which whoever wants gradients or watches it still gets)
     out = torch.empty(hidden, T, dtype=torch.float16, device=qkv.device)
     esz = qkv.element_size()
     # (whole tiles of aligned tokens are a kernel of their own behind either entry)

@@ -152,6 +152,62 @@ def test_feature_major_attention_on_ragged_sequences(built_library, batch, heads
         assert torch.all(o[:, T:] == 7.0) and torch.all(out[:lead] == 7.0) and torch.all(out[lead + hidden * ld_out:] == 7.0)
 
 
+def test_ragged_attention_is_left_to_torch_where_more_than_the_values_is_wanted(built_library, monkeypatch):
+    """A layer on 333 tokens with differentiable products in the place of the sparse ones: gradients of the input and of the
+    projections are those through torch's attention (here written out in fp32; the same operations twice, so what differs is the
+    order of library sums), which tensor subclasses, dispatch modes, vmap and forward-mode gradients get as well.  Values
+    alone come from the kernel, in gradient mode too."""
+    import torch.utils._python_dispatch as dispatch
+    import sspmm_amd.layers as layers_mod
+    hidden, heads, ffn, V, seq = 128, 2, 256, 8, 333
+    mk = lambda o, i, s: _vector_sparse_linear(o, i, V, 0.8, seed=s)
+    layer = SparseEncoderLayer(hidden, heads, ffn, mk(hidden, hidden, 1), mk(hidden, hidden, 2), mk(hidden, hidden, 3),
+                               mk(hidden, hidden, 4), mk(ffn, hidden, 5), mk(hidden, ffn, 6)).cuda().half()
+    dense = {n: getattr(layer, n).dense_weight() for n in ("qkv", "o", "ffn1_gelu", "ffn2")}
+    g = torch.Generator("cuda").manual_seed(8)
+    x0, direction = (torch.randn(hidden, seq, device="cuda", generator=g).half() for _ in range(2))
+
+    def attention(q, k, v, scale):
+        p = torch.softmax(q.float() @ k.float().transpose(-1, -2).contiguous() * scale, dim=-1)
+        return (p @ v.float()).half()
+
+    monkeypatch.setattr(torch.nn.functional, "scaled_dot_product_attention", attention)
+
+    def gradients():
+        x, w = x0.clone().requires_grad_(), {n: d.clone().requires_grad_() for n, d in dense.items()}
+        layer(x, 1, seq, linear=lambda name, lin, t: torch.nn.functional.gelu(w[name] @ t) if name == "ffn1_gelu" else w[name] @ t).backward(direction)
+        return [x.grad] + [w[n].grad for n in dense]
+
+    got, kernel = gradients(), layers_mod.attention_fm
+    with monkeypatch.context() as m:
+        m.setattr(layers_mod, "attention_fm", lambda *a, **kw: None)
+        want = gradients()
+    for a, b in zip(got, want):
+        assert a is not None and b.abs().max() > 0 and max_rel_err(a.float().cpu().numpy(), b.float().cpu().numpy()) <= 1e-2
+
+    qkv = torch.randn(3 * hidden, seq, device="cuda", generator=g).half()
+    call = lambda t: kernel(t, hidden, heads, 1, seq)  # noqa: E731
+
+    class Watcher(dispatch.TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Sub(torch.Tensor):
+        pass
+
+    assert call(qkv) is not None and call(qkv.clone().requires_grad_()) is None
+    assert call(qkv.as_subclass(Sub)) is None
+    with torch.no_grad():
+        assert call(qkv.clone().requires_grad_()) is not None
+        with Watcher():
+            assert call(qkv) is None
+        with torch.autograd.forward_ad.dual_level():
+            assert call(torch.autograd.forward_ad.make_dual(qkv, qkv)) is None
+        with torch.autocast("cuda"):
+            assert call(qkv) is None
+    assert torch.vmap(lambda t: torch.zeros(()) if call(t) is None else torch.ones(()))(qkv[None]).item() == 0
+
+
 def test_feature_major_attention_with_maxima_that_keep_growing(built_library):
     """Keys whose norm grows along the sequence: the running maximum of a query's scores rises by many units from one
     block of keys to the next, so the kernel moves the reference point of its exponentials again and again (it
