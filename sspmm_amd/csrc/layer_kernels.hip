@@ -401,6 +401,13 @@ __device__ __forceinline__ uint32_t att_pack(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, h);
 }
 
+// v with its infinities (and NaN) replaced by the largest finite number.
+__device__ __forceinline__ half8 att_bounded(half8 v) {
+  const _Float16 x = (_Float16)65504;
+  const half8 most = {x, x, x, x, x, x, x, x};
+  return __builtin_elementwise_max(__builtin_elementwise_min(v, most), -most);
+}
+
 struct AttentionArgs {
   const _Float16 *q, *k, *v;
   _Float16 *out;
@@ -445,10 +452,11 @@ __device__ __forceinline__ void att_store(_Float16 *p, uintx4 v, int left) {
 // probabilities are set to zero; the last block of queries likewise, without being stored.  Such calls ran on torch's attention
 // between two relayout copies, whose error against float64 is 2.7e-4 (12 heads, 500 tokens) where this kernel's is 2.9e-4, the
 // probabilities' rounding for the most part; so RAGGED adds what that rounding leaves as a second product: 2.1e-4, the rounding
-// of the result.  8 x 500 tokens: 25 us (21 without it, 16 for 8 x 512) against 69.
+// of the result.  8 x 500 tokens: 25 us (21 without it, 15 for 8 x 512) against 69.
 template <bool RAGGED>
 __global__ __launch_bounds__(kAttThreads, 3) void attention_fm_kernel(const AttentionArgs p) {
-  __shared__ __align__(16) unsigned char lds[kAttLds];
+  __shared__ __align__(16) unsigned char lds[kAttLds + (RAGGED ? 16 : 0)];
+  int *const again = reinterpret_cast<int *>(lds + kAttLds);  // (RAGGED)
   const int S = p.S, qblocks = (S + kAttQueries - 1) / kAttQueries, blocks = (S + kAttKeys - 1) / kAttKeys;
   // Workgroup ids go round-robin to the 8 XCDs, each with its own L2: the query blocks of one (batch element, head)
   // take ids 8 apart, so that the head's K and V are fetched from memory once and found in that L2 by the others.
@@ -483,6 +491,7 @@ __global__ __launch_bounds__(kAttThreads, 3) void attention_fm_kernel(const Atte
   *reinterpret_cast<uintx4 *>(k_tiles + l1) = kk[1];
   *reinterpret_cast<uintx4 *>(v_tiles + lv0) = vv[0];
   *reinterpret_cast<uintx4 *>(v_tiles + lv1) = vv[1];
+  if (RAGGED && tid == 0) *again = 0;
   __syncthreads();
 
   // ---- Wave w works on queries 32 * (w / 2) .. + 31 of the workgroup's 64 (two sets of 16) against keys
@@ -510,125 +519,156 @@ __global__ __launch_bounds__(kAttThreads, 3) void attention_fm_kernel(const Atte
   const float c = p.scale_log2e;  // > 0: the largest scaled score is the scaled largest score
   const uint32_t k_rd = (4 * g + (m >> 2)) * kAttPitchK + (m & 3) * 8 + (32 * khalf) * 2;
   const uint32_t v_rd = m * kAttPitchV + (4 * g) * 2 + (32 * khalf) * 2;
-  for (int kb = 0; kb < blocks; ++kb) {
-    const unsigned char *const k_tile = k_tiles + (kb & 1) * kAttTileK;
-    const unsigned char *const v_tile = v_tiles + (kb & 1) * kAttTileV;
-    const bool more = kb + 1 < blocks;  // uniform
-    if (more) {
-      const int off = (kb + 1) * kAttKeys;
-      kk[0] = att_load<RAGGED>(kg + g0 + off, left - off);
-      kk[1] = att_load<RAGGED>(kg + g1 + off, left - off);
-      vv[0] = att_load<RAGGED>(vg + g0 + off, left - off);
-      vv[1] = att_load<RAGGED>(vg + g1 + off, left - off);
-    }
-    // scores^T: s[set][kt], lane (m, g): keys 32 * khalf + 16kt + 4g .. + 3 of the block against query m of the set
-    floatx4 s[2][2] = {{zero, zero}, {zero, zero}};
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const unsigned char *a = k_tile + k_rd + (32 * u) * kAttPitchK + (16 * kt) * 2;
-        const uintx2 lo = att_read_tr(a), hi = att_read_tr(a + 16 * kAttPitchK);
-        AttOperand kop;
-        kop.u[0] = lo[0]; kop.u[1] = lo[1]; kop.u[2] = hi[0]; kop.u[3] = hi[1];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) s[j][kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kop.h, qop[j][u].h, s[j][kt], 0, 0, 0);
+  // what the two waves of a query half exchange at the end
+  floatx4 *const xo = reinterpret_cast<floatx4 *>(k_tiles) + qhalf * (2 * 4 * 64);  // [set][dt][lane]
+  float *const xs = reinterpret_cast<float *>(k_tiles + 2 * (2 * 4 * 64) * 16) + qhalf * (2 * 2 * 64);  // [set][max, sum][lane]
+  // What the rounding of the probabilities leaves (RAGGED) is of either sign or zero: against an infinite value it makes NaN where the
+  // probability alone makes infinity.  A workgroup with a NaN goes over its keys once more with V bounded in that product.
+  // 8 x 500 tokens: 24.2 us without the test for NaN, 25.4 with it; bounded the first time 26.7, a second copy of the loop 25.6.
+  for (bool bounded = false;; bounded = true) {
+    for (int kb = 0; kb < blocks; ++kb) {
+      const unsigned char *const k_tile = k_tiles + (kb & 1) * kAttTileK;
+      const unsigned char *const v_tile = v_tiles + (kb & 1) * kAttTileV;
+      const bool more = kb + 1 < blocks;  // uniform
+      if (more) {
+        const int off = (kb + 1) * kAttKeys;
+        kk[0] = att_load<RAGGED>(kg + g0 + off, left - off);
+        kk[1] = att_load<RAGGED>(kg + g1 + off, left - off);
+        vv[0] = att_load<RAGGED>(vg + g0 + off, left - off);
+        vv[1] = att_load<RAGGED>(vg + g1 + off, left - off);
       }
-    }
-    // keys of this lane's accumulators that lie in the sequence: those below (all of them in every block but the last)
-    const int keys_left = S - kb * kAttKeys - 32 * khalf - 4 * g;
-    const bool cut = RAGGED && (kb + 1) * kAttKeys > S;  // uniform
-    if (cut) {
+      // scores^T: s[set][kt], lane (m, g): keys 32 * khalf + 16kt + 4g .. + 3 of the block against query m of the set
+      floatx4 s[2][2] = {{zero, zero}, {zero, zero}};
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
+      for (int kt = 0; kt < 2; ++kt) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (16 * kt + r >= keys_left) s[0][kt][r] = s[1][kt][r] = -3.0e38f;
-    }
-    AttOperand rest[2];  // (RAGGED) what the rounding of the probabilities leaves
-    AttOperand pop[2];  // per set: contraction slots 0-3 = keys 4g .. + 3 of tile 0, slots 4-7 = the same keys of tile 1
+        for (int u = 0; u < 2; ++u) {
+          const unsigned char *a = k_tile + k_rd + (32 * u) * kAttPitchK + (16 * kt) * 2;
+          const uintx2 lo = att_read_tr(a), hi = att_read_tr(a + 16 * kAttPitchK);
+          AttOperand kop;
+          kop.u[0] = lo[0]; kop.u[1] = lo[1]; kop.u[2] = hi[0]; kop.u[3] = hi[1];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      float mx = s[j][0][0];
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[j][kt][r]);
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      // The reference point of the exponentials moves only when some query's maximum has grown by more than 8 in
-      // the base-2 domain (a wave-uniform decision): until then the probabilities are at most 2^8 times too large,
-      // which fp16 holds, the running sums and the context stay consistent with the old reference point, and the
-      // rescaling of the accumulators, which after the first block is nearly always by 1, is skipped.
-      const float new_max = fmaxf(run_max[j], mx);
-      if (__ballot((new_max - run_max[j]) * c > 8.0f) != 0) {
-        const float alpha = __builtin_amdgcn_exp2f(fmaxf((run_max[j] - new_max) * c, -126.0f));
-        run_max[j] = new_max;
-        run_sum[j] *= alpha;
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt) o[j][dt] *= alpha;
-      }
-      const float shift = -run_max[j] * c;
-      float part = 0.f;
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          s[j][kt][r] = __builtin_amdgcn_exp2f(fmaf(s[j][kt][r], c, shift));
-          if (cut && 16 * kt + r >= keys_left) s[j][kt][r] = 0.f;  // (a wave may have had no key at all yet)
-          part += s[j][kt][r];
+          for (int j = 0; j < 2; ++j) s[j][kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kop.h, qop[j][u].h, s[j][kt], 0, 0, 0);
         }
-      run_sum[j] += part;
-      pop[j].u[0] = att_pack(s[j][0][0], s[j][0][1]);
-      pop[j].u[1] = att_pack(s[j][0][2], s[j][0][3]);
-      pop[j].u[2] = att_pack(s[j][1][0], s[j][1][1]);
-      pop[j].u[3] = att_pack(s[j][1][2], s[j][1][3]);
-      if constexpr (RAGGED) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) rest[j].h[i] = (_Float16)(s[j][i >> 2][i & 3] - (float)pop[j].h[i]);
       }
-    }
+      // keys of this lane's accumulators that lie in the sequence: those below (all of them in every block but the last)
+      const int keys_left = S - kb * kAttKeys - 32 * khalf - 4 * g;
+      const bool cut = RAGGED && (kb + 1) * kAttKeys > S;  // uniform
+      if (cut) {
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-      const unsigned char *a = v_tile + v_rd + (16 * dt) * kAttPitchV;
-      const uintx2 lo = *reinterpret_cast<const uintx2 *>(a), hi = *reinterpret_cast<const uintx2 *>(a + 32);
-      AttOperand vop;
-      vop.u[0] = lo[0]; vop.u[1] = lo[1]; vop.u[2] = hi[0]; vop.u[3] = hi[1];
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (16 * kt + r >= keys_left) s[0][kt][r] = s[1][kt][r] = -3.0e38f;
+      }
+      AttOperand rest[2];  // (RAGGED) what the rounding of the probabilities leaves
+      AttOperand pop[2];  // per set: contraction slots 0-3 = keys 4g .. + 3 of tile 0, slots 4-7 = the same keys of tile 1
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        if constexpr (RAGGED) o[j][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vop.h, rest[j].h, o[j][dt], 0, 0, 0);
-        o[j][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vop.h, pop[j].h, o[j][dt], 0, 0, 0);
+        float mx = s[j][0][0];
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[j][kt][r]);
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        // The reference point of the exponentials moves only when some query's maximum has grown by more than 8 in
+        // the base-2 domain (a wave-uniform decision): until then the probabilities are at most 2^8 times too large,
+        // which fp16 holds, the running sums and the context stay consistent with the old reference point, and the
+        // rescaling of the accumulators, which after the first block is nearly always by 1, is skipped.
+        const float new_max = fmaxf(run_max[j], mx);
+        if (__ballot((new_max - run_max[j]) * c > 8.0f) != 0) {
+          const float alpha = __builtin_amdgcn_exp2f(fmaxf((run_max[j] - new_max) * c, -126.0f));
+          run_max[j] = new_max;
+          run_sum[j] *= alpha;
+#pragma unroll
+          for (int dt = 0; dt < 4; ++dt) o[j][dt] *= alpha;
+        }
+        const float shift = -run_max[j] * c;
+        float part = 0.f;
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            s[j][kt][r] = __builtin_amdgcn_exp2f(fmaf(s[j][kt][r], c, shift));
+            if (cut && 16 * kt + r >= keys_left) s[j][kt][r] = 0.f;  // (a wave may have had no key at all yet)
+            part += s[j][kt][r];
+          }
+        run_sum[j] += part;
+        pop[j].u[0] = att_pack(s[j][0][0], s[j][0][1]);
+        pop[j].u[1] = att_pack(s[j][0][2], s[j][0][3]);
+        pop[j].u[2] = att_pack(s[j][1][0], s[j][1][1]);
+        pop[j].u[3] = att_pack(s[j][1][2], s[j][1][3]);
+        if constexpr (RAGGED) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) rest[j].h[i] = (_Float16)(s[j][i >> 2][i & 3] - (float)pop[j].h[i]);
+        }
+      }
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) {
+        const unsigned char *a = v_tile + v_rd + (16 * dt) * kAttPitchV;
+        const uintx2 lo = *reinterpret_cast<const uintx2 *>(a), hi = *reinterpret_cast<const uintx2 *>(a + 32);
+        AttOperand vop;
+        vop.u[0] = lo[0]; vop.u[1] = lo[1]; vop.u[2] = hi[0]; vop.u[3] = hi[1];
+        half8 vrest = vop.h;
+        if (RAGGED && __builtin_expect(bounded, 0)) vrest = att_bounded(vrest);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          if constexpr (RAGGED) o[j][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vrest, rest[j].h, o[j][dt], 0, 0, 0);
+          o[j][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vop.h, pop[j].h, o[j][dt], 0, 0, 0);
+        }
+      }
+      if (more) {  // the other buffer: every wave finished reading it before the barrier that ended the previous block
+        unsigned char *const kn = k_tiles + ((kb + 1) & 1) * kAttTileK, *const vn = v_tiles + ((kb + 1) & 1) * kAttTileV;
+        *reinterpret_cast<uintx4 *>(kn + l0) = kk[0];
+        *reinterpret_cast<uintx4 *>(kn + l1) = kk[1];
+        *reinterpret_cast<uintx4 *>(vn + lv0) = vv[0];
+        *reinterpret_cast<uintx4 *>(vn + lv1) = vv[1];
+      }
+      __syncthreads();
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      run_sum[j] += __shfl_xor(run_sum[j], 16, 64);
+      run_sum[j] += __shfl_xor(run_sum[j], 32, 64);
+    }
+
+    // ---- The two waves of a query half merge: the one with the upper keys leaves its state in LDS (over the K tiles:
+    // the loop's last barrier is behind every read of them), the other adds it to its own.
+    if constexpr (RAGGED) {
+      float sum = 0.f;
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) sum += (o[j][dt][0] + o[j][dt][1]) + (o[j][dt][2] + o[j][dt][3]);
+      const bool nan = sum != sum;  // (or infinities of both signs)
+      if (__ballot(nan) != 0 && lane == 0) *again = 1;
+    }
+    if (khalf == 1) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) xo[(j * 4 + dt) * 64 + lane] = o[j][dt];
+        xs[(j * 2 + 0) * 64 + lane] = run_max[j];
+        xs[(j * 2 + 1) * 64 + lane] = run_sum[j];
       }
     }
-    if (more) {  // the other buffer: every wave finished reading it before the barrier that ended the previous block
-      unsigned char *const kn = k_tiles + ((kb + 1) & 1) * kAttTileK, *const vn = v_tiles + ((kb + 1) & 1) * kAttTileV;
-      *reinterpret_cast<uintx4 *>(kn + l0) = kk[0];
-      *reinterpret_cast<uintx4 *>(kn + l1) = kk[1];
-      *reinterpret_cast<uintx4 *>(vn + lv0) = vv[0];
-      *reinterpret_cast<uintx4 *>(vn + lv1) = vv[1];
+    __syncthreads();
+    if (!RAGGED || bounded || __builtin_amdgcn_readfirstlane(*again) == 0) break;
+    __syncthreads();
+    *reinterpret_cast<uintx4 *>(k_tiles + l0) = att_load<RAGGED>(kg + g0, left);
+    *reinterpret_cast<uintx4 *>(k_tiles + l1) = att_load<RAGGED>(kg + g1, left);
+    *reinterpret_cast<uintx4 *>(v_tiles + lv0) = att_load<RAGGED>(vg + g0, left);
+    *reinterpret_cast<uintx4 *>(v_tiles + lv1) = att_load<RAGGED>(vg + g1, left);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      run_max[j] = -3.0e38f;
+      run_sum[j] = 0.f;
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) o[j][dt] = zero;
     }
     __syncthreads();
   }
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    run_sum[j] += __shfl_xor(run_sum[j], 16, 64);
-    run_sum[j] += __shfl_xor(run_sum[j], 32, 64);
-  }
-
-  // ---- The two waves of a query half merge: the one with the upper keys leaves its state in LDS (over the K tiles:
-  // the loop's last barrier is behind every read of them), the other adds it to its own.
-  floatx4 *const xo = reinterpret_cast<floatx4 *>(k_tiles) + qhalf * (2 * 4 * 64);  // [set][dt][lane]
-  float *const xs = reinterpret_cast<float *>(k_tiles + 2 * (2 * 4 * 64) * 16) + qhalf * (2 * 2 * 64);  // [set][max, sum][lane]
-  if (khalf == 1) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt) xo[(j * 4 + dt) * 64 + lane] = o[j][dt];
-      xs[(j * 2 + 0) * 64 + lane] = run_max[j];
-      xs[(j * 2 + 1) * 64 + lane] = run_sum[j];
-    }
-  }
-  __syncthreads();
   if (khalf == 0) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {

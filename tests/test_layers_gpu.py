@@ -152,6 +152,21 @@ def test_feature_major_attention_on_ragged_sequences(built_library, batch, heads
         assert torch.all(o[:, T:] == 7.0) and torch.all(out[:lead] == 7.0) and torch.all(out[lead + hidden * ld_out:] == 7.0)
 
 
+@pytest.mark.parametrize("seq", [1, 37, 63, 64, 100, 333])
+def test_feature_major_attention_keeps_infinite_values(built_library, seq):
+    """One infinite or NaN value: its feature is infinite or NaN for every query, whole blocks or not (scores within a few units of each
+    other, so that no probability vanishes in fp16), and the features beside it are what they are without it."""
+    from sspmm_amd.layers import attention_fm
+    qkv = (torch.randn(3 * 64, seq, device="cuda", generator=torch.Generator("cuda").manual_seed(seq)) * 0.5).half()
+    plain = attention_fm(qkv, 64, 1, 1, seq)
+    for feature, value in ((5, float("inf")), (21, -float("inf")), (40, float("nan"))):
+        qkv[128 + feature, seq // 2] = value
+    got = attention_fm(qkv, 64, 1, 1, seq)
+    assert torch.all(got[5] == float("inf")) and torch.all(got[21] == -float("inf")) and torch.all(got[40].isnan())
+    rest = [f for f in range(64) if f not in (5, 21, 40)]
+    assert torch.equal(got[rest], plain[rest])
+
+
 def test_ragged_attention_is_left_to_torch_where_more_than_the_values_is_wanted(built_library, monkeypatch):
     """A layer on 333 tokens with differentiable products in the place of the sparse ones: gradients of the input and of the
     projections are those through torch's attention (here written out in fp32; the same operations twice, so what differs is the
