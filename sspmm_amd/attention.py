@@ -273,7 +273,7 @@ def _rows_norm_applies(ln, x):
     E, w, b = x.size(-1), ln.weight, ln.bias
     return (_plain_module(ln, torch.nn.LayerNorm) and E in ROW_WIDTHS and ln.normalized_shape == (E,) and w is not None and
             all(t is None or (type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float16 and t.device == x.device and
-                              t.is_contiguous() and t.data_ptr() % 16 == 0) for t in (w, b)))
+                              t.shape == (E,) and t.is_contiguous() and t.data_ptr() % 16 == 0) for t in (w, b)))
 
 
 BLOCK_FEATURES = 1 << 20  # hidden or output features that block_dense takes at most

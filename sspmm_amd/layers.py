@@ -150,8 +150,9 @@ def add_layernorm(x, a, ln):
     w, b = ln.weight, ln.bias
     whole = T % 4 == 0
     ok = (x.dtype == torch.float16 and x.is_cuda and x.is_contiguous() and H <= 4096 and
-          (a is None or (a.dtype == torch.float16 and a.is_contiguous() and a.shape == x.shape)) and
-          w is not None and w.dtype == torch.float16 and tuple(ln.normalized_shape) == (H,))
+          (a is None or (a.dtype == torch.float16 and a.is_contiguous() and a.shape == x.shape and a.device == x.device)) and
+          w is not None and tuple(ln.normalized_shape) == (H,) and
+          all(t is None or (t.dtype == torch.float16 and t.shape == (H,) and t.is_contiguous() and t.device == x.device) for t in (w, b)))
     if ok and not whole:
         # (tokens that are no multiple of 4 had torch's module, which whoever wants gradients or watches it still gets)
         dev = x.get_device()
@@ -263,7 +264,8 @@ def _tail_norm(ln, features, dev):
         return None
     own = ln._parameters
     w, b = own.get("weight"), own.get("bias")
-    if not (_plain_tensor(w, torch.float16, dev) and (b is None or _plain_tensor(b, torch.float16, dev))):
+    if not (_plain_tensor(w, torch.float16, dev) and w.shape == (features,) and
+            (b is None or (_plain_tensor(b, torch.float16, dev) and b.shape == (features,)))):
         return None
     return w.data_ptr(), None if b is None else b.data_ptr(), float(ln.eps)
 

@@ -148,6 +148,22 @@ def test_argument_errors_of_the_encoder_tail(built_library):
                 assert encoder_tail_fits(hidden, ffn, 64, V) == (L.sspmm_encoder_tail_fits(hidden, ffn, 64, V) == 1), (hidden, ffn, V)
 
 
+def test_norm_weights_of_another_length_do_not_reach_a_kernel():
+    """A LayerNorm whose weight or bias has been replaced by one of another length is left to the module, which refuses it: the
+    kernels read as many elements as there are features."""
+    import torch
+    from sspmm_amd.attention import _rows_norm_applies
+    from sspmm_amd.layers import _tail_norm
+    E, x = 128, torch.zeros(2, 128, dtype=torch.float16)
+    made = lambda: torch.nn.LayerNorm(E).half()  # noqa: E731
+    assert _tail_norm(made(), E, -1) is not None and _rows_norm_applies(made(), x)
+    for name in ("weight", "bias"):
+        for shape in ((E - 16,), (E + 16,), (2, E // 2), (0,)):
+            ln = made()
+            setattr(ln, name, torch.nn.Parameter(torch.ones(shape, dtype=torch.float16)))
+            assert _tail_norm(ln, E, -1) is None and not _rows_norm_applies(ln, x), (name, shape)
+
+
 def test_python_operator_rejects_bad_arguments(built_library):
     import torch
     import sspmm_amd

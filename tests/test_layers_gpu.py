@@ -96,6 +96,28 @@ def _attention_reference(q, k, v, batch, heads, seq, scale):
     return (p @ f(v)).permute(1, 3, 0, 2).reshape(heads * d, batch * seq)
 
 
+@pytest.mark.parametrize("T", [64, 61])
+def test_feature_major_add_layernorm_reads_only_operands_of_its_sizes(built_library, T):
+    """Weights of another length or type and a residual that is elsewhere go to the module, which refuses them."""
+    from sspmm_amd.layers import add_layernorm
+    H = 128
+    x = torch.ones(H, T, dtype=torch.float16, device="cuda")
+    with torch.no_grad():
+        for name in ("weight", "bias"):
+            for t in (torch.ones(H - 16), torch.ones(2, H // 2)):
+                ln = torch.nn.LayerNorm(H).cuda().half()
+                setattr(ln, name, torch.nn.Parameter(t.cuda().half()))
+                with pytest.raises(RuntimeError):
+                    add_layernorm(x, None, ln)
+        ln = torch.nn.LayerNorm(H).cuda().half()
+        with pytest.raises(RuntimeError):
+            add_layernorm(x, x.cpu(), ln)
+        want = add_layernorm(x, x, ln)
+        for t in (torch.zeros(2 * H).cuda().half()[::2], torch.zeros(H).cuda().half()):
+            ln.bias = torch.nn.Parameter(t)
+            assert torch.equal(add_layernorm(x, x, ln), want)
+
+
 @pytest.mark.parametrize("batch,heads,seq", [(1, 1, 64), (2, 3, 128), (3, 2, 192), (8, 12, 512), (1, 2, 320), (1, 1, 1024)])
 def test_feature_major_attention_matches_fp32_attention(built_library, batch, heads, seq):
     """sspmm_attention_fm_f16 through the C ABI, operands as three row ranges of one fused projection."""
