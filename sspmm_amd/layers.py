@@ -338,13 +338,15 @@ class SparseEncoderLayer(torch.nn.Module):
         ctx = torch.nn.functional.scaled_dot_product_attention(c[0], c[1], c[2], scale=1.0 / math.sqrt(d))
         return ctx.permute(1, 3, 0, 2).reshape(self.hidden, batch * seq)
 
-    def _one_launch_tail(self, x):
+    def _one_launch_tail(self, x, context):
         """What encoder_tail takes besides the activations, where everything behind the attention may run in that one launch
         and is ahead so: nothing but the values is wanted, plain layers and norms, sizes that a workgroup's LDS holds."""
         if type(x) is not torch.Tensor or x.dim() != 2 or x.size(1) < TAIL_TOKENS:  # (small calls are not kept waiting by the rest)
             return None
-        H = self.hidden
-        if not (type(self) is SparseEncoderLayer and x.is_cuda and x.dtype == torch.float16 and x.is_contiguous() and x.size(0) == H):
+        H, dev = self.hidden, x.get_device()
+        if not (type(self) is SparseEncoderLayer and x.is_cuda and x.dtype == torch.float16 and x.is_contiguous() and x.size(0) == H and
+                type(context) is torch.Tensor and context.shape == x.shape and context.dtype == x.dtype and context.get_device() == dev and
+                context.is_contiguous()):
             return None
         own = self._modules
         o, ffn1, ffn2 = own.get("o"), own.get("ffn1"), own.get("ffn2")
@@ -355,7 +357,6 @@ class SparseEncoderLayer(torch.nn.Module):
         vectors = sum(m._buffers["column_indices"].numel() for m in (o, ffn1, ffn2))
         if not (encoder_tail_fits(H, F, T, V) and encoder_tail_pays(H, T, vectors, _cus(x.device)) and _eager_inference()):
             return None
-        dev = x.get_device()
         parts = (_tail_weight(o, H, H, V, dev), _tail_norm(own.get("ln1"), H, dev), _tail_weight(ffn1, H, F, V, dev),
                  _tail_weight(ffn2, F, H, V, dev), _tail_norm(own.get("ln2"), H, dev))
         return None if None in parts else (F, V) + parts
@@ -365,13 +366,10 @@ class SparseEncoderLayer(torch.nn.Module):
         "ffn1_gelu", "ffn2"; "ffn1_gelu" is the first feed-forward product with the GELU behind it) is evaluated
         (the benchmark passes a dense matmul there to time the same layer without sparsity)."""
         f = linear or (lambda name, layer, t: layer(t))
-        tail = self._one_launch_tail(x) if linear is None else None
-        if tail is not None:
-            context = self._attention(self.qkv(x), batch, seq)
-            if context.shape == x.shape and context.dtype == x.dtype and context.device == x.device:
-                return encoder_tail(x, context.contiguous(), *tail)
-            return self._tail(f, x, context)
-        return self._tail(f, x, self._attention(f("qkv", self.qkv, x), batch, seq))
+        context = self._attention(f("qkv", self.qkv, x), batch, seq)
+        # (the weights are looked up when the launch is next: what has run until here may have replaced them)
+        tail = self._one_launch_tail(x, context) if linear is None else None
+        return self._tail(f, x, context) if tail is None else encoder_tail(x, context, *tail)
 
     def _tail(self, f, x, context):
         a = f("o", self.o, context)

@@ -422,6 +422,33 @@ def test_encoder_layers_tail_in_one_launch_matches_the_separate_launches(built_l
     assert len(calls) == 2
 
 
+def test_encoder_layers_tail_runs_on_the_weights_of_that_moment(built_library, monkeypatch):
+    """A hook behind the projections that gives the layer other weights: the launch behind the attention has their addresses,
+    not those of the arrays that went away (looked at without launching), and its result is the one with them."""
+    import sspmm_amd.layers as layers_mod
+    hidden, ffn, V, seq = 128, 256, 8, 64
+    mk = lambda o, i, s: _vector_sparse_linear(o, i, V, 0.8, seed=s)
+    layer = SparseEncoderLayer(hidden, 2, ffn, mk(hidden, hidden, 1), mk(hidden, hidden, 2), mk(hidden, hidden, 3),
+                               mk(hidden, hidden, 4), mk(ffn, hidden, 5), mk(hidden, ffn, 6)).cuda().half().eval()
+    x = torch.randn(hidden, seq, device="cuda", generator=torch.Generator("cuda").manual_seed(9)).half()
+    monkeypatch.setattr(layers_mod, "encoder_tail_pays", lambda *a: True)
+    monkeypatch.setattr(layers_mod, "TAIL_TOKENS", 1)
+    new = [-lin.values for lin in (layer.o, layer.ffn1, layer.ffn2)]
+
+    def replace(*_):
+        layer.o.values, layer.ffn1.values, layer.ffn2.values = (t.clone() for t in new)
+
+    layer.qkv.register_forward_hook(replace)
+    seen = []
+    with torch.no_grad():
+        with monkeypatch.context() as m:
+            m.setattr(layers_mod, "encoder_tail", lambda x, context, F, V, o, n1, f1, f2, n2: seen.extend(w[2] for w in (o, f1, f2)))
+            layer(x, 1, seq)
+        assert seen == [lin.values.data_ptr() for lin in (layer.o, layer.ffn1, layer.ffn2)]
+        want = layer(x, 1, seq, linear=lambda name, lin, t: lin(t))
+        assert max_rel_err(layer(x, 1, seq).float().cpu().numpy(), want.float().cpu().numpy()) <= 2.0 ** -8
+
+
 @pytest.mark.parametrize("H", [40, 200, 512, 768, 1000, 1100])
 @pytest.mark.parametrize("T", [1, 2, 3, 5, 15, 18, 63, 65, 130, 1021])
 def test_feature_major_add_layernorm_on_any_number_of_tokens(built_library, H, T):
