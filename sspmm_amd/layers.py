@@ -183,19 +183,21 @@ def attention_fm(qkv, hidden, heads, batch, seq, scale=None):
     from . import _lib
     d = hidden // heads
     T = batch * seq
+    whole = seq % 64 == 0
     if not (qkv.dtype == torch.float16 and qkv.is_cuda and qkv.is_contiguous() and tuple(qkv.shape) == (3 * hidden, T) and
-            d == 64 and hidden == heads * d and batch >= 1 and
-            1 <= seq <= (16384 if seq % 64 == 0 and T % 8 == 0 else ATTENTION_FM_RAGGED)):
+            d == 64 and hidden == heads * d and 1 <= seq <= (16384 if whole else ATTENTION_FM_RAGGED)):
         return None
-    if seq % 64 and not (type(qkv) is torch.Tensor and _eager() and not (torch.is_grad_enabled() and qkv.requires_grad)):
-        return None  # (ragged lengths had torch's attention, which whoever wants gradients or watches it still gets)
+    scale = float(1.0 / math.sqrt(d) if scale is None else scale)
+    # (ragged lengths had torch's attention, which takes any scale, and which whoever wants gradients or watches it still gets)
+    if not whole and not (batch >= 1 and 0 < scale <= 3.0e38 and type(qkv) is torch.Tensor and _eager() and
+                          not (torch.is_grad_enabled() and qkv.requires_grad)):
+        return None
     out = torch.empty(hidden, T, dtype=torch.float16, device=qkv.device)
     esz = qkv.element_size()
-    # (whole tiles of aligned tokens are a kernel of their own behind either entry)
-    rc = _lib.call(_lib.lib().sspmm_attention_fm_ragged_f16, qkv.device, batch, heads, seq, d, qkv.data_ptr(),
-                   qkv.data_ptr() + hidden * T * esz, qkv.data_ptr() + 2 * hidden * T * esz, T, out.data_ptr(), T,
-                   float(1.0 / math.sqrt(d) if scale is None else scale))
-    _lib.check(rc, "sspmm_attention_fm_ragged_f16")
+    L = _lib.lib()
+    rc = _lib.call(L.sspmm_attention_fm_f16 if whole else L.sspmm_attention_fm_ragged_f16, qkv.device, batch, heads, seq, d, qkv.data_ptr(),
+                   qkv.data_ptr() + hidden * T * esz, qkv.data_ptr() + 2 * hidden * T * esz, T, out.data_ptr(), T, scale)
+    _lib.check(rc, "sspmm_attention_fm_f16")
     return out
 
 
@@ -326,7 +328,7 @@ class SparseEncoderLayer(torch.nn.Module):
 
     def _attention(self, qkv, batch, seq):
         """qkv: [3 * hidden, batch*seq] feature-major; returns the context [hidden, batch*seq].  One HIP kernel that
-        reads and writes the feature-major layout (sspmm_attention_fm_ragged_f16 of the C ABI) where its shape limits hold
+        reads and writes the feature-major layout (sspmm_attention_fm_f16 of the C ABI and its ragged form) where its shape limits hold
         (head size 64).  Otherwise torch's attention between two relayout copies:
         one brings the three projections into the [batch, heads, seq, head size] layout it wants contiguous (on
         strided views of the feature-major activations it runs ten times slower), one brings the context back."""

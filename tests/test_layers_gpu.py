@@ -278,6 +278,23 @@ def test_feature_major_attention_rejects_what_it_does_not_cover(built_library):
     torch.cuda.synchronize()
 
 
+def test_attention_fm_takes_and_refuses_what_it_did(built_library):
+    """Scales that the kernel does not take are an error for whole blocks and somebody else's for other lengths, where empty
+    batches are as well; whole blocks of an empty batch are an empty context; projections that begin at any element are no
+    whole blocks."""
+    from sspmm_amd.layers import attention_fm
+    z = lambda *shape: torch.zeros(*shape, dtype=torch.float16, device="cuda")  # noqa: E731
+    for scale in (0.0, -0.125, float("nan"), float("inf")):
+        assert attention_fm(z(192, 63), 64, 1, 1, 63, scale) is None
+        with pytest.raises(RuntimeError):
+            attention_fm(z(192, 64), 64, 1, 1, 64, scale)
+    assert attention_fm(z(192, 0), 64, 1, 0, 63) is None and attention_fm(z(192, 0), 64, 1, 1, 0) is None
+    assert attention_fm(z(192, 0), 64, 1, 0, 64).shape == (64, 0)
+    with pytest.raises(RuntimeError):
+        attention_fm(z(192 * 64 + 1)[1:].view(192, 64), 64, 1, 1, 64)
+    assert attention_fm(z(192 * 63 + 1)[1:].view(192, 63), 64, 1, 1, 63) is not None
+
+
 def test_encoder_layer_at_the_benchmark_shape_takes_the_attention_kernel(built_library):
     """hidden 768, 12 heads, 8 x 512 tokens: the layer with the feature-major attention kernel against the same layer
     with torch's attention between relayout copies."""
