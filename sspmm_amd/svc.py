@@ -79,7 +79,7 @@ class _ReadBack:
     """Device values on their way to the host: what is queued behind this runs on, and wait() lasts until the copy is done."""
 
     def __init__(self, values):
-        self._host = torch.empty(values.shape, dtype=values.dtype, pin_memory=True)
+        self._host = torch.empty(values.shape, dtype=values.dtype, device="cpu", pin_memory=True)
         self._host.copy_(values, non_blocking=True)
         self._done = torch.cuda.Event()
         self._done.record()

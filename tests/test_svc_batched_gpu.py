@@ -204,6 +204,13 @@ def test_extents_on_their_way_to_the_host_stay_with_their_batch(built_library, h
     _check_matrices(batch, ptr, groups, range(4))
 
 
+def test_stacks_where_the_gpu_is_the_default_device(built_library):
+    """(what goes to the host lives there)"""
+    with torch.device("cuda"):
+        batch, ptr, groups = _stacked(np.random.default_rng(10), [40, 3, 8, 100])
+        _check_matrices(batch, ptr, groups, range(4))
+
+
 def _check_matrices(batch, ptr, groups, matrices):
     for i in matrices:
         own = ptr[groups[i]:groups[i + 1] + 1]
