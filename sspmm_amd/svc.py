@@ -78,7 +78,8 @@ class _RowPointer:
 class _ReadBack:
     """Device values on their way to the host: what is queued behind this runs on, and wait() lasts until the copy is done."""
 
-    def __init__(self, values):
+    def __init__(self, values, stream):
+        self.stream = stream
         self._host = torch.empty(values.shape, dtype=values.dtype, device="cpu", pin_memory=True)
         self._host.copy_(values, non_blocking=True)
         self._done = torch.cuda.Event()
@@ -86,13 +87,17 @@ class _ReadBack:
 
     def wait(self):
         self._done.synchronize()
-        return self._host.tolist()
+        return self._host.numpy()
+
+
+# Groups up to which svc_batched sends the row pointer ahead to the host (4 MB of pinned memory, which torch keeps for the next
+# call; the copy is a hundredth of the merge whatever the size)
+_AHEAD_GROUPS = 1 << 20
 
 
 def _split_row_ptr(count, groups, mat_groups, whole):
     """(all matrices' row pointers from zero, one after the other; the first vector of each and the end of the last)"""
-    own = torch.empty(groups + count, dtype=torch.int32, device=whole.device)
-    bounds = torch.empty(count + 1, dtype=torch.int32, device=whole.device)
+    own, bounds = torch.empty(groups + 2 * count + 1, dtype=torch.int32, device=whole.device).split((groups + count, count + 1))
     _lib.check(_lib.call(_lib.lib().svc_split_row_ptr, whole.device, count, groups, mat_groups.data_ptr(), whole.data_ptr(),
                          own.data_ptr(), bounds.data_ptr()), "svc_split_row_ptr")
     return own, bounds
@@ -133,10 +138,11 @@ class SvcBatch:
         # (row pointer from zero, first vector, end) of matrix i, whose groups are g0 .. g1 - 1.  Of a row pointer that
         # svc_batched made and nobody else has seen, one launch rebases all matrices' and one read-back brings their
         # extents: twenty matrices one by one took a launch each (0.4 ms a pass, 0.3 ms like this), and with a
-        # read-back each 1.2 ms.  svc_batched queues both between its phases (`ahead`), so that the host has the extents while
-        # the merge still runs and takes the next stack (twenty matrices 297 -> 212 us a pass).  Any other one is a caller's
-        # tensor (of any type, stride, length and device), written in ways that leave no trace on the host: those go one by
-        # one.  A piece of the split is handed out once (what a caller writes into it is not in the next one), on the stream
+        # read-back each 1.2 ms.  svc_batched sends the row pointer itself to the host between its phases (`ahead`), so that the
+        # host has the extents while the merge still runs and takes the next stack (twenty matrices, pass after pass 319 -> 234 us;
+        # with the launch in svc_batched too 229, but 14 us more for callers who never ask).  Any other one is a
+        # caller's tensor (of any type, stride, length and device), written in ways that leave no trace on the host: those go one
+        # by one.  A piece of the split is handed out once (what a caller writes into it is not in the next one), on the stream
         # that it was allocated on, and in the inference mode that it was made in.
         p = self._row_ptr
         whole = p.whole
@@ -146,12 +152,9 @@ class SvcBatch:
             return ptr - lo, lo, hi
         stream, split = _lib.stream_of(whole.device), p.split
         if split is None:
-            count, ahead = len(self), p.__dict__.pop("ahead", None)  # (by one thread only)
-            if ahead is not None and ahead[2] == stream and ahead[0].is_inference() == torch.is_inference_mode_enabled():
-                own, bounds = ahead[0], ahead[1].wait()
-            else:
-                own, bounds = _split_row_ptr(count, self._first[-1], self._mat_groups, whole)
-                bounds = bounds.tolist()
+            ahead = p.ahead
+            own, bounds = _split_row_ptr(len(self), self._first[-1], self._mat_groups, whole)
+            bounds = ahead.wait()[self._groups].tolist() if ahead is not None and ahead.stream == stream else bounds.tolist()
             sizes = [b - a + 1 for a, b in zip(self._first, self._first[1:])]
             p.split = split = (bounds, dict(enumerate(own.split(sizes))), stream, own.is_inference())
         bounds, own, own_stream, inference = split
@@ -167,7 +170,9 @@ class SvcBatch:
         return SvcResult(ptr, self.vec_col[lo:hi], None if self.vec_val is None else self.vec_val[lo * self.V:hi * self.V], hi - lo)
 
     def to_host(self):
-        ptr = self._row_ptr.whole.cpu().numpy()
+        p = self._row_ptr
+        ahead = p.ahead  # (there only while it is what the device has)
+        ptr = p.whole.cpu().numpy() if ahead is None or ahead.stream != _lib.stream_of(p.whole.device) else ahead.wait()
         n = int(ptr[-1])
         col = self.vec_col[:n].cpu().numpy()
         val = None if self.vec_val is None else self.vec_val[:n * self.V].cpu().numpy()
@@ -209,8 +214,8 @@ def svc_batched(mat_rows, K_max, row_ptr, col_ind, csr_val, V, order="cpython", 
 
     mat_rows: host int array [count + 1], first row of every matrix in the stack (as stack_csr returns it);
     row_ptr[M_total + 1], col_ind[nnz]: int32 GPU tensors of the stacked CSR; csr_val: fp16 GPU tensor or None.
-    Nothing is waited for: both phases are queued on the current stream, between them the matrices' extents, on their way
-    to the host for matrix().  Returns an SvcBatch."""
+    Nothing is waited for: both phases are queued on the current stream, between them a copy of the row pointer to the
+    host, for matrix().  Returns an SvcBatch."""
     import numpy as np
     if order not in _ORDERS:
         raise ValueError("order must be 'cpython' or 'sorted'")
@@ -222,7 +227,7 @@ def svc_batched(mat_rows, K_max, row_ptr, col_ind, csr_val, V, order="cpython", 
         raise ValueError("row_ptr and col_ind must live on the GPU")
     mat_rows = np.asarray(mat_rows, dtype=np.int64)
     count, M_total = mat_rows.size - 1, int(mat_rows[-1])
-    rows = np.diff(mat_rows)
+    rows = mat_rows[1:] - mat_rows[:-1]
     if count < 0 or row_ptr.numel() != M_total + 1 or (rows < 0).any():
         raise ValueError("mat_rows must be non-decreasing with mat_rows[-1] + 1 == len(row_ptr)")
     groups_of = np.zeros(count + 1, dtype=np.int64)
@@ -232,7 +237,7 @@ def svc_batched(mat_rows, K_max, row_ptr, col_ind, csr_val, V, order="cpython", 
     dev = row_ptr.device
     nnz = col_ind.numel()
     with torch.cuda.device(dev):
-        stream = torch.cuda.current_stream().cuda_stream
+        stream = _lib.stream_of(dev)
         d_rows, capturing, ahead = torch.from_numpy(mat_rows.astype(np.int32)), torch.cuda.is_current_stream_capturing(), None
         # (from pinned memory the copy waits for nothing; a stream that is captured refuses the other one, as it has to: a replay
         # would read the numbers from memory that has gone to others)
@@ -246,9 +251,8 @@ def svc_batched(mat_rows, K_max, row_ptr, col_ind, csr_val, V, order="cpython", 
             _lib.check(L.svc_count_batched(count, groups, d_rows.data_ptr(), M_total, K_max, V, row_ptr.data_ptr(),
                                            col_ind.data_ptr(), nnz, _ORDERS[order], d_groups.data_ptr(),
                                            vec_row_ptr.data_ptr(), ws.data_ptr(), stream), "svc_count_batched")
-            if not capturing:
-                own, bounds = _split_row_ptr(count, groups, d_groups, vec_row_ptr)
-                ahead = (own, _ReadBack(bounds), stream)
+            if not capturing and 0 < groups <= _AHEAD_GROUPS:
+                ahead = _ReadBack(vec_row_ptr, stream)
             _lib.check(L.svc_fill_batched(count, groups, d_rows.data_ptr(), M_total, K_max, V, row_ptr.data_ptr(),
                                           col_ind.data_ptr(), 0 if csr_val is None else csr_val.data_ptr(), nnz,
                                           _ORDERS[order], vec_row_ptr.data_ptr(), ws.data_ptr(), vec_col.data_ptr(),

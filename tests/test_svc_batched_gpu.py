@@ -204,6 +204,31 @@ def test_extents_on_their_way_to_the_host_stay_with_their_batch(built_library, h
     _check_matrices(batch, ptr, groups, range(4))
 
 
+def test_callers_who_take_no_matrix_do_not_pay_for_them(built_library, monkeypatch):
+    """The matrices' own row pointers are made for matrix() alone; to_host() has the row pointer that svc_batched sent, as long as
+    nobody else can have written it, before and after matrix()."""
+    import sys
+    svc_mod, made = sys.modules["sspmm_amd.svc"], []
+    split = svc_mod._split_row_ptr
+    monkeypatch.setattr(svc_mod, "_split_row_ptr", lambda *a: (made.append(1), split(*a))[1])
+    batch, ptr, groups = _stacked(np.random.default_rng(11), [40, 3, 8, 100])
+    rebased = lambda p: [[x - p[a] for x in p[a:b + 1]] for a, b in zip(groups, groups[1:])]  # noqa: E731
+    got = lambda: [t[0].tolist() for t in batch.to_host()]  # noqa: E731
+    assert got() == rebased(ptr) and not made
+    first = batch.to_host()[0][0]
+    first[:] = -1                                   # (what is handed out is the caller's)
+    assert got() == rebased(ptr) and not made
+    _check_matrices(batch, ptr, groups, range(4))
+    assert len(made) == 1 and got() == rebased(ptr)
+    other = [p - (i % 3 if 0 < i else 0) for i, p in enumerate(ptr)]
+    batch.vec_row_ptr.copy_(torch.tensor(other, dtype=torch.int32))
+    assert got() == rebased(other) and len(made) == 1
+    batch, ptr, groups = _stacked(np.random.default_rng(12), [40, 8])
+    whole = batch.vec_row_ptr                       # (before anything else was asked for)
+    whole[1:] += 1
+    assert got() == rebased([0] + [p + 1 for p in ptr[1:]]) and len(made) == 1
+
+
 def test_stacks_where_the_gpu_is_the_default_device(built_library):
     """(what goes to the host lives there)"""
     with torch.device("cuda"):
