@@ -68,8 +68,10 @@ class _RowPointer:
     """The row pointer of a stack and what matrix() may keep of it: as long as it is `alone`, nobody but the batch (and
     its shallow copies, which share this object) has the tensor, so nobody can have written it."""
 
+    ahead = None  # (for those that come out of an older pickle)
+
     def __init__(self, whole):
-        self.whole, self.alone, self.split, self.ahead = whole, False, None, None
+        self.whole, self.alone, self.split = whole, False, None
 
     def __getstate__(self):  # (deep copies and pickles: what is on its way to the host stays with the original)
         return dict(self.__dict__, ahead=None)
@@ -120,6 +122,10 @@ class SvcBatch:
         self._mat_groups = mat_groups       # the same on the device, or None
         self._row_ptr = _RowPointer(vec_row_ptr)
         self.vec_col, self.vec_val = vec_col, vec_val
+
+    def __setstate__(self, state):
+        self.__dict__.update(state)
+        self._first = [int(g) for g in self._groups]  # (older pickles have the array alone)
 
     @property
     def vec_row_ptr(self):

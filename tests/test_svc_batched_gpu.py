@@ -147,6 +147,19 @@ def test_extents_follow_the_row_pointer():
             b.matrix(i)
 
 
+def test_a_stack_pickled_before_it_had_a_list_of_its_first_groups():
+    """The state that a batch had when it kept the array of first groups and the row pointer alone (host tensors: no launches)."""
+    import pickle
+    from sspmm_amd.svc import SvcBatch
+    groups = np.array([0, 2, 2, 4])
+    b = SvcBatch(8, np.array([16, 0, 16]), None, groups, torch.tensor([0, 2, 5, 5, 9], dtype=torch.int32), torch.arange(9, dtype=torch.int32),
+                 None, torch.from_numpy(groups.astype(np.int32)))
+    b.__dict__.pop("_first")
+    b._row_ptr.__dict__.pop("ahead", None)
+    old = pickle.loads(pickle.dumps(b))
+    assert [old.matrix(i).num_vec for i in range(3)] == [5, 0, 4] and [t[0].tolist() for t in old.to_host()] == [[0, 2, 5], [0], [0, 0, 4]]
+
+
 @pytest.mark.parametrize("rows", [[16], [0, 0], [0, 24, 0, 0, 7, 300, 0], [8] * 70])
 def test_row_pointers_of_a_stack_are_each_matrix_s_own(built_library, rows):
     """Empty matrices at either end and in a row, more matrices than a wave has lanes; a second call and one on another
