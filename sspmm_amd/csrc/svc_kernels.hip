@@ -794,16 +794,19 @@ __device__ __forceinline__ int compact_table32(const Table32 &t, uint32_t slots,
   return kept;
 }
 
-// The same where the list is in LDS and the table is a construction's last: a wave has at most eight words, which stay in
+// The same where the list is in LDS and the table is a construction's last: a wave has at most MOST words, which stay in
 // registers between the count and the result, and the lists' entries are all read before any is written, so that the pass
 // is four LDS round trips instead of one or two per word.  `words`: 2 * WAVES ints that nothing else uses.
-template <int THREADS>
+// MOST: words a wave can have.  Every one of them is worked on, which a group of a few columns pays for once per row: 8 of at most two
+// for four waves and 512 slots cost 1024 groups of 8 rows of one entry 98 us, 2 of them 91 (and 93 before there was this pass); one for
+// tables of up to 64 slots a wave in the other kernels 2048 such groups 88 -> 85 (87), 125 groups of 8 rows of 16 86 -> 81.
+template <int THREADS, int MOST>
 __device__ __forceinline__ int compact_in_lds(const Table32 &t, uint32_t slots, int *words, int *list, int *before, OrderCheck &check) {
-  constexpr int WAVES = THREADS / 64, MOST = 8;
+  constexpr int WAVES = THREADS / 64;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const uint32_t n_words = slots >= 64u ? slots / 64u : 1u;
-  const uint32_t per_wave = (n_words + WAVES - 1u) / WAVES;  // <= MOST: 512 slots a wave, 8192 sixteen
+  const uint32_t per_wave = (n_words + WAVES - 1u) / WAVES;  // <= MOST: 512 slots for one wave and four, 8192 for sixteen
   const uint32_t w_beg = min(n_words, (uint32_t)wave * per_wave), mine = min(n_words, w_beg + per_wave) - w_beg;
   uint32_t x[MOST], rank[MOST];
 #pragma unroll
@@ -1091,7 +1094,9 @@ __device__ __forceinline__ uint32_t rebuild_in_lds(Table32 &t, uint32_t *tables,
     __builtin_amdgcn_wave_barrier();
   }
   t.slots = tables + table_offset(last);
-  n = compact_in_lds<THREADS>(t, last, words, list, before, check);
+  if constexpr (THREADS == 256) n = compact_in_lds<THREADS, 2>(t, last, words, list, before, check);
+  else if (last <= (uint32_t)THREADS) n = compact_in_lds<THREADS, 1>(t, last, words, list, before, check);
+  else n = compact_in_lds<THREADS, 8>(t, last, words, list, before, check);
   return last;
 }
 
@@ -1607,11 +1612,12 @@ hipError_t launch_svc_fill(const SvcArgs &args, int order, const uint16_t *csr_v
   if ((e = fork_streams(ss, stream, st, 1)) != hipSuccess) return e;
   // (from here on the helper is joined back into the caller's stream whatever happens)
   e = launch_fast_class<1024, true>(a, min(m_vec, cus), large ? 2 : 1, 1, kLargeKeys, 8192, key_bits, st[0], 81 * 1024);
-  // Four waves per small group as long as the chip holds all groups at once that way (the registers leave four such
+  // Four waves per small group as long as the chip holds all groups at once that way (the registers leave five such
   // workgroups on a CU): a group's chain of placements is then what is waited for, and four waves shorten it.  Uneven (power-law)
-  // matrices, one wave / four: 8192 x 2000, 8 a row (1024 groups) 163 / 126 us; 1024 groups of 280 columns 186 / 169, of 8 to
-  // 128 level, of 32 out of 1024 columns 10 % slower.  With more groups than that they queue, four times as many of them at a time with one
-  // wave each: 2048 groups of 128 columns 155 / 191 us, 4096 168 / 315, 8192 229 / 553; 2^20 x 65536, 3 a row, 1.4 / 4.6 ms.
+  // matrices, one wave / four: 8192 x 2000, 8 a row (1024 groups) 154 / 127 us, 2400 x 2000 142 / 123, 8192 x 4096, 16 a row 151 / 141;
+  // even ones of 1024 groups: 288 columns 149 / 140, 128 level, 64 106 / 110, 8 85 / 91.  With more groups than that they queue, and
+  // four times as many of them at a time with one wave each are ahead: 2048 groups of 64 columns 109 / 144, of 288 153 / 190,
+  // 4096 of 64 122 / 190; 1536 (the first queue little) 107 / 113 and 156 / 153.
   if (e == hipSuccess)
     e = m_vec <= 4 * cus ? launch_fast_class<256, true>(a, m_vec, 0, 0, kSmallKeys, 512, key_bits, st[1])
                          : launch_fast_class<64, true>(a, min(m_vec, 32 * cus), 0, 0, kSmallKeys, 512, key_bits, st[1]);

@@ -137,6 +137,25 @@ def test_either_side_of_every_table_size(oracle, built_library, keys):
         _compare_with_oracle(oracle, csr, V)
 
 
+@pytest.mark.parametrize("groups", [257, 1100])
+@pytest.mark.parametrize("keys", [1, 4, 5, 18, 19, 76, 77, 150, 306])
+def test_either_side_of_every_table_size_in_many_groups(oracle, built_library, keys, groups):
+    """The same table sizes in groups that are many enough for four waves each (more than there are CUs, no more than four times as
+    many) and for one, beside a wide group: all columns in the first row, one row after the other, and a last row that brings
+    nothing new."""
+    rng = np.random.default_rng(keys + groups)
+    V, K = 8, 100000
+    rows = []
+    for g in range(groups):
+        cols = np.sort(np.append(rng.integers(0, K - 1, 2000 if g == groups // 2 else keys - 1), K - 1))
+        cols = np.unique(cols)
+        parts = ([cols] + [cols[:0]] * (V - 1), np.array_split(cols, V), np.array_split(cols, V - 1) + [cols])[g % 3]
+        rows += [np.sort(p) for p in parts]
+    ptr = np.concatenate([[0], np.cumsum([r.size for r in rows])]).astype(np.int32)
+    flat = np.concatenate(rows).astype(np.int32)
+    _compare_with_oracle(oracle, synth.Csr(len(rows), K, ptr, flat, rng.standard_normal(flat.size).astype(np.float16)), V)
+
+
 @pytest.mark.parametrize("keys", [5, 40, 200, 700, 2500, 4000])
 def test_member_rows_that_bring_nothing_new(oracle, built_library, keys):
     """CPython rebuilds the set for every member row, also for an empty row and for a row whose columns are all
