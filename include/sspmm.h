@@ -122,8 +122,9 @@ int sspmm_linear_f16(int m_vec, int V, int N, int K, const int32_t *row_offsets,
  * Wo is [hidden, hidden], W1 [ffn, hidden], W2 [hidden, ffn], each row offsets, column indices and
  * values as for sspmm_linear_f16, biases and beta or NULL.  Every activation is rounded to fp16, sums
  * and statistics are fp32.  out may be neither x nor context.
- * Hidden up to 1024, hidden and ffn multiples of V and together up to about 4300 (they share a CU's LDS);
- * values 16-byte aligned, activations at any element, any number of tokens.  Other sizes: error.
+ * Hidden up to 1024, hidden and ffn multiples of V and together up to 4048 for every hidden, with V = 8 up to 4136
+ * (they share a CU's LDS; a narrow hidden leaves some more, which sspmm_encoder_tail_fits tells); values 16-byte
+ * aligned, activations at any element, up to 2^24 tokens.  Other sizes: error.
  * ---------------------------------------------------------------------------------------- */
 int sspmm_encoder_tail_fits(int hidden, int ffn, int tokens, int V); /* 1 where the launch takes these sizes, else 0 */
 int sspmm_encoder_tail_f16(int hidden, int ffn, int tokens, int V, const sspmm_half_t *x,

@@ -647,14 +647,16 @@ static constexpr uint32_t layout_buffer_off(int L, int NQ, uint32_t rows, uint32
 static constexpr int wave_lds_bytes(int V) { return val_tile_bytes(V); }
 
 // Ring slots: steps whose loads are in flight or waiting in registers.  A step is long beside the L2's answer (sixteen waves
-// share the CU), so two steps ahead, three with slabs of two column tiles, whose steps are the shortest, cover it; a deeper
-// ring delays the first step of every item and keeps more loads in a memory pipeline that the stores of C need.
-// Six slots (V = 8; five for V = 16) / three: A 2048 x 512 at 90 %, N = 256, batch 128, fp32 C 56.2 / 53.6 us (55.8 / 55.5 on another
-// card), at 70 %, batch 64
-// 45.4 / 43.6, 1536 x 1024 at 80 %, N = 500, batch 32 44.6 / 43.1, V = 16 level; two tiles, 2048 x 2048 at 80 %, N = 512, batch 16,
-// fp16 C six 60.3, five 60.1, four 60.1, three 61.2, at 90 %, N = 256, fp32 23.0, 22.7, 22.2, 22.4.  One tile (the encoder layer's
-// tail, 3 to 36 steps a wave and product): layer of 768 features, 8 x 512 tokens, V = 16 / 8 at 90 % two slots 69.3 / 97.9, three
-// 63.3 / 84.0, five 65.0 / 84.9.
+// share the CU), so two steps ahead, three with slabs of two column tiles, whose steps are the shortest, cover it.  What a deeper
+// ring costs has not been told apart: it delays the first step of every item, keeps more loads in a memory pipeline that the
+// stores of C need, and takes 6 to 17 vector registers more and scalar ones that spill (in 38 of the 56 slab kernels; now in none).
+// us with six slots (V = 16: five) / as it is, side by side on one card.  64 columns, V = 8: A 2048 x 512 at 90 %, N = 256, batch 128, fp32
+// C 57.2 / 56.7 (56.2 / 53.6 and 55.8 / 55.5 on two others), at 70 %, batch 64 47.9 / 46.9, 1536 x 1024 at 80 %, N = 500, batch 32, fp16
+// 45.0 / 44.1; V = 16: 59.2 / 59.0, 2048 x 256 at 70 %, N = 512, batch 64 56.5 / 55.5, at 90 % 56.8 / 57.4.  128 columns (fp16 C):
+// V = 8, 2048 x 512 at 90 % 41.4 / 39.5, at 50 % 57.3 / 53.6; V = 16 32.8 / 32.2, 2048 x 256 at 50 % 41.1 / 41.4.  32 columns,
+// 2048 x 2048, N = 512, batch 16, V = 8 at 80 % six 66.2, five 66.1, four 65.3, three 65.9, at 90 % 42.3, 41.5, 40.8, 41.3.  One tile (the encoder
+// layer's tail, 3 to 36 steps a wave and product): layer of 768 features, 8 x 512 tokens, V = 16 / 8 at 90 % two slots 69.3 / 97.9,
+// three 63.3 / 84.0, five 65.0 / 84.9.
 static constexpr int slab_ring(int NQ) { return NQ == 2 ? 4 : 3; }
 
 template <int V>

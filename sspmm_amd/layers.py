@@ -170,8 +170,10 @@ def add_layernorm(x, a, ln):
     return out
 
 
-# Longest sequence that is no multiple of 64 for which the kernel is ahead of torch's attention between two relayout copies: 12 heads,
-# 8 x 500 tokens 25 us against 69, 4 x 2000 130 against 217, 5000 261 against 285, and level from there on (the copies are linear).
+# Longest sequence that is no multiple of 64 for which the kernel is ahead of torch's attention between two relayout copies whatever the
+# batch: 12 heads, 8 x 500 tokens 25 us against 69, 4 x 2000 136 against 215, 2 x 4001 267 against 463; 5000 tokens are ahead with few
+# heads and behind with many (2 x 12 heads 410 / 472 us, 8 x 16 1990 / 2000), 6001 behind from 24 heads on (565 / 561), 12001 well behind
+# (2170 / 1666): torch's kernel has larger tiles, and the copies, which are linear, stop counting.
 ATTENTION_FM_RAGGED = 4096
 
 
@@ -217,12 +219,17 @@ TAIL_TOKENS = 1024
 
 def encoder_tail_pays(hidden, tokens, vectors, cus):
     """Whether the one launch is ahead of the five it replaces; `vectors`: stored vectors of its three weights.  A workgroup of
-    16 tokens, one per CU, takes as long however few of them there are: some 28 us and 0.45 us per thousand vectors, where the
-    separate launches' time follows the tokens.  Layer with 768 features (replayed, so that the host plays no part), separate / one
-    launch, us: V = 16 at 90 % (33 000 vectors) 512 tokens 47 / 55, 1024 57 / 57, 4096 89 / 69; V = 8 at 90 % (66 000) 1024
-    60 / 74, 2048 76 / 80, 3072 96 / 86, 4096 107 / 88; V = 8 at 50 % (330 000) 1536 117 / 180, 4096 210 / 205.  Beyond one
-    workgroup per CU a nearly empty last round costs a whole one: 8192 tokens 144 / 123, 7168 137 / 120, and narrow or dense weights
-    are level there (256 features V = 8 at 50 % 90 / 92, 512 at 50 % 203 / 210)."""
+    16 tokens, one per CU, takes as long however few of them there are: a layer with it some 35 us and 0.44 us per thousand
+    vectors, where the separate launches' time follows the tokens.  Layer with 768 features (replayed, so that the host plays
+    no part), separate / one launch, us: V = 16 at 90 % (33 000 vectors) 512 tokens 42 / 49, 1024 52 / 51, 4096 82 / 64; V = 8 at 90 %
+    (66 000) 1024 57 / 68, 2048 74 / 75, 3072 89 / 81, 4096 99 / 83; at 85 % (99 000) 2048 79 / 89, 3072 99 / 95, 4096 109 / 96; at 80 %
+    (132 000) 3072 110 / 110, 4096 121 / 111, 8192 206 / 210; V = 16 at 50 % (165 000) 4096 142 / 131, 8192 242 / 247; V = 8 at 70 %
+    (199 000) 4096 143 / 140, at 50 % (332 000) 1536 117 / 190, 4096 192 / 200.  Called one by one the separate launches keep the host
+    busy for 72 us and these 40, so where the device's times are level or a little apart the one launch is ahead: 512 features, V = 8 at 90 %,
+    1024 tokens 43 / 48 replayed, 71 / 49 called.  Beyond one workgroup per CU a nearly empty last round costs a whole one:
+    8192 tokens 134 / 115 (V = 16 at 90 %) and 183 / 179 (99 000 vectors), 6144 137 / 138 (66 000) and 158 / 171 (99 000); 512 features and 88 000
+    vectors, 7168 tokens 144 / 151.  Narrower layers are ahead there as well (256 features, V = 8 at 90 %, 8192 tokens 66 / 55) and
+    have the separate launches."""
     if vectors > 100000 or tokens < max(TAIL_TOKENS, vectors // 30):
         return False
     per_round = 16 * cus

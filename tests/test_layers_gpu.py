@@ -439,6 +439,42 @@ def test_encoder_layers_tail_in_one_launch_matches_the_separate_launches(built_l
     assert len(calls) == 2
 
 
+@pytest.mark.parametrize("V", [8, 16])
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("hidden,ffn,tokens", [(64, 128, 1), (128, 64, 15), (320, 1280, 37), (768, 3072, 333), (512, 2048, 1100), (1024, 1024, 64)])
+def test_encoder_layers_tail_matches_dense_fp32_products(built_library, V, bias, hidden, ffn, tokens):
+    """The one launch against products with the densified weights in fp32, GELU and norms by torch in fp32, rounded to fp16 where the
+    kernel rounds (projections, sums, norms, hidden features): nothing of this library computes the comparison.  An
+    activation may land on the fp16 next to it (2^-11 relative), which the norms and products behind it carry on: 2^-8 of the largest."""
+    import sspmm_amd.layers as layers_mod
+    g = torch.Generator("cuda").manual_seed(hidden + tokens + V)
+    rand = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    o, f1, f2 = (_vector_sparse_linear(a, b, V, 0.9, seed=a + b + i) for i, (a, b) in enumerate(((hidden, hidden), (ffn, hidden), (hidden, ffn))))
+    n1, n2 = torch.nn.LayerNorm(hidden).cuda().half(), torch.nn.LayerNorm(hidden).cuda().half()
+    with torch.no_grad():
+        for t in (n1, n2):
+            t.weight.copy_(1 + 0.1 * rand(hidden))
+            t.bias.copy_(0.1 * rand(hidden))
+        for lin in (o, f1, f2):
+            lin.bias = rand(lin.out_features).half() if bias else None
+        x, context = rand(hidden, tokens).half(), rand(hidden, tokens).half()
+        dev = x.get_device()
+        got = layers_mod.encoder_tail(x, context, ffn, V, layers_mod._tail_weight(o, hidden, hidden, V, dev), layers_mod._tail_norm(n1, hidden, dev),
+                                      layers_mod._tail_weight(f1, hidden, ffn, V, dev), layers_mod._tail_weight(f2, ffn, hidden, V, dev),
+                                      layers_mod._tail_norm(n2, hidden, dev))
+
+        def product(lin, t):
+            y = lin.dense_weight().float() @ t.float()
+            return y if lin.bias is None else y + lin.bias.float()[:, None]
+
+        def norm(ln, s):
+            return torch.nn.functional.layer_norm(s.t().float(), (hidden,), ln.weight.float(), ln.bias.float(), ln.eps).t().half()
+
+        n = norm(n1, x + product(o, context).half())
+        want = norm(n2, n + product(f2, torch.nn.functional.gelu(product(f1, n)).half()).half())
+    assert max_rel_err(got.float().cpu().numpy(), want.float().cpu().numpy()) <= 2.0 ** -8
+
+
 def test_encoder_layers_tail_runs_on_the_weights_of_that_moment(built_library, monkeypatch):
     """A hook behind the projections that gives the layer other weights: the launch behind the attention has their addresses,
     not those of the arrays that went away (looked at without launching), and its result is the one with them."""
