@@ -303,16 +303,20 @@ def _plain_linear(m, x, in_features, out_features, multiple):
                               t.is_contiguous() and t.data_ptr() % 16 == 0) for t in (w, b)))
 
 
+# (bound once: _eager is asked by calls of a few microseconds)
+_nn_module, _forward_ad = torch.nn.modules.module, torch.autograd.forward_ad
+_tracing, _compiling, _autocast = torch.jit.is_tracing, torch.compiler.is_compiling, torch.is_autocast_enabled
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+_transforms = torch._C._functorch.maybe_current_level
+
+
 def _eager():
     """Nothing watches the operators: no forward-mode gradients, no tracing or compiling, no autocast, no modes or module hooks
     that want to see every one of them."""
-    nn_module = torch.nn.modules.module
-    return not (torch.jit.is_tracing() or torch.compiler.is_compiling() or
-                torch.is_autocast_enabled("cuda") or torch.autograd.forward_ad._current_level >= 0 or
-                torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack() or
-                torch._C._functorch.maybe_current_level() is not None or
-                nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks or
-                nn_module._global_backward_hooks or nn_module._global_backward_pre_hooks)
+    return not (_tracing() or _compiling() or _autocast("cuda") or _forward_ad._current_level >= 0 or
+                _dispatch_modes() or _function_modes() or _transforms() is not None or
+                _nn_module._global_forward_hooks or _nn_module._global_forward_pre_hooks or
+                _nn_module._global_backward_hooks or _nn_module._global_backward_pre_hooks)
 
 
 def _eager_inference():

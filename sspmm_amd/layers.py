@@ -18,6 +18,7 @@ import math
 import numpy as np
 import torch
 
+from . import _lib
 from .attention import _eager, _eager_inference, _plain_module
 from .spmm import linear as linear_op, spmm
 from .svc import svc
@@ -29,6 +30,8 @@ class SparseLinear(torch.nn.Module):
     Build one with `from_dense` (a dense weight whose zero pattern is already vector-structured
     or not: RowMerge on the GPU packs whatever is there) or `from_cvse` (arrays as the SpMM
     takes them)."""
+
+    plan = None  # (until make_plan; here, so that a call without one does not go through the module's lookup of what it lacks: 1 us)
 
     def __init__(self, in_features, out_features, vec_length, row_offsets, column_indices, values, bias=None,
                  out_dtype=torch.float16, activation=None):
@@ -113,7 +116,7 @@ class SparseLinear(torch.nn.Module):
         act = self.activation if activation == "layer" else activation
         if x.dim() != 2 or x.size(0) != self.in_features:
             raise ValueError("x must be [in_features, tokens] = [%d, *], got %s" % (self.in_features, tuple(x.shape)))
-        plan = getattr(self, "plan", None)
+        plan = self.plan
         if plan is not None and x.size(1) > plan.max_N:
             plan = None
         fuse = plan is None and self.out_dtype == torch.float16 and (self.bias is None or self.bias.dtype == torch.float16)
@@ -141,24 +144,28 @@ class SparseLinear(torch.nn.Module):
         return torch.from_numpy(W).to(self.values.device)
 
 
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _of_features(t, features, dev):
+    """Whether t is one contiguous fp16 value per feature on GPU dev."""
+    return t.dtype == torch.float16 and t.get_device() == dev and t.dim() == 1 and t.numel() == features and t.is_contiguous()
+
+
 def add_layernorm(x, a, ln):
     """LayerNorm over the features of the feature-major sum x + a ([features, tokens] fp16; a may be None) with the
     weights of `ln` (a torch.nn.LayerNorm over `features`).  One HIP kernel (sspmm_add_layernorm_f16 of the C ABI)
     where its shape limits hold, torch on transposed copies otherwise."""
-    from . import _lib
-    H, T = x.shape
-    w, b = ln.weight, ln.bias
+    shape, dev = x.shape, x.get_device()
+    (H, T), w, b = shape, ln.weight, ln.bias
     whole = T % 4 == 0
     ok = (x.dtype == torch.float16 and x.is_cuda and x.is_contiguous() and H <= 4096 and
-          (a is None or (a.dtype == torch.float16 and a.is_contiguous() and a.shape == x.shape and a.device == x.device)) and
-          w is not None and tuple(ln.normalized_shape) == (H,) and
-          all(t is None or (t.dtype == torch.float16 and t.shape == (H,) and t.is_contiguous() and t.device == x.device) for t in (w, b)))
+          (a is None or (a.dtype == torch.float16 and a.is_contiguous() and a.shape == shape and a.get_device() == dev)) and
+          w is not None and tuple(ln.normalized_shape) == (H,) and _of_features(w, H, dev) and (b is None or _of_features(b, H, dev)))
     if ok and not whole:
         # (tokens that are no multiple of 4 had torch's module, which whoever wants gradients or watches it still gets)
-        dev = x.get_device()
         ok = (0 < T <= 1 << 30 and _plain_module(ln, torch.nn.LayerNorm) and _eager_inference() and type(x) is torch.Tensor and
-              (a is None or (type(a) is torch.Tensor and a.get_device() == dev)) and _plain_tensor(w, torch.float16, dev) and
-              (b is None or _plain_tensor(b, torch.float16, dev)))
+              (a is None or type(a) is torch.Tensor) and type(w) in _PLAIN and (b is None or type(b) in _PLAIN))
     if not ok:
         s = x if a is None else x + a
         return ln(s.t()).t().contiguous()
@@ -182,7 +189,6 @@ def attention_fm(qkv, hidden, heads, batch, seq, scale=None):
     [3 * hidden, batch * seq] fp16 (rows 0 .. hidden-1 the queries, then keys, then values; token b * seq + s in
     column b * seq + s); returns the context [hidden, batch * seq], or None where the kernel's shape limits do not
     hold or, with sequences that are no multiple of 64, more than the values is wanted (the caller then takes another route)."""
-    from . import _lib
     d = hidden // heads
     T = batch * seq
     whole = seq % 64 == 0
@@ -264,7 +270,7 @@ def _tail_weight(m, in_features, out_features, V, dev):
 
 
 def _plain_tensor(t, dtype, dev):
-    return type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == dtype and t.get_device() == dev and t.is_contiguous()
+    return type(t) in _PLAIN and t.dtype == dtype and t.get_device() == dev and t.is_contiguous()
 
 
 def _tail_norm(ln, features, dev):
@@ -273,8 +279,7 @@ def _tail_norm(ln, features, dev):
         return None
     own = ln._parameters
     w, b = own.get("weight"), own.get("bias")
-    if not (_plain_tensor(w, torch.float16, dev) and w.shape == (features,) and
-            (b is None or (_plain_tensor(b, torch.float16, dev) and b.shape == (features,)))):
+    if not (type(w) in _PLAIN and _of_features(w, features, dev) and (b is None or (type(b) in _PLAIN and _of_features(b, features, dev)))):
         return None
     return w.data_ptr(), None if b is None else b.data_ptr(), float(ln.eps)
 
@@ -282,7 +287,6 @@ def _tail_norm(ln, features, dev):
 def encoder_tail(x, context, ffn, V, o, norm1, ffn1, ffn2, norm2):
     """LayerNorm2(n + ffn2(gelu(ffn1(n)))) with n = LayerNorm1(x + o(context)) on feature-major activations
     [hidden, tokens] fp16 in one launch; the weights and norms as _tail_weight and _tail_norm give them."""
-    from . import _lib
     out = torch.empty_like(x)
     rc = _lib.call(_lib.lib().sspmm_encoder_tail_f16, x.device, x.size(0), ffn, x.size(1), V, x.data_ptr(),
                    context.data_ptr(), *o, *norm1, *ffn1, *ffn2, *norm2, out.data_ptr())

@@ -83,3 +83,41 @@ def test_svc_in_a_graph(built_library):
         torch.cuda.synchronize()
         assert torch.equal(vrp, eager.vec_row_ptr) and torch.equal(vcol, eager.vec_col) and torch.equal(vval, eager.vec_val)
         _between_replays()
+
+
+@pytest.mark.parametrize("batch,seq,one_launch", [(3, 333, False), (4, 320, True), (3, 347, True)])
+def test_encoder_layer_in_a_graph(built_library, monkeypatch, batch, seq, one_launch):
+    """The attention on any number of tokens, the norms on any number and all that follows the attention in one launch, recorded
+    once and replayed on other activations."""
+    from sspmm_amd import layers
+    hidden, ffn, V = 128, 256, 8
+
+    def sparse(o, i, seed):
+        vs = synth.vector_sparse(o, i, V, 0.9, seed=seed, std=0.05)
+        return layers.SparseLinear.from_cvse(i, V, dev(vs.row_offsets), dev(vs.col_idx), dev(vs.values))
+
+    layer = layers.SparseEncoderLayer(hidden, 2, ffn, *(sparse(hidden, hidden, s) for s in range(4)), sparse(ffn, hidden, 5),
+                                      sparse(hidden, ffn, 6)).cuda().half().eval()
+    launches, tail = [], layers.encoder_tail
+    monkeypatch.setattr(layers, "encoder_tail", lambda *a: (launches.append(1), tail(*a))[1])
+    monkeypatch.setattr(layers, "TAIL_TOKENS", 1 if one_launch else 1 << 30)
+    g = torch.Generator("cuda").manual_seed(seq)
+    xs = [torch.randn(hidden, batch * seq, device="cuda", generator=g).half() for _ in range(3)]
+    x, s = xs[0].clone(), torch.cuda.Stream()
+    with torch.no_grad():
+        wants = [layer(t, batch, seq).clone() for t in xs]
+        assert len(launches) == (3 if one_launch else 0)
+        s.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(s):
+            layer(x, batch, seq)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            out = layer(x, batch, seq)
+    for t, want in zip(xs + xs[:1], wants + wants[:1]):
+        x.copy_(t)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        _between_replays()
