@@ -798,8 +798,10 @@ __device__ __forceinline__ int compact_table32(const Table32 &t, uint32_t slots,
 // registers between the count and the result, and the lists' entries are all read before any is written, so that the pass
 // is four LDS round trips instead of one or two per word.  `words`: 2 * WAVES ints that nothing else uses.
 // MOST: words a wave can have.  Every one of them is worked on, which a group of a few columns pays for once per row: 8 of at most two
-// for four waves and 512 slots cost 1024 groups of 8 rows of one entry 98 us, 2 of them 91 (and 93 before there was this pass); one for
-// tables of up to 64 slots a wave in the other kernels 2048 such groups 88 -> 85 (87), 125 groups of 8 rows of 16 86 -> 81.
+// for four waves and 512 slots cost 1024 groups of 8 rows of one entry 98 us, 2 of them 91 (and 93 before there was this pass); 1 for
+// a lone wave's tables of up to 64 slots 2048 such groups 88 -> 85 (87).  Sixteen waves have the eight alone: a shorter pass beside it
+// helps a matrix of few groups (125 of 8 rows of 16 86 -> 81) and is more code for the groups of thousands of columns to walk through
+// (16384 power-law rows 166 -> 168).
 template <int THREADS, int MOST>
 __device__ __forceinline__ int compact_in_lds(const Table32 &t, uint32_t slots, int *words, int *list, int *before, OrderCheck &check) {
   constexpr int WAVES = THREADS / 64;
@@ -1095,7 +1097,7 @@ __device__ __forceinline__ uint32_t rebuild_in_lds(Table32 &t, uint32_t *tables,
   }
   t.slots = tables + table_offset(last);
   if constexpr (THREADS == 256) n = compact_in_lds<THREADS, 2>(t, last, words, list, before, check);
-  else if (last <= (uint32_t)THREADS) n = compact_in_lds<THREADS, 1>(t, last, words, list, before, check);
+  else if (THREADS == 64 && last <= 64u) n = compact_in_lds<THREADS, 1>(t, last, words, list, before, check);
   else n = compact_in_lds<THREADS, 8>(t, last, words, list, before, check);
   return last;
 }
