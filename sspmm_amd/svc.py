@@ -78,10 +78,11 @@ class _RowPointer:
 
 
 class _ReadBack:
-    """Device values on their way to the host: what is queued behind this runs on, and wait() lasts until the copy is done."""
+    """Device values on their way to the host: what is queued behind this runs on, and wait() lasts until the copy is done.
+    whole: they are the row pointer, not the matrices' extents alone."""
 
-    def __init__(self, values, stream):
-        self.stream = stream
+    def __init__(self, values, stream, whole):
+        self.stream, self.whole = stream, whole
         self._host = torch.empty(values.shape, dtype=values.dtype, device="cpu", pin_memory=True)
         self._host.copy_(values, non_blocking=True)
         self._done = torch.cuda.Event()
@@ -92,9 +93,10 @@ class _ReadBack:
         return self._host.numpy()
 
 
-# Groups up to which svc_batched sends the row pointer ahead to the host (4 MB of pinned memory, which torch keeps for the next
-# call; the copy is a hundredth of the merge whatever the size)
-_AHEAD_GROUPS = 1 << 20
+# Values that svc_batched sends ahead to the host at most, 16 KB: the row pointer where it is that small, the matrices' extents (by a
+# launch) where they are.  Larger copies go another way, of which the first ones keep the host waiting for 5 to 7 ms each (96 matrices
+# of 12288 groups: four of the first 40 calls).
+_AHEAD = 4096
 
 
 def _split_row_ptr(count, groups, mat_groups, whole):
@@ -144,9 +146,9 @@ class SvcBatch:
         # (row pointer from zero, first vector, end) of matrix i, whose groups are g0 .. g1 - 1.  Of a row pointer that
         # svc_batched made and nobody else has seen, one launch rebases all matrices' and one read-back brings their
         # extents: twenty matrices one by one took a launch each (0.4 ms a pass, 0.3 ms like this), and with a
-        # read-back each 1.2 ms.  svc_batched sends the row pointer itself to the host between its phases (`ahead`), so that the
-        # host has the extents while the merge still runs and takes the next stack (twenty matrices, pass after pass 319 -> 234 us;
-        # with the launch in svc_batched too 229, but 14 us more for callers who never ask).  Any other one is a
+        # read-back each 1.2 ms.  svc_batched sends the row pointer, or the extents, to the host between its phases (`ahead`), so that the
+        # host has the extents while the merge still runs and takes the next stack (twenty matrices, pass after pass 290-320 -> 195-235 us;
+        # with the launch in svc_batched the same, but 14 us more for callers who never ask).  Any other one is a
         # caller's tensor (of any type, stride, length and device), written in ways that leave no trace on the host: those go one
         # by one.  A piece of the split is handed out once (what a caller writes into it is not in the next one), on the stream
         # that it was allocated on, and in the inference mode that it was made in.
@@ -160,7 +162,9 @@ class SvcBatch:
         if split is None:
             ahead = p.ahead
             own, bounds = _split_row_ptr(len(self), self._first[-1], self._mat_groups, whole)
-            bounds = ahead.wait()[self._groups].tolist() if ahead is not None and ahead.stream == stream else bounds.tolist()
+            if ahead is not None and ahead.stream == stream:
+                bounds = ahead.wait()[self._groups] if ahead.whole else ahead.wait()
+            bounds = bounds.tolist()
             sizes = [b - a + 1 for a, b in zip(self._first, self._first[1:])]
             p.split = split = (bounds, dict(enumerate(own.split(sizes))), stream, own.is_inference())
         bounds, own, own_stream, inference = split
@@ -178,7 +182,7 @@ class SvcBatch:
     def to_host(self):
         p = self._row_ptr
         ahead = p.ahead  # (there only while it is what the device has)
-        ptr = p.whole.cpu().numpy() if ahead is None or ahead.stream != _lib.stream_of(p.whole.device) else ahead.wait()
+        ptr = ahead.wait() if ahead is not None and ahead.whole and ahead.stream == _lib.stream_of(p.whole.device) else p.whole.cpu().numpy()
         n = int(ptr[-1])
         col = self.vec_col[:n].cpu().numpy()
         val = None if self.vec_val is None else self.vec_val[:n * self.V].cpu().numpy()
@@ -220,8 +224,8 @@ def svc_batched(mat_rows, K_max, row_ptr, col_ind, csr_val, V, order="cpython", 
 
     mat_rows: host int array [count + 1], first row of every matrix in the stack (as stack_csr returns it);
     row_ptr[M_total + 1], col_ind[nnz]: int32 GPU tensors of the stacked CSR; csr_val: fp16 GPU tensor or None.
-    Nothing is waited for: both phases are queued on the current stream, between them a copy of the row pointer to the
-    host, for matrix().  Returns an SvcBatch."""
+    Nothing is waited for: both phases are queued on the current stream, between them a copy of the row pointer (or of the
+    matrices' extents) to the host, for matrix().  Returns an SvcBatch."""
     import numpy as np
     if order not in _ORDERS:
         raise ValueError("order must be 'cpython' or 'sorted'")
@@ -257,8 +261,9 @@ def svc_batched(mat_rows, K_max, row_ptr, col_ind, csr_val, V, order="cpython", 
             _lib.check(L.svc_count_batched(count, groups, d_rows.data_ptr(), M_total, K_max, V, row_ptr.data_ptr(),
                                            col_ind.data_ptr(), nnz, _ORDERS[order], d_groups.data_ptr(),
                                            vec_row_ptr.data_ptr(), ws.data_ptr(), stream), "svc_count_batched")
-            if not capturing and 0 < groups <= _AHEAD_GROUPS:
-                ahead = _ReadBack(vec_row_ptr, stream)
+            if not capturing and groups > 0 and min(groups, count) < _AHEAD:
+                whole = groups < _AHEAD
+                ahead = _ReadBack(vec_row_ptr if whole else _split_row_ptr(count, groups, d_groups, vec_row_ptr)[1], stream, whole)
             _lib.check(L.svc_fill_batched(count, groups, d_rows.data_ptr(), M_total, K_max, V, row_ptr.data_ptr(),
                                           col_ind.data_ptr(), 0 if csr_val is None else csr_val.data_ptr(), nnz,
                                           _ORDERS[order], vec_row_ptr.data_ptr(), ws.data_ptr(), vec_col.data_ptr(),

@@ -242,6 +242,18 @@ def test_callers_who_take_no_matrix_do_not_pay_for_them(built_library, monkeypat
     assert got() == rebased([0] + [p + 1 for p in ptr[1:]]) and len(made) == 1
 
 
+@pytest.mark.parametrize("ahead", [4096, 8, 2])
+def test_extents_whatever_went_ahead(built_library, monkeypatch, ahead):
+    """The row pointer, the matrices' extents or nothing on its way to the host: twenty groups of four matrices against what may be sent."""
+    import sys
+    monkeypatch.setattr(sys.modules["sspmm_amd.svc"], "_AHEAD", ahead)
+    batch, ptr, groups = _stacked(np.random.default_rng(13), [40, 3, 8, 100])
+    sent = batch._row_ptr.ahead
+    assert (sent is None) == (ahead == 2) and (sent is None or sent.whole == (ahead == 4096))
+    _check_matrices(batch, ptr, groups, range(4))
+    assert [t[0].tolist() for t in batch.to_host()] == [[x - ptr[a] for x in ptr[a:b + 1]] for a, b in zip(groups, groups[1:])]
+
+
 def test_stacks_where_the_gpu_is_the_default_device(built_library):
     """(what goes to the host lives there)"""
     with torch.device("cuda"):
