@@ -213,12 +213,13 @@ def pack_weights(linears, rows_per_wave):
     """The weights of torch.nn.Linear modules in the order in which block_dense's kernel loads them, each a tensor of its
     own out of one allocation, by one launch; rows_per_wave[i] = embed / 4 for out_proj and linear2, 64 for the others."""
     n = len(linears)
-    shapes = [m.weight.shape for m in linears]
+    weights = [_weights(m)[0] for m in linears]
+    shapes = [w.shape for w in weights]
     sizes = [r * c for r, c in shapes]
-    device = linears[0].weight.device
+    device = weights[0].device
     packed = torch.empty(sum(sizes), dtype=torch.float16, device=device)
     ints = ctypes.c_int32 * n
-    rc = _lib.call(_lib.lib().sspmm_block_pack_f16, device, n, (ctypes.c_void_p * n)(*[m.weight.data_ptr() for m in linears]),
+    rc = _lib.call(_lib.lib().sspmm_block_pack_f16, device, n, (ctypes.c_void_p * n)(*[w.data_ptr() for w in weights]),
                    ints(*[r for r, _ in shapes]), ints(*[c for _, c in shapes]), ints(*rows_per_wave), packed.data_ptr())
     _lib.check(rc, "sspmm_block_pack_f16")
     return packed.split(sizes)
@@ -243,15 +244,17 @@ def block_dense(x, attn, block, norm, tail=None, keep_x=False, packed=None, head
         own = [] if attn is None else [block.out_proj, block.linear1, block.linear2]
         if own or tail is not None:
             packed = pack_weights(own + ([] if tail is None else [tail]), [E // 4, 64, E // 4][:len(own)] + [64] * (tail is not None))
+    last = (None, None) if tail is None else (packed[-1].data_ptr(), _ptr(_weights(tail)[1]))
+    gamma_n, beta_n = _weights(norm)
     if attn is None:
         own = (None, None, None, None, 0.0, 0, None, None, None, None)
     else:
-        proj, up, down, ln = block.out_proj, block.linear1, block.linear2, block.layer_norm2
-        own = (packed[0].data_ptr(), _ptr(proj.bias), _ptr(ln.weight), _ptr(ln.bias), float(ln.eps), up.out_features,
-               packed[1].data_ptr(), _ptr(up.bias), packed[2].data_ptr(), _ptr(down.bias))
-    last = (None, None) if tail is None else (packed[-1].data_ptr(), _ptr(tail.bias))
+        proj, up, down, ln = _parts(block, "out_proj", "linear1", "linear2", "layer_norm2")
+        gamma, beta = _weights(ln)
+        own = (packed[0].data_ptr(), _ptr(_weights(proj)[1]), _ptr(gamma), _ptr(beta), float(ln.eps), up.out_features,
+               packed[1].data_ptr(), _ptr(_weights(up)[1]), packed[2].data_ptr(), _ptr(_weights(down)[1]))
     rc = _lib.call(_lib.lib().sspmm_block_dense_f16, x.device, outer, inner, E, x.data_ptr(), stride[0], stride[1], _ptr(pos), float(scale),
-                   _ptr(attn), *own, _ptr(norm.weight), _ptr(norm.bias), float(norm.eps), n_out, head_dim, *last, _ptr(kept), out.data_ptr())
+                   _ptr(attn), *own, _ptr(gamma_n), _ptr(beta_n), float(norm.eps), n_out, head_dim, *last, _ptr(kept), out.data_ptr())
     _lib.check(rc, "sspmm_block_dense_f16")
     return kept, out
 
@@ -268,12 +271,50 @@ def _plain_module(m, kind):
             "forward" not in m.__dict__)
 
 
+# A module's parameters, buffers and modules by way of its __getattr__ are 0.3 us each, and a forward pass of four blocks asks for some
+# two hundred of them: 260 us of the host a pass, where the device takes 230 for two sequences of 4096 tokens.  These look where it
+# would (what a program has put elsewhere is found there): 192 us, and the pass 238 -> 219.
+def _weights(m):
+    """(m.weight, m.bias)"""
+    own = m._parameters
+    try:
+        return own["weight"], own["bias"]
+    except KeyError:
+        return m.weight, m.bias
+
+
+def _parts(m, *names):
+    """m's modules of these names"""
+    own = m._modules
+    try:
+        return [own[n] for n in names]
+    except KeyError:
+        return [getattr(m, n) for n in names]
+
+
+def _pattern(block):
+    own = block._buffers
+    try:
+        return own["row_offsets"], own["column_indices"]
+    except KeyError:
+        return block.row_offsets, block.column_indices
+
+
+_TENSORS = (torch.Tensor, torch.nn.Parameter)
+
+
+def _operand(t, device, shape):
+    """Whether a kernel on GPU `device` may read t, of this shape, as it lies."""
+    return (type(t) in _TENSORS and t.dtype is torch.float16 and t.get_device() == device and t.shape == shape and t.is_contiguous() and
+            t.data_ptr() % 16 == 0)
+
+
 def _rows_norm_applies(ln, x):
     """Whether add_layernorm_rows may stand in for ln on activations like x."""
-    E, w, b = x.size(-1), ln.weight, ln.bias
-    return (_plain_module(ln, torch.nn.LayerNorm) and E in ROW_WIDTHS and ln.normalized_shape == (E,) and w is not None and
-            all(t is None or (type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float16 and t.device == x.device and
-                              t.shape == (E,) and t.is_contiguous() and t.data_ptr() % 16 == 0) for t in (w, b)))
+    if not _plain_module(ln, torch.nn.LayerNorm):
+        return False
+    E, device, (w, b) = x.size(-1), x.get_device(), _weights(ln)
+    return (E in ROW_WIDTHS and ln.normalized_shape == (E,) and _operand(w, device, (E,)) and (b is None or _operand(b, device, (E,))))
 
 
 BLOCK_FEATURES = 1 << 20  # hidden or output features that block_dense takes at most
@@ -295,12 +336,9 @@ def _plain_linear(m, x, in_features, out_features, multiple):
     whose weights a kernel may read as they lie, for activations like x."""
     if not _plain_module(m, torch.nn.Linear):
         return False
-    w, b = m.weight, m.bias
-    return (m.in_features == in_features and m.out_features % multiple == 0 and m.out_features <= BLOCK_FEATURES and
-            out_features in (None, m.out_features) and
-            w.shape == (m.out_features, in_features) and (b is None or b.shape == (m.out_features,)) and
-            all(t is None or (type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float16 and t.device == x.device and
-                              t.is_contiguous() and t.data_ptr() % 16 == 0) for t in (w, b)))
+    outs, device, (w, b) = m.out_features, x.get_device(), _weights(m)
+    return (m.in_features == in_features and outs % multiple == 0 and outs <= BLOCK_FEATURES and (out_features is None or outs == out_features) and
+            _operand(w, device, (outs, in_features)) and (b is None or _operand(b, device, (outs,))))
 
 
 # (bound once: _eager is asked by calls of a few microseconds)
@@ -417,8 +455,8 @@ class SparseAttentionEncoder(torch.nn.Module):
 
     def _fused_norms_apply(self, x):
         return (len(self.blocks) > 0 and _rows_operand(x) and _eager_inference() and _rows_norm_applies(self.layer_norm, x) and
-                all(_plain_module(b, SparseAttentionBlock) and "attention" not in b.__dict__ and _rows_norm_applies(b.layer_norm1, x) and
-                    _rows_norm_applies(b.layer_norm2, x) for b in self.blocks))
+                all(_plain_module(b, SparseAttentionBlock) and "attention" not in b.__dict__ and
+                    all([_rows_norm_applies(n, x) for n in _parts(b, "layer_norm1", "layer_norm2")]) for b in self.blocks))
 
     def _blocks_with_fused_norms(self, x):
         """The blocks and the final LayerNorm with every residual sum in the launch of the LayerNorm behind it, also
@@ -441,32 +479,39 @@ class SparseAttentionEncoder(torch.nn.Module):
         """(where the fused norms do) heads that one launch of attention takes, and products that block_dense does and is
         ahead with (see BLOCK_WEIGHTS)"""
         seq, bsz, E = x.shape
-        return E in BLOCK_WIDTHS and packed_attention_fits(seq, bsz, 3 * E) and all(
-            b.embed_dim == E and E % b.num_heads == 0 and E // b.num_heads in FUSED_HEAD_WIDTHS and
-            _plain_linear(b.in_proj, x, E, 3 * E, 64) and _plain_linear(b.out_proj, x, E, E, 64) and
-            _plain_linear(b.linear1, x, E, None, 256) and _plain_linear(b.linear2, x, b.linear1.out_features, E, 64) and
-            (E * b.linear1.out_features <= BLOCK_WEIGHTS or seq * bsz > 4096)
-            for b in self.blocks)
+        if not (E in BLOCK_WIDTHS and packed_attention_fits(seq, bsz, 3 * E)):
+            return False
+        for b in self.blocks:
+            into, out, up, down = _parts(b, "in_proj", "out_proj", "linear1", "linear2")
+            if not (b.embed_dim == E and E % b.num_heads == 0 and E // b.num_heads in FUSED_HEAD_WIDTHS and
+                    _plain_linear(into, x, E, 3 * E, 64) and _plain_linear(out, x, E, E, 64) and
+                    _plain_linear(up, x, E, None, 256) and _plain_linear(down, x, up.out_features, E, 64) and
+                    (E * up.out_features <= BLOCK_WEIGHTS or seq * bsz > 4096)):
+                return False
+        return True
 
     def _fused_blocks(self, x, pe, scale):
         """(x * scale) + pe through the blocks and the head.  Two launches per block: its attention, and all that follows up to the next block's projection (or the head)."""
         E, blocks = x.size(-1), list(self.blocks)
-        head = _plain_linear(self.linear, x, E, None, 64) and E * self.linear.out_features <= BLOCK_WEIGHTS
-        linears, rows = [blocks[0].in_proj], [64]
+        final, linear = _parts(self, "layer_norm", "linear")
+        head = _plain_linear(linear, x, E, None, 64) and E * linear.out_features <= BLOCK_WEIGHTS
+        into, norms = [_parts(b, "in_proj")[0] for b in blocks], [_parts(b, "layer_norm1")[0] for b in blocks]
+        linears, rows = [into[0]], [64]
         for i, blk in enumerate(blocks):
-            tail = [blocks[i + 1].in_proj] if i + 1 < len(blocks) else [self.linear] * head
-            linears += [blk.out_proj, blk.linear1, blk.linear2] + tail
+            tail = [into[i + 1]] if i + 1 < len(blocks) else [linear] * head
+            linears += _parts(blk, "out_proj", "linear1", "linear2") + tail
             rows += [E // 4, 64, E // 4] + [64] * len(tail)
         packed = pack_weights(linears, rows)
 
         def attention(blk, qkv):
             # (in the pattern's own order: the longest rows last, which row_indices asks for, cost 1 to 4 %)
-            return sparse_attention_split(None, blk.row_offsets, blk.column_indices, qkv, float(qkv.size(-1)) ** -0.5, blk.vec_length)
+            offsets, columns = _pattern(blk)
+            return sparse_attention_split(None, offsets, columns, qkv, float(qkv.size(-1)) ** -0.5, blk.vec_length)
 
-        x, qkv = block_dense(x, None, None, blocks[0].layer_norm1, blocks[0].in_proj, True, packed[:1], E // blocks[0].num_heads, pe, scale)
-        for i, (blk, nxt) in enumerate(zip(blocks, blocks[1:])):
-            x, qkv = block_dense(x, attention(blk, qkv), blk, nxt.layer_norm1, nxt.in_proj, True, packed[1 + 4 * i:5 + 4 * i],
-                                 E // nxt.num_heads)
-        out = block_dense(x, attention(blocks[-1], qkv), blocks[-1], self.layer_norm, self.linear if head else None,
+        x, qkv = block_dense(x, None, None, norms[0], into[0], True, packed[:1], E // blocks[0].num_heads, pe, scale)
+        for i, blk in enumerate(blocks[:-1]):
+            x, qkv = block_dense(x, attention(blk, qkv), blk, norms[i + 1], into[i + 1], True, packed[1 + 4 * i:5 + 4 * i],
+                                 E // blocks[i + 1].num_heads)
+        out = block_dense(x, attention(blocks[-1], qkv), blocks[-1], final, linear if head else None,
                           packed=packed[4 * len(blocks) - 3:])[1]
-        return out if head else self.linear(out)
+        return out if head else linear(out)
