@@ -225,7 +225,29 @@ def pack_weights(linears, rows_per_wave):
     return packed.split(sizes)
 
 
-def block_dense(x, attn, block, norm, tail=None, keep_x=False, packed=None, head_dim=0, pos=None, scale=1.0):
+def fold_blocks(blocks, linears, rows_per_wave):
+    """pack_weights(linears, rows_per_wave), and in the same launch linear1 and linear2 of every block as the one linear map they
+    are, there being nothing between them: (packed, [(matrix, affine) per block]) for block_dense's `folded`."""
+    n, f, E = len(linears), len(blocks), blocks[0].embed_dim
+    weights = [_weights(m)[0] for m in linears]
+    shapes = [w.shape for w in weights]
+    sizes = [r * c for r, c in shapes]
+    device = weights[0].device
+    pairs = [_parts(b, "linear1", "linear2") for b in blocks]
+    up, down = [_weights(a) for a, _ in pairs], [_weights(b) for _, b in pairs]
+    packed = torch.empty(sum(sizes) + f * E * E, dtype=torch.float16, device=device)
+    affine = torch.empty((f, 2 * E), dtype=torch.float32, device=device)
+    ints, ptrs, some = ctypes.c_int32 * n, ctypes.c_void_p * n, ctypes.c_void_p * f
+    rc = _lib.call(_lib.lib().sspmm_block_fold_f16, device, n, ptrs(*[w.data_ptr() for w in weights]), ints(*[r for r, _ in shapes]),
+                   ints(*[c for _, c in shapes]), ints(*rows_per_wave), packed.data_ptr(), f, E, (ctypes.c_int32 * f)(*[a.out_features for a, _ in pairs]),
+                   some(*[w.data_ptr() for w, _ in up]), some(*[_ptr(b) for _, b in up]), some(*[w.data_ptr() for w, _ in down]),
+                   some(*[_ptr(b) for _, b in down]), packed.data_ptr() + 2 * sum(sizes), affine.data_ptr())
+    _lib.check(rc, "sspmm_block_fold_f16")
+    parts = packed.split(sizes + f * [E * E])
+    return parts[:n], list(zip(parts[n:], affine))
+
+
+def block_dense(x, attn, block, norm, tail=None, keep_x=False, packed=None, head_dim=0, pos=None, scale=1.0, folded=None):
     """(x', out): everything between the attention of `block` and the next one's in one launch, on token-major activations
     [seq, batch, embed] fp16:
         s = out_proj(attn) + x, x' = linear2(linear1(layer_norm2(s))) + x, h = norm(x'), out = tail(h) or h itself.
@@ -233,7 +255,8 @@ def block_dense(x, attn, block, norm, tail=None, keep_x=False, packed=None, head
     attn is dense, and so are the results.  x' is only returned with keep_x.  packed: pack_weights of out_proj, linear1 and
     linear2 (where there is attn) and tail (where there is one), in this order.  head_dim: out as
     [tail.out_features / embed, batch, embed / head_dim, seq, head_dim], for sparse_attention_split.  pos
-    [seq, embed]: x is an embedding, and (x * scale) + pos stands in its place, each rounded to fp16."""
+    [seq, embed]: x is an embedding, and (x * scale) + pos stands in its place, each rounded to fp16.  folded: linear1 and linear2 as
+    fold_blocks leaves them (with attn, without pos), packed then that of out_proj and tail."""
     outer, inner, E = x.shape
     n_out = 0 if tail is None else tail.out_features
     shape = (n_out // E, inner, E // head_dim, outer, head_dim) if head_dim else (outer, inner, n_out or E)
@@ -246,6 +269,14 @@ def block_dense(x, attn, block, norm, tail=None, keep_x=False, packed=None, head
             packed = pack_weights(own + ([] if tail is None else [tail]), [E // 4, 64, E // 4][:len(own)] + [64] * (tail is not None))
     last = (None, None) if tail is None else (packed[-1].data_ptr(), _ptr(_weights(tail)[1]))
     gamma_n, beta_n = _weights(norm)
+    if folded is not None:
+        proj, ln = _parts(block, "out_proj", "layer_norm2")
+        gamma, beta = _weights(ln)
+        rc = _lib.call(_lib.lib().sspmm_block_dense_folded_f16, x.device, outer, inner, E, x.data_ptr(), stride[0], stride[1], _ptr(attn), packed[0].data_ptr(),
+                       _ptr(_weights(proj)[1]), _ptr(gamma), _ptr(beta), float(ln.eps), folded[0].data_ptr(), folded[1].data_ptr(),
+                       _ptr(gamma_n), _ptr(beta_n), float(norm.eps), n_out, head_dim, *last, _ptr(kept), out.data_ptr())
+        _lib.check(rc, "sspmm_block_dense_folded_f16")
+        return kept, out
     if attn is None:
         own = (None, None, None, None, 0.0, 0, None, None, None, None)
     else:
@@ -499,9 +530,9 @@ class SparseAttentionEncoder(torch.nn.Module):
         linears, rows = [into[0]], [64]
         for i, blk in enumerate(blocks):
             tail = [into[i + 1]] if i + 1 < len(blocks) else [linear] * head
-            linears += _parts(blk, "out_proj", "linear1", "linear2") + tail
-            rows += [E // 4, 64, E // 4] + [64] * len(tail)
-        packed = pack_weights(linears, rows)
+            linears += _parts(blk, "out_proj") + tail
+            rows += [E // 4] + [64] * len(tail)
+        packed, folded = fold_blocks(blocks, linears, rows)
 
         def attention(blk, qkv):
             # (in the pattern's own order: the longest rows last, which row_indices asks for, cost 1 to 4 %)
@@ -510,8 +541,8 @@ class SparseAttentionEncoder(torch.nn.Module):
 
         x, qkv = block_dense(x, None, None, norms[0], into[0], True, packed[:1], E // blocks[0].num_heads, pe, scale)
         for i, blk in enumerate(blocks[:-1]):
-            x, qkv = block_dense(x, attention(blk, qkv), blk, norms[i + 1], into[i + 1], True, packed[1 + 4 * i:5 + 4 * i],
-                                 E // blocks[i + 1].num_heads)
+            x, qkv = block_dense(x, attention(blk, qkv), blk, norms[i + 1], into[i + 1], True, packed[1 + 2 * i:3 + 2 * i],
+                                 E // blocks[i + 1].num_heads, folded=folded[i])
         out = block_dense(x, attention(blocks[-1], qkv), blocks[-1], final, linear if head else None,
-                          packed=packed[4 * len(blocks) - 3:])[1]
+                          packed=packed[2 * len(blocks) - 1:], folded=folded[-1])[1]
         return out if head else linear(out)

@@ -16,6 +16,12 @@
 // + i of tile j, accumulator i, lane group g): residual loads, LDS writes and stores are 16-byte pieces, of which the
 // four lane groups make 64 consecutive bytes.
 //
+// There is nothing between the two linear layers, so the encoder's forward pass has them multiplied first (fold_rows, once a pass)
+// and runs W2 W1 as one matrix: 0.33 M products a token in the place of 0.85, and 0.65 MB of weights to stream instead of
+// 1.6.  256 features, 1024 hidden ones, in a model: 8192 tokens 26.7 -> 16.3 us a launch, 32768 tokens 61 -> 36.5; what packs the weights and
+// multiplies them takes 12.9 us a pass for four blocks, where packing all took 7.6.  (Both layers, for callers that bring them packed:
+// the rest of this paragraph.)
+//
 // The weights a workgroup streams from L2 are 1.6 MB at 256 features and 1024 hidden ones, 25k cycles at the 64 bytes a
 // cycle of a CU, whatever TM, and the products 384 cycles per token.  The loads of the next two units (eight 16-byte
 // loads of a wave each) are in flight throughout, also across the products' boundaries; four units, at 64 registers more, were
@@ -34,6 +40,7 @@
 #include <stdint.h>
 
 #include "block_kernels.h"
+#include "lane_ops.h"
 
 namespace sspmm {
 
@@ -44,6 +51,12 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 
 constexpr int kChunk = 256;  // hidden (or output) features a workgroup makes at a time, 64 per wave
+
+typedef uint32_t uintx2 __attribute__((ext_vector_type(2)));
+typedef short shortx4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uintx2 fold_read_tr(const unsigned char *p) {
+  return __builtin_bit_cast(uintx2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) shortx4 *)p));
+}
 
 // Workgroup barrier that orders LDS only: global loads in flight stay in flight.
 __device__ __forceinline__ void lds_barrier() {
@@ -214,12 +227,15 @@ __device__ __forceinline__ void layer_norm(floatx4 (&v)[TT][NJ], const uint16_t 
 
 constexpr int block_waves(int E, int TM) { return TM == 16 || (TM == 64 && E < 512) ? 2 : 1; }  // per SIMD
 
-template <int E, int TM, bool ATTN>
+enum Part { kNoAttention, kTwoLayers, kFolded };  // what lies in front of the last LayerNorm
+
+template <int E, int TM, Part PART>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves(E, TM), block_waves(E, TM)))) void block_dense_kernel(const BlockDenseArgs p) {
   constexpr int NT = E / 64, TT = TM / 16, D = 2;
-  constexpr int kPitchA = E * 2 + 16, kPitchH = kChunk * 2 + 16;
+  constexpr int kPitchA = E * 2 + 32, kPitchH = kChunk * 2 + 32;
   __shared__ __align__(16) unsigned char act[TM * kPitchA];  // attention's output, then n, then h
-  __shared__ __align__(16) unsigned char hid[TM * kPitchH];  // kChunk hidden features
+  __shared__ __align__(16) unsigned char hid[PART == kTwoLayers ? TM * kPitchH : 16];  // kChunk hidden features
+  __shared__ __align__(16) float affine[PART == kFolded ? 2 * E : 4];
   __shared__ float part[8 * TM];
 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -233,9 +249,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
   uintx4 w[D][8];
   const int t_row = p.wt && wave * 64 < p.n_out ? wave * 64 : 0;
   // (where nothing follows, the loads ahead go to the matrix at hand once more)
-  const Weights tail = p.wt ? weights<4>(p.wt, p.n_out, E, t_row, 0) : weights<4>(p.w1, p.mlp, E, wave * 64, 0);
+  const Weights tail = p.wt ? weights<4>(p.wt, p.n_out, E, t_row, 0)
+                       : PART == kFolded ? weights<4>(p.w2, E, E, 0, 0) : weights<4>(p.w1, p.mlp, E, wave * 64, 0);
   const Weights wo = weights<NT>(p.wo, E, E, wave * (16 * NT), 0);
-  if constexpr (ATTN)
+  if constexpr (PART != kNoAttention)
     issue_first<NT, D>(w, wo);
   else if (p.wt)
     issue_first<4, D>(w, tail);
@@ -266,12 +283,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
   }
 
   floatx4 v[TT][NT];
-  if constexpr (ATTN) {
-    const Weights w1 = weights<4>(p.w1, p.mlp, E, wave * 64, 0);
-    const Weights w2 = weights<NT>(p.w2, E, p.mlp, wave * (16 * NT), 0);
+  if constexpr (PART != kNoAttention) {
+    const Weights w1 = PART == kFolded ? Weights() : weights<4>(p.w1, p.mlp, E, wave * 64, 0);
+    const Weights w2 = weights<NT>(p.w2, E, PART == kFolded ? E : p.mlp, wave * (16 * NT), 0);
     half8 bias[NT / 2], bias2[NT / 2];
     feature_values<NT>(bias, p.bo, first, 0.f);
-    feature_values<NT>(bias2, p.b2, first, 0.f);
+    if constexpr (PART == kFolded) {
+#pragma unroll
+      for (int i = 0; i < 2 * E; i += 1024)
+        if (i + 4 * (int)threadIdx.x < 2 * E)
+          *reinterpret_cast<floatx4 *>(affine + i + 4 * threadIdx.x) = *reinterpret_cast<const floatx4 *>(p.affine + i + 4 * threadIdx.x);
+    } else {
+      feature_values<NT>(bias2, p.b2, first, 0.f);
+    }
     constexpr int kPieces = E / 8, kRows = 256 / kPieces;
     const int piece = threadIdx.x % kPieces, row0 = threadIdx.x / kPieces;
 #pragma unroll
@@ -285,7 +309,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
       for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[t][j][i] = value(bias, j, i);
-    gemm<TT, NT, E, kPitchA, 4, D>(v, act_op, wo, w1, w);
+    gemm<TT, NT, E, kPitchA, PART == kFolded ? NT : 4, D>(v, act_op, wo, PART == kFolded ? w2 : w1, w);
 #pragma unroll
     for (int t = 0; t < TT; ++t)
 #pragma unroll
@@ -302,39 +326,56 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
 #pragma unroll
     for (int t = 0; t < TT; ++t) put_row<NT>(act + (t * 16 + m) * kPitchA + first * 2, v[t]);
     lds_barrier();
-#pragma unroll
-    for (int t = 0; t < TT; ++t)
-#pragma unroll
-      for (int j = 0; j < NT; ++j)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[t][j][i] = value(bias2, j, i) + value(x[t], j, i);
-    for (int c = 0; c < p.mlp; c += kChunk) {
-      floatx4 h[TT][4];
-      half8 bias1[2];
-      feature_values<4>(bias1, p.b1, c + chunk_first, 0.f);
+    if constexpr (PART == kFolded) {
 #pragma unroll
       for (int t = 0; t < TT; ++t)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) h[t][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-      Weights up = w1, down = w2, then = tail;
-      up.base += (uint32_t)c * (E * 2u);
-      down.base += (uint32_t)(c / Unit<NT>::K) * Unit<NT>::kBytes;
-      if (c + kChunk < p.mlp) {
-        then = up;
-        then.base += kChunk * (E * 2u);
+        for (int j = 0; j < NT; ++j) v[t][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+      gemm<TT, NT, E, kPitchA, 4, D>(v, act_op, w2, tail, w);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const int f = first + 32 * (j >> 1) + 4 * (j & 1);
+        const floatx4 scale = *reinterpret_cast<const floatx4 *>(affine + f), shift = *reinterpret_cast<const floatx4 *>(affine + E + f);
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[t][j][i] = __builtin_fmaf(v[t][j][i], scale[i], shift[i]) + value(x[t], j, i);
       }
-      gemm<TT, 4, E, kPitchA, NT, D>(h, act_op, up, down, w);
-      lds_barrier();  // the previous chunk has been read
+    } else {
 #pragma unroll
-      for (int t = 0; t < TT; ++t) {
+      for (int t = 0; t < TT; ++t)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < NT; ++j)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) h[t][j][i] += value(bias1, j, i);
-        put_row<4>(hid + (t * 16 + m) * kPitchH + chunk_first * 2, h[t]);
+          for (int i = 0; i < 4; ++i) v[t][j][i] = value(bias2, j, i) + value(x[t], j, i);
+      for (int c = 0; c < p.mlp; c += kChunk) {
+        floatx4 h[TT][4];
+        half8 bias1[2];
+        feature_values<4>(bias1, p.b1, c + chunk_first, 0.f);
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) h[t][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+        Weights up = w1, down = w2, then = tail;
+        up.base += (uint32_t)c * (E * 2u);
+        down.base += (uint32_t)(c / Unit<NT>::K) * Unit<NT>::kBytes;
+        if (c + kChunk < p.mlp) {
+          then = up;
+          then.base += kChunk * (E * 2u);
+        }
+        gemm<TT, 4, E, kPitchA, NT, D>(h, act_op, up, down, w);
+        lds_barrier();  // the previous chunk has been read
+#pragma unroll
+        for (int t = 0; t < TT; ++t) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) h[t][j][i] += value(bias1, j, i);
+          put_row<4>(hid + (t * 16 + m) * kPitchH + chunk_first * 2, h[t]);
+        }
+        lds_barrier();
+        gemm<TT, NT, kChunk, kPitchH, 4, D>(v, hid_op, down, then, w);
       }
-      lds_barrier();
-      gemm<TT, NT, kChunk, kPitchH, 4, D>(v, hid_op, down, then, w);
     }
   } else {
 #pragma unroll
@@ -408,11 +449,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
 
 // Up to BlockPackArgs::kMost matrices into the order in which the waves above load them: groups of 16 * NJ rows, in each units of
 // K columns, in each a 1 KB piece per step of 32 columns and tile, in that the 16 bytes of every lane.
-__global__ __launch_bounds__(256) void block_pack_kernel(const BlockPackArgs p) {
+__device__ __forceinline__ void pack_piece(const BlockPackArgs &p, uint32_t block, uint32_t threads) {
   int i = 0;
-  while (i + 1 < p.count && blockIdx.x >= p.m[i + 1].first_block) ++i;
+  while (i + 1 < p.count && block >= p.m[i + 1].first_block) ++i;
   const BlockPackArgs::Matrix &a = p.m[i];
-  const uint32_t at = (blockIdx.x - a.first_block) * 256u + threadIdx.x;  // 16-byte piece of the packed matrix
+  const uint32_t at = (block - a.first_block) * threads + threadIdx.x;  // 16-byte piece of the packed matrix
   const uint32_t cols = a.cols, nj = a.group / 16u, ku = nj == 8 ? 32u : 64u;
   if (at >= (uint32_t)a.rows * (cols / 8u)) return;
   const uint32_t lane = at & 63u, m = lane & 15u, g = lane >> 4, frag = at >> 6;
@@ -423,14 +464,126 @@ __global__ __launch_bounds__(256) void block_pack_kernel(const BlockPackArgs p) 
   reinterpret_cast<uintx4 *>(a.dst)[at] = *reinterpret_cast<const uintx4 *>(a.src + (size_t)row * cols + k);
 }
 
+__global__ __launch_bounds__(256) void block_pack_kernel(const BlockPackArgs p) { pack_piece(p, blockIdx.x, 256); }
+
+// Sixteen rows of W2 W1, and of W2 b1 + b2.  Sixteen waves: E / 64 of them take 64 columns each, and as many groups of them as that
+// leaves a share of the hidden features each; the shares are added up in LDS in their order.  A wave's 32 rows of W1 pass through an
+// LDS stage of its own, whose transpose reads make the operand (32 hidden features x 16 columns); W2's rows are the operand as they lie.
+// A row is scaled by a power of two before it is rounded to fp16, which needs its largest element: a workgroup therefore makes whole rows
+// and streams all of W1 through one CU, 512 KB for 256 x 1024: 5 of the 12.5 us at 64 bytes a cycle, some 3 for the sums and 2 to start.
+// Four steps of loads ahead instead of two are level (12.7), loads without a condition, the last ones repeated, slower (13.5).
+constexpr uint32_t kFoldPitch = 160;
+template <int E>
+__device__ void fold_rows(const BlockFoldArgs::Pair &a, int row0, unsigned char *lds) {
+  constexpr int CG = E / 64, KS = 16 / CG, DEPTH = 2, PER = E / 64;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), m = lane & 15, g = lane >> 4;
+  const int cg = wave % CG, ks = wave / CG, share = a.mlp / KS;
+  const uint16_t *const left = a.w2 + (size_t)(row0 + m) * a.mlp + ks * share + 8 * g;
+  const uint16_t *const right = a.w1 + (size_t)(ks * share + (lane >> 3)) * E + cg * 64 + (lane & 7) * 8;
+  unsigned char *const stage = lds + wave * (32 * kFoldPitch);
+  unsigned char *const dst = stage + (lane >> 3) * kFoldPitch + (lane & 7) * 16;
+  const unsigned char *const src = stage + (8 * g + (m >> 2)) * kFoldPitch + (m & 3) * 8;
+  uintx4 l[DEPTH], r[DEPTH][4];
+  const auto fetch = [&](int d, int k) {
+    l[d] = *reinterpret_cast<const uintx4 *>(left + k);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[d][i] = *reinterpret_cast<const uintx4 *>(right + (size_t)(k + 8 * i) * E);
+  };
+  floatx4 acc[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d)
+    if (32 * d < share) fetch(d, 32 * d);
+  for (int k = 0; k < share; k += 32 * DEPTH) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      const int at = k + 32 * d;
+      if (32 * DEPTH > 256 / KS && at >= share) continue;  // (uniform; a share is a multiple of 256 / KS)
+      // (LDS operations of a wave execute in order: these writes land behind the previous step's reads)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) *reinterpret_cast<uintx4 *>(dst + 8 * i * kFoldPitch) = r[d][i];
+      const half8 w = __builtin_bit_cast(half8, l[d]);
+      if (at + 32 * DEPTH < share) fetch(d, at + 32 * DEPTH);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const uintx2 lo = fold_read_tr(src + 32 * t), hi = fold_read_tr(src + 4 * kFoldPitch + 32 * t);
+        const uintx4 b = {lo[0], lo[1], hi[0], hi[1]};
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, __builtin_bit_cast(half8, b), acc[t], 0, 0, 0);
+      }
+    }
+  }
+  const int row = row0 + wave;
+  const uint16_t *const w2 = a.w2 + (size_t)row * a.mlp;
+  float shift = 0.f;
+  if (a.b1)
+    for (int k = lane * 8; k < a.mlp; k += 512) {
+      const half8 w = *reinterpret_cast<const half8 *>(w2 + k), b = *reinterpret_cast<const half8 *>(a.b1 + k);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) shift += (float)w[i] * (float)b[i];
+    }
+  shift = wave_sum_all(shift);
+  __syncthreads();
+  constexpr int kSums = E + 16;  // (the four rows a store touches at different banks)
+  float *const sums = reinterpret_cast<float *>(lds);  // [KS][16][kSums]
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sums[(ks * 16 + 4 * g + i) * kSums + cg * 64 + 16 * t + m] = acc[t][i];
+  __syncthreads();
+  // a wave per row, PER columns per lane
+  float c[PER], most = 0.f;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    c[i] = 0.f;
+#pragma unroll
+    for (int q = 0; q < KS; ++q) c[i] += sums[(q * 16 + wave) * kSums + lane * PER + i];
+    most = fmaxf(most, fabsf(c[i]));
+  }
+  most = wave_max_all(most);
+  // (a row of zeros, and one with an infinity or a NaN, as they are)
+  const int up = most > 0.f && most < INFINITY ? min(max(13 - (int)((__float_as_uint(most) >> 23) - 127u), -100), 100) : 0;
+  const float factor = __uint_as_float((uint32_t)(127 + up) << 23);
+  if (lane == 0) {
+    a.affine[row] = __uint_as_float((uint32_t)(127 - up) << 23);
+    a.affine[E + row] = shift + (a.b2 ? (float)*reinterpret_cast<const _Float16 *>(a.b2 + row) : 0.f);
+  }
+  // where block_pack_kernel puts element (row, k)
+  constexpr uint32_t kGroup = E / 4, NJ = kGroup / 16, KU = NJ == 8 ? 32 : 64;
+  const uint32_t in_group = (uint32_t)row % kGroup, k = (uint32_t)lane * PER;
+  const uint32_t tile = in_group / 32u * 2u + ((in_group >> 2) & 1u), mm = ((in_group >> 3) & 3u) * 4u + (in_group & 3u);
+  const uint32_t piece = ((uint32_t)row / kGroup * (E / KU) + k / KU) * (NJ * KU / 32u) + (k % KU) / 32u * NJ + tile;
+  _Float16 *const out = reinterpret_cast<_Float16 *>(a.dst) + piece * 512u + ((k % 32u) / 8u * 16u + mm) * 8u + k % 8u;
+  typedef _Float16 halves __attribute__((ext_vector_type(PER)));
+  halves h;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) h[i] = (_Float16)(c[i] * factor);
+  *reinterpret_cast<halves *>(out) = h;
+}
+
+template <int E>
+__global__ __launch_bounds__(1024) void block_prepare_kernel(const BlockFoldArgs f, const BlockPackArgs p) {
+  __shared__ __align__(16) unsigned char lds[16 * 32 * kFoldPitch];
+  const uint32_t folds = (uint32_t)f.count * (E / 16);
+  if (blockIdx.x < folds) {
+    // (workgroups eight apart share an XCD: one pair's on as few of them as can be, each of which fetches W1 once)
+    const uint32_t id = (blockIdx.x & 7u) * (folds / 8u) + (blockIdx.x >> 3);
+    fold_rows<E>(f.m[id / (E / 16)], (int)(id % (E / 16)) * 16, lds);
+  } else {
+    pack_piece(p, blockIdx.x - folds, 1024);
+  }
+}
+
 template <int E, int TM>
 hipError_t launch(const BlockDenseArgs &p, hipStream_t stream) {
   const long long blocks = (p.tokens + TM - 1) / TM;
   if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-  if (p.attn)
-    hipLaunchKernelGGL((block_dense_kernel<E, TM, true>), dim3((unsigned)blocks), dim3(256), 0, stream, p);
+  if (!p.attn)
+    hipLaunchKernelGGL((block_dense_kernel<E, TM, kNoAttention>), dim3((unsigned)blocks), dim3(256), 0, stream, p);
+  else if (p.affine)
+    hipLaunchKernelGGL((block_dense_kernel<E, TM, kFolded>), dim3((unsigned)blocks), dim3(256), 0, stream, p);
   else
-    hipLaunchKernelGGL((block_dense_kernel<E, TM, false>), dim3((unsigned)blocks), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((block_dense_kernel<E, TM, kTwoLayers>), dim3((unsigned)blocks), dim3(256), 0, stream, p);
   return hipGetLastError();
 }
 
@@ -457,6 +610,18 @@ bool block_dense_applies(int E, int mlp, int n_out) {
 
 hipError_t launch_block_pack(const BlockPackArgs &p, uint32_t blocks, hipStream_t stream) {
   hipLaunchKernelGGL(block_pack_kernel, dim3(blocks), dim3(256), 0, stream, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_block_prepare(int E, const BlockFoldArgs &folds, const BlockPackArgs &packs, uint32_t pack_blocks, hipStream_t stream) {
+  const dim3 grid((uint32_t)folds.count * (uint32_t)(E / 16) + pack_blocks);
+  if (grid.x == 0) return hipSuccess;
+  switch (E) {
+    case 128: hipLaunchKernelGGL(block_prepare_kernel<128>, grid, dim3(1024), 0, stream, folds, packs); break;
+    case 256: hipLaunchKernelGGL(block_prepare_kernel<256>, grid, dim3(1024), 0, stream, folds, packs); break;
+    case 512: hipLaunchKernelGGL(block_prepare_kernel<512>, grid, dim3(1024), 0, stream, folds, packs); break;
+    default: return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
 

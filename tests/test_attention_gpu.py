@@ -547,6 +547,90 @@ def test_packed_weights_hold_every_fragment_where_the_kernel_reads_it(built_libr
         assert np.array_equal(packed[i].cpu().numpy(), want[i]), i
 
 
+def _two_layers(E, mlp, count, g, size=1.0, bias=True):
+    from sspmm_amd.attention import SparseAttentionBlock
+    none = torch.zeros(1, dtype=torch.int32)
+    blocks = []
+    for _ in range(count):
+        b = SparseAttentionBlock(E, mlp, E // 32, none, none, none).cuda().half()
+        with torch.no_grad():
+            for m in (b.linear1, b.linear2):
+                m.weight.copy_(torch.randn(m.weight.shape, device="cuda", generator=g) * size * m.in_features ** -0.5)
+                m.bias.copy_(torch.randn(m.bias.shape, device="cuda", generator=g))
+            for m in (b.layer_norm1, b.layer_norm2):
+                m.weight.copy_(1 + 0.2 * torch.randn(E, device="cuda", generator=g))
+                m.bias.copy_(torch.randn(E, device="cuda", generator=g))
+        if not bias:
+            b.linear1.bias = b.linear2.bias = b.out_proj.bias = None
+        blocks.append(b)
+    return blocks
+
+
+@pytest.mark.parametrize("E,mlp,count,size,bias", [(128, 256, 1, 1.0, True), (128, 1280, 17, 2.0 ** -9, True), (256, 256, 2, 1.0, False),
+                                                   (256, 1024, 33, 4.0, True), (512, 512, 3, 1.0, True), (512, 256, 1, 2.0 ** -6, True)])
+def test_two_linear_layers_as_one_matrix(built_library, E, mlp, count, size, bias):
+    """What one to three launches leave of pairs of linear layers, against their product in float64: an element's rounding to fp16 (2^-11
+    of it, or half the smallest step of fp16, 2^-25, next to a largest element of 2^13 or more), and that of the fp32 sums, 2^-24 of their
+    terms each.  Weights whose products fp16 would not hold unscaled, a row of zeros, and one that overflows fp32."""
+    from sspmm_amd.attention import fold_blocks, pack_weights
+    g = torch.Generator("cuda").manual_seed(E + mlp)
+    blocks = _two_layers(E, mlp, count, g, size, bias)
+    with torch.no_grad():
+        blocks[0].linear2.weight[3] = 0
+        blocks[-1].linear2.weight[5, 7] = float("inf")
+    packed, folded = fold_blocks(blocks, [b.out_proj for b in blocks], [E // 4] * count)
+    group = E // 4
+    nj, unit = group // 16, 32 if group == 128 else 64
+    for b, (matrix, affine) in zip(blocks, folded):
+        got = matrix.cpu().numpy().astype(np.float64).reshape(E // group, E // unit, unit // 32, nj // 2, 2, 4, 4, 4, 8)
+        # (the inverse of the order in which the waves load: see test_packed_weights_hold_every_fragment_where_the_kernel_reads_it)
+        got = got.transpose(0, 3, 6, 4, 7, 1, 2, 5, 8).reshape(E, E)
+        down, shift = affine.cpu().numpy().astype(np.float64).reshape(2, E)
+        w1, w2 = (m.weight.detach().cpu().numpy().astype(np.float64) for m in (b.linear1, b.linear2))
+        b1, b2 = ((m.bias.detach().cpu().numpy().astype(np.float64) if bias else np.zeros(m.out_features)) for m in (b.linear1, b.linear2))
+        with np.errstate(invalid="ignore"):
+            want, terms, want_shift = w2 @ w1, np.abs(w2) @ np.abs(w1), w2 @ b1 + b2
+            finite = np.isfinite(want).all(1)
+            assert finite.sum() == E - (b is blocks[-1]) and not np.isfinite(got[~finite]).any()
+            most = np.abs(got).max(1)
+            assert (np.log2(down) % 1 == 0).all() and ((most[finite] >= 2 ** 13) & (most[finite] <= 2 ** 14) | (most[finite] == 0)).all()
+            bound = 2.0 ** -11 * np.abs(want) + (2.0 ** -25 * down)[:, None] + mlp * 2.0 ** -24 * terms
+            assert (np.abs(got * down[:, None] - want)[finite] <= bound[finite]).all()
+            assert (np.abs(shift - want_shift)[finite] <= (mlp * 2.0 ** -24 * (np.abs(w2) @ np.abs(b1)) + 2.0 ** -23 * np.abs(b2) + 1e-30)[finite]).all()
+    for one, other in zip(packed, pack_weights([b.out_proj for b in blocks], [E // 4] * count)):
+        assert torch.equal(one, other)
+
+
+@pytest.mark.parametrize("E,mlp,n_out,outer,inner", [(128, 256, 128, 1, 1), (128, 512, 64, 70, 61), (256, 1024, 768, 37, 3), (256, 256, 64, 1433, 3),
+                                                     (256, 512, 256, 2731, 3), (512, 256, 1536, 19, 1), (512, 512, 64, 1366, 3), (512, 256, 512, 2731, 3)])
+def test_block_dense_on_one_matrix_for_two_layers(built_library, E, mlp, n_out, outer, inner):
+    """Every width and tile of tokens (16, 32, 64) with a last tile that is not full; with and without a tail, x', biases.  The bound is
+    that of test_block_dense_in_one_launch, which has one rounding more."""
+    lin = lambda m, t: t @ m.weight.double().t() + (0 if m.bias is None else m.bias.double())  # noqa: E731
+    ln = lambda m, t: torch.nn.functional.layer_norm(t, m.normalized_shape, m.weight.double(), m.bias.double(), m.eps)  # noqa: E731
+    from sspmm_amd.attention import block_dense, fold_blocks
+    g = torch.Generator("cuda").manual_seed(E + outer)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g).half()  # noqa: E731
+    for bias in (True, False):
+        blk, = _two_layers(E, mlp, 1, g, bias=bias)
+        norm, tail = torch.nn.LayerNorm(E).cuda().half(), torch.nn.Linear(E, n_out, bias=bias).cuda().half()
+        attn, x = rnd(outer, inner, E), (rnd(inner, outer, E) * 2 + 1).transpose(0, 1)
+        for last, keep in ((tail, True), (None, False)):
+            with torch.no_grad():
+                packed, folded = fold_blocks([blk], [blk.out_proj] + [tail] * (last is not None), [E // 4] + [64] * (last is not None))
+                kept, got = block_dense(x, attn, blk, norm, last, keep_x=keep, packed=packed, folded=folded[0])
+                n = ln(blk.layer_norm2, lin(blk.out_proj, attn.double()) + x.double()).half().double()
+                want_x = (lin(blk.linear2, lin(blk.linear1, n)) + x.double()).half().double()
+                h = ln(norm, want_x)
+                want = h if last is None else lin(last, h.half().double())
+                assert ((got.double() - want).abs().max() <= 4 * 2 ** -11 * want.abs().max()).item()
+                assert (kept is None) if not keep else ((kept.double() - want_x).abs().max() <= 4 * 2 ** -11 * want_x.abs().max()).item()
+                if last is not None and n_out % E == 0:
+                    for d in (32, 64, 128):
+                        split = block_dense(x, attn, blk, norm, last, packed=packed, folded=folded[0], head_dim=d)[1]
+                        assert torch.equal(split, got.view(outer, inner, n_out // E, E // d, d).permute(2, 1, 3, 0, 4))
+
+
 @pytest.mark.parametrize("embed,heads,mlp,V", [(128, 4, 512, 8), (256, 8, 1024, 16), (512, 8, 512, 8), (192, 6, 512, 8), (1024, 16, 512, 16)])
 def test_encoder_against_float64(built_library, embed, heads, mlp, V):
     """The whole model on each of its routes (two launches a block, fused norms, and for 192 features the modules) against dense

@@ -121,6 +121,26 @@ def test_argument_errors_of_the_dense_block_entries(built_library):
     assert L.sspmm_block_pack_f16(1, None, None, None, None, p, None) == 1
     assert L.sspmm_block_pack_f16(0, None, None, None, None, None, None) == 0
 
+    def folded(outer=2, inner=3, E=128, x=p, attn=p, wo=p, w21=p, affine=p, n_out=128, head_dim=0, wt=p, x_out=p, out=p):
+        return L.sspmm_block_dense_folded_f16(outer, inner, E, x, 384, 128, attn, wo, p, p, p, 1e-5, w21, affine, p, p, 1e-5, n_out, head_dim, wt, p,
+                                              x_out, out, None)
+
+    for bad in (dict(outer=-1), dict(E=64), dict(E=192), dict(n_out=96), dict(n_out=0), dict(wt=None), dict(x=None), dict(attn=None), dict(wo=None),
+                dict(w21=None), dict(affine=None), dict(affine=p + 8), dict(w21=p + 2), dict(out=None), dict(head_dim=16)):
+        assert folded(**bad) == 1, bad
+    assert folded(outer=0) == 0 and folded(inner=0, attn=None) == 0
+
+    def fold(count=1, src=p, folds=1, E=128, mlp=256, w1=p, b1=p, w2=p, b2=p, w21=p, affine=p):
+        one = lambda v: (C.c_void_p * 1)(v)  # noqa: E731
+        return L.sspmm_block_fold_f16(count, one(src), (C.c_int32 * 1)(256), (C.c_int32 * 1)(128), (C.c_int32 * 1)(32), p, folds, E, (C.c_int32 * 1)(mlp),
+                                      one(w1), one(b1), one(w2), one(b2), w21, affine, None)
+
+    for bad in (dict(count=-1), dict(src=None), dict(folds=-1), dict(E=64), dict(E=0), dict(mlp=0), dict(mlp=128), dict(mlp=-256),
+                dict(mlp=(1 << 20) + 256), dict(w1=None), dict(w2=None), dict(w1=p + 2), dict(b1=p + 8), dict(w2=p + 4), dict(w21=None), dict(w21=p + 8),
+                dict(affine=None), dict(affine=p + 4)):
+        assert fold(**bad) == 1, bad
+    assert L.sspmm_block_fold_f16(0, None, None, None, None, None, 0, 256, None, None, None, None, None, None, None, None) == 0
+
     assert L.svc_split_row_ptr(-1, 4, p, p, p, p, None) == 1 and L.svc_split_row_ptr(1, 4, p, None, p, p, None) == 1
     assert L.svc_split_row_ptr(0, 0, None, None, None, None, None) == 0
 
