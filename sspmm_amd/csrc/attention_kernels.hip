@@ -502,13 +502,16 @@ hipError_t launch_softmax(const SoftmaxArgs &a, int V, hipStream_t stream) {
 // The probabilities enter the product rounded to fp16 before the division by the sum (the three launches round
 // after it); sums are fp32 throughout.
 // The launch is bound by the stream of gathered rows from the L2 into the CUs (256 bytes per stored vector and batch
-// element; measured 21 TB/s on 4096 keys, 90 % masked, 48 heads), not by waves in flight: two waves per SIMD with
-// the registers that allows measured 2-7 % faster than three, and four (which spills) 75 % slower.  Column indices
-// fetched in blocks of 64 with one coalesced load and handed out with lane permutes, as the sddmm kernel does, take
-// 11 % of the address unit's work away and cost 10 % in time here (124 -> 137 us): the permutes queue in the LDS pipe
-// behind the stage's writes and reads.  One index per lane of a quad (a 4-byte load) passed round with DPP moves
-// measures the same as the 16-byte load, run against it on one box (128.6 and 128.7 us): it is the 64 bytes a
-// cycle of the cache's data path that bound the launch, not the count of load instructions.
+// element; 22 TB/s on 4096 keys, 90 % masked, once there are rows for every wave).  What it can be given is loads in flight: rows in registers
+// for one step and one stage that k's and v's pass through in turn take 106 registers and 5 KB of LDS a wave, four waves per SIMD, where two
+// sets of rows and two stages (160 registers, two waves) had 20.9 TB/s.  4096 keys, 64 features, 8 / 16 / 32 / 64 (element, head) pairs, V = 8:
+// 27.6 / 49.2 / 90.8 / 167.8 -> 26.0 / 45.6 / 82.2 / 154.5 us, V = 16: 15.1 / 27.8 / 51.0 / 97.3 -> 14.9 / 25.4 / 47.6 / 89.2; one pair, two
+// waves a CU, 9.1 -> 9.6.  32 features (six waves) 19.0 / 33.1 / 60.6 / 112.7 -> 18.3 / 33.8 / 60.7 / 112.4, 128 (two) 46.2 / 84.3 / 156 / 308
+// -> 45.2 / 81.9 / 152 / 302; five waves at 64 features, eight at 32, three at 128 are level or slower, and so are two stages.  Neither what a
+// wave computes nor its column indices count: two heads per wave, which share the indices and the addresses, are level (27.6 -> 29, 106 -> 107), and
+// indices handed out with lane permutes, as the sddmm kernel does, slower (124 -> 137 us: the permutes queue in the LDS pipe).
+// K and V of 256 keys at a time in LDS, every CU fetching all of them for its 64 vector-rows, would read the L2 a seventh as often; it was built and
+// is level at 32 pairs (85-93 us) and slower below (36 us at 8): its waves wait for each other at every panel.
 namespace {
 
 typedef short shortx4 __attribute__((ext_vector_type(4)));
@@ -535,15 +538,16 @@ __device__ __forceinline__ float quad_rows_sum(float x) {
 
 }  // namespace
 
+constexpr int attention_waves(int F) { return F == 64 ? 4 : F == 32 ? 6 : 2; }  // per SIMD
+
 // F: features per row of q, k and v (32, 64 or 128).  A row is F * 2 bytes = LPR 16-byte pieces, a load instruction
 // brings 64 / LPR rows, a step of 32 rows takes L = LPR / 2 of them per operand; lane (jr, pc) fetches piece pc of the
 // rows of k slots L * jr .. L * jr + L - 1, whose column indices it reads as L consecutive ints.
 template <int V, int F>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(F == 32 ? 4 : 2, F == 32 ? 4 : 2))) void sparse_attention_kernel(const AttentionArgs p) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(attention_waves(F), attention_waves(F)))) void sparse_attention_kernel(const AttentionArgs p) {
   constexpr int LPR = F / 8, L = LPR / 2, NC = F / 32, NT = F / 16;
-  constexpr uint32_t kRowBytes = F * 2u, kPitch = kRowBytes + 16u;  // staged rows padded by 16 bytes against bank conflicts
-  __shared__ __align__(16) unsigned char stage_k[32 * kPitch];
-  __shared__ __align__(16) unsigned char stage_v[32 * kPitch];
+  constexpr uint32_t kRowBytes = F * 2u, kPitch = kRowBytes + 32u;  // (sixteen rows' pieces, read four at a time, then touch every bank as often)
+  __shared__ __align__(16) unsigned char stage[32 * kPitch];
   const uint32_t w = xcd_work_index(p.per_xcd);
   if (w >= p.total_work) return;
   const uint32_t r = w % (uint32_t)p.m_vec;
@@ -577,18 +581,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(F == 32 ? 4 
   for (int c = 0; c < NC; ++c)  // (rows past V: beyond the descriptor, zeros)
     q[c] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(srd_q, n < V ? (uint32_t)n * q_row + (32u * c + 8u * g) * 2u : 0xfffffff0u, 0, 0));
 
-  unsigned char *const k_dst = stage_k + (uint32_t)(L * jr) * kPitch + (uint32_t)pc * 16u;
-  unsigned char *const v_dst = stage_v + (uint32_t)(L * jr) * kPitch + (uint32_t)pc * 16u;
-  const unsigned char *const k_rd = stage_k + (uint32_t)n * kPitch + (uint32_t)g * 16u;
-  const unsigned char *const v_rd = stage_v + (uint32_t)(4 * g + (n >> 2)) * kPitch + (uint32_t)(n & 3) * 8u;
+  unsigned char *const dst = stage + (uint32_t)(L * jr) * kPitch + (uint32_t)pc * 16u;
+  const unsigned char *const k_rd = stage + (uint32_t)n * kPitch + (uint32_t)g * 16u;
+  const unsigned char *const v_rd = stage + (uint32_t)(4 * g + (n >> 2)) * kPitch + (uint32_t)(n & 3) * 8u;
   const uint32_t piece_off = (uint32_t)pc * 16u;
   const float scale2 = p.scale * 1.4426950408889634f;
 
   struct Head {
     uint32_t c[L];
-  };
-  struct Body {
-    uintx4 k[L], v[L];
   };
   const auto load_head = [&](int kc) {
     Head h;
@@ -606,25 +606,35 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(F == 32 ? 4 
     }
     return h;
   };
-  const auto load_body = [&](Body &b, const Head &h, int kc) {
-    uint32_t ok[L], ov[L];
+  struct Places {
+    uint32_t k[L], v[L];
+  };
+  const auto places = [&](const Head &h, int kc) {
+    Places o;
 #pragma unroll
     for (int i = 0; i < L; ++i) {
-      ok[i] = __umul24(h.c[i], k_row) + piece_off;  // (both factors below 2^24: the launcher's caller checks the row pitch)
-      ov[i] = __umul24(h.c[i], v_row) + piece_off;
+      o.k[i] = __umul24(h.c[i], k_row) + piece_off;  // (both factors below 2^24: the launcher's caller checks the row pitch)
+      o.v[i] = __umul24(h.c[i], v_row) + piece_off;
     }
     if (kc + 32 > end) {  // (uniform) the row's last step: slots past its end fetch zeros
 #pragma unroll
       for (int i = 0; i < L; ++i) {
         const bool live = kc + L * jr + i < end;
-        ok[i] = live ? ok[i] : k_bytes;
-        ov[i] = live ? ov[i] : v_bytes;
+        o.k[i] = live ? o.k[i] : k_bytes;
+        o.v[i] = live ? o.v[i] : v_bytes;
       }
     }
+    return o;
+  };
+  uintx4 k[L], v[L];
+  const auto fetch = [&](uintx4 (&rows)[L], const __amdgpu_buffer_rsrc_t &srd, const uint32_t (&at)[L]) {
 #pragma unroll
-    for (int i = 0; i < L; ++i) b.k[i] = __builtin_bit_cast(uintx4, __builtin_amdgcn_raw_buffer_load_b128(srd_k, ok[i], 0, 0));
+    for (int i = 0; i < L; ++i) rows[i] = __builtin_bit_cast(uintx4, __builtin_amdgcn_raw_buffer_load_b128(srd, at[i], 0, 0));
+  };
+  // (LDS operations of a wave execute in order: the writes land behind the reads of what the stage held before)
+  const auto put = [&](const uintx4 (&rows)[L]) {
 #pragma unroll
-    for (int i = 0; i < L; ++i) b.v[i] = __builtin_bit_cast(uintx4, __builtin_amdgcn_raw_buffer_load_b128(srd_v, ov[i], 0, 0));
+    for (int i = 0; i < L; ++i) *reinterpret_cast<uintx4 *>(dst + i * kPitch) = rows[i];
   };
 
   floatx4 acc[NT];
@@ -632,13 +642,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(F == 32 ? 4 
   for (int u = 0; u < NT; ++u) acc[u] = floatx4{0.f, 0.f, 0.f, 0.f};
   float run_max = -INFINITY, run_sum = 0.f;  // of query n; the sum only over this lane's share of the keys
 
-  const auto contract = [&](const Body &b, int kc) {
-    // (LDS operations of a wave execute in order: these writes land behind the previous step's reads)
-#pragma unroll
-    for (int i = 0; i < L; ++i) *reinterpret_cast<uintx4 *>(k_dst + i * kPitch) = b.k[i];
-#pragma unroll
-    for (int i = 0; i < L; ++i) *reinterpret_cast<uintx4 *>(v_dst + i * kPitch) = b.v[i];
-    float x[8];
+  float x[8];
+  const auto scores = [&] {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       floatx4 s = {0.f, 0.f, 0.f, 0.f};
@@ -650,6 +655,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(F == 32 ? 4 
 #pragma unroll
       for (int i = 0; i < 4; ++i) x[4 * t + i] = s[i] * scale2;
     }
+  };
+  const auto softmax_and_product = [&](int kc) {
     if (kc + 32 > end) {  // (uniform)
 #pragma unroll
       for (int t = 0; t < 2; ++t)
@@ -685,28 +692,25 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(F == 32 ? 4 
     }
   };
 
-  // Column indices run two steps ahead of the arithmetic, the rows of k and v one (two sets, used alternately).
-  Body b0, b1;
-  Head h0 = load_head(beg), h1 = load_head(beg + 32);
-  load_body(b0, h0, beg);
-  int kc = beg;  // the step held in b0
-  for (;;) {
-    if (kc + 32 >= end) {
-      contract(b0, kc);
-      break;
+  // Column indices run two steps ahead of the arithmetic, the rows of k and v one: a step's rows pass through the stage, k's and then
+  // v's, and the next step's are on their way as soon as the registers are free.
+  const Head now = load_head(beg);
+  Head ahead = load_head(beg + 32);
+  Places at = places(now, beg);
+  fetch(k, srd_k, at.k);
+  fetch(v, srd_v, at.v);
+  for (int kc = beg; kc < end; kc += 32) {
+    put(k);
+    const bool more = kc + 32 < end;
+    if (more) {
+      at = places(ahead, kc + 32);
+      fetch(k, srd_k, at.k);
+      ahead = load_head(kc + 64);
     }
-    h0 = load_head(kc + 64);
-    load_body(b1, h1, kc + 32);
-    contract(b0, kc);
-    kc += 32;
-    if (kc + 32 >= end) {
-      contract(b1, kc);
-      break;
-    }
-    h1 = load_head(kc + 64);
-    load_body(b0, h0, kc + 32);
-    contract(b1, kc);
-    kc += 32;
+    scores();
+    put(v);
+    if (more) fetch(v, srd_v, at.v);
+    softmax_and_product(kc);
   }
 
   const float inv = 1.0f / quad_rows_sum(run_sum);
