@@ -365,6 +365,9 @@ hipError_t launch_add_layernorm_rows(int E, const AddLayerNormRows &p, hipStream
 // registers.  The context goes back through LDS and is written feature-major in whole 128-byte lines.  Bound by
 // HBM in bytes (q, k, v read once, out written once: 8 * hidden * tokens bytes; a head's K and V are re-read by its
 // seq / 64 workgroups from L2), by the exponentials and the LDS reads in time.
+// 8 x 512 tokens, 12 heads, inside the layer: 18.0 -> 17.0 us with the maxima exchanged by lane swaps instead of permutes through the LDS, V's
+// operands read ahead of the exponentials and the sums taken of pairs of rounded probabilities (the error against float64 2.55 - 2.92e-4 ->
+// 2.26 - 2.91e-4).
 typedef uint32_t uintx2 __attribute__((ext_vector_type(2)));
 typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 typedef short shortx4 __attribute__((ext_vector_type(4)));
@@ -395,6 +398,13 @@ __device__ __forceinline__ uintx2 att_read_tr(const unsigned char *p) {
   return __builtin_bit_cast(uintx2, v);
 }
 
+// Maximum over the four lanes n, n + 16, n + 32, n + 48, in each of them.
+__device__ __forceinline__ float att_max4(float x) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
 __device__ __forceinline__ uint32_t att_pack(float lo, float hi) {
   typedef _Float16 half2v __attribute__((ext_vector_type(2)));
   const half2v h = {(_Float16)lo, (_Float16)hi};
@@ -561,6 +571,18 @@ __global__ __launch_bounds__(kAttThreads, 3) void attention_fm_kernel(const Atte
           for (int r = 0; r < 4; ++r)
             if (16 * kt + r >= keys_left) s[0][kt][r] = s[1][kt][r] = -3.0e38f;
       }
+      // V's operands are read ahead of the exponentials (RAGGED, whose products take more registers, reads them where it uses them)
+      AttOperand vops[4];
+      const auto read_v = [&](int dt) {
+        const unsigned char *a = v_tile + v_rd + (16 * dt) * kAttPitchV;
+        const uintx2 lo = *reinterpret_cast<const uintx2 *>(a), hi = *reinterpret_cast<const uintx2 *>(a + 32);
+        vops[dt].u[0] = lo[0]; vops[dt].u[1] = lo[1]; vops[dt].u[2] = hi[0]; vops[dt].u[3] = hi[1];
+      };
+      if constexpr (!RAGGED) {
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) read_v(dt);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       AttOperand rest[2];  // (RAGGED) what the rounding of the probabilities leaves
       AttOperand pop[2];  // per set: contraction slots 0-3 = keys 4g .. + 3 of tile 0, slots 4-7 = the same keys of tile 1
 #pragma unroll
@@ -570,8 +592,12 @@ __global__ __launch_bounds__(kAttThreads, 3) void attention_fm_kernel(const Atte
         for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
           for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[j][kt][r]);
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        if constexpr (RAGGED) {  // (25.9 us at 8 x 500 tokens, 26.2 with the lane swaps)
+          mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+          mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        } else {
+          mx = att_max4(mx);
+        }
         // The reference point of the exponentials moves only when some query's maximum has grown by more than 8 in
         // the base-2 domain (a wave-uniform decision): until then the probabilities are at most 2^8 times too large,
         // which fp16 holds, the running sums and the context stay consistent with the old reference point, and the
@@ -592,13 +618,20 @@ __global__ __launch_bounds__(kAttThreads, 3) void attention_fm_kernel(const Atte
           for (int r = 0; r < 4; ++r) {
             s[j][kt][r] = __builtin_amdgcn_exp2f(fmaf(s[j][kt][r], c, shift));
             if (cut && 16 * kt + r >= keys_left) s[j][kt][r] = 0.f;  // (a wave may have had no key at all yet)
-            part += s[j][kt][r];
+            if (RAGGED) part += s[j][kt][r];
           }
         run_sum[j] += part;
         pop[j].u[0] = att_pack(s[j][0][0], s[j][0][1]);
         pop[j].u[1] = att_pack(s[j][0][2], s[j][0][3]);
         pop[j].u[2] = att_pack(s[j][1][0], s[j][1][1]);
         pop[j].u[3] = att_pack(s[j][1][2], s[j][1][3]);
+        if constexpr (!RAGGED) {
+          // the sum of what the product takes: the rounding of the largest probabilities cancels in the quotient
+          typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+          const half2v ones = {(_Float16)1, (_Float16)1};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) run_sum[j] = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2v, pop[j].u[i]), ones, run_sum[j], false);
+        }
         if constexpr (RAGGED) {
 #pragma unroll
           for (int i = 0; i < 8; ++i) rest[j].h[i] = (_Float16)(s[j][i >> 2][i & 3] - (float)pop[j].h[i]);
@@ -606,10 +639,8 @@ __global__ __launch_bounds__(kAttThreads, 3) void attention_fm_kernel(const Atte
       }
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt) {
-        const unsigned char *a = v_tile + v_rd + (16 * dt) * kAttPitchV;
-        const uintx2 lo = *reinterpret_cast<const uintx2 *>(a), hi = *reinterpret_cast<const uintx2 *>(a + 32);
-        AttOperand vop;
-        vop.u[0] = lo[0]; vop.u[1] = lo[1]; vop.u[2] = hi[0]; vop.u[3] = hi[1];
+        if (RAGGED) read_v(dt);
+        const AttOperand vop = vops[dt];
         half8 vrest = vop.h;
         if (RAGGED && __builtin_expect(bounded, 0)) vrest = att_bounded(vrest);
 #pragma unroll
