@@ -505,8 +505,8 @@ hipError_t launch_softmax(const SoftmaxArgs &a, int V, hipStream_t stream) {
 // element; 22 TB/s on 4096 keys, 90 % masked, once there are rows for every wave).  What it can be given is loads in flight: rows in registers
 // for one step and one stage that k's and v's pass through in turn take 106 registers and 5 KB of LDS a wave, four waves per SIMD, where two
 // sets of rows and two stages (160 registers, two waves) had 20.9 TB/s.  4096 keys, 64 features, 8 / 16 / 32 / 64 (element, head) pairs, V = 8:
-// 27.6 / 49.2 / 90.8 / 167.8 -> 26.0 / 45.6 / 82.2 / 154.5 us, V = 16: 15.1 / 27.8 / 51.0 / 97.3 -> 14.9 / 25.4 / 47.6 / 89.2; one pair, two
-// waves a CU, 9.1 -> 9.6.  32 features (six waves) 19.0 / 33.1 / 60.6 / 112.7 -> 18.3 / 33.8 / 60.7 / 112.4, 128 (two) 46.2 / 84.3 / 156 / 308
+// 27.6 / 49.2 / 90.8 / 167.8 -> 25.5 / 44.9 / 82.3 / 153.6 us, V = 16: 15.1 / 27.8 / 51.0 / 97.3 -> 14.7 / 25.8 / 46.0 / 88.1; one pair, two
+// waves a CU, 9.1 -> 9.3 (9.6 with the scores scaled before their maximum and the sums taken in fp32: twelve instructions a step more).  32 features (six waves) 19.0 / 33.1 / 60.6 / 112.7 -> 18.3 / 33.8 / 60.7 / 112.4, 128 (two) 46.2 / 84.3 / 156 / 308
 // -> 45.2 / 81.9 / 152 / 302; five waves at 64 features, eight at 32, three at 128 are level or slower, and so are two stages.  Neither what a
 // wave computes nor its column indices count: two heads per wave, which share the indices and the addresses, are level (27.6 -> 29, 106 -> 107), and
 // indices handed out with lane permutes, as the sddmm kernel does, slower (124 -> 137 us: the permutes queue in the LDS pipe).
@@ -653,7 +653,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(attention_wa
         s = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, q[c], s, 0, 0, 0);
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) x[4 * t + i] = s[i] * scale2;
+      for (int i = 0; i < 4; ++i) x[4 * t + i] = s[i];
     }
   };
   const auto softmax_and_product = [&](int kc) {
@@ -665,7 +665,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(attention_wa
           if (kc + 16 * t + 4 * g + i >= end) x[4 * t + i] = -INFINITY;
     }
     float mx = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
-    mx = quad_rows_max(mx);  // finite: the step's first slot is always a stored vector
+    mx = quad_rows_max(mx) * scale2;  // finite: the step's first slot is always a stored vector
     const float new_max = fmaxf(run_max, mx);
     if (__builtin_amdgcn_ballot_w64(new_max > run_max)) {  // (uniform) some query's maximum moved
       const float alpha = __builtin_amdgcn_exp2f(run_max - new_max);
@@ -674,15 +674,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(attention_wa
       for (int u = 0; u < NT; ++u) acc[u] *= alpha;
       run_max = new_max;
     }
-    float e[8], sum = 0.f;
+    half8 pb;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      e[i] = __builtin_amdgcn_exp2f(x[i] - run_max);
-      sum += e[i];
+    for (int i = 0; i < 8; ++i) pb[i] = (_Float16)__builtin_amdgcn_exp2f(__builtin_fmaf(x[i], scale2, -run_max));
+    // (the sum of what the product takes: the rounding of the largest probabilities cancels in the quotient)
+    const uintx4 pairs = __builtin_bit_cast(uintx4, pb);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+      const half2v ones = {(_Float16)1, (_Float16)1};
+      run_sum = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2v, (uint32_t)pairs[i]), ones, run_sum, false);
     }
-    run_sum += sum;
-    const half8 pb = {(_Float16)e[0], (_Float16)e[1], (_Float16)e[2], (_Float16)e[3],
-                      (_Float16)e[4], (_Float16)e[5], (_Float16)e[6], (_Float16)e[7]};
 #pragma unroll
     for (int u = 0; u < NT; ++u) {
       const uintx2 lo = lds_read_tr(v_rd + 32u * u);
