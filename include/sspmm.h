@@ -443,6 +443,17 @@ int sspmm_block_dense_f16(int outer, int inner, int E, const sspmm_half_t *x, in
                           sspmm_half_t *out, void *hip_stream);
 
 /*
+ * sspmm_block_dense_f16 without attn, on an embedding that has not been looked up: row (i, j) of x is row
+ * tokens[i * token_outer + j * token_inner] of table [vocab, E] (4- or 8-byte integers, 0 <= token < vocab; a token outside
+ * is a row of NaN), fp16(x * x_scale) + pos[i] stands in its place.
+ */
+int sspmm_block_embed_f16(int outer, int inner, int E, const void *tokens, int token_bytes, int64_t token_outer,
+                          int64_t token_inner, const sspmm_half_t *table, int64_t vocab, const sspmm_half_t *pos,
+                          float x_scale, const sspmm_half_t *gamma_n, const sspmm_half_t *beta_n, float eps_n, int n_out,
+                          int head_dim, const sspmm_half_t *wt, const sspmm_half_t *bt, sspmm_half_t *x_out,
+                          sspmm_half_t *out, void *hip_stream);
+
+/*
  * Weight matrices [rows, cols] (row-major, 16-byte aligned) into the order in which sspmm_block_dense_f16 loads them,
  * one after the other into dst: the same elements, fragment by fragment of a matrix instruction.  group[i] =
  * 32, 64 or 128 rows belong to one wave; rows[i] a multiple of it, cols[i] of 64.  The four arrays are host

@@ -53,6 +53,7 @@ SIGNATURES = {
     "sspmm_block_pack_f16": (_int, [_int, _vp, _vp, _vp, _vp, _vp, _vp]),
     "sspmm_block_dense_f16": (_int, [_int, _int, _int, _vp, _i64, _i64, _vp, ctypes.c_float, _vp, _vp, _vp, _vp, _vp, ctypes.c_float, _int, _vp, _vp, _vp, _vp,
                                      _vp, _vp, ctypes.c_float, _int, _int, _vp, _vp, _vp, _vp, _vp]),
+    "sspmm_block_embed_f16": (_int, [_int, _int, _int, _vp, _int, _i64, _i64, _vp, _i64, _vp, ctypes.c_float, _vp, _vp, ctypes.c_float, _int, _int] + [_vp] * 5),
     "sspmm_block_fold_f16": (_int, [_int, _vp, _vp, _vp, _vp, _vp, _int, _int] + [_vp] * 8),
     "sspmm_block_dense_folded_f16": (_int, [_int, _int, _int, _vp, _i64, _i64] + [_vp] * 5 + [ctypes.c_float] + [_vp] * 4 + [ctypes.c_float, _int, _int] +
                                      [_vp] * 5),

@@ -247,7 +247,7 @@ def fold_blocks(blocks, linears, rows_per_wave):
     return parts[:n], list(zip(parts[n:], affine))
 
 
-def block_dense(x, attn, block, norm, tail=None, keep_x=False, packed=None, head_dim=0, pos=None, scale=1.0, folded=None):
+def block_dense(x, attn, block, norm, tail=None, keep_x=False, packed=None, head_dim=0, pos=None, scale=1.0, folded=None, table=None):
     """(x', out): everything between the attention of `block` and the next one's in one launch, on token-major activations
     [seq, batch, embed] fp16:
         s = out_proj(attn) + x, x' = linear2(linear1(layer_norm2(s))) + x, h = norm(x'), out = tail(h) or h itself.
@@ -256,13 +256,21 @@ def block_dense(x, attn, block, norm, tail=None, keep_x=False, packed=None, head
     linear2 (where there is attn) and tail (where there is one), in this order.  head_dim: out as
     [tail.out_features / embed, batch, embed / head_dim, seq, head_dim], for sparse_attention_split.  pos
     [seq, embed]: x is an embedding, and (x * scale) + pos stands in its place, each rounded to fp16.  folded: linear1 and linear2 as
-    fold_blocks leaves them (with attn, without pos), packed then that of out_proj and tail."""
-    outer, inner, E = x.shape
+    fold_blocks leaves them (with attn, without pos), packed then that of out_proj and tail.  table (without attn, with pos): x are
+    tokens [batch, seq], and the embedding is read from the table's rows."""
+    outer, inner, E = x.shape if table is None else (x.size(1), x.size(0), table.size(1))
     n_out = 0 if tail is None else tail.out_features
     shape = (n_out // E, inner, E // head_dim, outer, head_dim) if head_dim else (outer, inner, n_out or E)
     out = torch.empty(shape, dtype=torch.float16, device=x.device)
     kept = torch.empty((outer, inner, E), dtype=torch.float16, device=x.device) if keep_x else None
     stride = x.stride()
+    if table is not None:
+        gamma_n, beta_n = _weights(norm)
+        rc = _lib.call(_lib.lib().sspmm_block_embed_f16, x.device, outer, inner, E, x.data_ptr(), x.element_size(), stride[1], stride[0], table.data_ptr(),
+                       table.size(0), pos.data_ptr(), float(scale), _ptr(gamma_n), _ptr(beta_n), float(norm.eps), n_out, head_dim, packed[-1].data_ptr(),
+                       _ptr(_weights(tail)[1]), _ptr(kept), out.data_ptr())
+        _lib.check(rc, "sspmm_block_embed_f16")
+        return kept, out
     if packed is None:
         own = [] if attn is None else [block.out_proj, block.linear1, block.linear2]
         if own or tail is not None:
@@ -470,11 +478,18 @@ class SparseAttentionEncoder(torch.nn.Module):
 
     def forward(self, tokens, dense_masks=None):
         """tokens: int [batch, seq] -> [seq, batch, num_class]."""
-        out, scale = self.encoder(tokens), self.embed_dim ** 0.5
+        scale = self.embed_dim ** 0.5
+        if dense_masks is None:
+            table = self._table(tokens)
+            if table is not None:
+                (batch, seq), pe = tokens.shape, self._positions(tokens.size(1), table)
+                if pe is not None and _eager_inference() and self._norms_apply(table) and self._blocks_apply(table, seq, batch):
+                    return self._fused_blocks(tokens, pe, scale, table)
+        out = self.encoder(tokens)
         if dense_masks is None and out.dim() == 3:
-            x, pe = out.transpose(0, 1), self.pe[:tokens.size(1)].to(out.dtype)
-            if pe.shape == (x.size(0), 1, x.size(2)) and _rows_operand(pe) and pe.is_contiguous() and pe.device == x.device and \
-                    self._fused_norms_apply(x) and self._fused_blocks_apply(x):
+            x = out.transpose(0, 1)
+            pe = self._positions(tokens.size(1), x)
+            if pe is not None and self._fused_norms_apply(x) and self._blocks_apply(x, x.size(0), x.size(1)):
                 return self._fused_blocks(x, pe, scale)
         out = out * scale
         out = out.transpose(0, 1) + self.pe[:tokens.size(1)].to(out.dtype)
@@ -484,10 +499,28 @@ class SparseAttentionEncoder(torch.nn.Module):
             out = blk(out, None if dense_masks is None else dense_masks[i])
         return self.linear(self.layer_norm(out))
 
-    def _fused_norms_apply(self, x):
-        return (len(self.blocks) > 0 and _rows_operand(x) and _eager_inference() and _rows_norm_applies(self.layer_norm, x) and
+    def _table(self, tokens):
+        """The embedding's weight, where a kernel may look the tokens' rows up in it; None otherwise."""
+        encoder, = _parts(self, "encoder")
+        if not (type(tokens) is torch.Tensor and tokens.is_cuda and tokens.dim() == 2 and tokens.numel() > 0 and
+                tokens.dtype in (torch.int64, torch.int32) and _plain_module(encoder, torch.nn.Embedding) and encoder.max_norm is None):
+            return None
+        weight = encoder._parameters.get("weight")
+        shape = (encoder.num_embeddings, self.embed_dim)
+        return weight if weight is not None and shape[0] > 0 and _operand(weight, tokens.get_device(), shape) else None
+
+    def _positions(self, seq, like):
+        """The first rows of pe as a kernel reads them next to `like`, or None."""
+        pe = self.pe[:seq].to(like.dtype)
+        return pe if pe.shape == (seq, 1, like.size(-1)) and _rows_operand(pe) and pe.is_contiguous() and pe.device == like.device else None
+
+    def _norms_apply(self, x):
+        return (len(self.blocks) > 0 and _rows_norm_applies(_parts(self, "layer_norm")[0], x) and
                 all(_plain_module(b, SparseAttentionBlock) and "attention" not in b.__dict__ and
                     all([_rows_norm_applies(n, x) for n in _parts(b, "layer_norm1", "layer_norm2")]) for b in self.blocks))
+
+    def _fused_norms_apply(self, x):
+        return _rows_operand(x) and _eager_inference() and self._norms_apply(x)
 
     def _blocks_with_fused_norms(self, x):
         """The blocks and the final LayerNorm with every residual sum in the launch of the LayerNorm behind it, also
@@ -506,10 +539,10 @@ class SparseAttentionEncoder(torch.nn.Module):
             x, h = add_norm(x, y, self.layer_norm if last else self.blocks[i + 1].layer_norm1, keep_sum=not last)
         return h
 
-    def _fused_blocks_apply(self, x):
+    def _blocks_apply(self, x, seq, bsz):
         """(where the fused norms do) heads that one launch of attention takes, and products that block_dense does and is
-        ahead with (see BLOCK_WEIGHTS)"""
-        seq, bsz, E = x.shape
+        ahead with (see BLOCK_WEIGHTS).  x: an operand on the device, of the blocks' width."""
+        E = x.size(-1)
         if not (E in BLOCK_WIDTHS and packed_attention_fits(seq, bsz, 3 * E)):
             return False
         for b in self.blocks:
@@ -521,11 +554,13 @@ class SparseAttentionEncoder(torch.nn.Module):
                 return False
         return True
 
-    def _fused_blocks(self, x, pe, scale):
-        """(x * scale) + pe through the blocks and the head.  Two launches per block: its attention, and all that follows up to the next block's projection (or the head)."""
-        E, blocks = x.size(-1), list(self.blocks)
+    def _fused_blocks(self, x, pe, scale, table=None):
+        """(x * scale) + pe through the blocks and the head (x: an embedding, or with table the tokens to look up in it).  Two launches per
+        block: its attention, and all that follows up to the next block's projection (or the head)."""
+        like = x if table is None else table
+        E, blocks = like.size(-1), list(self.blocks)
         final, linear = _parts(self, "layer_norm", "linear")
-        head = _plain_linear(linear, x, E, None, 64) and E * linear.out_features <= BLOCK_WEIGHTS
+        head = _plain_linear(linear, like, E, None, 64) and E * linear.out_features <= BLOCK_WEIGHTS
         into, norms = [_parts(b, "in_proj")[0] for b in blocks], [_parts(b, "layer_norm1")[0] for b in blocks]
         linears, rows = [into[0]], [64]
         for i, blk in enumerate(blocks):
@@ -539,7 +574,8 @@ class SparseAttentionEncoder(torch.nn.Module):
             offsets, columns = _pattern(blk)
             return sparse_attention_split(None, offsets, columns, qkv, float(qkv.size(-1)) ** -0.5, blk.vec_length)
 
-        x, qkv = block_dense(x, None, None, norms[0], into[0], True, packed[:1], E // blocks[0].num_heads, pe, scale)
+        x, qkv = block_dense(x, None, None, norms[0], into[0], True, packed[:1], E // blocks[0].num_heads, pe, scale,
+                             table=table)
         for i, blk in enumerate(blocks[:-1]):
             x, qkv = block_dense(x, attention(blk, qkv), blk, norms[i + 1], into[i + 1], True, packed[1 + 2 * i:3 + 2 * i],
                                  E // blocks[i + 1].num_heads, folded=folded[i])

@@ -20,6 +20,9 @@ struct BlockDenseArgs {
   long long x_outer, x_inner;
   const uint16_t *pos;                       // nullable: x is an embedding, fp16(x * x_scale) + pos[token / inner] in its place
   float x_scale;
+  const void *ids;                           // nullable (without attn, with pos): row i of x is row ids[(i / inner) * x_outer + (i % inner) * x_inner]
+  int wide_ids;                              // of `vocab` rows at x, NaN where there is none; int64 instead of int32
+  long long vocab;
   const uint16_t *attn;                      // nullable, and the next two lines with it
   const uint16_t *wo, *bo, *gamma2, *beta2;
   const uint16_t *w1, *b1, *w2, *b2;

@@ -22,6 +22,10 @@
 // multiplies them takes 12.9 us a pass for four blocks, where packing all took 7.6.  (Both layers, for callers that bring them packed:
 // the rest of this paragraph.)
 //
+// The launch in front of the first block looks the tokens up in the embedding's table itself: as a launch of its own the lookup wrote
+// and this one read tokens x E halfs that no one else wants (256 features, four blocks: 8192 tokens 194 -> 180 us the forward pass,
+// 32768 tokens 546 -> 507).
+//
 // The weights a workgroup streams from L2 are 1.6 MB at 256 features and 1024 hidden ones, 25k cycles at the 64 bytes a
 // cycle of a CU, whatever TM, and the products 384 cycles per token.  The loads of the next two units (eight 16-byte
 // loads of a wave each) are in flight throughout, also across the products' boundaries; four units, at 64 registers more, were
@@ -268,7 +272,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
 #pragma unroll
     for (int t = 0; t < TT; ++t) {
       const uint32_t r = r0 + (uint32_t)min(t * 16 + m, left - 1), q = r / (uint32_t)p.inner;
-      load_row<NT>(x[t], p.x + (q0 + q) * p.x_outer + (long long)(r - q * (uint32_t)p.inner) * p.x_inner + first);
+      const long long at = (q0 + q) * p.x_outer + (long long)(r - q * (uint32_t)p.inner) * p.x_inner;
+      if (PART == kNoAttention && p.ids) {  // (uniform)
+        const long long id = p.wide_ids ? static_cast<const long long *>(p.ids)[at] : static_cast<const int *>(p.ids)[at];
+        const bool there = id >= 0 && id < p.vocab;
+        load_row<NT>(x[t], p.x + (there ? id : 0) * E + first);
+        if (!there) {
+#pragma unroll
+          for (int j = 0; j < NT / 2; ++j)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) x[t][j][i] = (_Float16)__builtin_nanf("");
+        }
+      } else {
+        load_row<NT>(x[t], p.x + at + first);
+      }
       if (p.pos) {  // (uniform) fp16(x * scale) + pos, rounded as an activation in between
         half8 at[NT / 2];
         load_row<NT>(at, p.pos + (q0 + q) * E + first);

@@ -652,6 +652,7 @@ static int block_dense(int outer, int inner, int E, const sspmm_half_t *x, int64
   p.eps_n = eps_n;
   p.mlp = attn ? mlp : 0;
   p.affine = affine;
+  p.ids = nullptr;
   p.n_out = n_out;
   p.head_dim = head_dim;
   p.x_out = x_out;
@@ -677,6 +678,44 @@ int sspmm_block_dense_folded_f16(int outer, int inner, int E, const sspmm_half_t
   if (outer > 0 && inner > 0 && (!attn || !affine)) return kInvalid;
   return block_dense(outer, inner, E, x, x_outer, x_inner, nullptr, 1.f, attn, wo, bo, gamma2, beta2, eps2, 0, nullptr, nullptr, w21, nullptr, affine,
                      gamma_n, beta_n, eps_n, n_out, head_dim, wt, bt, x_out, out, hip_stream);
+}
+
+int sspmm_block_embed_f16(int outer, int inner, int E, const void *tokens, int token_bytes, int64_t token_outer, int64_t token_inner,
+                          const sspmm_half_t *table, int64_t vocab, const sspmm_half_t *pos, float x_scale, const sspmm_half_t *gamma_n,
+                          const sspmm_half_t *beta_n, float eps_n, int n_out, int head_dim, const sspmm_half_t *wt, const sspmm_half_t *bt,
+                          sspmm_half_t *x_out, sspmm_half_t *out, void *hip_stream) {
+  if (outer < 0 || inner < 0 || !sspmm::block_dense_applies(E, 256, n_out)) return kInvalid;
+  if (outer == 0 || inner == 0) return 0;
+  if (!tokens || !table || !pos || !out || (token_bytes != 4 && token_bytes != 8) || reinterpret_cast<uintptr_t>(tokens) % (uintptr_t)token_bytes ||
+      token_outer < 0 || token_inner < 0 || vocab < 1 || (wt != nullptr) != (n_out > 0))
+    return kInvalid;
+  if (head_dim != 0 && ((head_dim != 32 && head_dim != 64 && head_dim != 128) || n_out % E)) return kInvalid;
+  uintptr_t bits = 0;
+  for (const sspmm_half_t *q : {table, pos, gamma_n, beta_n, wt, bt, (const sspmm_half_t *)x_out, (const sspmm_half_t *)out})
+    bits |= reinterpret_cast<uintptr_t>(q);
+  if (bits % 16) return kInvalid;
+  sspmm::BlockDenseArgs p{};
+  p.ids = tokens;
+  p.wide_ids = token_bytes == 8;
+  p.vocab = vocab;
+  p.tokens = (long long)outer * inner;
+  p.inner = inner;
+  p.x = table;
+  p.x_outer = token_outer;
+  p.x_inner = token_inner;
+  p.pos = pos;
+  p.x_scale = x_scale;
+  p.gamma_n = gamma_n;
+  p.beta_n = beta_n;
+  p.wt = wt;
+  p.bt = bt;
+  p.eps_n = eps_n;
+  p.n_out = n_out;
+  p.head_dim = head_dim;
+  p.x_out = x_out;
+  p.norm_out = wt ? nullptr : out;
+  p.out = out;
+  return (int)sspmm::launch_block_dense(E, p, static_cast<hipStream_t>(hip_stream));
 }
 
 int sspmm_attention_fm_f16(int batch, int heads, int seq, int head_dim, const sspmm_half_t *q, const sspmm_half_t *k,

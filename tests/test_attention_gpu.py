@@ -631,6 +631,61 @@ def test_block_dense_on_one_matrix_for_two_layers(built_library, E, mlp, n_out, 
                         assert torch.equal(split, got.view(outer, inner, n_out // E, E // d, d).permute(2, 1, 3, 0, 4))
 
 
+@pytest.mark.parametrize("E,outer,inner", [(128, 5, 1), (128, 1367, 3), (256, 37, 3), (256, 1400, 3), (512, 2731, 3), (512, 19, 2)])
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+def test_block_dense_looks_tokens_up(built_library, E, outer, inner, dtype):
+    """The rows of a table in the place of the embedding, for every width and tile of tokens: the same bits, whatever the tokens'
+    strides; a token that is no row of the table makes a row of NaN and leaves the others alone."""
+    from sspmm_amd.attention import block_dense, pack_weights
+    g = torch.Generator("cuda").manual_seed(E + outer)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g).half()  # noqa: E731
+    norm, tail = torch.nn.LayerNorm(E).cuda().half(), torch.nn.Linear(E, 3 * E).cuda().half()
+    table, pos = rnd(50, E), rnd(outer, 1, E)
+    wide = torch.randint(0, 50, (2 * inner, 3 * outer), device="cuda", generator=g).to(dtype)
+    with torch.no_grad():
+        packed = pack_weights([tail], [64])
+        for tokens in (wide[:inner, :outer].contiguous(), wide[::2, ::3], wide[:inner, :outer].t().contiguous().t()):
+            assert tokens.shape == (inner, outer)
+            x = table[tokens.long()].transpose(0, 1)
+            for d in (0, 32):
+                want = block_dense(x, None, None, norm, tail, True, packed, d, pos, 11.3)
+                got = block_dense(tokens, None, None, norm, tail, True, packed, d, pos, 11.3, table=table)
+                assert torch.equal(want[0], got[0]) and torch.equal(want[1], got[1])
+        tokens = wide[:inner, :outer].contiguous()
+        tokens[0, 1], tokens[inner - 1, 0] = 50, -1
+        kept, out = block_dense(tokens, None, None, norm, tail, True, packed, 0, pos, 11.3, table=table)
+    lost = ((tokens < 0) | (tokens >= 50)).t()
+    assert torch.equal(kept.isnan().all(-1), lost) and torch.equal(out.isnan().any(-1), lost)
+
+
+def test_encoder_looks_tokens_up_in_its_first_launch(built_library):
+    """Tokens of either type and any strides give the bits of the embedding called as a module, which a hook on it, a limit on the
+    rows' norm and tokens that a kernel does not read get."""
+    from sspmm_amd import attention as A
+    model = A.SparseAttentionEncoder(50, 128, 4, 0.9, 96, 256, 64, vec_length=8, layers=2, seed=2).cuda().half().eval()
+    tokens = torch.randint(0, 50, (3, 96), device="cuda", generator=torch.Generator("cuda").manual_seed(1))
+    tables, plain = [], A.block_dense
+    A.block_dense = lambda *args, **kw: (tables.append(kw.get("table")), plain(*args, **kw))[1]
+    try:
+        with torch.no_grad():
+            got = [model(t) for t in (tokens, tokens.int(), tokens.t().contiguous().t(), torch.stack([tokens, tokens], -1)[..., 1])]
+            assert len(tables) == 12 and all((t is model.encoder.weight) == (i % 3 == 0) for i, t in enumerate(tables))
+            del tables[:]
+            seen = []
+            handle = model.encoder.register_forward_hook(lambda m, i, o: seen.append(1))
+            want = model(tokens)
+            handle.remove()
+            assert seen and all(torch.equal(want, t) for t in got)
+            model.encoder.max_norm = 1e4
+            assert torch.equal(model(tokens), want)
+            model.encoder.max_norm = None
+            assert len(tables) == 6 and all(t is None for t in tables)
+            with pytest.raises(RuntimeError):
+                model(tokens.short())
+    finally:
+        A.block_dense = plain
+
+
 @pytest.mark.parametrize("embed,heads,mlp,V", [(128, 4, 512, 8), (256, 8, 1024, 16), (512, 8, 512, 8), (192, 6, 512, 8), (1024, 16, 512, 16)])
 def test_encoder_against_float64(built_library, embed, heads, mlp, V):
     """The whole model on each of its routes (two launches a block, fused norms, and for 192 features the modules) against dense

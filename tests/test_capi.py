@@ -130,6 +130,16 @@ def test_argument_errors_of_the_dense_block_entries(built_library):
         assert folded(**bad) == 1, bad
     assert folded(outer=0) == 0 and folded(inner=0, attn=None) == 0
 
+    def embed(outer=2, inner=3, E=128, tokens=p, size=8, t_outer=1, t_inner=2, table=p, vocab=7, pos=p, n_out=128, head_dim=0, wt=p, bt=p, x_out=p, out=p):
+        return L.sspmm_block_embed_f16(outer, inner, E, tokens, size, t_outer, t_inner, table, vocab, pos, 1.0, p, p, 1e-5, n_out, head_dim, wt, bt,
+                                       x_out, out, None)
+
+    for bad in (dict(outer=-1), dict(inner=-1), dict(E=64), dict(tokens=None), dict(tokens=p + 4), dict(tokens=p + 2, size=4), dict(size=2),
+                dict(t_outer=-1), dict(t_inner=-2), dict(table=None), dict(table=p + 8), dict(vocab=0), dict(pos=None), dict(pos=p + 2), dict(n_out=96),
+                dict(n_out=0), dict(wt=None), dict(head_dim=48), dict(bt=p + 8), dict(x_out=p + 4), dict(out=None)):
+        assert embed(**bad) == 1, bad
+    assert embed(outer=0) == 0 and embed(inner=0, tokens=None) == 0
+
     def fold(count=1, src=p, folds=1, E=128, mlp=256, w1=p, b1=p, w2=p, b2=p, w21=p, affine=p):
         one = lambda v: (C.c_void_p * 1)(v)  # noqa: E731
         return L.sspmm_block_fold_f16(count, one(src), (C.c_int32 * 1)(256), (C.c_int32 * 1)(128), (C.c_int32 * 1)(32), p, folds, E, (C.c_int32 * 1)(mlp),
