@@ -174,36 +174,48 @@ __device__ __forceinline__ uintx2 lds_read_tr(const unsigned char *lds_base, uin
   return __builtin_bit_cast(uintx2, v);
 }
 
+// The 32 x V halfs of a step, spread over the 64 lanes.  The address unit passes a load of 16 or of 8 bytes a lane on in sixteen cycles,
+// however many of its lanes take part (6.8 and 7.2 ns a wave and CU from the first-level cache), one of 4 bytes in four or five (2.2): the 512 bytes of V = 8
+// come in two loads of 4 bytes a lane, the 1 KB of V = 16 in one of 16.  2048 x 512 at 90 %, N = 256, batch 128, fp32 C 54.6 -> 53.1 us; the staged kernel,
+// 16 x 2000 x 2000 at 90 %, N = 64 9.13 -> 8.78.
 template <int V>
-struct SlabVals;  // the 32 x V halfs of a step, spread over the 64 lanes
+struct SlabVals;
 template <>
 struct SlabVals<8> {
-  typedef uintx2 type;  // 8 bytes per lane
+  struct type {
+    uint32_t lo, hi;  // 4 bytes of the first 256 and of the second
+  };
+  static constexpr uint32_t kLane = 4u;
   static __device__ __forceinline__ type load(__amdgpu_buffer_rsrc_t srd, uint32_t off) {
-    return __builtin_bit_cast(uintx2, __builtin_amdgcn_raw_buffer_load_b64(srd, off, 0, 0));
+    return {(uint32_t)__builtin_amdgcn_raw_buffer_load_b32(srd, off, 0, 0), (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(srd, off + 256u, 0, 0)};
+  }
+  static __device__ __forceinline__ void put(unsigned char *tile_lane, const type &v) {
+    reinterpret_cast<uint32_t *>(tile_lane)[0] = v.lo;
+    reinterpret_cast<uint32_t *>(tile_lane)[64] = v.hi;
   }
 };
 template <>
 struct SlabVals<16> {
   typedef uintx4 type;  // 16 bytes per lane
+  static constexpr uint32_t kLane = 16u;
   static __device__ __forceinline__ type load(__amdgpu_buffer_rsrc_t srd, uint32_t off) {
     return __builtin_bit_cast(uintx4, __builtin_amdgcn_raw_buffer_load_b128(srd, off, 0, 0));
   }
+  static __device__ __forceinline__ void put(unsigned char *tile_lane, const type &v) { *reinterpret_cast<type *>(tile_lane) = v; }
 };
 
 // One chunk = 32 consecutive non-zero vectors of a vector-row.  Its loads form a chain of two
 // memory round trips (column indices, then the rows of B they name), so they are issued in two
 // stages, one step apart: while chunk s is contracted, the gathers of chunk s + 1 and the column
 // indices of chunk s + 2 are in flight.
-// SHARED_COLS: the column indices come as one dword per lane and the lanes that need one fetch it from there with a
-// lane permute (the address unit takes sixteen cycles for a load instruction of a wave whatever it carries: the
-// eight indices a lane needs, loaded by the lane itself, cost two of them).  Pays where that unit bounds the kernel
-// (one wave per vector-row, many in flight); where a single long row is the critical path (the split-row kernel)
-// the permutes' latency costs more than the instruction saves.
-template <int V, bool SHARED_COLS = true>
+// The eight lanes that start a group of sixteen load an index each of the eight that the group needs (the others the same
+// ones: one load of 4 bytes a lane), and the group hands their rows' offsets round in the additions of the lanes' own (DPP).  A lane permute
+// per index instead keeps the LDS busy, two loads of 16 bytes a lane the address unit: permutes / this, V = 8, 2048 x 1024 at 80 %, N = 1024
+// 7.85 / 7.41 us, 768 x 3072 at 70 %, N = 2048, fp16 18.0 / 17.1, 1024 x 1152 at 90 %, N = 1225 6.88 / 6.77; V = 16, 2304 x 768 at 90 %,
+// N = 4096, fp16 8.05 / 7.77, 1024 x 2304 at 80 %, N = 3136 13.0 / 12.8; loads / this, in the split-row kernel, 3072 x 4608 at 98 %, N = 4096 14.9 / 14.4.
+template <int V>
 struct ChunkHead {   // stage 1: what does not depend on other loads
-  uint32_t cols;     // SHARED_COLS: column index of k slot lane % 32
-  uintx4 c0, c1;     // otherwise: column indices of k slots 8g .. 8g+7
+  uint32_t cols;     // column index of k slot 8 (lane / 16) + lane % 8
   typename SlabVals<V>::type vraw;  // the lane's share of the chunk's 32 x V values, as they lie in memory
   int kc;            // first vector of the chunk
 };
@@ -230,35 +242,31 @@ struct Chunk {
   typename ChunkRaw<CPL>::type raw[8];  // raw[j] = CPL halfs (columns n0+CPL*m..) of the row of B named by k slot 8g+j
 };
 
-template <int V, bool SHARED_COLS>
-__device__ __forceinline__ void load_head(ChunkHead<V, SHARED_COLS> &h, int kc, int g, __amdgpu_buffer_rsrc_t srd_cols,
+template <int V>
+__device__ __forceinline__ void load_head(ChunkHead<V> &h, int kc, int g, __amdgpu_buffer_rsrc_t srd_cols,
                                           __amdgpu_buffer_rsrc_t srd_vals, uint32_t vals_lane_off) {
   h.kc = kc;
   // srd_cols / srd_vals end at this vector-row's last vector: slots past it read as zero.
-  if (SHARED_COLS) {
-    h.cols = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(srd_cols, (kc + (int)(threadIdx.x & 31)) * 4, 0, 0);
-  } else {
-    const int kb = kc + 8 * g;
-    h.c0 = __builtin_bit_cast(uintx4, __builtin_amdgcn_raw_buffer_load_b128(srd_cols, kb * 4, 0, 0));
-    h.c1 = __builtin_bit_cast(uintx4, __builtin_amdgcn_raw_buffer_load_b128(srd_cols, kb * 4 + 16, 0, 0));
-  }
-  // one coalesced load of the chunk's values (vals_lane_off = lane * V bytes); vectors past the row read as zero
+  h.cols = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(srd_cols, (kc + 8 * g + (int)(threadIdx.x & 7)) * 4, 0, 0);
+  // one coalesced load of the chunk's values (vals_lane_off = lane * SlabVals<V>::kLane); vectors past the row read as zero
   h.vraw = SlabVals<V>::load(srd_vals, (uint32_t)kc * (V * 2) + vals_lane_off);
 }
 
+// off[j] = x of lane j of the sixteen + y.  (x of a lane whose own columns lie beyond N is a row's offset like any other.)
+template <int J = 0>
+__device__ __forceinline__ void row_offsets(uint32_t (&off)[8], uint32_t x, uint32_t y) {
+  off[J] = (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x150 + J, 0xf, 0xf, true) + y;
+  if constexpr (J < 7) row_offsets<J + 1>(off, x, y);
+}
+
 // (also sends the chunk's values to the value tile `tile_lane` points into: the lane's slot of the tile)
-template <int CPL, int V, bool SHARED_COLS>
-__device__ __forceinline__ void load_body(Chunk<CPL> &c, const ChunkHead<V, SHARED_COLS> &h, int end, int g, __amdgpu_buffer_rsrc_t srd_b,
-                                          uint32_t lane_n2, uint32_t lane_col_off, uint32_t b_bytes,
+template <int CPL, int V>
+__device__ __forceinline__ void load_body(Chunk<CPL> &c, const ChunkHead<V> &h, int end, int g, __amdgpu_buffer_rsrc_t srd_b,
+                                          uint32_t n2, uint32_t lane_col_off, uint32_t b_bytes,
                                           unsigned char *tile_lane) {
   const int kb = h.kc + 8 * g;
   uint32_t off[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const uint32_t col = SHARED_COLS ? (uint32_t)__builtin_amdgcn_ds_bpermute((8 * g + j) * 4, (int)h.cols)
-                                     : (j < 4 ? h.c0[j] : h.c1[j - 4]);
-    off[j] = __umul24(col, lane_n2) + lane_col_off;
-  }
+  row_offsets(off, __umul24(h.cols, n2), lane_col_off);
   if (h.kc + 32 > end) {  // wave-uniform: only the last chunk of a vector-row can be partial
 #pragma unroll
     for (int j = 0; j < 8; ++j) off[j] = (kb + j < end) ? off[j] : b_bytes;
@@ -267,7 +275,7 @@ __device__ __forceinline__ void load_body(Chunk<CPL> &c, const ChunkHead<V, SHAR
   for (int j = 0; j < 8; ++j) {
     c.raw[j] = ChunkRaw<CPL>::load(srd_b, off[j]);
   }
-  *reinterpret_cast<typename SlabVals<V>::type *>(tile_lane) = h.vraw;
+  SlabVals<V>::put(tile_lane, h.vraw);
 }
 
 // tile_op: the lane's address for the transpose reads of the chunk's value tile
@@ -355,10 +363,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
   const int col = (int)tile * (16 * CPL) + m * CPL;
   const bool col_ok = col < p.N;
   const int ncol = min(col, p.N - CPL);  // (unit_col for pieces of CPL columns)
-  // Lanes whose columns lie beyond N aim every gather at the first byte past B.
-  const uint32_t lane_n2 = col_ok ? (uint32_t)p.N * 2u : 0u;
+  // Lanes whose columns lie beyond N aim every gather past B (round the 32 bits of an offset, where B is that large, at some
+  // row of it: nothing that such a lane computes is stored).
+  const uint32_t n2 = (uint32_t)p.N * 2u;
   const uint32_t lane_col_off = col_ok ? (uint32_t)ncol * 2u : b_bytes;
-  constexpr uint32_t kLaneBytes = V * 2u * 32u / 64u;
+  constexpr uint32_t kLaneBytes = SlabVals<V>::kLane;
   const uint32_t vals_lane_off = (uint32_t)lane * kLaneBytes;
   // where the lane writes its share of a value tile, and where its transpose reads start (rows 8g + m/4 of the tile)
   unsigned char *const tw0 = val_tiles[0] + lane * kLaneBytes, *const tw1 = val_tiles[1] + lane * kLaneBytes;
@@ -382,7 +391,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
     Chunk<CPL> c0, c1;
     load_head(h0, beg, g, srd_cols, srd_vals, vals_lane_off);
     load_head(h1, beg + 32, g, srd_cols, srd_vals, vals_lane_off);
-    load_body(c0, h0, end, g, srd_b, lane_n2, lane_col_off, b_bytes, tw0);
+    load_body(c0, h0, end, g, srd_b, n2, lane_col_off, b_bytes, tw0);
     int kc = beg + 32;  // first vector of the chunk whose body is loaded next
     for (;;) {
       if (kc >= end) {
@@ -390,7 +399,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
         break;
       }
       load_head(h0, kc + 32, g, srd_cols, srd_vals, vals_lane_off);
-      load_body(c1, h1, end, g, srd_b, lane_n2, lane_col_off, b_bytes, tw1);
+      load_body(c1, h1, end, g, srd_b, n2, lane_col_off, b_bytes, tw1);
       mac_chunk<CPL, V>(c0, acc, tr0);
       kc += 32;
       if (kc >= end) {
@@ -398,7 +407,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
         break;
       }
       load_head(h1, kc + 32, g, srd_cols, srd_vals, vals_lane_off);
-      load_body(c0, h0, end, g, srd_b, lane_n2, lane_col_off, b_bytes, tw0);
+      load_body(c0, h0, end, g, srd_b, n2, lane_col_off, b_bytes, tw0);
       mac_chunk<CPL, V>(c1, acc, tr1);
       kc += 32;
     }
@@ -457,9 +466,9 @@ __device__ __forceinline__ void gather_accumulate(floatx4 (&acc)[8], const SpmmA
   const __amdgpu_buffer_rsrc_t srd_cols = make_srd(p.col_idx, (uint32_t)end * 4u);
   const __amdgpu_buffer_rsrc_t srd_vals = make_srd(vals, (uint32_t)end * (V * 2u));
   const __amdgpu_buffer_rsrc_t srd_b = make_srd(bmat, b_bytes);
-  const uint32_t lane_n2 = col_ok ? (uint32_t)p.N * 2u : 0u;
+  const uint32_t n2 = (uint32_t)p.N * 2u;
   const uint32_t lane_col_off = col_ok ? (uint32_t)ncol * 2u : b_bytes;
-  constexpr uint32_t kLaneBytes = V * 2u * 32u / 64u;
+  constexpr uint32_t kLaneBytes = SlabVals<V>::kLane;
   const uint32_t vals_lane_off = (uint32_t)lane * kLaneBytes;
   unsigned char *const tw0 = val_tiles[0] + lane * kLaneBytes, *const tw1 = val_tiles[1] + lane * kLaneBytes;
   const uint32_t a_off = (uint32_t)(8 * g + (m >> 2)) * (V * 2u) + (uint32_t)(m & 3) * 8u;
@@ -467,11 +476,11 @@ __device__ __forceinline__ void gather_accumulate(floatx4 (&acc)[8], const SpmmA
 #pragma unroll
   for (int q = 0; q < 8; ++q) acc[q] = floatx4{0.f, 0.f, 0.f, 0.f};
   if (beg >= sub_end) return;
-  ChunkHead<V, false> h0, h1;
+  ChunkHead<V> h0, h1;
   Chunk<8> c0, c1;
   load_head(h0, beg, g, srd_cols, srd_vals, vals_lane_off);
   load_head(h1, beg + 32, g, srd_cols, srd_vals, vals_lane_off);
-  load_body(c0, h0, end, g, srd_b, lane_n2, lane_col_off, b_bytes, tw0);
+  load_body(c0, h0, end, g, srd_b, n2, lane_col_off, b_bytes, tw0);
   int kc = beg + 32;  // first vector of the chunk whose body is loaded next
   for (;;) {
     if (kc >= sub_end) {
@@ -479,7 +488,7 @@ __device__ __forceinline__ void gather_accumulate(floatx4 (&acc)[8], const SpmmA
       break;
     }
     load_head(h0, kc + 32, g, srd_cols, srd_vals, vals_lane_off);
-    load_body(c1, h1, end, g, srd_b, lane_n2, lane_col_off, b_bytes, tw1);
+    load_body(c1, h1, end, g, srd_b, n2, lane_col_off, b_bytes, tw1);
     mac_chunk<8, V>(c0, acc, tr0);
     kc += 32;
     if (kc >= sub_end) {
@@ -487,7 +496,7 @@ __device__ __forceinline__ void gather_accumulate(floatx4 (&acc)[8], const SpmmA
       break;
     }
     load_head(h1, kc + 32, g, srd_cols, srd_vals, vals_lane_off);
-    load_body(c0, h0, end, g, srd_b, lane_n2, lane_col_off, b_bytes, tw0);
+    load_body(c0, h0, end, g, srd_b, n2, lane_col_off, b_bytes, tw0);
     mac_chunk<8, V>(c1, acc, tr1);
     kc += 32;
   }
@@ -730,7 +739,7 @@ __device__ __forceinline__ void slab_issue(SlabLoads<V> &r, int row, int kc, int
   r.col[1] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(srd_cols, (kc + (int)slot0) * 4 + 16, 0, 0);
   // The value descriptor ends with the vector-row: vectors past it read as zero.
   const __amdgpu_buffer_rsrc_t srd_vals = make_srd(vals, (uint32_t)end * (V * 2u));
-  constexpr uint32_t kLaneBytes = V * 2u * 32u / 64u;
+  constexpr uint32_t kLaneBytes = SlabVals<V>::kLane;
   r.vraw = SlabVals<V>::load(srd_vals, (uint32_t)kc * (V * 2u) + (uint32_t)lane * kLaneBytes);
 }
 
@@ -941,7 +950,7 @@ __device__ __forceinline__ void slab_process_item(const SlabCtx<V, OutT> &x, uns
     if (head.valid) cursor_advance(head, rows);
   }
   // the value tile of the first step
-  *reinterpret_cast<typename SlabVals<V>::type *>(x.val_dst) = ld[0].vraw;
+  SlabVals<V>::put(x.val_dst, ld[0].vraw);
 
   const uint32_t lane_base = x.b_lane_off + slab_base + lds_address(lds);  // slab_base is a multiple of 32 (128 for swizzled rows), the LDS base of 128
   // Accumulators are cleared by an MFMA of two zero operands: four instructions on the otherwise
@@ -990,7 +999,7 @@ __device__ __forceinline__ void slab_process_item(const SlabCtx<V, OutT> &x, uns
       }
       // the next step's value tile goes to LDS behind the reads above (LDS operations of a wave
       // execute in order; unconditionally: after the last step it is zeros that nobody reads)
-      *reinterpret_cast<typename SlabVals<V>::type *>(x.val_dst) = ld[nxt].vraw;
+      SlabVals<V>::put(x.val_dst, ld[nxt].vraw);
 
 #pragma unroll
       for (int q = 0; q < NQ; ++q) acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[q].h, a.h, acc[q], 0, 0, 0);
@@ -1106,7 +1115,7 @@ __global__ __launch_bounds__(kSlabThreads) void spmm_slab_kernel(const SpmmArgs 
   SlabCtx<V, OutT> x;
   x.lane = lane;
   x.val_tile = lds + tiles_off + wave * wave_lds_bytes(V);
-  constexpr uint32_t kLaneBytes = V * 2u * 32u / 64u;
+  constexpr uint32_t kLaneBytes = SlabVals<V>::kLane;
   x.val_dst = x.val_tile + lane * kLaneBytes;
   // value tile rows are V*2 bytes; transpose read h picks rows 8g + 4h + m/4
   x.a_off = (uint32_t)(8 * g + (m >> 2)) * (V * 2u) + (uint32_t)(m & 3) * 8u;
@@ -1401,7 +1410,7 @@ __global__ __launch_bounds__(kSlabThreads) void encoder_tail_kernel(const Encode
   SlabCtx<V, _Float16> x;
   x.lane = lane;
   x.val_tile = lds + at.tiles + wave * wave_lds_bytes(V);
-  x.val_dst = x.val_tile + lane * (V * 2u * 32u / 64u);
+  x.val_dst = x.val_tile + lane * SlabVals<V>::kLane;
   x.a_off = (uint32_t)(8 * g + (m >> 2)) * (V * 2u) + (uint32_t)(m & 3) * 8u;
   x.slot0 = (uint32_t)(8 * g + (m >> 2));
   x.b_lane_off = (uint32_t)(m & 3) * 8u;
@@ -1452,9 +1461,19 @@ __global__ __launch_bounds__(kSlabThreads) void encoder_tail_kernel(const Encode
 // rows a 16-lane group reads fall into different banks.
 static constexpr uint32_t kStagePitch = 144;
 
+// off[i] = x of lane i of the quad + y: a quad loads the four indices that it needs one a lane.  With four a lane in one load the
+// address unit, which carries the rows of B too, is busy for sixteen cycles instead of five: 16 x 2000 x 2000 at 90 %, N = 64 8.78 -> 8.63 us (V = 8), 32 x 4096 x 4096
+// at 95 % 19.5 -> 18.9 (V = 16), the balanced kernel on 16384 rows of 16 vectors at the mean, N = 256 17.2 -> 16.9; N = 64 7.80 -> 7.86.
+__device__ __forceinline__ void quad_offsets(uint32_t (&off)[4], uint32_t x, uint32_t y) {
+  off[0] = (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x00, 0xf, 0xf, true) + y;
+  off[1] = (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x55, 0xf, 0xf, true) + y;
+  off[2] = (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xaa, 0xf, 0xf, true) + y;
+  off[3] = (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xff, 0xf, 0xf, true) + y;
+}
+
 template <int V>
 struct StageHead {  // what does not depend on other loads
-  uintx4 cols;      // column indices of k slots 4j .. 4j+3, j = lane / 8
+  uint32_t cols;    // column index of k slot 4 (lane / 8) + lane % 4
   typename SlabVals<V>::type vraw;
   int kc;
 };
@@ -1469,6 +1488,7 @@ struct StageBody {
 template <int V>
 struct StageLane {
   int j, pc;            // the lane fetches 16-byte piece pc of the rows named by k slots 4j .. 4j+3
+  int slot;             // and loads the index of one of them
   uint32_t vals_lane_off, a_off, b_rd;
   unsigned char *tile_dst, *stage_dst;
   const unsigned char *val_tile;
@@ -1476,7 +1496,8 @@ struct StageLane {
     const int m = lane & 15, g = lane >> 4;
     j = lane >> 3;
     pc = lane & 7;
-    constexpr uint32_t kLaneBytes = V * 2u * 32u / 64u;
+    slot = 4 * j + (lane & 3);
+    constexpr uint32_t kLaneBytes = SlabVals<V>::kLane;
     vals_lane_off = (uint32_t)lane * kLaneBytes;
     val_tile = tile;
     tile_dst = tile + lane * kLaneBytes;
@@ -1493,16 +1514,15 @@ struct StageLane {
 template <int V>
 __device__ __forceinline__ void stage_accumulate(floatx4 (&acc)[4], const StageLane<V> &x, __amdgpu_buffer_rsrc_t srd_cols,
                                                  __amdgpu_buffer_rsrc_t srd_vals, __amdgpu_buffer_rsrc_t srd_b, int beg,
-                                                 int end, uint32_t lane_n2, uint32_t lane_col_off, uint32_t b_bytes) {
+                                                 int end, uint32_t n2, uint32_t lane_col_off, uint32_t b_bytes) {
   const auto load_head = [&](StageHead<V> &h, int kc) {
     h.kc = kc;
-    h.cols = __builtin_bit_cast(uintx4, __builtin_amdgcn_raw_buffer_load_b128(srd_cols, (kc + 4 * x.j) * 4, 0, 0));
+    h.cols = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(srd_cols, (kc + x.slot) * 4, 0, 0);
     h.vraw = SlabVals<V>::load(srd_vals, (uint32_t)kc * (V * 2u) + x.vals_lane_off);
   };
   const auto load_body = [&](StageBody<V> &c, const StageHead<V> &h) {
     uint32_t off[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) off[i] = __umul24(h.cols[i], lane_n2) + lane_col_off;
+    quad_offsets(off, __umul24(h.cols, n2), lane_col_off);
     if (h.kc + 32 > end) {  // wave-uniform: only the last chunk of a vector-row can be partial
 #pragma unroll
       for (int i = 0; i < 4; ++i) off[i] = (h.kc + 4 * x.j + i < end) ? off[i] : b_bytes;
@@ -1516,7 +1536,7 @@ __device__ __forceinline__ void stage_accumulate(floatx4 (&acc)[4], const StageL
     // (LDS operations of a wave execute in order: these writes land behind the previous chunk's reads)
 #pragma unroll
     for (int i = 0; i < 4; ++i) *reinterpret_cast<uintx4 *>(x.stage_dst + i * kStagePitch) = c.piece[i];
-    *reinterpret_cast<typename SlabVals<V>::type *>(x.tile_dst) = c.vraw;
+    SlabVals<V>::put(x.tile_dst, c.vraw);
     Half8Bits a;
     {
       const uintx2 lo = lds_read_tr(x.val_tile, x.a_off);
@@ -1567,7 +1587,7 @@ __device__ __forceinline__ void stage_accumulate(floatx4 (&acc)[4], const StageL
 // forms them (same steps, same order).
 template <int V, typename OutT>
 __device__ __forceinline__ void stage_stream(const StageLane<V> &x, const int32_t *col_idx, const uint16_t *vals,
-                                             __amdgpu_buffer_rsrc_t srd_b, uint32_t lane_n2, uint32_t lane_col_off, uint32_t b_bytes,
+                                             __amdgpu_buffer_rsrc_t srd_b, uint32_t n2, uint32_t lane_col_off, uint32_t b_bytes,
                                              const void *first_item, int count, int lane, const SlabStore<V, OutT, 4> &out,
                                              __amdgpu_buffer_rsrc_t srd_c, uint32_t c_vrow_bytes) {
   // the bundle's items, one per lane (row, first vector, end): a uniform index reads one back without memory
@@ -1602,13 +1622,12 @@ __device__ __forceinline__ void stage_stream(const StageLane<V> &x, const int32_
   const auto load_head = [&](StageHead<V> &h, const Step &d) {
     const uint32_t recs = d.valid ? (uint32_t)d.end : 0u;
     h.kc = d.kc;
-    h.cols = __builtin_bit_cast(uintx4, __builtin_amdgcn_raw_buffer_load_b128(make_srd(col_idx, recs * 4u), (d.kc + 4 * x.j) * 4, 0, 0));
+    h.cols = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(make_srd(col_idx, recs * 4u), (d.kc + x.slot) * 4, 0, 0);
     h.vraw = SlabVals<V>::load(make_srd(vals, recs * (V * 2u)), (uint32_t)d.kc * (V * 2u) + x.vals_lane_off);
   };
   const auto load_body = [&](StageBody<V> &c, const StageHead<V> &h, const Step &d) {
     uint32_t off[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) off[i] = __umul24(h.cols[i], lane_n2) + lane_col_off;
+    quad_offsets(off, __umul24(h.cols, n2), lane_col_off);
     if (h.kc + 32 > d.end) {  // wave-uniform: only the last step of a vector-row can be partial
 #pragma unroll
       for (int i = 0; i < 4; ++i) off[i] = (h.kc + 4 * x.j + i < d.end) ? off[i] : b_bytes;
@@ -1624,7 +1643,7 @@ __device__ __forceinline__ void stage_stream(const StageLane<V> &x, const int32_
   const auto contract = [&](const StageBody<V> &c, const Step &d) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) *reinterpret_cast<uintx4 *>(x.stage_dst + i * kStagePitch) = c.piece[i];
-    *reinterpret_cast<typename SlabVals<V>::type *>(x.tile_dst) = c.vraw;
+    SlabVals<V>::put(x.tile_dst, c.vraw);
     Half8Bits a;
     {
       const uintx2 lo = lds_read_tr(x.val_tile, x.a_off);
@@ -1704,14 +1723,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(V == 8 ? 5 :
   // Lanes whose columns lie beyond N aim every gather at the first byte past B, where loads return zero.
   const int col = (int)tile * 64 + 8 * x.pc, ncol = unit_col(col, p.N);
   const bool col_ok = col < p.N;
-  const uint32_t lane_n2 = col_ok ? (uint32_t)p.N * 2u : 0u;
+  const uint32_t n2 = (uint32_t)p.N * 2u;
   const uint32_t lane_col_off = col_ok ? (uint32_t)ncol * 2u : b_bytes;
   floatx4 acc[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) acc[q] = floatx4{0.f, 0.f, 0.f, 0.f};
   // (the bias of the lane's output row is fetched before the loop so that the row's end does not wait for it)
   const float b = bias_of_row(p, (int64_t)row * V + (lane & (V - 1)));
-  stage_accumulate<V>(acc, x, srd_cols, srd_vals, srd_b, beg, end, lane_n2, lane_col_off, b_bytes);
+  stage_accumulate<V>(acc, x, srd_cols, srd_vals, srd_b, beg, end, n2, lane_col_off, b_bytes);
   if (has_epilogue(p)) {  // (uniform) every accumulator of lane (m, g) belongs to output row m of the vector-row
 #pragma unroll
     for (int q = 0; q < 4; ++q)
@@ -1826,7 +1845,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
       SlabStore<V, OutT, 4> out;
       out.init(lane, (int)tile * 64, p.N);
       stage_stream<V, OutT>(x, p.col_idx, p.values + (int64_t)batch * p.stride_values,
-                            make_srd(p.B + (int64_t)batch * p.stride_B, b_bytes), col_ok ? (uint32_t)p.N * 2u : 0u,
+                            make_srd(p.B + (int64_t)batch * p.stride_B, b_bytes), (uint32_t)p.N * 2u,
                             col_ok ? (uint32_t)ncol * 2u : b_bytes, b_bytes, s.items + first, last - first, lane, out,
                             make_srd(reinterpret_cast<OutT *>(p.C) + (int64_t)batch * p.stride_C, (uint32_t)p.m_vec * c_vrow_bytes),
                             c_vrow_bytes);
@@ -1844,12 +1863,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     // Lanes whose columns lie beyond N aim every gather at the first byte past B, where loads return zero.
     const int col = (int)tile * 64 + 8 * x.pc, ncol = unit_col(col, p.N);
     const bool col_ok = col < p.N;
-    const uint32_t lane_n2 = col_ok ? (uint32_t)p.N * 2u : 0u;
+    const uint32_t n2 = (uint32_t)p.N * 2u;
     const uint32_t lane_col_off = col_ok ? (uint32_t)ncol * 2u : b_bytes;
     floatx4 acc[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) acc[q] = floatx4{0.f, 0.f, 0.f, 0.f};
-    stage_accumulate<V>(acc, x, srd_cols, srd_vals, srd_b, kbeg, kend, lane_n2, lane_col_off, b_bytes);
+    stage_accumulate<V>(acc, x, srd_cols, srd_vals, srd_b, kbeg, kend, n2, lane_col_off, b_bytes);
 
     if (split_id >= 0) {
       const uint32_t n_slots = (uint32_t)s.header[kHdrSlots], n_split = (uint32_t)s.header[kHdrSplitRows];
