@@ -54,7 +54,7 @@ __device__ __forceinline__ uint32_t xcd_work_index(uint32_t per_xcd) {
 // WHOLE: F = 32 * NC exactly, no piece to test for: vector instructions are what the kernel waits for (2000 keys, 16 heads,
 // 64 features 11.3 -> 10.7 us, 128: 17.5 -> 16.2; 4096 keys, 48 heads, 64: 79.6 -> 76.2; 16 heads, 256: 109 -> 96).  Two groups
 // of vectors per step, with twice the rows in flight, measured 3 to 8 % slower.
-template <int V, int NC, bool WHOLE>
+template <int V, int NC, bool WHOLE, bool SHARED>
 __global__ __launch_bounds__(64) void sddmm_kernel(const SddmmArgs p) {
   constexpr uint32_t kStageRow = NC * 64u + 16u;  // bytes: room for 32 * NC features, and the padding
   __shared__ __align__(16) unsigned char stage[2][16 * kStageRow];
@@ -107,15 +107,19 @@ __global__ __launch_bounds__(64) void sddmm_kernel(const SddmmArgs p) {
   struct Pieces {
     uintx4 d[NC];
   };
-  // The column indices come in blocks of 64 (four groups), one per lane in one fully coalesced load, a block
-  // ahead; the lanes that fetch a row then pick its column out of the block with a lane permute.  (A load per
-  // group, eight lanes asking for the same index, costs the memory pipeline sixteen quarter-wave passes for 64
-  // bytes, and this kernel is bound by that pipeline.)
+  // Column indices: one load of 4 bytes a lane per load of rows, the lanes of a row asking for the same index (five cycles of the address unit),
+  // or, SHARED, blocks of 64 of them (four groups), one per lane, a block ahead, out of which the lanes pick theirs with a lane permute.  16 heads of
+  // 2000 keys, 64 features 10.54 (blocks) / 10.04 us, 512 keys, 8 heads 3.29 / 3.16, 128 features, 2048 keys, 16 heads 15.7 / 15.4, 256 features
+  // 30.3 / 28.2; but of 64 features with more waves than are resident at once the address unit is what they wait for: 2048 keys, 48 heads, V = 16
+  // 16.2 / 16.6, 4096 keys, 48 heads 77.0 / 78.4 (32 features 18.7 / 18.1, 128 28.2 / 27.7).
   int blk_base = beg;
-  uint32_t blk0 = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(srd_cols, (beg + lane) * 4, 0, 0);
-  uint32_t blk1 = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(srd_cols, (beg + 64 + lane) * 4, 0, 0);
+  uint32_t blk0 = 0, blk1 = 0;
+  if constexpr (SHARED) {
+    blk0 = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(srd_cols, (beg + lane) * 4, 0, 0);
+    blk1 = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(srd_cols, (beg + 64 + lane) * 4, 0, 0);
+  }
   auto load_cols = [&](int kc) {  // (called with kc rising by 16 from beg)
-    if (kc - blk_base >= 64) {
+    if (SHARED && kc - blk_base >= 64) {
       blk_base += 64;
       blk0 = blk1;
       blk1 = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(srd_cols, (blk_base + 64 + lane) * 4, 0, 0);
@@ -123,7 +127,8 @@ __global__ __launch_bounds__(64) void sddmm_kernel(const SddmmArgs p) {
     Cols x;
 #pragma unroll
     for (int i = 0; i < NC; ++i)
-      x.c[i] = (uint32_t)__builtin_amdgcn_ds_bpermute((kc - blk_base + (int)ld_row[i]) * 4, (int)blk0);
+      x.c[i] = SHARED ? (uint32_t)__builtin_amdgcn_ds_bpermute((kc - blk_base + (int)ld_row[i]) * 4, (int)blk0)
+                      : (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(srd_cols, (kc + (int)ld_row[i]) * 4, 0, 0);
     return x;
   };
   auto load_rows = [&](Pieces &b, const Cols &x) {
@@ -209,9 +214,13 @@ static hipError_t launch_sddmm_nc(const SddmmArgs &a, hipStream_t stream) {
   p.per_xcd = (p.total_work + 7u) / 8u;
   if (p.total_work == 0) return hipSuccess;
   if (a.F == 32 * NC)
-    hipLaunchKernelGGL((sddmm_kernel<V, NC, true>), dim3(p.per_xcd * 8u), dim3(64), 0, stream, p);
+    // (8192 waves: 32 for every CU; 32 heads of 2048 keys, V = 8, are level)
+    if (NC == 2 && p.total_work > 8192u)
+      hipLaunchKernelGGL((sddmm_kernel<V, NC, true, NC == 2>), dim3(p.per_xcd * 8u), dim3(64), 0, stream, p);
+    else
+      hipLaunchKernelGGL((sddmm_kernel<V, NC, true, false>), dim3(p.per_xcd * 8u), dim3(64), 0, stream, p);
   else
-    hipLaunchKernelGGL((sddmm_kernel<V, NC, false>), dim3(p.per_xcd * 8u), dim3(64), 0, stream, p);
+    hipLaunchKernelGGL((sddmm_kernel<V, NC, false, false>), dim3(p.per_xcd * 8u), dim3(64), 0, stream, p);
   return hipGetLastError();
 }
 

@@ -57,6 +57,25 @@ def test_sddmm_row_length_tails_and_permutation(oracle, built_library, per_row):
 
 
 @pytest.mark.parametrize("V", [8, 16])
+def test_sddmm_of_many_waves_reads_its_indices_in_blocks(oracle, built_library, V):
+    """64 features and more than 8192 waves: indices in blocks of 64, rows that end at and around a block's end."""
+    K, F, batch = 200, 64, 431
+    lens = [0, 1, 15, 16, 17, 47, 48, 49, 63, 64, 65, 79, 80, 81, 127, 128, 129, 143, 193, 200]
+    rng = np.random.default_rng(V)
+    cols = np.concatenate([rng.permutation(K)[:n] for n in lens]).astype(np.int32)
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    assert (batch - 1) * len(lens) > 8192 >= len(lens)
+    lhs = rng.integers(-3, 4, (batch, len(lens) * V, F)).astype(np.float16)  # (every product and sum is representable)
+    rhs = rng.integers(-3, 4, (batch, K, F)).astype(np.float16)
+    got = sspmm_amd.bsddmm(None, dev(off), dev(cols), dev(lhs), dev(rhs), V)
+    torch.cuda.synchronize()
+    for b in (0, batch // 2, batch - 1):
+        want = oracle.sddmm(len(lens), V, off, cols, lhs[b], rhs[b])
+        assert np.array_equal(got[b].cpu().numpy(), want)
+        assert torch.equal(got[b], sspmm_amd.sddmm(None, dev(off), dev(cols), dev(lhs[b]), dev(rhs[b]), V))
+
+
+@pytest.mark.parametrize("V", [8, 16])
 def test_softmax_matches_oracle_and_rows_sum_to_one(oracle, built_library, V):
     rng = np.random.default_rng(7)
     lens = np.array([0, 1, 5, 64, 65, 200, 0, 1000, 3, 256, 257, 512, 513])  # around what a wave keeps in registers
