@@ -35,6 +35,9 @@ struct BlockDenseArgs {
   int head_dim;                              // out as [n_out / E, inner, E / head_dim, tokens / inner, head_dim]; 0: as [tokens, n_out]
   uint16_t *x_out;                           // nullable: x' is not needed
   uint16_t *norm_out, *out;
+  long long outer;                           // (these three by launch_block_dense) tokens / inner
+  uint32_t inner_magic;                      // 0: a division
+  int inner_shift;
 };
 
 // Weight matrices [out features, in features] as torch.nn.Linear keeps them, in the order in which block_dense loads them.

@@ -34,12 +34,12 @@
 // row: from torch's layout it reads 64 bytes of each of sixteen rows, which lie 512 to 2048 bytes apart on a few of the L2's
 // channels, and 32 tokens per workgroup took 61 us instead of 27 (8192 tokens).
 //
-// 256 features, 1024 hidden, 768 out, with the LayerNorms: 8192 tokens 26 us, 32768 tokens 58 us (0.9 PFLOP/s) back to
-// back, 27 and 63 between the attention launches of a model, against 104 (the host) and 121 for the four library products
-// and two LayerNorm launches.  Counters of the launches in a model: the CU's path to its first-level cache passes 64 bytes
-// a cycle and is used for 64 % of the cycles at 8192 tokens and 73 % at 32768 (two workgroups per CU fetch the weights
-// each), nearly all of it weights; the matrix units are busy for 24 and 47 %, LDS for 15 and 29 %.  The rest at 8192 tokens
-// is waiting: a SIMD holds one wave there, and nothing covers its LayerNorms, barriers and the start of a product.
+// 256 features, 1024 hidden, 768 out, with the LayerNorms, both layers / folded: 8192 tokens 25.7 / 16.5 us, 32768 tokens 62.6 / 38.5,
+// against 104 (the host) and 121 for the four library products and two LayerNorm launches.  Where a folded launch's cycles go: 8192 tokens
+// 26 000: 4000 until the attention's output is there, 2400 to 2700 a product of 256 x 256 (2048 at 64 bytes of weights a cycle), 1900 a LayerNorm, 1300 the
+// stores of 256 outputs; 32768 tokens 58 000, 12 to 13 000 of them until all workgroups' 33 MB are there, and the stores at the end, 7 us of them, as
+// exposed.  Without gain: loads of x and the attention's output in front of the first weights, the weights fetched into L2 ahead by a load a thread,
+// four units of the last product's weights in flight, the last product's bias in its accumulators (its load waits for the stores).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -52,6 +52,7 @@ namespace {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 
 constexpr int kChunk = 256;  // hidden (or output) features a workgroup makes at a time, 64 per wave
@@ -173,59 +174,52 @@ __device__ __forceinline__ void put_row(unsigned char *p, const floatx4 (&v)[NJ]
   }
 }
 
-// Sum over a token's features of one value per lane and token tile: over the four lane groups, then over the four
-// waves through `part` [4][TM].  One barrier; the next use of `part` needs another one in between.
-template <int TT>
-__device__ __forceinline__ void token_sums(float (&s)[TT], float *part, int wave, int lane) {
-#pragma unroll
-  for (int t = 0; t < TT; ++t) {
-    s[t] += __shfl_xor(s[t], 16, 64);
-    s[t] += __shfl_xor(s[t], 32, 64);
-    part[wave * (TT * 16) + t * 16 + (lane & 15)] = s[t];  // (the four lane groups hold the same sum)
-  }
-  lds_barrier();
-#pragma unroll
-  for (int t = 0; t < TT; ++t) {
-    const float *q = part + t * 16 + (lane & 15);
-    s[t] = (q[0] + q[TT * 16]) + (q[2 * TT * 16] + q[3 * TT * 16]);
-  }
+// Sum over the four lane groups, in each of them.
+__device__ __forceinline__ float groups_sum(float v) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
-// v = LayerNorm(v) over the E features of every token, statistics in fp32, mean first.
+// v = LayerNorm(v) over the E features of every token, statistics in fp32.  s: the lane's sums of v.  A wave takes the mean of its E / 4
+// features of a token and the squares' sum about it, and the four waves' pairs are put together as Chan, Golub and LeVeque do (1979): one
+// exchange through `part` [4][TM] and one barrier, where the mean first and then the squares about it took two.  At 8192 tokens of 256
+// features nothing runs beside it: with lane permutes, two exchanges, and gamma and beta loaded here, behind the weights in flight, the two LayerNorms took
+// 2680 and 2340 of a workgroup's 27 300 cycles, now (lane swaps, gamma and beta in LDS from the start) 1880 and 1930.
 template <int TT, int NJ, int E>
-__device__ __forceinline__ void layer_norm(floatx4 (&v)[TT][NJ], const uint16_t *gamma, const uint16_t *beta, float eps, int first,
-                                           float *part, int wave, int lane) {
-  half8 w[NJ / 2], b[NJ / 2];
-  feature_values<NJ>(w, gamma, first, 1.f);
-  feature_values<NJ>(b, beta, first, 0.f);
-  float s[TT];
+__device__ __forceinline__ void layer_norm(floatx4 (&v)[TT][NJ], float (&s)[TT], const uint16_t *gamma_beta, float eps, int first, floatx2 *part,
+                                           int wave, int lane) {
 #pragma unroll
   for (int t = 0; t < TT; ++t) {
-    s[t] = 0.f;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) s[t] += (v[t][j][0] + v[t][j][1]) + (v[t][j][2] + v[t][j][3]);
-  }
-  token_sums<TT>(s, part, wave, lane);
-#pragma unroll
-  for (int t = 0; t < TT; ++t) {
-    const float mean = s[t] * (1.0f / (float)E);
-    s[t] = 0.f;
+    s[t] = groups_sum(s[t]) * (4.0f / (float)E);
+    float q = 0.f;
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        v[t][j][i] -= mean;
-        s[t] += v[t][j][i] * v[t][j][i];
+        v[t][j][i] -= s[t];
+        q = __builtin_fmaf(v[t][j][i], v[t][j][i], q);
       }
+    part[wave * (TT * 16) + t * 16 + (lane & 15)] = floatx2{s[t], groups_sum(q)};  // (the four lane groups hold the same)
   }
-  token_sums<TT>(s, part + 4 * TT * 16, wave, lane);
+  lds_barrier();
+  half8 w[NJ / 2], b[NJ / 2];
+  load_row<NJ>(w, gamma_beta + first);
+  load_row<NJ>(b, gamma_beta + E + first);
 #pragma unroll
   for (int t = 0; t < TT; ++t) {
-    const float rstd = rsqrtf(s[t] * (1.0f / (float)E) + eps);
+    const floatx2 *const at = part + t * 16 + (lane & 15);
+    const floatx2 x0 = at[0], x1 = at[TT * 16], x2 = at[2 * TT * 16], x3 = at[3 * TT * 16];
+    const float mean = ((x0[0] + x1[0]) + (x2[0] + x3[0])) * 0.25f;
+    const float d0 = x0[0] - mean, d1 = x1[0] - mean, d2 = x2[0] - mean, d3 = x3[0] - mean;
+    const float between = (d0 * d0 + d1 * d1) + (d2 * d2 + d3 * d3);
+    const float q = (x0[1] + x1[1]) + (x2[1] + x3[1]);
+    const float rstd = rsqrtf(q * (1.0f / (float)E) + between * 0.25f + eps), shift = (s[t] - mean) * rstd;
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[t][j][i] = v[t][j][i] * rstd * value(w, j, i) + value(b, j, i);
+      for (int i = 0; i < 4; ++i) v[t][j][i] = __builtin_fmaf(v[t][j][i], rstd, shift) * value(w, j, i) + value(b, j, i);
   }
 }
 
@@ -240,7 +234,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
   __shared__ __align__(16) unsigned char act[TM * kPitchA];  // attention's output, then n, then h
   __shared__ __align__(16) unsigned char hid[PART == kTwoLayers ? TM * kPitchH : 16];  // kChunk hidden features
   __shared__ __align__(16) float affine[PART == kFolded ? 2 * E : 4];
-  __shared__ float part[8 * TM];
+  __shared__ __align__(16) uint16_t norms[4 * E];  // gamma and beta of both LayerNorms
+  __shared__ __align__(8) floatx2 part[4 * TM];
 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int m = lane & 15, g = lane >> 4;
@@ -249,6 +244,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
   const int first = wave * (16 * NT) + g * 8;  // the lane's first feature of E
   const int chunk_first = wave * 64 + g * 8;         // and of a chunk
   const unsigned char *const act_op = act + m * kPitchA + g * 16, *const hid_op = hid + m * kPitchH + g * 16;
+
+  float one = 1.f;  // (the compiler does not see it: a product with it and a sum are one instruction that takes halfs as they are)
+  asm("" : "+s"(one));
 
   uintx4 w[D][8];
   const int t_row = p.wt && wave * 64 < p.n_out ? wave * 64 : 0;
@@ -261,17 +259,38 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
   else if (p.wt)
     issue_first<4, D>(w, tail);
 
+  // token / inner, of the workgroup's first and of a number below inner + 64 (a product with 2^(31 + l) / inner, l = log2 inner rounded up, which is
+  // exact below 2^31; the division takes the scalar unit 150 instructions and a lane 20, with nothing beside them)
+  const auto outer_of = [&](long long t) -> long long {
+    if (p.inner == 1) return t;
+    return p.inner_magic ? (long long)(__umulhi((uint32_t)t, p.inner_magic) >> p.inner_shift) : t / p.inner;
+  };
+  const auto inner_of = [&](uint32_t r) -> uint32_t {
+    if (p.inner == 1) return r;
+    return p.inner_magic ? __umulhi(r, p.inner_magic) >> p.inner_shift : r / (uint32_t)p.inner;
+  };
+
+#pragma unroll
+  for (int i = 0; i < 4 * E; i += 256 * 8) {  // (256 features: 128 threads take a piece each)
+    const int at = i + (int)threadIdx.x * 8, which = at / E;
+    if (at < 4 * E && (PART != kNoAttention || which >= 2)) {
+      const uint16_t *const from = which == 0 ? p.gamma2 : which == 1 ? p.beta2 : which == 2 ? p.gamma_n : p.beta_n;
+      const uint32_t none = which & 1 ? 0u : 0x3c003c00u;
+      *reinterpret_cast<uintx4 *>(norms + at) = from ? *reinterpret_cast<const uintx4 *>(from + at % E) : uintx4{none, none, none, none};
+    }
+  }
+
   // the lane's share of x, fetched once
   half8 x[TT][NT / 2];
   if (p.x_inner == E && p.x_outer == p.inner * E && !p.pos) {
 #pragma unroll
     for (int t = 0; t < TT; ++t) load_row<NT>(x[t], p.x + (t0 + min(t * 16 + m, left - 1)) * E + first);
   } else {
-    const long long q0 = t0 / p.inner;
+    const long long q0 = outer_of(t0);
     const uint32_t r0 = (uint32_t)(t0 - q0 * p.inner);
 #pragma unroll
     for (int t = 0; t < TT; ++t) {
-      const uint32_t r = r0 + (uint32_t)min(t * 16 + m, left - 1), q = r / (uint32_t)p.inner;
+      const uint32_t r = r0 + (uint32_t)min(t * 16 + m, left - 1), q = inner_of(r);
       const long long at = (q0 + q) * p.x_outer + (long long)(r - q * (uint32_t)p.inner) * p.x_inner;
       if (PART == kNoAttention && p.ids) {  // (uniform)
         const long long id = p.wide_ids ? static_cast<const long long *>(p.ids)[at] : static_cast<const int *>(p.ids)[at];
@@ -325,21 +344,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
 #pragma unroll
       for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[t][j][i] = value(bias, j, i);
-    gemm<TT, NT, E, kPitchA, PART == kFolded ? NT : 4, D>(v, act_op, wo, PART == kFolded ? w2 : w1, w);
-#pragma unroll
-    for (int t = 0; t < TT; ++t)
-#pragma unroll
-      for (int j = 0; j < NT; ++j)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[t][j][i] += value(x[t], j, i);
+        for (int i = 0; i < 4; ++i) v[t][j][i] = __builtin_fmaf(value(bias, j, i), one, value(x[t], j, i));
     // (or the compiler keeps the widened values for the second use, at twice the registers)
 #pragma unroll
     for (int t = 0; t < TT; ++t)
 #pragma unroll
       for (int j = 0; j < NT / 2; ++j) asm("" : "+v"(x[t][j]));
-    layer_norm<TT, NT, E>(v, p.gamma2, p.beta2, p.eps2, first, part, wave, lane);
-    // (every wave is past its product: the sums' barriers lie in between)
+    gemm<TT, NT, E, kPitchA, PART == kFolded ? NT : 4, D>(v, act_op, wo, PART == kFolded ? w2 : w1, w);
+    float s[TT];
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+      s[t] = 0.f;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) s[t] += (v[t][j][0] + v[t][j][1]) + (v[t][j][2] + v[t][j][3]);
+    }
+    layer_norm<TT, NT, E>(v, s, norms, p.eps2, first, part, wave, lane);
+    // (every wave is past its product: the sums' barrier lies in between)
 #pragma unroll
     for (int t = 0; t < TT; ++t) put_row<NT>(act + (t * 16 + m) * kPitchA + first * 2, v[t]);
     lds_barrier();
@@ -356,7 +376,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
 #pragma unroll
         for (int t = 0; t < TT; ++t)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) v[t][j][i] = __builtin_fmaf(v[t][j][i], scale[i], shift[i]) + value(x[t], j, i);
+          for (int i = 0; i < 4; ++i) v[t][j][i] = __builtin_fmaf(v[t][j][i], scale[i], __builtin_fmaf(value(x[t], j, i), one, shift[i]));
       }
     } else {
 #pragma unroll
@@ -364,7 +384,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) v[t][j][i] = value(bias2, j, i) + value(x[t], j, i);
+          for (int i = 0; i < 4; ++i) v[t][j][i] = __builtin_fmaf(value(bias2, j, i), one, value(x[t], j, i));
       for (int c = 0; c < p.mlp; c += kChunk) {
         floatx4 h[TT][4];
         half8 bias1[2];
@@ -403,16 +423,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
         for (int i = 0; i < 4; ++i) v[t][j][i] = value(x[t], j, i);
   }
   // x' as it is stored is what its LayerNorm reads
+  float s[TT];
 #pragma unroll
   for (int t = 0; t < TT; ++t) {
+    s[t] = 0.f;
 #pragma unroll
-    for (int j = 0; j < NT; ++j)
+    for (int j = 0; j < NT; j += 2) {
+      half8 h;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[t][j][i] = (float)(_Float16)v[t][j][i];
-    if (p.x_out && t * 16 + m < left) put_row<NT>(reinterpret_cast<unsigned char *>(p.x_out + (t0 + t * 16 + m) * E + first), v[t]);
+      for (int i = 0; i < 4; ++i) {
+        h[i] = (_Float16)v[t][j][i];
+        h[4 + i] = (_Float16)v[t][j + 1][i];
+      }
+      if (p.x_out && t * 16 + m < left) *reinterpret_cast<half8 *>(p.x_out + (t0 + t * 16 + m) * E + first + j * 16) = h;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v[t][j][i] = (float)h[i];
+        v[t][j + 1][i] = (float)h[4 + i];
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) s[t] = __builtin_fmaf((float)h[i], one, s[t]);
+    }
   }
 
-  layer_norm<TT, NT, E>(v, p.gamma_n, p.beta_n, p.eps_n, first, part, wave, lane);
+  layer_norm<TT, NT, E>(v, s, norms + 2 * E, p.eps_n, first, part, wave, lane);
   if (!p.wt) {
 #pragma unroll
     for (int t = 0; t < TT; ++t)
@@ -423,13 +457,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
   for (int t = 0; t < TT; ++t) put_row<NT>(act + (t * 16 + m) * kPitchA + first * 2, v[t]);
   lds_barrier();
   Weights cur = tail;
-  const long long outer = p.tokens / p.inner, q0 = t0 / p.inner;
+  const long long outer = p.outer, q0 = p.head_dim ? outer_of(t0) : 0;
   const uint32_t r0 = (uint32_t)(t0 - q0 * p.inner);
   const int head_shift = p.head_dim ? __builtin_ctz((unsigned)p.head_dim) : 0;
   for (int c = wave * 64; c < p.n_out; c += kChunk) {  // (no barrier from here on)
     floatx4 o[TT][4];
     half8 bias[2];
     feature_values<4>(bias, p.bt, c + g * 8, 0.f);
+    uint32_t r_first = r0;
+    asm volatile("" : "+s"(r_first));  // (the rows' places are made anew for every chunk: kept, they cost registers that spill)
 #pragma unroll
     for (int t = 0; t < TT; ++t)
 #pragma unroll
@@ -448,7 +484,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
         if (p.head_dim == 0) {
           put_row<4>(reinterpret_cast<unsigned char *>(p.out + (t0 + t * 16 + m) * p.n_out + c + g * 8), o[t]);
         } else {  // (a head is at least as wide as the 32 features of two tiles)
-          const uint32_t r = r0 + (uint32_t)(t * 16 + m), i = r / (uint32_t)p.inner;  // token (q0 + i, r - i * inner)
+          const uint32_t r = r_first + (uint32_t)(t * 16 + m), i = inner_of(r);  // token (q0 + i, r - i * inner)
           uint16_t *const row = p.out + (r - i * (uint32_t)p.inner) * (E * outer) + (q0 + i) * p.head_dim + g * 8;
 #pragma unroll
           for (int j = 0; j < 4; j += 2) {
@@ -610,7 +646,8 @@ hipError_t launch(const BlockDenseArgs &p, hipStream_t stream) {
 // CU one: 8192 tokens of 128, 256, 512 features 15, 26, 56 us against 18, 30, 73; 10000 tokens 25, 43, 101 against 18, 31, 73.
 // Up to 4096 tokens 16 do the same, and a workgroup's chain of products and LayerNorms is shorter: 2048 tokens 10.0, 17.5, 43 us
 // against 12.3, 20.1, 48 with 32 (without attention 4.6, 7.4, 17 against 5.6, 9.2, 20), 4096 tokens 10.9, 19.3, 46 against 12.6, 21.2,
-// 49; 8192 tokens without attention 7.6, 14.2, 36 against 6.6, 11.1, 25.
+// 49; 8192 tokens without attention 7.6, 14.2, 36 against 6.6, 11.1, 25.  (Both linear layers, LayerNorms of two exchanges.)  Folded, 256 features,
+// 16 / 32 / 64 tokens: 8192 tokens 21 / 16.5 / 19.7, 32768 75 / 50 / 38.5.
 template <int E>
 hipError_t launch_for_width(const BlockDenseArgs &p, hipStream_t stream) {
   if (p.tokens <= 256 * 16) return launch<E, 16>(p, stream);
@@ -642,7 +679,17 @@ hipError_t launch_block_prepare(int E, const BlockFoldArgs &folds, const BlockPa
   return hipGetLastError();
 }
 
-hipError_t launch_block_dense(int E, const BlockDenseArgs &p, hipStream_t stream) {
+hipError_t launch_block_dense(int E, const BlockDenseArgs &args, hipStream_t stream) {
+  BlockDenseArgs p = args;
+  p.outer = p.tokens / p.inner;
+  p.inner_magic = 0;
+  p.inner_shift = 0;
+  if (p.inner > 1 && p.tokens < (1ll << 31) && p.inner < (1ll << 31) - 64) {
+    int l = 1;
+    while ((1ll << l) < p.inner) ++l;
+    p.inner_magic = (uint32_t)((1ull << (31 + l)) / (unsigned long long)p.inner + 1u);
+    p.inner_shift = l - 1;
+  }
   switch (E) {
     case 128: return launch_for_width<128>(p, stream);
     case 256: return launch_for_width<256>(p, stream);

@@ -650,6 +650,29 @@ def test_block_dense_on_one_matrix_for_two_layers(built_library, E, mlp, n_out, 
                         assert torch.equal(split, got.view(outer, inner, n_out // E, E // d, d).permute(2, 1, 3, 0, 4))
 
 
+@pytest.mark.parametrize("E,outer,inner", [(128, 2000, 1), (256, 1001, 2), (256, 700, 5), (128, 37, 7), (256, 9, 31), (512, 5, 64), (128, 3, 1000), (256, 2, 4097)])
+def test_block_dense_finds_a_tokens_place(built_library, E, outer, inner):
+    """Token / inner by a product: the bits of one long sequence, whatever it is cut into, x batch-major, out dense and split into
+    heads, and an embedding's positions; LayerNorms without weights are those with ones and zeros."""
+    from sspmm_amd.attention import block_dense, fold_blocks
+    g = torch.Generator("cuda").manual_seed(E + inner)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g).half()  # noqa: E731
+    blk, = _two_layers(E, 256, 1, g)
+    norm, tail = torch.nn.LayerNorm(E).cuda().half(), torch.nn.Linear(E, E).cuda().half()
+    plain = torch.nn.LayerNorm(E, elementwise_affine=False)
+    x, attn, pos, T = rnd(inner, outer, E).transpose(0, 1), rnd(outer, inner, E), rnd(outer, 1, E), outer * inner
+    with torch.no_grad():
+        packed, folded = fold_blocks([blk], [blk.out_proj, tail], [E // 4, 64])
+        whole = block_dense(x.reshape(T, 1, E), attn.view(T, 1, E), blk, norm, tail, True, packed, 0, folded=folded[0])
+        kept, got = block_dense(x, attn, blk, norm, tail, True, packed, 0, folded=folded[0])
+        split = block_dense(x, attn, blk, plain, tail, False, packed, 32, folded=folded[0])[1]
+        assert torch.equal(kept.view(T, 1, E), whole[0]) and torch.equal(got.view(T, 1, E), whole[1])
+        assert torch.equal(split, got.view(outer, inner, 1, E // 32, 32).permute(2, 1, 3, 0, 4))
+        want = block_dense(x.reshape(T, 1, E), None, None, norm, tail, True, packed[1:], 0, pos.expand(outer, inner, E).reshape(T, 1, E), 3.0)
+        kept, got = block_dense(x, None, None, plain, tail, True, packed[1:], 0, pos, 3.0)
+        assert torch.equal(kept.view(T, 1, E), want[0]) and torch.equal(got.view(T, 1, E), want[1])
+
+
 @pytest.mark.parametrize("E,outer,inner", [(128, 5, 1), (128, 1367, 3), (256, 37, 3), (256, 1400, 3), (512, 2731, 3), (512, 19, 2)])
 @pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
 def test_block_dense_looks_tokens_up(built_library, E, outer, inner, dtype):
