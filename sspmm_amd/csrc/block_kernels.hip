@@ -63,13 +63,6 @@ __device__ __forceinline__ uintx2 fold_read_tr(const unsigned char *p) {
   return __builtin_bit_cast(uintx2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) shortx4 *)p));
 }
 
-// Workgroup barrier that orders LDS only: global loads in flight stay in flight.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 template <int NJ>
 struct Unit {  // what is loaded together: NJ tiles of 16 features x K values of k
   static constexpr int K = NJ == 8 ? 32 : 64;
@@ -174,14 +167,6 @@ __device__ __forceinline__ void put_row(unsigned char *p, const floatx4 (&v)[NJ]
   }
 }
 
-// Sum over the four lane groups, in each of them.
-__device__ __forceinline__ float groups_sum(float v) {
-  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
-
 // v = LayerNorm(v) over the E features of every token, statistics in fp32.  s: the lane's sums of v.  A wave takes the mean of its E / 4
 // features of a token and the squares' sum about it, and the four waves' pairs are put together as Chan, Golub and LeVeque do (1979): one
 // exchange through `part` [4][TM] and one barrier, where the mean first and then the squares about it took two.  At 8192 tokens of 256
@@ -192,7 +177,7 @@ __device__ __forceinline__ void layer_norm(floatx4 (&v)[TT][NJ], float (&s)[TT],
                                            int wave, int lane) {
 #pragma unroll
   for (int t = 0; t < TT; ++t) {
-    s[t] = groups_sum(s[t]) * (4.0f / (float)E);
+    s[t] = sum_over_rows(s[t]) * (4.0f / (float)E);
     float q = 0.f;
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
@@ -201,7 +186,7 @@ __device__ __forceinline__ void layer_norm(floatx4 (&v)[TT][NJ], float (&s)[TT],
         v[t][j][i] -= s[t];
         q = __builtin_fmaf(v[t][j][i], v[t][j][i], q);
       }
-    part[wave * (TT * 16) + t * 16 + (lane & 15)] = floatx2{s[t], groups_sum(q)};  // (the four lane groups hold the same)
+    part[wave * (TT * 16) + t * 16 + (lane & 15)] = floatx2{s[t], sum_over_rows(q)};  // (the four lane groups hold the same)
   }
   lds_barrier();
   half8 w[NJ / 2], b[NJ / 2];

@@ -698,8 +698,8 @@ struct SlabCursor {
 
 struct SlabRows {      // what the cursors need to find rows
   const intx4 *table;  // LDS: n_rows entries (row, first vector, end vector, 1) and an all-zero entry behind them
-  int *counter;        // LDS: the number of positions claimed so far (in the entry behind the table's last)
-  int n_rows, lane;
+  int *counter;        // LDS: the number of positions claimed so far, behind those of the waves' first rows (in the entry behind the table's last)
+  int n_rows, lane, wave;
 };
 
 // Lane 0 takes the next position (the append instruction that would do it for a whole wave addresses only the
@@ -712,7 +712,7 @@ __device__ __forceinline__ int cursor_claim(const SlabRows &rows, int spent) {
 }
 
 __device__ __forceinline__ void cursor_prefetch(SlabCursor &c, const SlabRows &rows) {
-  const int idx = __builtin_amdgcn_readfirstlane(c.claim);
+  const int idx = __builtin_amdgcn_readfirstlane(c.claim) + kSlabWaves;  // (the first sixteen go to the waves in their order, unasked)
   c.next = rows.table[min(idx, rows.n_rows)];  // positions beyond the block read the all-zero entry: not valid
   c.claim = cursor_claim(rows, c.claim);
 }
@@ -928,28 +928,36 @@ struct SlabCtx {
   uint32_t c_vrow_bytes;
 };
 
-// One wave's share of a work item: the vector-rows it claims from the item's row table,
-// against the slab at byte offset slab_base of LDS.
-template <int V, typename OutT, int NQ, int L, bool RAGGED, typename Out>
-__device__ __forceinline__ void slab_process_item(const SlabCtx<V, OutT> &x, unsigned char *lds, uint32_t slab_base,
-                                                  const SlabRows &rows, const uint16_t *vals,
-                                                  __amdgpu_buffer_rsrc_t srd_c, const Out &out) {
+// One wave's share of a work item: the vector-rows it claims from the item's row table, against the slab at byte offset
+// slab_base of LDS.  slab_begin claims the first rows, brings their first steps on their way: it needs the row table, not
+// the slab.
+template <int V, int NQ>
+struct SlabRing {
   SlabCursor head;  // issues loads
+  SlabLoads<V> ld[slab_ring(NQ)];
+};
+template <int V, typename OutT, int NQ>
+__device__ __forceinline__ void slab_begin(SlabRing<V, NQ> &ring, const SlabCtx<V, OutT> &x, const SlabRows &rows, const uint16_t *vals) {
+  SlabCursor &head = ring.head;
+  head.next = rows.table[min(rows.wave, rows.n_rows)];
   head.claim = cursor_claim(rows, 0);
-  cursor_prefetch(head, rows);
   cursor_take_next(head, rows);
-  if (!head.valid) return;
-
-  constexpr int R = slab_ring(NQ);
-  SlabLoads<V> ld[R];
 #pragma unroll
-  for (int i = 0; i < R - 1; ++i) {
+  for (int i = 0; i < slab_ring(NQ) - 1; ++i) {
     // Loads are issued whether or not the head still has a step (an exhausted head has kc = end = 0:
     // the value load is out of bounds and returns zeros), so that the number of loads in flight
     // behind any ring slot is a compile-time constant and the waits below can be exact.
-    slab_issue<V>(ld[i], head.row, head.kc, head.end, head.valid, x.lane, x.slot0, x.srd_cols, vals);
+    slab_issue<V>(ring.ld[i], head.row, head.kc, head.end, head.valid, x.lane, x.slot0, x.srd_cols, vals);
     if (head.valid) cursor_advance(head, rows);
   }
+}
+template <int V, typename OutT, int NQ, int L, bool RAGGED, typename Out>
+__device__ __forceinline__ void slab_run(SlabRing<V, NQ> &ring, const SlabCtx<V, OutT> &x, unsigned char *lds, uint32_t slab_base,
+                                         const SlabRows &rows, const uint16_t *vals, __amdgpu_buffer_rsrc_t srd_c, const Out &out) {
+  constexpr int R = slab_ring(NQ);
+  SlabCursor &head = ring.head;
+  SlabLoads<V>(&ld)[R] = ring.ld;
+  if (!ld[0].valid) return;
   // the value tile of the first step
   SlabVals<V>::put(x.val_dst, ld[0].vraw);
 
@@ -1179,13 +1187,16 @@ __global__ __launch_bounds__(kSlabThreads) void spmm_slab_kernel(const SpmmArgs 
       // (the entries at rows_per_block and behind it are rewritten, all zeros, with every table)
       rows.counter = reinterpret_cast<int *>(lds + table_off + table_sel * table_bytes + (p.rows_per_block + 1u) * 16u);
       rows.lane = lane;
+      rows.wave = wave;
       SlabStore<V, OutT, NQ> out;
       out.init(lane, (int)cur.tile * (16 * NQ), p.N);
       // One buffer descriptor spans this batch element's C (the launcher checks it is at most 2 GiB).
       const __amdgpu_buffer_rsrc_t srd_c = make_srd(reinterpret_cast<OutT *>(p.C) + (int64_t)cur.batch * p.stride_C,
                                                     (uint32_t)p.m_vec * x.c_vrow_bytes);
-      slab_process_item<V, OutT, NQ, L, RAGGED>(x, lds, layout_buffer_off(L, NQ, zero_row + 1u, slab_sel), rows, p.values + (int64_t)cur.batch * p.stride_values,
-                                 srd_c, out);
+      SlabRing<V, NQ> ring;
+      const uint16_t *const vals = p.values + (int64_t)cur.batch * p.stride_values;
+      slab_begin(ring, x, rows, vals);
+      slab_run<V, OutT, NQ, L, RAGGED>(ring, x, lds, layout_buffer_off(L, NQ, zero_row + 1u, slab_sel), rows, vals, srd_c, out);
     }
     if (!has_next) break;
 
@@ -1248,10 +1259,11 @@ __global__ __launch_bounds__(kSlabThreads) void spmm_slab_kernel(const SpmmArgs 
 //   LDS: x (then x + a, then its LayerNorm, then that + y): hidden rows; the context, then the hidden features: ffn rows; a zero
 //   row behind either; value tiles, row tables of the three products, biases.  The workgroups of 64 consecutive tokens share
 //   an XCD (ids 8 apart), so that a line of x, context or result crosses the fabric once.
-// 768 features, 3072 hidden, V = 16 at 90 %, 4096 tokens (a workgroup per CU): 42 us, where the five launches took 5, 11, 15, 14
-// and 11; the layer 82 -> 62 us.  1200 steps of 32 vectors a workgroup: bound by the step's chain (value tile to LDS and
+// 768 features, 3072 hidden, V = 16 at 90 %, 4096 tokens (a workgroup per CU): 39 us, where the five launches took 5, 11, 15, 14
+// and 11; the layer 82 -> 59.6 us.  1200 steps of 32 vectors a workgroup: bound by the step's chain (value tile to LDS and
 // back, rows of the slab, MFMA) on four waves per SIMD, 29 ns a step and CU as in the slab kernel, and by the 7 us of vector
-// instructions of 49 000 GELUs.
+// instructions of 49 000 GELUs.  Of a workgroup's 71 000 cycles 5800 are the row tables' way to LDS, 10 800, 22 600 and 13 200 the products
+// (the first with x's and the context's), 900 the start of each, 2 to 3000 the wait for the last wave, 3700 a LayerNorm.
 struct SlabTailStore {
   unsigned char *rows;   // LDS: row r of the product at rows + 32 r
   const _Float16 *bias;  // LDS
@@ -1273,39 +1285,61 @@ struct SlabTailStore {
 
 // LayerNorm of the 16 tokens over H rows (16 waves; H <= 1024), statistics in fp32, mean first.  dst: the rows' own place, or
 // memory with `pitch` elements between rows, `left` of the thread's four tokens.  Contains barriers; every thread must call it.
+// gamma and beta of a thread's rows are fetched in front of the first product.  A LayerNorm is a chain on four waves per SIMD, the same 4600 cycles
+// for 256 features as for 768: every step of it counts.  (7100 with the sums put together by sixteen reads a thread, all four components in every exchange
+// and gamma loaded here, 9600 with the vector-memory drain of the general barrier too.)
+struct SlabTailNormWeights {
+  _Float16 w[4], b[4];
+  __device__ __forceinline__ void load(const uint16_t *gamma, const uint16_t *beta, int H) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int h = (threadIdx.x >> 2) + u * (kSlabThreads / 4);
+      w[u] = (_Float16)1;
+      b[u] = (_Float16)0;
+      if (h < H) {
+        w[u] = reinterpret_cast<const _Float16 *>(gamma)[h];
+        if (beta) b[u] = reinterpret_cast<const _Float16 *>(beta)[h];
+      }
+    }
+  }
+};
+// Sums over the lanes of a wave with the same lane % 4, of component 0, 2, 1, 3 of v in the first to fourth sixteen lanes: the exchanges
+// that add two lanes' values up carry two components at a time.
+__device__ __forceinline__ float slab_tail_token_sum(const floatx4 &v) {
+  const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[0]), __float_as_uint(v[1]), false, false);
+  const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[2]), __float_as_uint(v[3]), false, false);
+  const float a = __uint_as_float(p[0]) + __uint_as_float(p[1]), b = __uint_as_float(q[0]) + __uint_as_float(q[1]);
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  float c = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  c += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(c), 0x128, 0xf, 0xf, false));  // rotated by 8 in each 16
+  c += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(c), 0x124, 0xf, 0xf, false));  // and by 4
+  return c;
+}
 template <bool TO_MEMORY, bool RAGGED>
-__device__ __forceinline__ void slab_tail_norm(unsigned char *rows, int H, const _Float16 *gamma, const _Float16 *beta, float eps,
-                                               floatx4 (*red)[kSlabWaves][4], _Float16 *dst, int64_t pitch, int left) {
+__device__ __forceinline__ void slab_tail_norm(unsigned char *rows, int H, const SlabTailNormWeights &weights, float eps,
+                                               float (*red)[16][kSlabWaves], float *own, _Float16 *dst, int64_t pitch, int left) {
   constexpr int TRIP = 4, kGroups = kSlabThreads / 4;
   const int tid = threadIdx.x, tl = tid & 3, rg = tid >> 2, lane = tid & 63, wave = tid >> 6;
   half4 s[TRIP];
-  float w[TRIP], b[TRIP];
   floatx4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int u = 0; u < TRIP; ++u) {
     const int h = rg + u * kGroups;
     s[u] = half4{0, 0, 0, 0};
-    w[u] = 1.0f;
-    b[u] = 0.0f;
-    if (h < H) {
-      s[u] = *reinterpret_cast<const half4 *>(rows + h * 32 + tl * 8);
-      w[u] = (float)gamma[h];
-      if (beta) b[u] = (float)beta[h];
-    }
+    if (h < H) s[u] = *reinterpret_cast<const half4 *>(rows + h * 32 + tl * 8);
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[i] += (float)s[u][i];
   }
   floatx4 stat[2];  // mean, 1 / deviation
 #pragma unroll
   for (int pass = 0; pass < 2; ++pass) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] = sum_over_quads(acc[i]);
-    if (lane < 4) red[pass][wave][tl] = acc;
-    __syncthreads();
-    floatx4 sum = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int v = 0; v < kSlabWaves; ++v) sum += red[pass][v][tl];
-    stat[pass] = sum;
+    const float mine = slab_tail_token_sum(acc);
+    if ((lane & 12) == 0) red[pass][4 * tl + 2 * (lane >> 4 & 1) + (lane >> 5)][wave] = mine;
+    lds_barrier();
+    const floatx4 four = *reinterpret_cast<const floatx4 *>(&red[pass][lane & 15][4 * (lane >> 4)]);
+    const float all = sum_over_rows((four[0] + four[1]) + (four[2] + four[3]));
+    if (lane < 16) own[lane] = all;
+    stat[pass] = *reinterpret_cast<const floatx4 *>(own + 4 * tl);
     if (pass == 0) {
       stat[0] *= 1.0f / (float)H;
       acc = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -1328,7 +1362,7 @@ __device__ __forceinline__ void slab_tail_norm(unsigned char *rows, int H, const
     if (h >= H) break;
     half4 o;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = (_Float16)(((float)s[u][i] - stat[0][i]) * stat[1][i] * w[u] + b[u]);
+    for (int i = 0; i < 4; ++i) o[i] = (_Float16)(((float)s[u][i] - stat[0][i]) * stat[1][i] * (float)weights.w[u] + (float)weights.b[u]);
     if (!TO_MEMORY) *reinterpret_cast<half4 *>(rows + h * 32 + tl * 8) = o;
     else if (left > 0) store_four<RAGGED>(dst + (int64_t)h * pitch + 4 * tl, o, left);
   }
@@ -1349,7 +1383,7 @@ __host__ __device__ inline SlabTailLds slab_tail_lds(int V, int hidden, int ffn)
     at += (rows[i] / (uint32_t)V + 2u) * 16u;
   }
   o.red = at;
-  at += 2u * kSlabWaves * 4u * 16u;
+  at += 2u * 16u * kSlabWaves * 4u;
   for (int i = 0; i < 3; ++i) {
     o.bias[i] = at;
     at += rows[i] * 2u;
@@ -1370,6 +1404,16 @@ __global__ __launch_bounds__(kSlabThreads) void encoder_tail_kernel(const Encode
   const SlabTailLds at = slab_tail_lds(V, H, F);
   const int left = p.tokens - first - 4 * (tid & 3);  // tokens from the thread's four on
 
+  // The row tables first: the first product's first steps are on their way while x and the context arrive, and those of the second and
+  // the third before the barrier in front of them, beside the slower waves, the LayerNorm and what it waits for.
+  intx4 entry[3];
+  const int out_rows[3] = {H, F, H};
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const int n = out_rows[i] / V;
+    entry[i] = intx4{0, 0, 0, 0};
+    if (tid < n) entry[i] = intx4{tid, p.w[i].row_offsets[tid], p.w[i].row_offsets[tid + 1], 1};
+  }
   const _Float16 *const xg = reinterpret_cast<const _Float16 *>(p.x) + first, *const cg = reinterpret_cast<const _Float16 *>(p.context) + first;
   half4 xs[4], cs[4];
 #pragma unroll
@@ -1381,20 +1425,48 @@ __global__ __launch_bounds__(kSlabThreads) void encoder_tail_kernel(const Encode
       xs[u] = load_four<RAGGED>(xg + (int64_t)h * p.tokens + 4 * (tid & 3), left);
     }
   }
-  const int out_rows[3] = {H, F, H};
+  // (at most 1024 rows, and as many hidden ones as have 32 bytes of LDS each)
+  constexpr int kTrips[3] = {1, 160 * 1024 / 32 / kSlabThreads, 1};
+  _Float16 bias[3][kTrips[1]];
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int u = 0; u < kTrips[i]; ++u) {
+      const int r = tid + u * kSlabThreads;
+      bias[i][u] = (_Float16)0;
+      if (r < out_rows[i] && p.w[i].bias) bias[i][u] = reinterpret_cast<const _Float16 *>(p.w[i].bias)[r];
+    }
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+    if (tid < out_rows[i] / V + 2) reinterpret_cast<intx4 *>(lds + at.tables[i])[tid] = entry[i];
+  lds_barrier();
+
+  SlabCtx<V, _Float16> x[3];
+  SlabRows rows[3];
+  SlabRing<V, 1> ring[3];
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     const int n = out_rows[i] / V;
-    intx4 *const table = reinterpret_cast<intx4 *>(lds + at.tables[i]);
-    for (int r = tid; r < n + 2; r += kSlabThreads) {
-      intx4 e = {0, 0, 0, 0};
-      if (r < n) e = intx4{r, p.w[i].row_offsets[r], p.w[i].row_offsets[r + 1], 1};
-      table[r] = e;
-    }
-    _Float16 *const bias = reinterpret_cast<_Float16 *>(lds + at.bias[i]);
-    for (int r = tid; r < out_rows[i]; r += kSlabThreads)
-      bias[r] = p.w[i].bias ? reinterpret_cast<const _Float16 *>(p.w[i].bias)[r] : (_Float16)0;
+    x[i].lane = lane;
+    x[i].val_tile = lds + at.tiles + wave * wave_lds_bytes(V);
+    x[i].val_dst = x[i].val_tile + lane * SlabVals<V>::kLane;
+    x[i].a_off = (uint32_t)(4 * g + (m >> 2)) * (V * 2u) + (uint32_t)(m & 3) * 8u;
+    x[i].slot0 = (uint32_t)(4 * g + (m >> 2));
+    x[i].b_lane_off = (uint32_t)(m & 3) * 8u;
+    x[i].c_vrow_bytes = V * 32u;
+    x[i].zero_row = (uint32_t)(i == 2 ? F : H);
+    // (in scalar registers, or every load of column indices becomes a loop over the lanes' descriptors)
+    x[i].srd_cols = make_srd(p.w[i].col_idx, (uint32_t)__builtin_amdgcn_readfirstlane(p.w[i].row_offsets[n]) * 4u);
+    rows[i].table = reinterpret_cast<const intx4 *>(lds + at.tables[i]);
+    rows[i].n_rows = n;
+    rows[i].counter = reinterpret_cast<int *>(lds + at.tables[i] + (n + 1) * 16);
+    rows[i].lane = lane;
+    rows[i].wave = wave;
   }
+  slab_begin(ring[0], x[0], rows[0], p.w[0].values);
+  SlabTailNormWeights norm1, norm2;
+  norm1.load(p.gamma1, p.beta1, H);
+  norm2.load(p.gamma2, p.beta2, H);
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     const int h = (tid >> 2) + u * (kSlabThreads / 4);
@@ -1403,51 +1475,38 @@ __global__ __launch_bounds__(kSlabThreads) void encoder_tail_kernel(const Encode
       *reinterpret_cast<half4 *>(lds + at.wide + h * 32 + (tid & 3) * 8) = cs[u];
     }
   }
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int u = 0; u < kTrips[i]; ++u)
+      if (tid + u * kSlabThreads < out_rows[i]) reinterpret_cast<_Float16 *>(lds + at.bias[i])[tid + u * kSlabThreads] = bias[i][u];
   if (tid < 8) {  // the zero rows behind x and the context
     *reinterpret_cast<half4 *>(lds + (tid < 4 ? 0u : at.wide) + H * 32 + (tid & 3) * 8) = half4{0, 0, 0, 0};
   }
-  __syncthreads();
+  lds_barrier();
 
-  SlabCtx<V, _Float16> x;
-  x.lane = lane;
-  x.val_tile = lds + at.tiles + wave * wave_lds_bytes(V);
-  x.val_dst = x.val_tile + lane * SlabVals<V>::kLane;
-  x.a_off = (uint32_t)(4 * g + (m >> 2)) * (V * 2u) + (uint32_t)(m & 3) * 8u;
-  x.slot0 = (uint32_t)(4 * g + (m >> 2));
-  x.b_lane_off = (uint32_t)(m & 3) * 8u;
-  x.c_vrow_bytes = V * 32u;
-  floatx4(*const red)[kSlabWaves][4] = reinterpret_cast<floatx4(*)[kSlabWaves][4]>(lds + at.red);
+  float(*const red)[16][kSlabWaves] = reinterpret_cast<float(*)[16][kSlabWaves]>(lds + at.red);
+  float *const own = reinterpret_cast<float *>(lds + at.tiles + wave * wave_lds_bytes(V));  // (between the products the wave's value tile is free)
   SlabTailStore out;
   out.lane = lane;
   out.last = V - 1;
   // (unrolled: what differs between the products is known to the compiler)
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
-    const int n = (i == 1 ? F : H) / V;
-    const uint32_t table = at.tables[i];
-    SlabRows rows;
-    rows.table = reinterpret_cast<const intx4 *>(lds + table);
-    rows.n_rows = n;
-    rows.counter = reinterpret_cast<int *>(lds + table + (n + 1) * 16);
-    rows.lane = lane;
-    x.zero_row = (uint32_t)(i == 2 ? F : H);
-    // (in scalar registers, or every load of column indices becomes a loop over the lanes' descriptors)
-    x.srd_cols = make_srd(p.w[i].col_idx, (uint32_t)__builtin_amdgcn_readfirstlane(p.w[i].row_offsets[n]) * 4u);
     out.rows = lds + (i == 1 ? at.wide : 0u);
     out.bias = reinterpret_cast<const _Float16 *>(lds + at.bias[i]);
     out.act = i == 1 ? 1 : 0;
     out.add = i != 1;
-    slab_process_item<V, _Float16, 1, kXorSingle, false>(x, lds, i == 1 ? 0u : at.wide, rows, p.w[i].values, x.srd_cols, out);
-    __syncthreads();
+    slab_run<V, _Float16, 1, kXorSingle, false>(ring[i], x[i], lds, i == 1 ? 0u : at.wide, rows[i], p.w[i].values, x[i].srd_cols, out);
+    if (i < 2) slab_begin(ring[i < 2 ? i + 1 : 2], x[i < 2 ? i + 1 : 2], rows[i < 2 ? i + 1 : 2], p.w[i < 2 ? i + 1 : 2].values);
+    lds_barrier();
     if (i == 0) {
       if (tid < 4) *reinterpret_cast<half4 *>(lds + at.wide + F * 32 + tid * 8) = half4{0, 0, 0, 0};  // (the context has been read)
-      slab_tail_norm<false, RAGGED>(lds, H, reinterpret_cast<const _Float16 *>(p.gamma1), reinterpret_cast<const _Float16 *>(p.beta1), p.eps1, red,
-                                    nullptr, 0, left);
-      __syncthreads();
+      slab_tail_norm<false, RAGGED>(lds, H, norm1, p.eps1, red, own, nullptr, 0, left);
+      lds_barrier();
     }
   }
-  slab_tail_norm<true, RAGGED>(lds, H, reinterpret_cast<const _Float16 *>(p.gamma2), reinterpret_cast<const _Float16 *>(p.beta2), p.eps2, red,
-                               reinterpret_cast<_Float16 *>(p.out) + first, p.tokens, left);
+  slab_tail_norm<true, RAGGED>(lds, H, norm2, p.eps2, red, own, reinterpret_cast<_Float16 *>(p.out) + first, p.tokens, left);
 }
 
 // ------------------------------------------------------------------------------------------

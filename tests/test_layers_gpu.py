@@ -475,6 +475,15 @@ def test_encoder_layers_tail_matches_dense_fp32_products(built_library, V, bias,
     assert max_rel_err(got.float().cpu().numpy(), want.float().cpu().numpy()) <= 2.0 ** -8
 
 
+@pytest.mark.parametrize("V,hidden,ffn,tokens", [(16, 16, 4112, 20), (8, 64, 4096, 33), (8, 72, 64, 16), (16, 256, 96, 65), (16, 1024, 2048, 18)])
+def test_encoder_layers_tail_of_few_and_of_most_rows(built_library, V, hidden, ffn, tokens):
+    """Fewer vector-rows than a workgroup has waves, and as many hidden features as fit: the bound of the test above."""
+    from sspmm_amd.layers import encoder_tail_fits
+    assert encoder_tail_fits(hidden, ffn, tokens, V)
+    for bias in (True, False):
+        test_encoder_layers_tail_matches_dense_fp32_products(built_library, V, bias, hidden, ffn, tokens)
+
+
 def test_encoder_layers_tail_runs_on_the_weights_of_that_moment(built_library, monkeypatch):
     """A hook behind the projections that gives the layer other weights: the launch behind the attention has their addresses,
     not those of the arrays that went away (looked at without launching), and its result is the one with them."""
