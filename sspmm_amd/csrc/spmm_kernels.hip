@@ -1285,9 +1285,9 @@ struct SlabTailStore {
 
 // LayerNorm of the 16 tokens over H rows (16 waves; H <= 1024), statistics in fp32, mean first.  dst: the rows' own place, or
 // memory with `pitch` elements between rows, `left` of the thread's four tokens.  Contains barriers; every thread must call it.
-// gamma and beta of a thread's rows are fetched in front of the first product.  A LayerNorm is a chain on four waves per SIMD, the same 4600 cycles
-// for 256 features as for 768: every step of it counts.  (7100 with the sums put together by sixteen reads a thread, all four components in every exchange
-// and gamma loaded here, 9600 with the vector-memory drain of the general barrier too.)
+// gamma and beta of a thread's rows are fetched in front of the first product.  A LayerNorm is a chain on four waves per SIMD, 3300 cycles for 256
+// features as 3700 for 768: every step of it counts.  (768 features: 9600 with the waves' sums put together by sixteen reads a thread, all four components in every
+// exchange and gamma loaded here; 7100 with a read a lane for the sums and gamma in front of the barrier; 5000 with gamma at the start.)
 struct SlabTailNormWeights {
   _Float16 w[4], b[4];
   __device__ __forceinline__ void load(const uint16_t *gamma, const uint16_t *beta, int H) {
