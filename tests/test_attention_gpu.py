@@ -187,6 +187,32 @@ def test_one_launch_attention_row_lengths_permutation_and_large_scores(built_lib
     assert (one.float() - chain.float()).abs().max().item() <= 3e-2
 
 
+@pytest.mark.parametrize("gap", [7.0, 9.0, 10.5, 12.0])
+def test_one_launch_attentions_with_many_small_probabilities(built_library, gap):
+    """One key ahead of all others by gap^2 / 8, 6 to 18 in the exponent, so that the others' probabilities are small, subnormal in
+    fp16 or nothing there: together they are a good part of the sum.  A probability's rounding is 2^-25 at most there
+    (half a step), one for each key, and 2^-11 of it above; the result's rounding is 2^-11 of values of about one."""
+    from sspmm_amd.layers import attention_fm
+    keys, d = 4096, 64
+    x = np.float16(gap)
+    q, k = np.zeros((1, 64, d), np.float16), np.zeros((1, keys, d), np.float16)
+    q[..., 0], k[0, 0, 0] = x, x
+    v = np.where(np.arange(keys) % 2, 1.0, 0.5)[None, :, None].repeat(d, 2).astype(np.float16)
+    v[0, 0] = -1.0
+    bound = keys * 2.0 ** -25 + 2.0 ** -10
+    for V in (8, 16):
+        off = (np.arange(64 // V + 1) * keys).astype(np.int32)
+        cols = np.tile(np.arange(keys, dtype=np.int32), 64 // V)
+        want = _dense_attention(off, cols, V, q, k, v, 0.125)
+        got = sspmm_amd.fused_sparse_attention(None, dev(off), dev(cols), dev(q), dev(k), dev(v), 0.125, V)
+        assert np.abs(got.cpu().numpy() - want).max() <= bound
+    for seq in (keys, keys - 4):
+        qkv = np.concatenate([np.broadcast_to(q[0, :1], (seq, d)).T, k[0, :seq].T, v[0, :seq].T])
+        want = _dense_attention(np.array([0, seq], np.int32), np.arange(seq), 1, q[:, :1], k, v, 0.125)[0, 0]
+        got = attention_fm(dev(np.ascontiguousarray(qkv)), d, 1, 1, seq)
+        assert np.abs(got.cpu().numpy() - want[:, None]).max() <= bound
+
+
 def test_one_launch_attention_at_full_size_by_its_properties(built_library):
     """The benchmark's block (4096 tokens, 90 % of the vectors masked out, 48 heads of 64 features): with every row of
     v the same the probabilities of a row must add up to one, so every query gets that row back; columns stored in
