@@ -649,7 +649,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(attention_wa
   floatx4 acc[NT];
 #pragma unroll
   for (int u = 0; u < NT; ++u) acc[u] = floatx4{0.f, 0.f, 0.f, 0.f};
-  float run_max = -INFINITY, run_sum = 0.f;  // of query n; the sum only over this lane's share of the keys
+  float run_raw = -INFINITY, run_max = -INFINITY, run_sum = 0.f;  // of query n: maximum before and after the scale; the sum only over this lane's share of the keys
+  // Some query's scaled maximum lies beyond 2^10 (uniform).  An exponent x scale2 - run_max misses by the rounding of run_max, the same for every key: beyond 2^28
+  // the largest probability would be 2^16 or 0, so there the difference is taken first, which is 0 at the maximum; below 2^10 it is 2^-15 and cancels in the quotient.  Costs 2 us of 507 in
+  // a model of 8 x 4096 tokens; taken first everywhere it is the additions that the multiply-add saves.
+  bool far = false;
 
   float x[8];
   const auto scores = [&] {
@@ -674,18 +678,27 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(attention_wa
           if (kc + 16 * t + 4 * g + i >= end) x[4 * t + i] = -INFINITY;
     }
     float mx = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
-    mx = quad_rows_max(mx) * scale2;  // finite: the step's first slot is always a stored vector
-    const float new_max = fmaxf(run_max, mx);
-    if (__builtin_amdgcn_ballot_w64(new_max > run_max)) {  // (uniform) some query's maximum moved
-      const float alpha = __builtin_amdgcn_exp2f(run_max - new_max);
+    mx = quad_rows_max(mx);  // finite: the step's first slot is always a stored vector
+    const float new_raw = fmaxf(run_raw, mx);  // (scale2 > 0: the order of the scaled scores)
+    if (__builtin_amdgcn_ballot_w64(new_raw > run_raw)) {  // (uniform) some query's maximum moved
+      const float alpha = __builtin_amdgcn_exp2f((run_raw - new_raw) * scale2);
       run_sum *= alpha;
 #pragma unroll
       for (int u = 0; u < NT; ++u) acc[u] *= alpha;
-      run_max = new_max;
+      run_raw = new_raw;
+      run_max = new_raw * scale2;
+      far = __builtin_amdgcn_ballot_w64(fabsf(run_max) > 1024.f) != 0;
+    }
+    if (far) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = (x[i] - run_raw) * scale2;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = __builtin_fmaf(x[i], scale2, -run_max);
     }
     half8 pb;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) pb[i] = (_Float16)__builtin_amdgcn_exp2f(__builtin_fmaf(x[i], scale2, -run_max));
+    for (int i = 0; i < 8; ++i) pb[i] = (_Float16)__builtin_amdgcn_exp2f(x[i]);
     // (the sum of what the product takes: the rounding of the largest probabilities cancels in the quotient)
     const uintx4 pairs = __builtin_bit_cast(uintx4, pb);
 #pragma unroll

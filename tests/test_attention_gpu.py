@@ -213,6 +213,25 @@ def test_one_launch_attentions_with_many_small_probabilities(built_library, gap)
         assert np.abs(got.cpu().numpy() - want[:, None]).max() <= bound
 
 
+@pytest.mark.parametrize("V,d", [(8, 32), (8, 64), (16, 64), (8, 128), (16, 128)])
+def test_one_launch_attention_with_scores_of_any_size(built_library, V, d):
+    """Scaled scores from a fraction to 2^32, of either sign: the largest probability is one whatever fp32 makes of its exponent.  A
+    score is one exact product, so what is left is the rounding of the probabilities and of the result to fp16, 2^-11 each of values
+    up to one, and of the exponents, under 2^-14 while a maximum moves."""
+    keys, rows = 133, 64
+    rng = np.random.default_rng(V + d)
+    q, k = np.zeros((2, rows, d), np.float16), np.zeros((2, keys, d), np.float16)
+    q[..., 0] = np.exp2(rng.uniform(-8, 15.9, (2, rows))) * rng.choice([-1.0, 1.0], (2, rows))
+    k[..., 0] = np.exp2(rng.uniform(-4, 15.9, (2, keys)))
+    k[1] = np.sort(k[1], axis=0)  # (every step moves the maximum)
+    v = rng.uniform(-1, 1, (2, keys, d)).astype(np.float16)
+    off = (np.arange(rows // V + 1) * keys).astype(np.int32)
+    cols = np.tile(np.arange(keys, dtype=np.int32), rows // V)
+    want = _dense_attention(off, cols, V, q, k, v, 1.0)
+    got = sspmm_amd.fused_sparse_attention(None, dev(off), dev(cols), dev(q), dev(k), dev(v), 1.0, V).cpu().numpy()
+    assert np.abs(got - want).max() <= 2.0 ** -10 + 2.0 ** -13
+
+
 def test_one_launch_attention_at_full_size_by_its_properties(built_library):
     """The benchmark's block (4096 tokens, 90 % of the vectors masked out, 48 heads of 64 features): with every row of
     v the same the probabilities of a row must add up to one, so every query gets that row back; columns stored in
