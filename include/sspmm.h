@@ -468,16 +468,27 @@ int sspmm_block_pack_f16(int count, const sspmm_half_t *const *src, const int32_
  * packed in groups of E / 4 rows, each row times a power of two that puts its largest element between 2^13 and 2^14;
  * affine + i * 2 * E: what undoes that, E values, and W2 b1 + b2, E values.  b1[i] and b2[i] may be NULL.  E = 128, 256 or
  * 512, mlp[i] a multiple of 256 up to 2^20; 16-byte aligned pointers, b2[i] excepted.  The arrays of pointers and sizes are host memory and are read
- * before the call returns.
+ * before the call returns.  An element of w21 is rounded to fp16 (2^-11 of it, or 2^-38 of its row's largest), where the
+ * layers one after the other take the weights as they are and round the hidden features: what W1 cancels (a mean along its
+ * rows, a large beta2 that b1 takes back) is not cancelled then, and such weights lose up to a factor of |n| |W21| over
+ * |W2| |W1 n + b1|.  sspmm_block_fold_split_f16 also keeps what the rounding leaves: w21_rest + i * E * E, rounded to
+ * fp16 in turn, as w21 in all else, and the two together miss the fp32 sums by 2^-22 of an element or 2^-38 of the
+ * row's largest (w21_rest NULL: not kept).
  */
 int sspmm_block_fold_f16(int count, const sspmm_half_t *const *src, const int32_t *rows, const int32_t *cols,
                          const int32_t *group, sspmm_half_t *dst, int folds, int E, const int32_t *mlp,
                          const sspmm_half_t *const *w1, const sspmm_half_t *const *b1, const sspmm_half_t *const *w2,
                          const sspmm_half_t *const *b2, sspmm_half_t *w21, float *affine, void *hip_stream);
+int sspmm_block_fold_split_f16(int count, const sspmm_half_t *const *src, const int32_t *rows, const int32_t *cols,
+                               const int32_t *group, sspmm_half_t *dst, int folds, int E, const int32_t *mlp,
+                               const sspmm_half_t *const *w1, const sspmm_half_t *const *b1, const sspmm_half_t *const *w2,
+                               const sspmm_half_t *const *b2, sspmm_half_t *w21, sspmm_half_t *w21_rest, float *affine,
+                               void *hip_stream);
 
 /*
- * sspmm_block_dense_f16 with x' = n W21^T + (W2 b1 + b2) + x from what sspmm_block_fold_f16 leaves; attn is needed.  The hidden
- * features are never made, so nothing is rounded there, nor becomes infinite beyond what fp16 holds.
+ * sspmm_block_dense_f16 with x' = n W21^T + (W2 b1 + b2) + x from what sspmm_block_fold_f16 leaves, or (split) with
+ * n W21^T + n W21rest^T; attn is needed.  The hidden features are never made, so they are not rounded, and do not become
+ * infinite beyond what fp16 holds; W21 is what has been rounded (above).
  */
 int sspmm_block_dense_folded_f16(int outer, int inner, int E, const sspmm_half_t *x, int64_t x_outer, int64_t x_inner,
                                  const sspmm_half_t *attn, const sspmm_half_t *wo, const sspmm_half_t *bo,
@@ -486,6 +497,13 @@ int sspmm_block_dense_folded_f16(int outer, int inner, int E, const sspmm_half_t
                                  const sspmm_half_t *beta_n, float eps_n, int n_out, int head_dim,
                                  const sspmm_half_t *wt, const sspmm_half_t *bt, sspmm_half_t *x_out, sspmm_half_t *out,
                                  void *hip_stream);
+int sspmm_block_dense_split_f16(int outer, int inner, int E, const sspmm_half_t *x, int64_t x_outer, int64_t x_inner,
+                                const sspmm_half_t *attn, const sspmm_half_t *wo, const sspmm_half_t *bo,
+                                const sspmm_half_t *gamma2, const sspmm_half_t *beta2, float eps2,
+                                const sspmm_half_t *w21, const sspmm_half_t *w21_rest, const float *affine,
+                                const sspmm_half_t *gamma_n, const sspmm_half_t *beta_n, float eps_n, int n_out,
+                                int head_dim, const sspmm_half_t *wt, const sspmm_half_t *bt, sspmm_half_t *x_out,
+                                sspmm_half_t *out, void *hip_stream);
 
 /* ------------------------------------------------------------------------------------------
  * Dense attention on feature-major activations: out = softmax(Q^T K * scale) V per (batch element,

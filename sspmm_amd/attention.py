@@ -225,9 +225,13 @@ def pack_weights(linears, rows_per_wave):
     return packed.split(sizes)
 
 
+class FoldedLayers(tuple):
+    """(matrix, affine) of two linear layers with nothing between them, and `rest`, what the matrix's rounding to fp16 left."""
+
+
 def fold_blocks(blocks, linears, rows_per_wave):
     """pack_weights(linears, rows_per_wave), and in the same launch linear1 and linear2 of every block as the one linear map they
-    are, there being nothing between them: (packed, [(matrix, affine) per block]) for block_dense's `folded`."""
+    are, there being nothing between them: (packed, [FoldedLayers per block]) for block_dense's `folded`."""
     n, f, E = len(linears), len(blocks), blocks[0].embed_dim
     weights = [_weights(m)[0] for m in linears]
     shapes = [w.shape for w in weights]
@@ -235,16 +239,20 @@ def fold_blocks(blocks, linears, rows_per_wave):
     device = weights[0].device
     pairs = [_parts(b, "linear1", "linear2") for b in blocks]
     up, down = [_weights(a) for a, _ in pairs], [_weights(b) for _, b in pairs]
-    packed = torch.empty(sum(sizes) + f * E * E, dtype=torch.float16, device=device)
+    packed = torch.empty(sum(sizes) + 2 * f * E * E, dtype=torch.float16, device=device)
     affine = torch.empty((f, 2 * E), dtype=torch.float32, device=device)
     ints, ptrs, some = ctypes.c_int32 * n, ctypes.c_void_p * n, ctypes.c_void_p * f
-    rc = _lib.call(_lib.lib().sspmm_block_fold_f16, device, n, ptrs(*[w.data_ptr() for w in weights]), ints(*[r for r, _ in shapes]),
+    at = packed.data_ptr() + 2 * sum(sizes)
+    rc = _lib.call(_lib.lib().sspmm_block_fold_split_f16, device, n, ptrs(*[w.data_ptr() for w in weights]), ints(*[r for r, _ in shapes]),
                    ints(*[c for _, c in shapes]), ints(*rows_per_wave), packed.data_ptr(), f, E, (ctypes.c_int32 * f)(*[a.out_features for a, _ in pairs]),
                    some(*[w.data_ptr() for w, _ in up]), some(*[_ptr(b) for _, b in up]), some(*[w.data_ptr() for w, _ in down]),
-                   some(*[_ptr(b) for _, b in down]), packed.data_ptr() + 2 * sum(sizes), affine.data_ptr())
-    _lib.check(rc, "sspmm_block_fold_f16")
-    parts = packed.split(sizes + f * [E * E])
-    return parts[:n], list(zip(parts[n:], affine))
+                   some(*[_ptr(b) for _, b in down]), at, at + 2 * f * E * E, affine.data_ptr())
+    _lib.check(rc, "sspmm_block_fold_split_f16")
+    parts = packed.split(sizes + 2 * f * [E * E])
+    folded = [FoldedLayers(pair) for pair in zip(parts[n:], affine)]
+    for pair, rest in zip(folded, parts[n + f:]):
+        pair.rest = rest
+    return parts[:n], folded
 
 
 def block_dense(x, attn, block, norm, tail=None, keep_x=False, packed=None, head_dim=0, pos=None, scale=1.0, folded=None, table=None):
@@ -280,10 +288,10 @@ def block_dense(x, attn, block, norm, tail=None, keep_x=False, packed=None, head
     if folded is not None:
         proj, ln = _parts(block, "out_proj", "layer_norm2")
         gamma, beta = _weights(ln)
-        rc = _lib.call(_lib.lib().sspmm_block_dense_folded_f16, x.device, outer, inner, E, x.data_ptr(), stride[0], stride[1], _ptr(attn), packed[0].data_ptr(),
-                       _ptr(_weights(proj)[1]), _ptr(gamma), _ptr(beta), float(ln.eps), folded[0].data_ptr(), folded[1].data_ptr(),
+        rc = _lib.call(_lib.lib().sspmm_block_dense_split_f16, x.device, outer, inner, E, x.data_ptr(), stride[0], stride[1], _ptr(attn), packed[0].data_ptr(),
+                       _ptr(_weights(proj)[1]), _ptr(gamma), _ptr(beta), float(ln.eps), folded[0].data_ptr(), folded.rest.data_ptr(), folded[1].data_ptr(),
                        _ptr(gamma_n), _ptr(beta_n), float(norm.eps), n_out, head_dim, *last, _ptr(kept), out.data_ptr())
-        _lib.check(rc, "sspmm_block_dense_folded_f16")
+        _lib.check(rc, "sspmm_block_dense_split_f16")
         return kept, out
     if attn is None:
         own = (None, None, None, None, 0.0, 0, None, None, None, None)
@@ -357,14 +365,16 @@ def _rows_norm_applies(ln, x):
 
 
 BLOCK_FEATURES = 1 << 20  # hidden or output features that block_dense takes at most
-# Every workgroup of block_dense streams the weights whole, 64 bytes a cycle of a CU (256 features, 4096 hidden ones: 66 us a
-# block), where a library product spreads them over the chip.  Up to this many weights in a matrix the one launch is ahead all the
-# same, by what the separate launches cost the host: forward pass of one block at 64 to 4096 tokens, E x hidden features, in one launch /
-# as modules / modules with the norms fused, us: 256 x 4096 108 / 215 / 230, 512 x 4096 121-137 / 220 / 217, 256 x 8192
-# 109-121 / 225 / 230; twice as many 180-195 / 220 / 219 and 193-215 / 220 / 218, level for one block and behind once the
-# device is what is waited for (four blocks: 190 us of the device a block against 150 of the host).  From 8192 tokens
-# on there are workgroups for every CU and the one launch is ahead whatever the sizes: 512 x 16384, 8192 tokens 396 / 494 / 443 us,
-# 32768 tokens 1054 / 1449 / 1295; at 6144 tokens 365 / 406 / 359.  A head is level with the library's product at best when it is
+# However few tokens there are, a wide hidden layer costs the launch that multiplies the two linear layers its W1, which a CU streams
+# whole at 64 bytes a cycle for every sixteen rows (256 features: 8192 hidden ones 33 us more than 4096, whatever the number of
+# blocks), where library products spread the weights over the chip.  Up to this many weights in a matrix the two launches a block are ahead all
+# the same, by what the modules cost the host.  Forward pass, 64 / 512 / 4096 tokens, in these launches called one after the
+# other - as modules with the norms fused called / replayed from a graph, us: one block 256 x 4096 79 / 80 / 81 - 220 / 230 / 229, 45 / 52 / 96,
+# 256 x 8192 87 / 88 / 104 - 223 / 230 / 230, 47 / 58 / 124, four blocks of the latter 181 / 185 / 197 - 626 / 653 / 654, 164 / 186 / 454.  Twice as
+# many, 256 x 16384: 152 / 153 / 168 - 229 / 230 / 231, 58 / 70 / 176, and 512 x 8192 172 / 171 / 191 - 229 / 229 / 232, 54 / 72 / 174: called they are
+# ahead there too, replayed they would be 2.5 times as slow, so the line stays.  Beyond 4096 tokens these launches are ahead whatever the
+# sizes: 6144 tokens 512 x 16384 341 - 392, 390, 512 x 32768 590 - 668, 664, 256 x 65536 584 - 748, 750.  A head is level with the library's
+# product at best when it is
 # that large and behind beyond, with many tokens too: outputs in the launch / as a module, us of the device, 512 x 4096, 64 and
 # 32768 tokens 90 / 54 and 351 / 374, 512 x 8192 134 / 54 and 573 / 559, 256 x 65536 413 / 35 at 64 tokens and 814 / 487 at 8192.
 BLOCK_WEIGHTS = 1 << 21
@@ -562,12 +572,22 @@ class SparseAttentionEncoder(torch.nn.Module):
         final, linear = _parts(self, "layer_norm", "linear")
         head = _plain_linear(linear, like, E, None, 64) and E * linear.out_features <= BLOCK_WEIGHTS
         into, norms = [_parts(b, "in_proj")[0] for b in blocks], [_parts(b, "layer_norm1")[0] for b in blocks]
-        linears, rows = [into[0]], [64]
+        # (the two linear layers as one, in two matrices of E x E, where those are fewer weights than the two layers'.  Four blocks replayed, folded /
+        # two layers, us: 512 features, 256 hidden ones 169 / 148 at 512 tokens, 567 / 539 at 16384, 512 hidden 172 / 166, 569 / 570, 768 hidden
+        # 176 / 185, 572 / 600; 256 features, 256 hidden 74 / 72, 336 / 337, 512 hidden 76 / 83, 337 / 350)
+        fold = [_parts(b, "linear1")[0].out_features > E for b in blocks]
+        linears, rows, ends = [into[0]], [64], [1]
         for i, blk in enumerate(blocks):
             tail = [into[i + 1]] if i + 1 < len(blocks) else [linear] * head
-            linears += _parts(blk, "out_proj") + tail
-            rows += [E // 4] + [64] * len(tail)
-        packed, folded = fold_blocks(blocks, linears, rows)
+            linears += (_parts(blk, "out_proj") if fold[i] else _parts(blk, "out_proj", "linear1", "linear2")) + tail
+            rows += ([E // 4] if fold[i] else [E // 4, 64, E // 4]) + [64] * len(tail)
+            ends.append(len(linears))
+        if any(fold):
+            packed, pairs = fold_blocks([b for b, f in zip(blocks, fold) if f], linears, rows)
+            pairs = iter(pairs)
+            folded = [next(pairs) if f else None for f in fold]
+        else:
+            packed, folded = pack_weights(linears, rows), [None] * len(blocks)
 
         def attention(blk, qkv):
             # (in the pattern's own order: the longest rows last, which row_indices asks for, cost 1 to 4 %)
@@ -577,8 +597,8 @@ class SparseAttentionEncoder(torch.nn.Module):
         x, qkv = block_dense(x, None, None, norms[0], into[0], True, packed[:1], E // blocks[0].num_heads, pe, scale,
                              table=table)
         for i, blk in enumerate(blocks[:-1]):
-            x, qkv = block_dense(x, attention(blk, qkv), blk, norms[i + 1], into[i + 1], True, packed[1 + 2 * i:3 + 2 * i],
+            x, qkv = block_dense(x, attention(blk, qkv), blk, norms[i + 1], into[i + 1], True, packed[ends[i]:ends[i + 1]],
                                  E // blocks[i + 1].num_heads, folded=folded[i])
         out = block_dense(x, attention(blocks[-1], qkv), blocks[-1], final, linear if head else None,
-                          packed=packed[2 * len(blocks) - 1:], folded=folded[-1])[1]
+                          packed=packed[ends[-2]:], folded=folded[-1])[1]
         return out if head else linear(out)

@@ -32,6 +32,7 @@ struct BlockDenseArgs {
   int mlp, n_out;
   const float *affine;                       // nullable: w2 is the product W2 W1 of E x E, see launch_block_prepare; [2][E]: what undoes a row's
                                              // scaling, and W2 b1 + b2; w1, b1, b2 and mlp are not looked at
+  const uint16_t *rest;                      // nullable, with affine: what the rounding of w2's rows left
   int head_dim;                              // out as [n_out / E, inner, E / head_dim, tokens / inner, head_dim]; 0: as [tokens, n_out]
   uint16_t *x_out;                           // nullable: x' is not needed
   uint16_t *norm_out, *out;
@@ -55,12 +56,13 @@ hipError_t launch_block_pack(const BlockPackArgs &args, uint32_t blocks, hipStre
 
 // The same, first_block counting 1024 pieces each, and with it the products of pairs of linear layers with nothing between them:
 // n -> (n W1^T + b1) W2^T + b2 as one matrix [E, E], packed in groups of E / 4 rows, row o times 2^s(o) (its largest element then is
-// between 2^13 and 2^14, so that fp16 keeps what fp32 sums give whatever the weights' size), and affine = [2][E]: 2^-s and W2 b1 + b2.
+// between 2^13 and 2^14, so that fp16 keeps what fp32 sums give whatever the weights' size), what that rounding to fp16 leaves as a second
+// matrix, rounded to fp16 in turn, packed and scaled alike, and affine = [2][E]: 2^-s and W2 b1 + b2.
 struct BlockFoldArgs {
   static constexpr int kMost = 16;
   struct Pair {
     const uint16_t *w1, *b1, *w2, *b2;  // W1 [mlp, E], W2 [E, mlp]; b1 and b2 nullable
-    uint16_t *dst;
+    uint16_t *dst, *rest;               // rest nullable
     float *affine;
     int mlp;                            // a multiple of 256
   } m[kMost];

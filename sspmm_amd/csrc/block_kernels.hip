@@ -17,10 +17,14 @@
 // four lane groups make 64 consecutive bytes.
 //
 // There is nothing between the two linear layers, so the encoder's forward pass has them multiplied first (fold_rows, once a pass)
-// and runs W2 W1 as one matrix: 0.33 M products a token in the place of 0.85, and 0.65 MB of weights to stream instead of
-// 1.6.  256 features, 1024 hidden ones, in a model: 8192 tokens 26.7 -> 16.3 us a launch, 32768 tokens 61 -> 36.5; what packs the weights and
-// multiplies them takes 12.9 us a pass for four blocks, where packing all took 7.6.  (Both layers, for callers that bring them packed:
-// the rest of this paragraph.)
+// where that makes fewer weights: 0.39 M products a token in the place of 0.79, and 0.79 MB of weights to stream instead of
+// 1.6.  W2 W1 comes as two fp16 matrices, what it is rounded to and what the rounding left.  The layers one after the other take W1 and W2
+// as they are and round what comes out of W1, after all that W1 cancels (a mean along its rows against the LayerNorm's output, a bias
+// against beta): one rounded matrix, whose elements know nothing of that, misses float64 by up to fifteen times as much (256 x 1024, rows of
+// W1 with a mean of sixteen deviations: rms of x' 3.3e-3, the layers 3.6e-4), the two by less than the layers (2.9e-4), for 0.065 M products a token.
+// 256 features, 1024 hidden ones, in a model, both layers / one matrix / two: 8192 tokens 26.7 / 16.3 / 17.7 us a launch, 32768 tokens 61 / 38.3 / 40.0;
+// what packs the weights and multiplies them takes 13 us a pass for four blocks, where packing all took 7.6.  (Both layers, where they are the
+// narrower ones and for callers that bring them packed: the rest of this paragraph.)
 //
 // The launch in front of the first block looks the tokens up in the embedding's table itself: as a launch of its own the lookup wrote
 // and this one read tokens x E halfs that no one else wants (256 features, four blocks: 8192 tokens 194 -> 180 us the forward pass,
@@ -34,7 +38,7 @@
 // row: from torch's layout it reads 64 bytes of each of sixteen rows, which lie 512 to 2048 bytes apart on a few of the L2's
 // channels, and 32 tokens per workgroup took 61 us instead of 27 (8192 tokens).
 //
-// 256 features, 1024 hidden, 768 out, with the LayerNorms, both layers / folded: 8192 tokens 25.7 / 16.5 us, 32768 tokens 62.6 / 38.5,
+// 256 features, 1024 hidden, 768 out, with the LayerNorms, both layers / folded (this paragraph: one matrix): 8192 tokens 25.7 / 16.5 us, 32768 tokens 62.6 / 38.5,
 // against 104 (the host) and 121 for the four library products and two LayerNorm launches.  Where a folded launch's cycles go: 8192 tokens
 // 26 000: 4000 until the attention's output is there, 2400 to 2700 a product of 256 x 256 (2048 at 64 bytes of weights a cycle), 1900 a LayerNorm, 1300 the
 // stores of 256 outputs; 32768 tokens 58 000, 12 to 13 000 of them until all workgroups' 33 MB are there, and the stores at the end, 7 us of them, as
@@ -307,6 +311,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
   if constexpr (PART != kNoAttention) {
     const Weights w1 = PART == kFolded ? Weights() : weights<4>(p.w1, p.mlp, E, wave * 64, 0);
     const Weights w2 = weights<NT>(p.w2, E, PART == kFolded ? E : p.mlp, wave * (16 * NT), 0);
+    // (without it w2 twice, at half its scale: a branch around the product costs registers that spill at 512 features)
+    const Weights rest = PART == kFolded && p.rest ? weights<NT>(p.rest, E, E, wave * (16 * NT), 0) : w2;
+    const float share = p.rest ? 1.f : 0.5f;
     half8 bias[NT / 2], bias2[NT / 2];
     feature_values<NT>(bias, p.bo, first, 0.f);
     if constexpr (PART == kFolded) {
@@ -335,7 +342,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
     for (int t = 0; t < TT; ++t)
 #pragma unroll
       for (int j = 0; j < NT / 2; ++j) asm("" : "+v"(x[t][j]));
-    gemm<TT, NT, E, kPitchA, PART == kFolded ? NT : 4, D>(v, act_op, wo, PART == kFolded ? w2 : w1, w);
+    gemm<TT, NT, E, kPitchA, PART == kFolded ? NT : 4, D>(v, act_op, wo, PART == kFolded ? rest : w1, w);
     float s[TT];
 #pragma unroll
     for (int t = 0; t < TT; ++t) {
@@ -353,11 +360,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
       for (int t = 0; t < TT; ++t)
 #pragma unroll
         for (int j = 0; j < NT; ++j) v[t][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+      gemm<TT, NT, E, kPitchA, NT, D>(v, act_op, rest, w2, w);
       gemm<TT, NT, E, kPitchA, 4, D>(v, act_op, w2, tail, w);
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
         const int f = first + 32 * (j >> 1) + 4 * (j & 1);
-        const floatx4 scale = *reinterpret_cast<const floatx4 *>(affine + f), shift = *reinterpret_cast<const floatx4 *>(affine + E + f);
+        const floatx4 scale = *reinterpret_cast<const floatx4 *>(affine + f) * share, shift = *reinterpret_cast<const floatx4 *>(affine + E + f);
 #pragma unroll
         for (int t = 0; t < TT; ++t)
 #pragma unroll
@@ -593,10 +601,15 @@ __device__ void fold_rows(const BlockFoldArgs::Pair &a, int row0, unsigned char 
   const uint32_t piece = ((uint32_t)row / kGroup * (E / KU) + k / KU) * (NJ * KU / 32u) + (k % KU) / 32u * NJ + tile;
   _Float16 *const out = reinterpret_cast<_Float16 *>(a.dst) + piece * 512u + ((k % 32u) / 8u * 16u + mm) * 8u + k % 8u;
   typedef _Float16 halves __attribute__((ext_vector_type(PER)));
-  halves h;
+  halves h, rest;
 #pragma unroll
-  for (int i = 0; i < PER; ++i) h[i] = (_Float16)(c[i] * factor);
+  for (int i = 0; i < PER; ++i) {
+    h[i] = (_Float16)(c[i] * factor);
+    const float left = c[i] * factor - (float)h[i];  // (exact; of an infinity or a NaN nothing is left)
+    rest[i] = fabsf(left) < INFINITY ? (_Float16)left : (_Float16)0;
+  }
   *reinterpret_cast<halves *>(out) = h;
+  if (a.rest) *reinterpret_cast<halves *>(reinterpret_cast<_Float16 *>(a.rest) + (out - reinterpret_cast<_Float16 *>(a.dst))) = rest;
 }
 
 template <int E>
@@ -631,7 +644,7 @@ hipError_t launch(const BlockDenseArgs &p, hipStream_t stream) {
 // CU one: 8192 tokens of 128, 256, 512 features 15, 26, 56 us against 18, 30, 73; 10000 tokens 25, 43, 101 against 18, 31, 73.
 // Up to 4096 tokens 16 do the same, and a workgroup's chain of products and LayerNorms is shorter: 2048 tokens 10.0, 17.5, 43 us
 // against 12.3, 20.1, 48 with 32 (without attention 4.6, 7.4, 17 against 5.6, 9.2, 20), 4096 tokens 10.9, 19.3, 46 against 12.6, 21.2,
-// 49; 8192 tokens without attention 7.6, 14.2, 36 against 6.6, 11.1, 25.  (Both linear layers, LayerNorms of two exchanges.)  Folded, 256 features,
+// 49; 8192 tokens without attention 7.6, 14.2, 36 against 6.6, 11.1, 25.  (Both linear layers, LayerNorms of two exchanges.)  Folded (one matrix), 256 features,
 // 16 / 32 / 64 tokens: 8192 tokens 21 / 16.5 / 19.7, 32768 75 / 50 / 38.5.
 template <int E>
 hipError_t launch_for_width(const BlockDenseArgs &p, hipStream_t stream) {

@@ -564,7 +564,8 @@ int sspmm_add_layernorm_rows_f16(int outer, int inner, int E, const sspmm_half_t
 // Matrices to pack and, with E, pairs of linear layers to multiply, as many launches as the kernels' argument lists ask for.
 static int block_prepare(int count, const sspmm_half_t *const *src, const int32_t *rows, const int32_t *cols, const int32_t *group, sspmm_half_t *dst,
                          int folds, int E, const int32_t *mlp, const sspmm_half_t *const *w1, const sspmm_half_t *const *b1,
-                         const sspmm_half_t *const *w2, const sspmm_half_t *const *b2, sspmm_half_t *w21, float *affine, hipStream_t stream) {
+                         const sspmm_half_t *const *w2, const sspmm_half_t *const *b2, sspmm_half_t *w21, sspmm_half_t *rest, float *affine,
+                         hipStream_t stream) {
   if (count < 0 || (count > 0 && (!src || !rows || !cols || !group || !dst || reinterpret_cast<uintptr_t>(dst) % 16))) return kInvalid;
   for (int i = 0; i < count; ++i) {
     if (!src[i] || reinterpret_cast<uintptr_t>(src[i]) % 16 || (group[i] != 32 && group[i] != 64 && group[i] != 128)) return kInvalid;
@@ -583,7 +584,8 @@ static int block_prepare(int count, const sspmm_half_t *const *src, const int32_
     if (E) {
       sspmm::BlockFoldArgs f;
       for (f.count = 0; f.count < sspmm::BlockFoldArgs::kMost && folded < folds; ++f.count, ++folded)
-        f.m[f.count] = {w1[folded], b1[folded], w2[folded], b2[folded], w21 + (int64_t)folded * E * E, affine + (int64_t)folded * 2 * E, mlp[folded]};
+        f.m[f.count] = {w1[folded], b1[folded], w2[folded], b2[folded], w21 + (int64_t)folded * E * E, rest ? rest + (int64_t)folded * E * E : nullptr,
+                           affine + (int64_t)folded * 2 * E, mlp[folded]};
       e = sspmm::launch_block_prepare(E, f, p, blocks, stream);
     } else {
       e = sspmm::launch_block_pack(p, blocks, stream);
@@ -595,35 +597,43 @@ static int block_prepare(int count, const sspmm_half_t *const *src, const int32_
 
 int sspmm_block_pack_f16(int count, const sspmm_half_t *const *src, const int32_t *rows, const int32_t *cols, const int32_t *group,
                          sspmm_half_t *dst, void *hip_stream) {
-  return block_prepare(count, src, rows, cols, group, dst, 0, 0, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
+  return block_prepare(count, src, rows, cols, group, dst, 0, 0, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
                        static_cast<hipStream_t>(hip_stream));
 }
 
 int sspmm_block_fold_f16(int count, const sspmm_half_t *const *src, const int32_t *rows, const int32_t *cols, const int32_t *group,
                          sspmm_half_t *dst, int folds, int E, const int32_t *mlp, const sspmm_half_t *const *w1, const sspmm_half_t *const *b1,
                          const sspmm_half_t *const *w2, const sspmm_half_t *const *b2, sspmm_half_t *w21, float *affine, void *hip_stream) {
+  return sspmm_block_fold_split_f16(count, src, rows, cols, group, dst, folds, E, mlp, w1, b1, w2, b2, w21, nullptr, affine, hip_stream);
+}
+
+int sspmm_block_fold_split_f16(int count, const sspmm_half_t *const *src, const int32_t *rows, const int32_t *cols, const int32_t *group,
+                               sspmm_half_t *dst, int folds, int E, const int32_t *mlp, const sspmm_half_t *const *w1, const sspmm_half_t *const *b1,
+                               const sspmm_half_t *const *w2, const sspmm_half_t *const *b2, sspmm_half_t *w21, sspmm_half_t *w21_rest, float *affine,
+                               void *hip_stream) {
   if (folds < 0 || (E != 128 && E != 256 && E != 512)) return kInvalid;
   if (folds > 0 && (!mlp || !w1 || !b1 || !w2 || !b2 || !w21 || !affine)) return kInvalid;
-  if ((reinterpret_cast<uintptr_t>(w21) | reinterpret_cast<uintptr_t>(affine)) % 16) return kInvalid;
+  if ((reinterpret_cast<uintptr_t>(w21) | reinterpret_cast<uintptr_t>(w21_rest) | reinterpret_cast<uintptr_t>(affine)) % 16) return kInvalid;
   for (int i = 0; i < folds; ++i) {
     if (mlp[i] <= 0 || mlp[i] % 256 || mlp[i] > (1 << 20) || !w1[i] || !w2[i]) return kInvalid;
     if ((reinterpret_cast<uintptr_t>(w1[i]) | reinterpret_cast<uintptr_t>(w2[i]) | reinterpret_cast<uintptr_t>(b1[i])) % 16) return kInvalid;
   }
-  return block_prepare(count, src, rows, cols, group, dst, folds, E, mlp, w1, b1, w2, b2, w21, affine, static_cast<hipStream_t>(hip_stream));
+  return block_prepare(count, src, rows, cols, group, dst, folds, E, mlp, w1, b1, w2, b2, w21, w21_rest, affine, static_cast<hipStream_t>(hip_stream));
 }
 
 static int block_dense(int outer, int inner, int E, const sspmm_half_t *x, int64_t x_outer, int64_t x_inner, const sspmm_half_t *pos,
                        float x_scale, const sspmm_half_t *attn, const sspmm_half_t *wo, const sspmm_half_t *bo, const sspmm_half_t *gamma2, const sspmm_half_t *beta2,
                        float eps2, int mlp, const sspmm_half_t *w1, const sspmm_half_t *b1, const sspmm_half_t *w2,
-                       const sspmm_half_t *b2, const float *affine, const sspmm_half_t *gamma_n, const sspmm_half_t *beta_n, float eps_n, int n_out, int head_dim,
-                       const sspmm_half_t *wt, const sspmm_half_t *bt, sspmm_half_t *x_out, sspmm_half_t *out, void *hip_stream) {
+                       const sspmm_half_t *b2, const sspmm_half_t *rest, const float *affine, const sspmm_half_t *gamma_n, const sspmm_half_t *beta_n,
+                       float eps_n, int n_out, int head_dim, const sspmm_half_t *wt, const sspmm_half_t *bt, sspmm_half_t *x_out, sspmm_half_t *out,
+                       void *hip_stream) {
   if (outer < 0 || inner < 0 || !sspmm::block_dense_applies(E, attn && !affine ? mlp : 256, n_out)) return kInvalid;
   if (outer == 0 || inner == 0) return 0;
   if (!x || !out || x_outer < 0 || x_inner < 0 || x_outer % 8 || x_inner % 8 || (wt != nullptr) != (n_out > 0)) return kInvalid;
   if (attn && (!wo || !w2 || (!w1 && !affine))) return kInvalid;
   if (head_dim != 0 && ((head_dim != 32 && head_dim != 64 && head_dim != 128) || n_out % E)) return kInvalid;
   uintptr_t bits = reinterpret_cast<uintptr_t>(affine);
-  for (const sspmm_half_t *q : {x, pos, attn, wo, bo, gamma2, beta2, w1, b1, w2, b2, gamma_n, beta_n, wt, bt, (const sspmm_half_t *)x_out,
+  for (const sspmm_half_t *q : {x, pos, attn, wo, bo, gamma2, beta2, w1, b1, w2, b2, rest, gamma_n, beta_n, wt, bt, (const sspmm_half_t *)x_out,
                              (const sspmm_half_t *)out})
     bits |= reinterpret_cast<uintptr_t>(q);
   if (bits % 16) return kInvalid;
@@ -652,6 +662,7 @@ static int block_dense(int outer, int inner, int E, const sspmm_half_t *x, int64
   p.eps_n = eps_n;
   p.mlp = attn ? mlp : 0;
   p.affine = affine;
+  p.rest = rest;
   p.ids = nullptr;
   p.n_out = n_out;
   p.head_dim = head_dim;
@@ -666,8 +677,8 @@ int sspmm_block_dense_f16(int outer, int inner, int E, const sspmm_half_t *x, in
                           float eps2, int mlp, const sspmm_half_t *w1, const sspmm_half_t *b1, const sspmm_half_t *w2,
                           const sspmm_half_t *b2, const sspmm_half_t *gamma_n, const sspmm_half_t *beta_n, float eps_n, int n_out, int head_dim,
                           const sspmm_half_t *wt, const sspmm_half_t *bt, sspmm_half_t *x_out, sspmm_half_t *out, void *hip_stream) {
-  return block_dense(outer, inner, E, x, x_outer, x_inner, pos, x_scale, attn, wo, bo, gamma2, beta2, eps2, mlp, w1, b1, w2, b2, nullptr, gamma_n,
-                     beta_n, eps_n, n_out, head_dim, wt, bt, x_out, out, hip_stream);
+  return block_dense(outer, inner, E, x, x_outer, x_inner, pos, x_scale, attn, wo, bo, gamma2, beta2, eps2, mlp, w1, b1, w2, b2, nullptr, nullptr,
+                     gamma_n, beta_n, eps_n, n_out, head_dim, wt, bt, x_out, out, hip_stream);
 }
 
 int sspmm_block_dense_folded_f16(int outer, int inner, int E, const sspmm_half_t *x, int64_t x_outer, int64_t x_inner, const sspmm_half_t *attn,
@@ -675,8 +686,17 @@ int sspmm_block_dense_folded_f16(int outer, int inner, int E, const sspmm_half_t
                                  const sspmm_half_t *w21, const float *affine, const sspmm_half_t *gamma_n, const sspmm_half_t *beta_n,
                                  float eps_n, int n_out, int head_dim, const sspmm_half_t *wt, const sspmm_half_t *bt, sspmm_half_t *x_out,
                                  sspmm_half_t *out, void *hip_stream) {
+  return sspmm_block_dense_split_f16(outer, inner, E, x, x_outer, x_inner, attn, wo, bo, gamma2, beta2, eps2, w21, nullptr, affine, gamma_n, beta_n, eps_n,
+                                     n_out, head_dim, wt, bt, x_out, out, hip_stream);
+}
+
+int sspmm_block_dense_split_f16(int outer, int inner, int E, const sspmm_half_t *x, int64_t x_outer, int64_t x_inner, const sspmm_half_t *attn,
+                                const sspmm_half_t *wo, const sspmm_half_t *bo, const sspmm_half_t *gamma2, const sspmm_half_t *beta2, float eps2,
+                                const sspmm_half_t *w21, const sspmm_half_t *w21_rest, const float *affine, const sspmm_half_t *gamma_n,
+                                const sspmm_half_t *beta_n, float eps_n, int n_out, int head_dim, const sspmm_half_t *wt, const sspmm_half_t *bt,
+                                sspmm_half_t *x_out, sspmm_half_t *out, void *hip_stream) {
   if (outer > 0 && inner > 0 && (!attn || !affine)) return kInvalid;
-  return block_dense(outer, inner, E, x, x_outer, x_inner, nullptr, 1.f, attn, wo, bo, gamma2, beta2, eps2, 0, nullptr, nullptr, w21, nullptr, affine,
+  return block_dense(outer, inner, E, x, x_outer, x_inner, nullptr, 1.f, attn, wo, bo, gamma2, beta2, eps2, 0, nullptr, nullptr, w21, nullptr, w21_rest, affine,
                      gamma_n, beta_n, eps_n, n_out, head_dim, wt, bt, x_out, out, hip_stream);
 }
 

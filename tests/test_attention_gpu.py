@@ -635,7 +635,7 @@ def _two_layers(E, mlp, count, g, size=1.0, bias=True):
 def test_two_linear_layers_as_one_matrix(built_library, E, mlp, count, size, bias):
     """What one to three launches leave of pairs of linear layers, against their product in float64: an element's rounding to fp16 (2^-11
     of it, or half the smallest step of fp16, 2^-25, next to a largest element of 2^13 or more), and that of the fp32 sums, 2^-24 of their
-    terms each.  Weights whose products fp16 would not hold unscaled, a row of zeros, and one that overflows fp32."""
+    terms each.  Weights whose products fp16 would not hold unscaled, a row of zeros, and one with an infinity."""
     from sspmm_amd.attention import fold_blocks, pack_weights
     g = torch.Generator("cuda").manual_seed(E + mlp)
     blocks = _two_layers(E, mlp, count, g, size, bias)
@@ -669,7 +669,8 @@ def test_two_linear_layers_as_one_matrix(built_library, E, mlp, count, size, bia
                                                      (256, 512, 256, 2731, 3), (512, 256, 1536, 19, 1), (512, 512, 64, 1366, 3), (512, 256, 512, 2731, 3)])
 def test_block_dense_on_one_matrix_for_two_layers(built_library, E, mlp, n_out, outer, inner):
     """Every width and tile of tokens (16, 32, 64) with a last tile that is not full; with and without a tail, x', biases.  The bound is
-    that of test_block_dense_in_one_launch, which has one rounding more."""
+    that of test_block_dense_in_one_launch: the hidden features are not rounded, the matrix is to 2^-22 (what that is worth where the first layer
+    cancels, test_two_linear_layers_as_one_where_the_first_cancels says; here nothing does)."""
     lin = lambda m, t: t @ m.weight.double().t() + (0 if m.bias is None else m.bias.double())  # noqa: E731
     ln = lambda m, t: torch.nn.functional.layer_norm(t, m.normalized_shape, m.weight.double(), m.bias.double(), m.eps)  # noqa: E731
     from sspmm_amd.attention import block_dense, fold_blocks
@@ -693,6 +694,68 @@ def test_block_dense_on_one_matrix_for_two_layers(built_library, E, mlp, n_out, 
                     for d in (32, 64, 128):
                         split = block_dense(x, attn, blk, norm, last, packed=packed, folded=folded[0], head_dim=d)[1]
                         assert torch.equal(split, got.view(outer, inner, n_out // E, E // d, d).permute(2, 1, 3, 0, 4))
+
+
+def _unpacked(matrix, E):
+    """A folded matrix of E x E out of the order in which the waves load it."""
+    group = E // 4
+    nj, unit = group // 16, 32 if group == 128 else 64
+    w = matrix.cpu().numpy().astype(np.float64).reshape(E // group, E // unit, unit // 32, nj // 2, 2, 4, 4, 4, 8)
+    return w.transpose(0, 3, 6, 4, 7, 1, 2, 5, 8).reshape(E, E)
+
+
+@pytest.mark.parametrize("E,mlp,count", [(128, 256, 17), (128, 1280, 1), (256, 512, 3), (512, 256, 2)])
+def test_two_linear_layers_as_two_matrices(built_library, E, mlp, count):
+    """The matrix and what its rounding leaves hold 22 bits: of integers up to 15 the sums need 19 at most (225 x 1280), so the two are
+    the product itself.  Of an element that is not finite nothing is left."""
+    from sspmm_amd.attention import fold_blocks
+    g = torch.Generator("cuda").manual_seed(E + mlp)
+    blocks = _two_layers(E, mlp, count, g)
+    with torch.no_grad():
+        for b in blocks:
+            for m in (b.linear1, b.linear2):
+                m.weight.copy_(torch.randint(-15, 16, m.weight.shape, device="cuda", generator=g).half())
+        blocks[-1].linear2.weight[5, 7] = float("inf")
+        folded = fold_blocks(blocks, [b.out_proj for b in blocks], [E // 4] * count)[1]
+    for b, pair in zip(blocks, folded):
+        w1, w2 = (m.weight.detach().cpu().numpy().astype(np.float64) for m in (b.linear1, b.linear2))
+        down = pair[1][:E].cpu().numpy().astype(np.float64)[:, None]
+        matrix, rest = _unpacked(pair[0], E), _unpacked(pair.rest, E)
+        rows = np.arange(E) != (5 if b is blocks[-1] else -1)
+        assert np.array_equal(((matrix + rest) * down)[rows], (w2 @ w1)[rows]) and np.abs(rest).max() > 0
+        assert not np.isfinite(matrix[~rows]).any() and (rest[~rows] == 0).all()
+
+
+@pytest.mark.parametrize("E,mlp,tokens", [(128, 256, 333), (256, 1024, 500), (256, 512, 4100), (512, 1024, 40), (512, 512, 4100)])
+@pytest.mark.parametrize("kind", ["offset", "shift", "centred"])
+def test_two_linear_layers_as_one_where_the_first_cancels(built_library, E, mlp, tokens, kind):
+    """Rows of the first layer with a part that a LayerNorm's output of mean zero cancels, a large beta that the first bias takes back, and
+    rows without a mean under a beta: the largest and the root mean square of the error against float64 are no larger than those of the
+    layers one after the other, where these cancel before anything is rounded.  (Both end in a rounding to fp16; the output
+    projection is zero, and every second feature of a token 1 and -1, so that the LayerNorm's output is known exactly.)"""
+    from sspmm_amd.attention import block_dense, fold_blocks, pack_weights
+    g = torch.Generator("cuda").manual_seed(E + mlp + tokens)
+    blk, = _two_layers(E, mlp, 1, g)
+    gamma, beta = {"offset": (1.0, 0.0), "shift": (2.0 ** -4, 8.0), "centred": (0.25, 1.0)}[kind]
+    with torch.no_grad():
+        blk.out_proj.weight.zero_(), blk.out_proj.bias.zero_(), blk.linear2.bias.zero_()
+        blk.layer_norm2.weight.fill_(gamma), blk.layer_norm2.bias.fill_(beta)
+        w1, b1 = blk.linear1.weight, blk.linear1.bias
+        if kind == "offset":
+            w1.add_(torch.randn(mlp, 1, device="cuda", generator=g).half())  # (sixteen deviations of the rest at 256 features)
+        elif kind == "centred":
+            w1.sub_(w1.double().mean(1, keepdim=True).half())
+        b1.copy_(-(w1.double().sum(1) * beta).half())
+        sign = torch.rand(tokens, E, device="cuda", generator=g).argsort(1) % 2 * 2.0 - 1.0
+        x = sign.half().view(tokens, 1, E)
+        n = sign.double() * gamma + beta
+        want = (n @ w1.double().t() + b1.double()) @ blk.linear2.weight.double().t() + sign.double()
+        norm, attn = blk.layer_norm1, torch.zeros_like(x)
+        two = block_dense(x, attn, blk, norm, keep_x=True, packed=pack_weights([blk.out_proj, blk.linear1, blk.linear2], [E // 4, 64, E // 4]))[0]
+        packed, folded = fold_blocks([blk], [blk.out_proj], [E // 4])
+        one = block_dense(x, attn, blk, norm, keep_x=True, packed=packed, folded=folded[0])[0]
+    off = [(t.view(tokens, E).double() - want).abs() for t in (one, two)]
+    assert off[0].max() <= off[1].max() and off[0].square().mean() <= off[1].square().mean()
 
 
 @pytest.mark.parametrize("E,outer,inner", [(128, 2000, 1), (256, 1001, 2), (256, 700, 5), (128, 37, 7), (256, 9, 31), (512, 5, 64), (128, 3, 1000), (256, 2, 4097)])
@@ -796,3 +859,30 @@ def test_encoder_against_float64(built_library, embed, heads, mlp, V):
     error = ((got - want).norm() / want.norm()).item()
     print("embed %d: relative error %.2e" % (embed, error), flush=True)
     assert error <= 4 * 2.0 ** -11 / 3 ** 0.5
+
+
+@pytest.mark.parametrize("embed,mlps", [(128, (256, 512)), (256, (256, 512, 256)), (512, (512, 256, 768)), (256, (1024, 256, 512, 256))])
+def test_encoder_folds_the_layers_that_are_wider_than_the_model(built_library, embed, mlps):
+    """Blocks with hidden layers of both kinds behind one another: the bound of test_encoder_against_float64, against the same."""
+    import copy
+    from sspmm_amd import attention as A
+    model = A.SparseAttentionEncoder(50, embed, embed // 32, 0.8, 96, 256, 64, vec_length=8, layers=len(mlps), seed=3)
+    for b, n in zip(model.blocks, mlps):
+        b.linear1, b.linear2 = torch.nn.Linear(embed, n), torch.nn.Linear(n, embed)
+    model = model.cuda().half().eval()
+    tokens = torch.randint(0, 50, (3, 96), device="cuda", generator=torch.Generator("cuda").manual_seed(1))
+    masks, folds, plain = [], [], A.block_dense
+    for b in model.blocks:
+        mask = torch.zeros(12, 8, 96, dtype=torch.bool, device="cuda")
+        mask[torch.repeat_interleave(torch.arange(12, device="cuda"), b.row_offsets.diff().long()), :, b.column_indices.long()] = True
+        masks.append(mask.view(96, 96))
+    A.block_dense = lambda *args, **kw: (folds.append(kw.get("folded") is not None), plain(*args, **kw))[1]
+    try:
+        with torch.no_grad():
+            got = model(tokens).double()
+    finally:
+        A.block_dense = plain
+    assert folds == [False] + [n > embed for n in mlps]
+    with torch.no_grad():
+        want = copy.deepcopy(model).double()(tokens, masks)
+    assert (got - want).norm() / want.norm() <= 4 * 2.0 ** -11 / 3 ** 0.5

@@ -151,6 +151,15 @@ def test_argument_errors_of_the_dense_block_entries(built_library):
         assert fold(**bad) == 1, bad
     assert L.sspmm_block_fold_f16(0, None, None, None, None, None, 0, 256, None, None, None, None, None, None, None, None) == 0
 
+    # (with what the matrix's rounding leaves: the entries above are these without it)
+    split = lambda outer=2, rest=p, w21=p, affine=p, attn=p: L.sspmm_block_dense_split_f16(  # noqa: E731
+        outer, 3, 128, p, 384, 128, attn, p, p, p, p, 1e-5, w21, rest, affine, p, p, 1e-5, 128, 0, p, p, p, p, None)
+    assert all(split(**bad) == 1 for bad in (dict(rest=p + 8), dict(w21=None), dict(affine=None), dict(attn=None), dict(outer=-1)))
+    assert split(outer=0) == 0 and split(outer=0, rest=None) == 0
+    one = lambda v: (C.c_void_p * 1)(v)  # noqa: E731
+    assert L.sspmm_block_fold_split_f16(0, None, None, None, None, None, 1, 128, (C.c_int32 * 1)(256), one(p), one(p), one(p), one(p), p, p + 8, p, None) == 1
+    assert L.sspmm_block_fold_split_f16(0, None, None, None, None, None, 0, 256, None, None, None, None, None, None, None, None, None) == 0
+
     assert L.svc_split_row_ptr(-1, 4, p, p, p, p, None) == 1 and L.svc_split_row_ptr(1, 4, p, None, p, p, None) == 1
     assert L.svc_split_row_ptr(0, 0, None, None, None, None, None) == 0
 
