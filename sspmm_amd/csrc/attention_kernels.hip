@@ -514,8 +514,8 @@ hipError_t launch_softmax(const SoftmaxArgs &a, int V, hipStream_t stream) {
 // element; 22 TB/s on 4096 keys, 90 % masked, once there are rows for every wave).  What it can be given is loads in flight: rows in registers
 // for one step and one stage that k's and v's pass through in turn take 106 registers and 5 KB of LDS a wave, four waves per SIMD, where two
 // sets of rows and two stages (160 registers, two waves) had 20.9 TB/s.  4096 keys, 64 features, 8 / 16 / 32 / 64 (element, head) pairs, V = 8:
-// 27.6 / 49.2 / 90.8 / 167.8 -> 25.5 / 44.9 / 82.3 / 153.6 us, V = 16: 15.1 / 27.8 / 51.0 / 97.3 -> 14.7 / 25.8 / 46.0 / 88.1; one pair, two
-// waves a CU, 9.1 -> 9.3 (9.6 with the scores scaled before their maximum and the sums taken in fp32: twelve instructions a step more).  32 features (six waves) 19.0 / 33.1 / 60.6 / 112.7 -> 18.3 / 33.8 / 60.7 / 112.4, 128 (two) 46.2 / 84.3 / 156 / 308
+// 27.6 / 49.2 / 90.8 / 167.8 -> 25.5 / 44.9 / 82.3 / 153.6 us, V = 16: 15.1 / 27.8 / 51.0 / 97.3 -> 14.7 / 25.8 / 46.0 / 88.1 (sums of rounded probabilities; of the
+// exponentials, as now, measures the same, 8 pairs 21.06 / 21.13 replayed, 32 pairs 76.3 / 76.4, V = 16 13.25 / 13.16 and 45.1 / 44.8).  32 features (six waves) 19.0 / 33.1 / 60.6 / 112.7 -> 18.3 / 33.8 / 60.7 / 112.4, 128 (two) 46.2 / 84.3 / 156 / 308
 // -> 45.2 / 81.9 / 152 / 302; five waves at 64 features, eight at 32, three at 128 are level or slower, and so are two stages.  Neither what a
 // wave computes nor its column indices count: two heads per wave, which share the indices and the addresses, are level (27.6 -> 29, 106 -> 107), and
 // indices handed out with lane permutes, as the sddmm kernel does, slower (124 -> 137 us: the permutes queue in the LDS pipe).
@@ -697,16 +697,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(attention_wa
       for (int i = 0; i < 8; ++i) x[i] = __builtin_fmaf(x[i], scale2, -run_max);
     }
     half8 pb;
+    float sum = 0.f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) pb[i] = (_Float16)__builtin_amdgcn_exp2f(x[i]);
-    // (the sum of what the product takes: the rounding of the largest probabilities cancels in the quotient)
-    const uintx4 pairs = __builtin_bit_cast(uintx4, pb);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-      const half2v ones = {(_Float16)1, (_Float16)1};
-      run_sum = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2v, (uint32_t)pairs[i]), ones, run_sum, false);
+    for (int i = 0; i < 8; ++i) {
+      const float e = __builtin_amdgcn_exp2f(x[i]);
+      sum += e;  // (before the rounding: many probabilities that fp16 does not hold are a part of it)
+      pb[i] = (_Float16)e;
     }
+    run_sum += sum;
 #pragma unroll
     for (int u = 0; u < NT; ++u) {
       const uintx2 lo = lds_read_tr(v_rd + 32u * u);

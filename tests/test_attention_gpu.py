@@ -213,6 +213,32 @@ def test_one_launch_attentions_with_many_small_probabilities(built_library, gap)
         assert np.abs(got.cpu().numpy() - want[:, None]).max() <= bound
 
 
+def _one_key_ahead_of_many(keys, d):
+    """q, k, v: key 0 ahead of all others by 25.05 in the base-2 exponent at a scale of 1/8, so that each of their probabilities is just
+    under half the smallest that fp16 holds; their values are zero, key 0's is 2047/1024."""
+    a, b = np.float16(11.78125), np.float16(11.7890625)
+    assert 25.0 < float(a) * float(b) / 8 * np.log2(np.e) < 25.06
+    q, k, v = (np.zeros((1, n, d), np.float16) for n in (64, keys, keys))
+    q[..., 0], k[0, 0, 0], v[0, 0] = a, b, 2047 / 1024
+    return q, k, v
+
+
+# half a step of fp16 below two, and a few steps of the fp32 sums: without the others' probabilities in the sum the result is 0.95 steps off
+_MANY_KEYS_BOUND = 2.0 ** -11 + 2.0 ** -16
+
+
+@pytest.mark.parametrize("V,d", [(8, 32), (8, 64), (8, 128), (16, 32), (16, 64), (16, 128)])
+@pytest.mark.parametrize("pairs", [1, 40, 300])
+def test_one_launch_attention_sums_what_fp16_does_not_hold(built_library, V, d, pairs):
+    keys = 16384
+    q, k, v = _one_key_ahead_of_many(keys, d)
+    off = (np.arange(64 // V + 1) * keys).astype(np.int32)
+    cols = np.tile(np.arange(keys, dtype=np.int32), 64 // V)
+    want = _dense_attention(off, cols, V, q, k, v, 0.125)
+    got = sspmm_amd.fused_sparse_attention(None, dev(off), dev(cols), *(dev(t).expand(pairs, -1, -1).contiguous() for t in (q, k, v)), 0.125, V)
+    assert np.abs(got.cpu().numpy() - want).max() <= _MANY_KEYS_BOUND
+
+
 @pytest.mark.parametrize("V,d", [(8, 32), (8, 64), (16, 64), (8, 128), (16, 128)])
 def test_one_launch_attention_with_scores_of_any_size(built_library, V, d):
     """Scaled scores from a fraction to 2^32, of either sign: the largest probability is one whatever fp32 makes of its exponent.  A
