@@ -365,9 +365,9 @@ hipError_t launch_add_layernorm_rows(int E, const AddLayerNormRows &p, hipStream
 // registers.  The context goes back through LDS and is written feature-major in whole 128-byte lines.  Bound by
 // HBM in bytes (q, k, v read once, out written once: 8 * hidden * tokens bytes; a head's K and V are re-read by its
 // seq / 64 workgroups from L2), by the exponentials and the LDS reads in time.
-// 8 x 512 tokens, 12 heads, inside the layer: 18.0 -> 17.0 us with the maxima exchanged by lane swaps instead of permutes through the LDS, V's
-// operands read ahead of the exponentials and the sums taken of pairs of rounded probabilities (the error against float64 2.55 - 2.92e-4 ->
-// 2.26 - 2.91e-4).
+// 8 x 512 tokens, 12 heads, inside the layer: 18.0 -> 16.8 to 17.5 us with the maxima exchanged by lane swaps instead of permutes through the LDS and
+// V's operands read ahead of the exponentials.  (Sums of the probabilities as fp16 holds them, four dot products for eight additions, are level:
+// 17.0 and 17.1 in the same two runs.)
 typedef uint32_t uintx2 __attribute__((ext_vector_type(2)));
 typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 typedef short shortx4 __attribute__((ext_vector_type(4)));
@@ -618,20 +618,13 @@ __global__ __launch_bounds__(kAttThreads, 3) void attention_fm_kernel(const Atte
           for (int r = 0; r < 4; ++r) {
             s[j][kt][r] = __builtin_amdgcn_exp2f(fmaf(s[j][kt][r], c, shift));
             if (cut && 16 * kt + r >= keys_left) s[j][kt][r] = 0.f;  // (a wave may have had no key at all yet)
-            if (RAGGED) part += s[j][kt][r];
+            part += s[j][kt][r];
           }
         run_sum[j] += part;
         pop[j].u[0] = att_pack(s[j][0][0], s[j][0][1]);
         pop[j].u[1] = att_pack(s[j][0][2], s[j][0][3]);
         pop[j].u[2] = att_pack(s[j][1][0], s[j][1][1]);
         pop[j].u[3] = att_pack(s[j][1][2], s[j][1][3]);
-        if constexpr (!RAGGED) {
-          // the sum of what the product takes: the rounding of the largest probabilities cancels in the quotient
-          typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-          const half2v ones = {(_Float16)1, (_Float16)1};
-#pragma unroll
-          for (int i = 0; i < 4; ++i) run_sum[j] = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2v, pop[j].u[i]), ones, run_sum[j], false);
-        }
         if constexpr (RAGGED) {
 #pragma unroll
           for (int i = 0; i < 8; ++i) rest[j].h[i] = (_Float16)(s[j][i >> 2][i & 3] - (float)pop[j].h[i]);

@@ -239,6 +239,17 @@ def test_one_launch_attention_sums_what_fp16_does_not_hold(built_library, V, d, 
     assert np.abs(got.cpu().numpy() - want).max() <= _MANY_KEYS_BOUND
 
 
+def test_dense_attention_sums_what_fp16_does_not_hold(built_library):
+    """(The two waves that share queries keep sums of their own, so half of the keys would count: 0.48 steps of 0.97.)"""
+    from sspmm_amd.layers import attention_fm
+    seq = 16384
+    q, k, v = _one_key_ahead_of_many(seq, 64)
+    qkv = np.concatenate([np.broadcast_to(q[0, :1], (seq, 64)).T, k[0].T, v[0].T])
+    want = _dense_attention(np.array([0, seq], np.int32), np.arange(seq), 1, q[:, :1], k, v, 0.125)[0, 0]
+    got = attention_fm(dev(np.ascontiguousarray(qkv)), 64, 1, 1, seq)
+    assert np.abs(got.cpu().numpy() - want[:, None]).max() <= _MANY_KEYS_BOUND
+
+
 @pytest.mark.parametrize("V,d", [(8, 32), (8, 64), (16, 64), (8, 128), (16, 128)])
 def test_one_launch_attention_with_scores_of_any_size(built_library, V, d):
     """Scaled scores from a fraction to 2^32, of either sign: the largest probability is one whatever fp32 makes of its exponent.  A
