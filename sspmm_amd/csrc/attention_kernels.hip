@@ -716,24 +716,33 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(attention_wa
 
   // Column indices run two steps ahead of the arithmetic, the rows of k and v one: a step's rows pass through the stage, k's and then
   // v's, and the next step's are on their way as soon as the registers are free.
+  const auto in_order = [] { asm volatile("" ::: "memory"); };  // (left alone the compiler lets loads sink to their first use)
   const Head now = load_head(beg);
   Head ahead = load_head(beg + 32);
+  in_order();
   Places at = places(now, beg);
   fetch(k, srd_k, at.k);
   fetch(v, srd_v, at.v);
-  for (int kc = beg; kc < end; kc += 32) {
+  // The last step stands apart, and the loads stay in this order: where loads may or may not have been issued behind those that a write to
+  // LDS waits for, it waits for all.  4096 keys, 64 features, replayed, with one loop / now: V = 8, one pair 8.80 / 8.38 us, 2 9.45 / 9.2-9.3, 4 and more
+  // level; V = 16, 1 / 2 / 4 / 8 pairs 8.50 / 9.13 / 9.9 / 13.1 -> 8.07 / 8.64 / 9.41 / 13.1, 32 features 7.1 / 7.6 / 7.8 / 9.5 -> 6.7 / 7.15 / 7.4 / 9.4,
+  // 128 features 11.9 / 12.7 / 15.0 / 24.0 -> 11.2 / 12.1 / 14.4 / 24.1; 1024 waves on 1024 keys, V = 16 5.33 -> 5.11.
+  int kc = beg;
+  for (; kc + 32 < end; kc += 32) {
     put(k);
-    const bool more = kc + 32 < end;
-    if (more) {
-      at = places(ahead, kc + 32);
-      fetch(k, srd_k, at.k);
-      ahead = load_head(kc + 64);
-    }
+    at = places(ahead, kc + 32);
+    fetch(k, srd_k, at.k);
+    ahead = load_head(kc + 64);
     scores();
     put(v);
-    if (more) fetch(v, srd_v, at.v);
+    fetch(v, srd_v, at.v);
+    in_order();
     softmax_and_product(kc);
   }
+  put(k);
+  scores();
+  put(v);
+  softmax_and_product(kc);
 
   const float inv = 1.0f / quad_rows_sum(run_sum);
   if (n < V) {
