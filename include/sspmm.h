@@ -445,13 +445,19 @@ int sspmm_block_dense_f16(int outer, int inner, int E, const sspmm_half_t *x, in
 /*
  * sspmm_block_dense_f16 without attn, on an embedding that has not been looked up: row (i, j) of x is row
  * tokens[i * token_outer + j * token_inner] of table [vocab, E] (4- or 8-byte integers, 0 <= token < vocab; a token outside
- * is a row of NaN), fp16(x * x_scale) + pos[i] stands in its place.
+ * is a row of NaN), fp16(x * x_scale) + pos[i] stands in its place.  checked: *tokens_ok (device memory) becomes 0 where there is
+ * a token outside and is left alone otherwise; NULL: the same as without.
  */
 int sspmm_block_embed_f16(int outer, int inner, int E, const void *tokens, int token_bytes, int64_t token_outer,
                           int64_t token_inner, const sspmm_half_t *table, int64_t vocab, const sspmm_half_t *pos,
                           float x_scale, const sspmm_half_t *gamma_n, const sspmm_half_t *beta_n, float eps_n, int n_out,
                           int head_dim, const sspmm_half_t *wt, const sspmm_half_t *bt, sspmm_half_t *x_out,
                           sspmm_half_t *out, void *hip_stream);
+int sspmm_block_embed_checked_f16(int outer, int inner, int E, const void *tokens, int token_bytes, int64_t token_outer,
+                                  int64_t token_inner, const sspmm_half_t *table, int64_t vocab, const sspmm_half_t *pos,
+                                  float x_scale, const sspmm_half_t *gamma_n, const sspmm_half_t *beta_n, float eps_n,
+                                  int n_out, int head_dim, const sspmm_half_t *wt, const sspmm_half_t *bt,
+                                  sspmm_half_t *x_out, sspmm_half_t *out, int32_t *tokens_ok, void *hip_stream);
 
 /*
  * Weight matrices [rows, cols] (row-major, 16-byte aligned) into the order in which sspmm_block_dense_f16 loads them,
@@ -473,7 +479,8 @@ int sspmm_block_pack_f16(int count, const sspmm_half_t *const *src, const int32_
  * rows, a large beta2 that b1 takes back) is not cancelled then, and such weights lose up to a factor of |n| |W21| over
  * |W2| |W1 n + b1|.  sspmm_block_fold_split_f16 also keeps what the rounding leaves: w21_rest + i * E * E, rounded to
  * fp16 in turn, as w21 in all else, and the two together miss the fp32 sums by 2^-22 of an element or 2^-38 of the
- * row's largest (w21_rest NULL: not kept).
+ * row's largest (w21_rest NULL: not kept).  *tokens_ok becomes 1 where it is not NULL (for sspmm_block_embed_checked_f16
+ * behind it on the stream) and there is anything to pack or fold.
  */
 int sspmm_block_fold_f16(int count, const sspmm_half_t *const *src, const int32_t *rows, const int32_t *cols,
                          const int32_t *group, sspmm_half_t *dst, int folds, int E, const int32_t *mlp,
@@ -483,7 +490,7 @@ int sspmm_block_fold_split_f16(int count, const sspmm_half_t *const *src, const 
                                const int32_t *group, sspmm_half_t *dst, int folds, int E, const int32_t *mlp,
                                const sspmm_half_t *const *w1, const sspmm_half_t *const *b1, const sspmm_half_t *const *w2,
                                const sspmm_half_t *const *b2, sspmm_half_t *w21, sspmm_half_t *w21_rest, float *affine,
-                               void *hip_stream);
+                               int32_t *tokens_ok, void *hip_stream);
 
 /*
  * sspmm_block_dense_f16 with x' = n W21^T + (W2 b1 + b2) + x from what sspmm_block_fold_f16 leaves, or (split) with

@@ -54,8 +54,10 @@ SIGNATURES = {
     "sspmm_block_dense_f16": (_int, [_int, _int, _int, _vp, _i64, _i64, _vp, ctypes.c_float, _vp, _vp, _vp, _vp, _vp, ctypes.c_float, _int, _vp, _vp, _vp, _vp,
                                      _vp, _vp, ctypes.c_float, _int, _int, _vp, _vp, _vp, _vp, _vp]),
     "sspmm_block_embed_f16": (_int, [_int, _int, _int, _vp, _int, _i64, _i64, _vp, _i64, _vp, ctypes.c_float, _vp, _vp, ctypes.c_float, _int, _int] + [_vp] * 5),
+    "sspmm_block_embed_checked_f16": (_int, [_int, _int, _int, _vp, _int, _i64, _i64, _vp, _i64, _vp, ctypes.c_float, _vp, _vp, ctypes.c_float, _int, _int] +
+                                      [_vp] * 6),
     "sspmm_block_fold_f16": (_int, [_int, _vp, _vp, _vp, _vp, _vp, _int, _int] + [_vp] * 8),
-    "sspmm_block_fold_split_f16": (_int, [_int, _vp, _vp, _vp, _vp, _vp, _int, _int] + [_vp] * 9),
+    "sspmm_block_fold_split_f16": (_int, [_int, _vp, _vp, _vp, _vp, _vp, _int, _int] + [_vp] * 10),
     "sspmm_block_dense_folded_f16": (_int, [_int, _int, _int, _vp, _i64, _i64] + [_vp] * 5 + [ctypes.c_float] + [_vp] * 4 + [ctypes.c_float, _int, _int] +
                                      [_vp] * 5),
     "sspmm_block_dense_split_f16": (_int, [_int, _int, _int, _vp, _i64, _i64] + [_vp] * 5 + [ctypes.c_float] + [_vp] * 5 + [ctypes.c_float, _int, _int] +

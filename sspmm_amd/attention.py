@@ -229,10 +229,11 @@ class FoldedLayers(tuple):
     """(matrix, affine) of two linear layers with nothing between them, and `rest`, what the matrix's rounding to fp16 left."""
 
 
-def fold_blocks(blocks, linears, rows_per_wave):
+def fold_blocks(blocks, linears, rows_per_wave, tokens_ok=None):
     """pack_weights(linears, rows_per_wave), and in the same launch linear1 and linear2 of every block as the one linear map they
-    are, there being nothing between them: (packed, [FoldedLayers per block]) for block_dense's `folded`."""
-    n, f, E = len(linears), len(blocks), blocks[0].embed_dim
+    are, there being nothing between them: (packed, [FoldedLayers per block]) for block_dense's `folded`.
+    tokens_ok: an int32 that becomes one, for block_dense behind it."""
+    n, f, E = len(linears), len(blocks), linears[0].in_features
     weights = [_weights(m)[0] for m in linears]
     shapes = [w.shape for w in weights]
     sizes = [r * c for r, c in shapes]
@@ -246,7 +247,7 @@ def fold_blocks(blocks, linears, rows_per_wave):
     rc = _lib.call(_lib.lib().sspmm_block_fold_split_f16, device, n, ptrs(*[w.data_ptr() for w in weights]), ints(*[r for r, _ in shapes]),
                    ints(*[c for _, c in shapes]), ints(*rows_per_wave), packed.data_ptr(), f, E, (ctypes.c_int32 * f)(*[a.out_features for a, _ in pairs]),
                    some(*[w.data_ptr() for w, _ in up]), some(*[_ptr(b) for _, b in up]), some(*[w.data_ptr() for w, _ in down]),
-                   some(*[_ptr(b) for _, b in down]), at, at + 2 * f * E * E, affine.data_ptr())
+                   some(*[_ptr(b) for _, b in down]), at, at + 2 * f * E * E, affine.data_ptr(), _ptr(tokens_ok))
     _lib.check(rc, "sspmm_block_fold_split_f16")
     parts = packed.split(sizes + 2 * f * [E * E])
     folded = [FoldedLayers(pair) for pair in zip(parts[n:], affine)]
@@ -255,7 +256,7 @@ def fold_blocks(blocks, linears, rows_per_wave):
     return parts[:n], folded
 
 
-def block_dense(x, attn, block, norm, tail=None, keep_x=False, packed=None, head_dim=0, pos=None, scale=1.0, folded=None, table=None):
+def block_dense(x, attn, block, norm, tail=None, keep_x=False, packed=None, head_dim=0, pos=None, scale=1.0, folded=None, table=None, tokens_ok=None):
     """(x', out): everything between the attention of `block` and the next one's in one launch, on token-major activations
     [seq, batch, embed] fp16:
         s = out_proj(attn) + x, x' = linear2(linear1(layer_norm2(s))) + x, h = norm(x'), out = tail(h) or h itself.
@@ -265,7 +266,7 @@ def block_dense(x, attn, block, norm, tail=None, keep_x=False, packed=None, head
     [tail.out_features / embed, batch, embed / head_dim, seq, head_dim], for sparse_attention_split.  pos
     [seq, embed]: x is an embedding, and (x * scale) + pos stands in its place, each rounded to fp16.  folded: linear1 and linear2 as
     fold_blocks leaves them (with attn, without pos), packed then that of out_proj and tail.  table (without attn, with pos): x are
-    tokens [batch, seq], and the embedding is read from the table's rows."""
+    tokens [batch, seq], and the embedding is read from the table's rows; a token that is none of them makes a row of NaN, and 0 of tokens_ok."""
     outer, inner, E = x.shape if table is None else (x.size(1), x.size(0), table.size(1))
     n_out = 0 if tail is None else tail.out_features
     shape = (n_out // E, inner, E // head_dim, outer, head_dim) if head_dim else (outer, inner, n_out or E)
@@ -274,10 +275,10 @@ def block_dense(x, attn, block, norm, tail=None, keep_x=False, packed=None, head
     stride = x.stride()
     if table is not None:
         gamma_n, beta_n = _weights(norm)
-        rc = _lib.call(_lib.lib().sspmm_block_embed_f16, x.device, outer, inner, E, x.data_ptr(), x.element_size(), stride[1], stride[0], table.data_ptr(),
+        rc = _lib.call(_lib.lib().sspmm_block_embed_checked_f16, x.device, outer, inner, E, x.data_ptr(), x.element_size(), stride[1], stride[0], table.data_ptr(),
                        table.size(0), pos.data_ptr(), float(scale), _ptr(gamma_n), _ptr(beta_n), float(norm.eps), n_out, head_dim, packed[-1].data_ptr(),
-                       _ptr(_weights(tail)[1]), _ptr(kept), out.data_ptr())
-        _lib.check(rc, "sspmm_block_embed_f16")
+                       _ptr(_weights(tail)[1]), _ptr(kept), out.data_ptr(), _ptr(tokens_ok))
+        _lib.check(rc, "sspmm_block_embed_checked_f16")
         return kept, out
     if packed is None:
         own = [] if attn is None else [block.out_proj, block.linear1, block.linear2]
@@ -487,7 +488,8 @@ class SparseAttentionEncoder(torch.nn.Module):
         self.linear = torch.nn.Linear(embed_dim, num_class)
 
     def forward(self, tokens, dense_masks=None):
-        """tokens: int [batch, seq] -> [seq, batch, num_class]."""
+        """tokens: int [batch, seq] -> [seq, batch, num_class].  A token that is no row of the embedding's table is an error of the
+        device, as in torch.nn.Embedding."""
         scale = self.embed_dim ** 0.5
         if dense_masks is None:
             table = self._table(tokens)
@@ -582,12 +584,10 @@ class SparseAttentionEncoder(torch.nn.Module):
             linears += (_parts(blk, "out_proj") if fold[i] else _parts(blk, "out_proj", "linear1", "linear2")) + tail
             rows += ([E // 4] if fold[i] else [E // 4, 64, E // 4]) + [64] * len(tail)
             ends.append(len(linears))
-        if any(fold):
-            packed, pairs = fold_blocks([b for b, f in zip(blocks, fold) if f], linears, rows)
-            pairs = iter(pairs)
-            folded = [next(pairs) if f else None for f in fold]
-        else:
-            packed, folded = pack_weights(linears, rows), [None] * len(blocks)
+        ok = None if table is None else torch.empty(1, dtype=torch.int32, device=table.device)
+        packed, pairs = fold_blocks([b for b, f in zip(blocks, fold) if f], linears, rows, ok)
+        pairs = iter(pairs)
+        folded = [next(pairs) if f else None for f in fold]
 
         def attention(blk, qkv):
             # (in the pattern's own order: the longest rows last, which row_indices asks for, cost 1 to 4 %)
@@ -595,7 +595,10 @@ class SparseAttentionEncoder(torch.nn.Module):
             return sparse_attention_split(None, offsets, columns, qkv, float(qkv.size(-1)) ** -0.5, blk.vec_length)
 
         x, qkv = block_dense(x, None, None, norms[0], into[0], True, packed[:1], E // blocks[0].num_heads, pe, scale,
-                             table=table)
+                             table=table, tokens_ok=ok)
+        if ok is not None:
+            # (as torch's own lookup does; 1.7 us of the device and some 6 of the host, where the lookup as a launch of its own is 14 and more)
+            torch._assert_async(ok, "a token is no row of the embedding's table")
         for i, blk in enumerate(blocks[:-1]):
             x, qkv = block_dense(x, attention(blk, qkv), blk, norms[i + 1], into[i + 1], True, packed[ends[i]:ends[i + 1]],
                                  E // blocks[i + 1].num_heads, folded=folded[i])

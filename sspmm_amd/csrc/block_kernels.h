@@ -23,6 +23,7 @@ struct BlockDenseArgs {
   const void *ids;                           // nullable (without attn, with pos): row i of x is row ids[(i / inner) * x_outer + (i % inner) * x_inner]
   int wide_ids;                              // of `vocab` rows at x, NaN where there is none; int64 instead of int32
   long long vocab;
+  int *ids_ok;                               // nullable: becomes 0 where there is no such row
   const uint16_t *attn;                      // nullable, and the next two lines with it
   const uint16_t *wo, *bo, *gamma2, *beta2;
   const uint16_t *w1, *b1, *w2, *b2;
@@ -67,6 +68,7 @@ struct BlockFoldArgs {
     int mlp;                            // a multiple of 256
   } m[kMost];
   int count;
+  int *ids_ok;                          // nullable: set to 1, for BlockDenseArgs::ids_ok of a launch behind this one
 };
 hipError_t launch_block_prepare(int E, const BlockFoldArgs &folds, const BlockPackArgs &packs, uint32_t pack_blocks, hipStream_t stream);
 

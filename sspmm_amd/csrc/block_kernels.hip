@@ -286,6 +286,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_waves
         const bool there = id >= 0 && id < p.vocab;
         load_row<NT>(x[t], p.x + (there ? id : 0) * E + first);
         if (!there) {
+          if (p.ids_ok) *p.ids_ok = 0;
 #pragma unroll
           for (int j = 0; j < NT / 2; ++j)
 #pragma unroll
@@ -616,6 +617,7 @@ template <int E>
 __global__ __launch_bounds__(1024) void block_prepare_kernel(const BlockFoldArgs f, const BlockPackArgs p) {
   __shared__ __align__(16) unsigned char lds[16 * 32 * kFoldPitch];
   const uint32_t folds = (uint32_t)f.count * (E / 16);
+  if (f.ids_ok && blockIdx.x == 0 && threadIdx.x == 0) *f.ids_ok = 1;
   if (blockIdx.x < folds) {
     // (workgroups eight apart share an XCD: one pair's on as few of them as can be, each of which fetches W1 once)
     const uint32_t id = (blockIdx.x & 7u) * (folds / 8u) + (blockIdx.x >> 3);

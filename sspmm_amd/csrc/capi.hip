@@ -565,7 +565,7 @@ int sspmm_add_layernorm_rows_f16(int outer, int inner, int E, const sspmm_half_t
 static int block_prepare(int count, const sspmm_half_t *const *src, const int32_t *rows, const int32_t *cols, const int32_t *group, sspmm_half_t *dst,
                          int folds, int E, const int32_t *mlp, const sspmm_half_t *const *w1, const sspmm_half_t *const *b1,
                          const sspmm_half_t *const *w2, const sspmm_half_t *const *b2, sspmm_half_t *w21, sspmm_half_t *rest, float *affine,
-                         hipStream_t stream) {
+                         int32_t *tokens_ok, hipStream_t stream) {
   if (count < 0 || (count > 0 && (!src || !rows || !cols || !group || !dst || reinterpret_cast<uintptr_t>(dst) % 16))) return kInvalid;
   for (int i = 0; i < count; ++i) {
     if (!src[i] || reinterpret_cast<uintptr_t>(src[i]) % 16 || (group[i] != 32 && group[i] != 64 && group[i] != 128)) return kInvalid;
@@ -583,6 +583,7 @@ static int block_prepare(int count, const sspmm_half_t *const *src, const int32_
     hipError_t e;
     if (E) {
       sspmm::BlockFoldArgs f;
+      f.ids_ok = tokens_ok;
       for (f.count = 0; f.count < sspmm::BlockFoldArgs::kMost && folded < folds; ++f.count, ++folded)
         f.m[f.count] = {w1[folded], b1[folded], w2[folded], b2[folded], w21 + (int64_t)folded * E * E, rest ? rest + (int64_t)folded * E * E : nullptr,
                            affine + (int64_t)folded * 2 * E, mlp[folded]};
@@ -597,28 +598,30 @@ static int block_prepare(int count, const sspmm_half_t *const *src, const int32_
 
 int sspmm_block_pack_f16(int count, const sspmm_half_t *const *src, const int32_t *rows, const int32_t *cols, const int32_t *group,
                          sspmm_half_t *dst, void *hip_stream) {
-  return block_prepare(count, src, rows, cols, group, dst, 0, 0, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
+  return block_prepare(count, src, rows, cols, group, dst, 0, 0, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
                        static_cast<hipStream_t>(hip_stream));
 }
 
 int sspmm_block_fold_f16(int count, const sspmm_half_t *const *src, const int32_t *rows, const int32_t *cols, const int32_t *group,
                          sspmm_half_t *dst, int folds, int E, const int32_t *mlp, const sspmm_half_t *const *w1, const sspmm_half_t *const *b1,
                          const sspmm_half_t *const *w2, const sspmm_half_t *const *b2, sspmm_half_t *w21, float *affine, void *hip_stream) {
-  return sspmm_block_fold_split_f16(count, src, rows, cols, group, dst, folds, E, mlp, w1, b1, w2, b2, w21, nullptr, affine, hip_stream);
+  return sspmm_block_fold_split_f16(count, src, rows, cols, group, dst, folds, E, mlp, w1, b1, w2, b2, w21, nullptr, affine, nullptr, hip_stream);
 }
 
 int sspmm_block_fold_split_f16(int count, const sspmm_half_t *const *src, const int32_t *rows, const int32_t *cols, const int32_t *group,
                                sspmm_half_t *dst, int folds, int E, const int32_t *mlp, const sspmm_half_t *const *w1, const sspmm_half_t *const *b1,
                                const sspmm_half_t *const *w2, const sspmm_half_t *const *b2, sspmm_half_t *w21, sspmm_half_t *w21_rest, float *affine,
-                               void *hip_stream) {
+                               int32_t *tokens_ok, void *hip_stream) {
   if (folds < 0 || (E != 128 && E != 256 && E != 512)) return kInvalid;
   if (folds > 0 && (!mlp || !w1 || !b1 || !w2 || !b2 || !w21 || !affine)) return kInvalid;
-  if ((reinterpret_cast<uintptr_t>(w21) | reinterpret_cast<uintptr_t>(w21_rest) | reinterpret_cast<uintptr_t>(affine)) % 16) return kInvalid;
+  if ((reinterpret_cast<uintptr_t>(w21) | reinterpret_cast<uintptr_t>(w21_rest) | reinterpret_cast<uintptr_t>(affine)) % 16 || reinterpret_cast<uintptr_t>(tokens_ok) % 4)
+    return kInvalid;
   for (int i = 0; i < folds; ++i) {
     if (mlp[i] <= 0 || mlp[i] % 256 || mlp[i] > (1 << 20) || !w1[i] || !w2[i]) return kInvalid;
     if ((reinterpret_cast<uintptr_t>(w1[i]) | reinterpret_cast<uintptr_t>(w2[i]) | reinterpret_cast<uintptr_t>(b1[i])) % 16) return kInvalid;
   }
-  return block_prepare(count, src, rows, cols, group, dst, folds, E, mlp, w1, b1, w2, b2, w21, w21_rest, affine, static_cast<hipStream_t>(hip_stream));
+  return block_prepare(count, src, rows, cols, group, dst, folds, E, mlp, w1, b1, w2, b2, w21, w21_rest, affine, tokens_ok,
+                       static_cast<hipStream_t>(hip_stream));
 }
 
 static int block_dense(int outer, int inner, int E, const sspmm_half_t *x, int64_t x_outer, int64_t x_inner, const sspmm_half_t *pos,
@@ -704,9 +707,17 @@ int sspmm_block_embed_f16(int outer, int inner, int E, const void *tokens, int t
                           const sspmm_half_t *table, int64_t vocab, const sspmm_half_t *pos, float x_scale, const sspmm_half_t *gamma_n,
                           const sspmm_half_t *beta_n, float eps_n, int n_out, int head_dim, const sspmm_half_t *wt, const sspmm_half_t *bt,
                           sspmm_half_t *x_out, sspmm_half_t *out, void *hip_stream) {
+  return sspmm_block_embed_checked_f16(outer, inner, E, tokens, token_bytes, token_outer, token_inner, table, vocab, pos, x_scale, gamma_n, beta_n, eps_n,
+                                       n_out, head_dim, wt, bt, x_out, out, nullptr, hip_stream);
+}
+
+int sspmm_block_embed_checked_f16(int outer, int inner, int E, const void *tokens, int token_bytes, int64_t token_outer, int64_t token_inner,
+                                  const sspmm_half_t *table, int64_t vocab, const sspmm_half_t *pos, float x_scale, const sspmm_half_t *gamma_n,
+                                  const sspmm_half_t *beta_n, float eps_n, int n_out, int head_dim, const sspmm_half_t *wt, const sspmm_half_t *bt,
+                                  sspmm_half_t *x_out, sspmm_half_t *out, int32_t *tokens_ok, void *hip_stream) {
   if (outer < 0 || inner < 0 || !sspmm::block_dense_applies(E, 256, n_out)) return kInvalid;
   if (outer == 0 || inner == 0) return 0;
-  if (!tokens || !table || !pos || !out || (token_bytes != 4 && token_bytes != 8) || reinterpret_cast<uintptr_t>(tokens) % (uintptr_t)token_bytes ||
+  if (!tokens || !table || !pos || !out || reinterpret_cast<uintptr_t>(tokens_ok) % 4 || (token_bytes != 4 && token_bytes != 8) || reinterpret_cast<uintptr_t>(tokens) % (uintptr_t)token_bytes ||
       token_outer < 0 || token_inner < 0 || vocab < 1 || (wt != nullptr) != (n_out > 0))
     return kInvalid;
   if (head_dim != 0 && ((head_dim != 32 && head_dim != 64 && head_dim != 128) || n_out % E)) return kInvalid;
@@ -718,6 +729,7 @@ int sspmm_block_embed_f16(int outer, int inner, int E, const void *tokens, int t
   p.ids = tokens;
   p.wide_ids = token_bytes == 8;
   p.vocab = vocab;
+  p.ids_ok = tokens_ok;
   p.tokens = (long long)outer * inner;
   p.inner = inner;
   p.x = table;

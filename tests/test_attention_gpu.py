@@ -923,3 +923,24 @@ def test_encoder_folds_the_layers_that_are_wider_than_the_model(built_library, e
     with torch.no_grad():
         want = copy.deepcopy(model).double()(tokens, masks)
     assert (got - want).norm() / want.norm() <= 4 * 2.0 ** -11 / 3 ** 0.5
+
+
+@pytest.mark.parametrize("mlp", [256, 512])
+def test_encoder_refuses_tokens_outside_the_table(built_library, monkeypatch, mlp):
+    """As torch's lookup does, by an assertion on the device (looked at here, not made), with and without layers to fold; sequences beside are
+    what they are without such a token."""
+    from sspmm_amd.attention import SparseAttentionEncoder
+    model = SparseAttentionEncoder(50, 256, 8, 0.8, 96, mlp, 64, vec_length=8, layers=2, seed=2).cuda().half().eval()
+    tokens = torch.randint(0, 50, (3, 96), device="cuda", generator=torch.Generator("cuda").manual_seed(1))
+    seen = []
+    monkeypatch.setattr(torch, "_assert_async", lambda ok, *message: seen.append(ok))
+    with torch.no_grad():
+        want = model(tokens)
+        for bad in (50, -1, 1 << 40):
+            tokens[1, 17] = bad
+            got = model(tokens)
+            assert got[:, 1].isnan().any() and torch.equal(got[:, ::2], want[:, ::2])
+        tokens[1, 17] = 49
+        got = model(tokens)
+        assert not got.isnan().any()
+    assert [ok.item() for ok in seen] == [1, 0, 0, 0, 1]

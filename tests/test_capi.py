@@ -157,8 +157,11 @@ def test_argument_errors_of_the_dense_block_entries(built_library):
     assert all(split(**bad) == 1 for bad in (dict(rest=p + 8), dict(w21=None), dict(affine=None), dict(attn=None), dict(outer=-1)))
     assert split(outer=0) == 0 and split(outer=0, rest=None) == 0
     one = lambda v: (C.c_void_p * 1)(v)  # noqa: E731
-    assert L.sspmm_block_fold_split_f16(0, None, None, None, None, None, 1, 128, (C.c_int32 * 1)(256), one(p), one(p), one(p), one(p), p, p + 8, p, None) == 1
-    assert L.sspmm_block_fold_split_f16(0, None, None, None, None, None, 0, 256, None, None, None, None, None, None, None, None, None) == 0
+    assert L.sspmm_block_fold_split_f16(0, None, None, None, None, None, 1, 128, (C.c_int32 * 1)(256), one(p), one(p), one(p), one(p), p, p + 8, p, p, None) == 1
+    assert L.sspmm_block_fold_split_f16(0, None, None, None, None, None, 0, 128, None, None, None, None, None, None, None, None, p + 2, None) == 1
+    assert L.sspmm_block_fold_split_f16(0, None, None, None, None, None, 0, 256, None, None, None, None, None, None, None, None, p, None) == 0
+    checked = lambda outer, ok: L.sspmm_block_embed_checked_f16(outer, 3, 128, p, 8, 1, 2, p, 7, p, 1.0, p, p, 1e-5, 128, 0, p, p, p, p, ok, None)  # noqa: E731
+    assert checked(2, p + 2) == 1 and checked(-1, p) == 1 and checked(0, p) == 0
 
     assert L.svc_split_row_ptr(-1, 4, p, p, p, p, None) == 1 and L.svc_split_row_ptr(1, 4, p, None, p, p, None) == 1
     assert L.svc_split_row_ptr(0, 0, None, None, None, None, None) == 0
