@@ -944,3 +944,31 @@ def test_encoder_refuses_tokens_outside_the_table(built_library, monkeypatch, ml
         got = model(tokens)
         assert not got.isnan().any()
     assert [ok.item() for ok in seen] == [1, 0, 0, 0, 1]
+
+
+@pytest.mark.parametrize("where,name", [("linear1", "weight"), ("linear2", "bias"), ("out_proj", "weight"), ("in_proj", "bias"), ("layer_norm1", "weight"),
+                                        ("layer_norm2", "bias"), ("encoder", "weight"), ("linear", "weight"), ("layer_norm", "bias"),
+                                        ("block", "linear1"), ("block", "layer_norm2"), ("block", "column_indices"), ("model", "encoder")])
+def test_encoder_takes_an_instances_own_attribute_first(built_library, where, name):
+    """What a program has put into a module's __dict__ comes before the parameter, buffer or module of that name, as everywhere in torch."""
+    import copy
+    from sspmm_amd.attention import SparseAttentionEncoder
+    model = SparseAttentionEncoder(50, 128, 4, 0.8, 96, 256, 64, vec_length=8, layers=2, seed=2).cuda().half().eval()
+    tokens = torch.randint(0, 50, (2, 96), device="cuda", generator=torch.Generator("cuda").manual_seed(1))
+
+    def owner(m):
+        return {"block": m.blocks[1], "model": m}.get(where) or getattr(m if hasattr(m, where) else m.blocks[1], where)
+
+    with torch.no_grad():
+        want, old = copy.deepcopy(model), getattr(owner(model), name)
+        if isinstance(old, torch.nn.Module):
+            new = copy.deepcopy(old)
+            new.weight.copy_(torch.randn_like(new.weight) * 0.1)
+        else:
+            new = old.flip(0) if name == "column_indices" else torch.randn_like(old) * 0.1
+        setattr(owner(want), name, torch.nn.Parameter(new) if isinstance(old, torch.nn.Parameter) else new)
+        owner(model).__dict__[name] = new
+        assert getattr(owner(model), name) is new
+        assert torch.equal(model(tokens), want(tokens))
+        del owner(model).__dict__[name]
+        assert not torch.equal(model(tokens), want(tokens))
