@@ -260,6 +260,8 @@ def _tail_weight(m, in_features, out_features, V, dev):
             m.out_dtype == torch.float16 and m.__dict__.get("plan") is None):
         return None
     own = m._buffers
+    if not own.keys().isdisjoint(m.__dict__):  # (an attribute of the instance comes before a buffer; here and below)
+        return None
     off, col, val, bias = own.get("row_offsets"), own.get("column_indices"), own.get("values"), own.get("bias")
     if not (_plain_tensor(off, torch.int32, dev) and _plain_tensor(col, torch.int32, dev) and _plain_tensor(val, torch.float16, dev) and
             off.numel() == out_features // V + 1 and val.numel() >= col.numel() * V and
@@ -278,6 +280,8 @@ def _tail_norm(ln, features, dev):
     if not (_plain_module(ln, torch.nn.LayerNorm) and ln.normalized_shape == (features,)):
         return None
     own = ln._parameters
+    if not own.keys().isdisjoint(ln.__dict__):
+        return None
     w, b = own.get("weight"), own.get("bias")
     if not (type(w) in _PLAIN and _of_features(w, features, dev) and (b is None or (type(b) in _PLAIN and _of_features(b, features, dev)))):
         return None
@@ -362,6 +366,8 @@ class SparseEncoderLayer(torch.nn.Module):
                 context.is_contiguous()):
             return None
         own = self._modules
+        if not own.keys().isdisjoint(self.__dict__):
+            return None
         o, ffn1, ffn2 = own.get("o"), own.get("ffn1"), own.get("ffn2")
         if not (type(o) is SparseLinear and type(ffn1) is SparseLinear and type(ffn2) is SparseLinear and o.activation is None and
                 ffn2.activation is None):

@@ -484,6 +484,29 @@ def test_encoder_layers_tail_of_few_and_of_most_rows(built_library, V, hidden, f
         test_encoder_layers_tail_matches_dense_fp32_products(built_library, V, bias, hidden, ffn, tokens)
 
 
+@pytest.mark.parametrize("where,name", [("o", "values"), ("ffn1", "bias"), ("ln1", "weight"), ("layer", "ffn2")])
+def test_encoder_layers_tail_takes_an_instances_own_attribute_first(built_library, monkeypatch, where, name):
+    """What a program has put into a module's __dict__ comes before the parameter, buffer or module of that name."""
+    import copy
+    import sspmm_amd.layers as layers_mod
+    monkeypatch.setattr(layers_mod, "encoder_tail_pays", lambda *a: True)
+    monkeypatch.setattr(layers_mod, "TAIL_TOKENS", 1)
+    sp = [_vector_sparse_linear(o, i, 8, 0.8, seed=k, bias=torch.zeros(o, device="cuda").half())
+          for k, (o, i) in enumerate([(128, 128)] * 4 + [(256, 128), (128, 256)])]
+    layer = SparseEncoderLayer(128, 2, 256, *sp).cuda().half().eval()
+    x = torch.randn(128, 64, device="cuda", generator=torch.Generator("cuda").manual_seed(1)).half()
+    owner = layer if where == "layer" else getattr(layer, where)
+    old = getattr(owner, name)
+    new = copy.deepcopy(old)
+    with torch.no_grad():
+        (new.values if name == "ffn2" else new).mul_(0.5).add_(0.25)
+        owner.__dict__[name] = new
+        want = layer(x, 1, 64, linear=lambda n, lin, t: lin(t))
+        assert max_rel_err(layer(x, 1, 64).float().cpu().numpy(), want.float().cpu().numpy()) <= 2.0 ** -8
+        del owner.__dict__[name]
+        assert max_rel_err(layer(x, 1, 64).float().cpu().numpy(), want.float().cpu().numpy()) > 2.0 ** -8
+
+
 def test_encoder_layers_tail_runs_on_the_weights_of_that_moment(built_library, monkeypatch):
     """A hook behind the projections that gives the layer other weights: the launch behind the attention has their addresses,
     not those of the arrays that went away (looked at without launching), and its result is the one with them."""
