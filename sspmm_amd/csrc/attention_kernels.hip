@@ -47,7 +47,7 @@ __device__ __forceinline__ uint32_t xcd_work_index(uint32_t per_xcd) {
 // lanes would read 16 bytes each of sixteen different rows; instead the rows are fetched with
 // neighbouring lanes on neighbouring 16-byte pieces of one row (whole 128-byte lines for 64
 // features), written to a small LDS stage, and read back in the operand layout.  Rows of the
-// stage are padded by 16 bytes so that the sixteen rows a read touches spread over the banks.
+// stage are padded by 16 bytes (the reads still meet in some banks: a quarter of the LDS cycles at 64 features and 2000 keys).
 // NC MFMAs contract the features, and the lane ends up with rows 4g .. 4g+3 of vector m: eight
 // contiguous bytes of the output.  The column indices run two groups ahead of the arithmetic, the
 // rows of rhs one group (two stages, used alternately).
@@ -497,7 +497,7 @@ hipError_t launch_softmax(const SoftmaxArgs &a, int V, hipStream_t stream) {
 //
 // One wave per (vector-row, batch element), a step is 32 stored vectors.  The rows of k and of v the step names
 // are fetched as in the staged SpMM kernel (eight lanes on the eight 16-byte pieces of one 128-byte row, lane
-// (j, pc) = rows of k slots 4j .. 4j+3, piece pc) and written to two LDS stages with padded rows.
+// (j, pc) = rows of k slots 4j .. 4j+3, piece pc) and written to an LDS stage with padded rows, k's first and v's behind them.
 //   scores:  the staged rows of k are the MFMA's first operand (lane (n, g): features 32c + 8g .. of staged row
 //            16t + n), the V rows of q the second, held in registers for the whole row; the lane ends up with the
 //            scores of query n against staged rows 16t + 4g + r, r = 0 .. 3, t = 0, 1.
@@ -521,32 +521,6 @@ hipError_t launch_softmax(const SoftmaxArgs &a, int V, hipStream_t stream) {
 // indices handed out with lane permutes, as the sddmm kernel does, slower (124 -> 137 us: the permutes queue in the LDS pipe).
 // K and V of 256 keys at a time in LDS, every CU fetching all of them for its 64 vector-rows, would read the L2 a seventh as often; it was built and
 // is level at 32 pairs (85-93 us) and slower below (36 us at 8): its waves wait for each other at every panel.
-namespace {
-
-typedef short shortx4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ uintx2 lds_read_tr(const unsigned char *p) {
-  const shortx4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) shortx4 *)p);
-  return __builtin_bit_cast(uintx2, v);
-}
-
-// max / sum over the four lanes n, n + 16, n + 32, n + 48, in each of them
-__device__ __forceinline__ float quad_rows_max(float x) {
-  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-__device__ __forceinline__ float quad_rows_sum(float x) {
-  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
-
-
-}  // namespace
-
 constexpr int attention_waves(int F) { return F == 64 ? 4 : F == 32 ? 6 : 2; }  // per SIMD
 
 // F: features per row of q, k and v (32, 64 or 128).  A row is F * 2 bytes = LPR 16-byte pieces, a load instruction
@@ -678,7 +652,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(attention_wa
           if (kc + 16 * t + 4 * g + i >= end) x[4 * t + i] = -INFINITY;
     }
     float mx = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
-    mx = quad_rows_max(mx);  // finite: the step's first slot is always a stored vector
+    mx = max_over_rows(mx);  // finite: the step's first slot is always a stored vector
     const float new_raw = fmaxf(run_raw, mx);  // (scale2 > 0: the order of the scaled scores)
     if (__builtin_amdgcn_ballot_w64(new_raw > run_raw)) {  // (uniform) some query's maximum moved
       const float alpha = __builtin_amdgcn_exp2f((run_raw - new_raw) * scale2);
@@ -744,7 +718,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(attention_wa
   put(v);
   softmax_and_product(kc);
 
-  const float inv = 1.0f / quad_rows_sum(run_sum);
+  const float inv = 1.0f / sum_over_rows(run_sum);
   if (n < V) {
 #pragma unroll
     for (int u = 0; u < NT; ++u) {

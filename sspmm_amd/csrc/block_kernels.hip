@@ -11,7 +11,7 @@
 // Orientation: out^T[feature, token] = W (MFMA operand A, 16 features x 32 k) * act^T (operand B, 32 k x 16 tokens).
 // Both operands then are eight consecutive k per lane: W comes straight from global memory (row-major as torch keeps it;
 // a wave reads only the rows of its own features, so nothing is loaded twice by a workgroup and LDS is not involved),
-// act from LDS rows padded by 16 bytes (sixteen rows at sixteen different bank groups).  The rows of a wave's feature
+// act from LDS rows padded by 32 bytes (by 16 both layers took 59 us at 32768 tokens, by 32 or 48 56 to 58).  The rows of a wave's feature
 // tiles are dealt so that two tiles leave a lane eight consecutive features of one token (feature 32 (j / 2) + 8 g + 4 (j % 2)
 // + i of tile j, accumulator i, lane group g): residual loads, LDS writes and stores are 16-byte pieces, of which the
 // four lane groups make 64 consecutive bytes.
@@ -60,12 +60,6 @@ typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 
 constexpr int kChunk = 256;  // hidden (or output) features a workgroup makes at a time, 64 per wave
-
-typedef uint32_t uintx2 __attribute__((ext_vector_type(2)));
-typedef short shortx4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ uintx2 fold_read_tr(const unsigned char *p) {
-  return __builtin_bit_cast(uintx2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) shortx4 *)p));
-}
 
 template <int NJ>
 struct Unit {  // what is loaded together: NJ tiles of 16 features x K values of k
@@ -554,7 +548,7 @@ __device__ void fold_rows(const BlockFoldArgs::Pair &a, int row0, unsigned char 
       if (at + 32 * DEPTH < share) fetch(d, at + 32 * DEPTH);
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        const uintx2 lo = fold_read_tr(src + 32 * t), hi = fold_read_tr(src + 4 * kFoldPitch + 32 * t);
+        const two_words lo = lds_read_tr(src + 32 * t), hi = lds_read_tr(src + 4 * kFoldPitch + 32 * t);
         const uintx4 b = {lo[0], lo[1], hi[0], hi[1]};
         acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, __builtin_bit_cast(half8, b), acc[t], 0, 0, 0);
       }

@@ -1,4 +1,4 @@
-// Running sums and maxima over the lanes of a wave with lane moves inside the vector unit (DPP), and a workgroup's barrier.
+// Running sums and maxima over the lanes of a wave with lane moves inside the vector unit (DPP), transpose reads, and a workgroup's barrier.
 //
 // A permute through the LDS pipe (__shfl_up and the like) costs a kernel that has a wave or two per
 // SIMD, and so nothing to hide a latency behind, some 70 cycles each: six dependent ones per scan.
@@ -110,7 +110,13 @@ __device__ __forceinline__ void store_four(_Float16 *p, four_halfs v, int left) 
   }
 }
 
-// Sum of v over the lanes of the wave with the same lane % 16, in each of them.
+// Maximum, and below the sum, of v over the lanes of the wave with the same lane % 16, in each of them.
+__device__ __forceinline__ float max_over_rows(float v) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
 __device__ __forceinline__ float sum_over_rows(float v) {
   const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
@@ -123,6 +129,14 @@ __device__ __forceinline__ float sum_over_quads(float v) {
   v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, false));  // rotated by 8 in each 16
   v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xf, 0xf, false));  // and by 4
   return sum_over_rows(v);
+}
+
+// Transpose read of 16-bit elements from LDS: within 16 lanes, lane n receives element n of the four 32-byte runs addressed by lanes 0-3,
+// 4-7, 8-11, 12-15.
+typedef uint32_t two_words __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ two_words lds_read_tr(const unsigned char *p) {
+  typedef short four_shorts __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(two_words, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) four_shorts *)p));
 }
 
 // Workgroup barrier that orders LDS only: global loads in flight stay in flight.

@@ -370,8 +370,6 @@ hipError_t launch_add_layernorm_rows(int E, const AddLayerNormRows &p, hipStream
 // 17.0 and 17.1 in the same two runs.)
 typedef uint32_t uintx2 __attribute__((ext_vector_type(2)));
 typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
-typedef short shortx4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) shortx4 lds_shortx4;
 
 static constexpr int kAttThreads = 256;
 static constexpr int kAttD = 64;          // head size
@@ -392,19 +390,6 @@ union AttOperand {
   uint32_t u[4];
 };
 
-// Within 16 lanes, lane n receives element n of the four 32-byte runs addressed by lanes 0-3, 4-7, 8-11, 12-15.
-__device__ __forceinline__ uintx2 att_read_tr(const unsigned char *p) {
-  const shortx4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4 *)p);
-  return __builtin_bit_cast(uintx2, v);
-}
-
-// Maximum over the four lanes n, n + 16, n + 32, n + 48, in each of them.
-__device__ __forceinline__ float att_max4(float x) {
-  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
 __device__ __forceinline__ uint32_t att_pack(float lo, float hi) {
   typedef _Float16 half2v __attribute__((ext_vector_type(2)));
   const half2v h = {(_Float16)lo, (_Float16)hi};
@@ -517,7 +502,7 @@ __global__ __launch_bounds__(kAttThreads, 3) void attention_fm_kernel(const Atte
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const unsigned char *a = q_tile + (32 * u + 4 * g + (m >> 2)) * kAttPitchK + (32 * qhalf + 16 * j) * 2 + (m & 3) * 8;
-      const uintx2 lo = att_read_tr(a), hi = att_read_tr(a + 16 * kAttPitchK);
+      const uintx2 lo = lds_read_tr(a), hi = lds_read_tr(a + 16 * kAttPitchK);
       qop[j][u].u[0] = lo[0]; qop[j][u].u[1] = lo[1]; qop[j][u].u[2] = hi[0]; qop[j][u].u[3] = hi[1];
     }
 
@@ -554,7 +539,7 @@ __global__ __launch_bounds__(kAttThreads, 3) void attention_fm_kernel(const Atte
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           const unsigned char *a = k_tile + k_rd + (32 * u) * kAttPitchK + (16 * kt) * 2;
-          const uintx2 lo = att_read_tr(a), hi = att_read_tr(a + 16 * kAttPitchK);
+          const uintx2 lo = lds_read_tr(a), hi = lds_read_tr(a + 16 * kAttPitchK);
           AttOperand kop;
           kop.u[0] = lo[0]; kop.u[1] = lo[1]; kop.u[2] = hi[0]; kop.u[3] = hi[1];
 #pragma unroll
@@ -596,7 +581,7 @@ __global__ __launch_bounds__(kAttThreads, 3) void attention_fm_kernel(const Atte
           mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
           mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
         } else {
-          mx = att_max4(mx);
+          mx = max_over_rows(mx);
         }
         // The reference point of the exponentials moves only when some query's maximum has grown by more than 8 in
         // the base-2 domain (a wave-uniform decision): until then the probabilities are at most 2^8 times too large,

@@ -152,15 +152,15 @@ struct StoreRow<_Float16, 4> {
   }
 };
 
-// The value tile of a step: 32 vectors x V halfs as they lie in memory (vector-major), written to LDS with one
-// 8- or 16-byte store per lane and read back as the MFMA operand (lane (v, g): k = 8g .. 8g+7 of row v) by two
+// The value tile of a step: 32 vectors x V halfs as they lie in memory (vector-major), written to LDS with two
+// 4-byte stores or one of 16 per lane and read back as the MFMA operand (lane (v, g): k = 8g .. 8g+7 of row v) by two
 // ds_read_b64_tr_b16.  The V = 8 transpose read touches 16 bytes past its 512.
 static constexpr int val_tile_bytes(int V) { return V == 8 ? 528 : 1024; }
 
 typedef short shortx4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) shortx4 lds_shortx4;
 
-// The same read at an absolute LDS byte address (saves adding the base of the dynamic LDS array,
+// lds_read_tr at an absolute LDS byte address (saves adding the base of the dynamic LDS array,
 // which the compiler does not fold, to every address).
 __device__ __forceinline__ uintx2 lds_read_tr_abs(uint32_t lds_addr) {
   const shortx4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4 *)(uintptr_t)lds_addr);
@@ -168,10 +168,6 @@ __device__ __forceinline__ uintx2 lds_read_tr_abs(uint32_t lds_addr) {
 }
 __device__ __forceinline__ uint32_t lds_address(const unsigned char *p) {
   return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char *)p;
-}
-__device__ __forceinline__ uintx2 lds_read_tr(const unsigned char *lds_base, uint32_t byte_off) {
-  const shortx4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4 *)(lds_base + byte_off));
-  return __builtin_bit_cast(uintx2, v);
 }
 
 // The 32 x V halfs of a step, spread over the 64 lanes.  The address unit passes a load of 16 or of 8 bytes a lane on in sixteen cycles,
@@ -283,8 +279,8 @@ template <int CPL, int V>
 __device__ __forceinline__ void mac_chunk(const Chunk<CPL> &c, floatx4 (&acc)[CPL], const unsigned char *tile_op) {
   Half8Bits a;
   {
-    const uintx2 lo = lds_read_tr(tile_op, 0);
-    const uintx2 hi = lds_read_tr(tile_op, 4u * (V * 2u));
+    const uintx2 lo = lds_read_tr(tile_op);
+    const uintx2 hi = lds_read_tr(tile_op + 4u * (V * 2u));
     a.u[0] = lo[0]; a.u[1] = lo[1]; a.u[2] = hi[0]; a.u[3] = hi[1];
   }
 #pragma unroll
@@ -982,8 +978,8 @@ __device__ __forceinline__ void slab_run(SlabRing<V, NQ> &ring, const SlabCtx<V,
       // A operand: this step's value tile
       Half8Bits a;
       {
-        const uintx2 lo = lds_read_tr(x.val_tile, x.a_off);
-        const uintx2 hi = lds_read_tr(x.val_tile, x.a_off + 16u * (V * 2u));
+        const uintx2 lo = lds_read_tr(x.val_tile + x.a_off);
+        const uintx2 hi = lds_read_tr(x.val_tile + (x.a_off + 16u * (V * 2u)));
         a.u[0] = lo[0]; a.u[1] = lo[1]; a.u[2] = hi[0]; a.u[3] = hi[1];
       }
       // B operands: two column indices per lane; unused k slots of a partial step read the zero row
@@ -1599,8 +1595,8 @@ __device__ __forceinline__ void stage_accumulate(floatx4 (&acc)[4], const StageL
     SlabVals<V>::put(x.tile_dst, c.vraw);
     Half8Bits a;
     {
-      const uintx2 lo = lds_read_tr(x.val_tile, x.a_off);
-      const uintx2 hi = lds_read_tr(x.val_tile, x.a_off + 4u * (V * 2u));
+      const uintx2 lo = lds_read_tr(x.val_tile + x.a_off);
+      const uintx2 hi = lds_read_tr(x.val_tile + (x.a_off + 4u * (V * 2u)));
       a.u[0] = lo[0]; a.u[1] = lo[1]; a.u[2] = hi[0]; a.u[3] = hi[1];
     }
 #pragma unroll
@@ -1706,8 +1702,8 @@ __device__ __forceinline__ void stage_stream(const StageLane<V> &x, const int32_
     SlabVals<V>::put(x.tile_dst, c.vraw);
     Half8Bits a;
     {
-      const uintx2 lo = lds_read_tr(x.val_tile, x.a_off);
-      const uintx2 hi = lds_read_tr(x.val_tile, x.a_off + 4u * (V * 2u));
+      const uintx2 lo = lds_read_tr(x.val_tile + x.a_off);
+      const uintx2 hi = lds_read_tr(x.val_tile + (x.a_off + 4u * (V * 2u)));
       a.u[0] = lo[0]; a.u[1] = lo[1]; a.u[2] = hi[0]; a.u[3] = hi[1];
     }
 #pragma unroll
@@ -2211,7 +2207,7 @@ static bool whole_pieces(const SpmmArgs &a, bool out_f16) {
 // kernel alone, now below the 6.9 us of the call; 128 x 2659 at 80 %, N = 30: 86 -> 11 us a call; 512-wide encoder layer on
 // 7 x 101 tokens 238 -> 154 us.  The error against float64 is a quarter to all of the scalar kernel's on fourteen such products
 // (7e-8 to 1.7e-7 where it has 1.8e-7 to 6e-7).
-// The value vectors are fetched with 8-byte (V = 8) or 16-byte (V = 16) loads per lane from aligned memory; 24-bit
+// The value vectors are fetched with two 4-byte (V = 8) or one 16-byte (V = 16) loads per lane from aligned memory; 24-bit
 // multiplies bound K and 2N; one buffer descriptor must span B.
 static bool mfma_kernels_apply(const SpmmArgs &a, bool out_f16) {
   const uint64_t b_bytes = (uint64_t)a.K * (uint64_t)a.N * 2u;
