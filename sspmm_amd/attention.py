@@ -139,7 +139,8 @@ def sparse_attention_packed(row_indices, row_offsets, column_indices, qkv, num_h
 
 def sparse_attention_split(row_indices, row_offsets, column_indices, qkv, scaling, vec_length):
     """The same from a projection split into heads: qkv [3, batch, heads, seq, d] -> [seq, batch, heads * d].  A head's
-    rows then lie side by side, which the gathers take 3 to 9 % faster than rows 3 * batch * embed elements apart."""
+    rows then lie side by side instead of 3 * batch * embed elements apart: 4096 keys, 32 pairs of element and head, 32 / 64 / 128 features, V = 8
+    59.2 -> 54.2, 76.4 -> 75.7, 152 -> 147 us, V = 16 32.7 -> 29.7, 44.1 -> 43.3, 84.4 -> 82.7, 4 pairs 10.3 -> 8.9, 12.3 -> 12.2, 21.5 -> 21.4."""
     _check_pattern(row_indices, row_offsets, column_indices, vec_length)
     _check_half("qkv", qkv)
     if qkv.dim() != 5 or qkv.size(0) != 3 or qkv.size(-1) not in FUSED_HEAD_WIDTHS:

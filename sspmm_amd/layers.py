@@ -225,17 +225,18 @@ TAIL_TOKENS = 1024
 
 def encoder_tail_pays(hidden, tokens, vectors, cus):
     """Whether the one launch is ahead of the five it replaces; `vectors`: stored vectors of its three weights.  A workgroup of
-    16 tokens, one per CU, takes as long however few of them there are: a layer with it some 35 us and 0.44 us per thousand
+    16 tokens, one per CU, takes as long however few of them there are: a layer with it some 35 us and 0.45 us per thousand
     vectors, where the separate launches' time follows the tokens.  Layer with 768 features (replayed, so that the host plays
-    no part), separate / one launch, us: V = 16 at 90 % (33 000 vectors) 512 tokens 42 / 49, 1024 52 / 51, 4096 82 / 64; V = 8 at 90 %
-    (66 000) 1024 57 / 68, 2048 74 / 75, 3072 89 / 81, 4096 99 / 83; at 85 % (99 000) 2048 79 / 89, 3072 99 / 95, 4096 109 / 96; at 80 %
-    (132 000) 3072 110 / 110, 4096 121 / 111, 8192 206 / 210; V = 16 at 50 % (165 000) 4096 142 / 131, 8192 242 / 247; V = 8 at 70 %
-    (199 000) 4096 143 / 140, at 50 % (332 000) 1536 117 / 190, 4096 192 / 200.  Called one by one the separate launches keep the host
-    busy for 72 us and these 40, so where the device's times are level or a little apart the one launch is ahead: 512 features, V = 8 at 90 %,
-    1024 tokens 43 / 48 replayed, 71 / 49 called.  Beyond one workgroup per CU a nearly empty last round costs a whole one:
-    8192 tokens 134 / 115 (V = 16 at 90 %) and 183 / 179 (99 000 vectors), 6144 137 / 138 (66 000) and 158 / 171 (99 000); 512 features and 88 000
-    vectors, 7168 tokens 144 / 151.  Narrower layers are ahead there as well (256 features, V = 8 at 90 %, 8192 tokens 66 / 55) and
-    have the separate launches."""
+    no part), separate / one launch, us: V = 16 at 90 % (33 000 vectors) 512 tokens 41 / 45, 1024 52 / 47, 2048 63 / 53, 4096 83 / 59; V = 8 at 90 %
+    (66 000) 1024 56 / 65, 2048 72 / 71, 3072 89 / 77, 4096 100 / 79; at 85 % (99 000) 2048 79 / 83, 3072 99 / 89, 4096 111 / 92; at 80 %
+    (133 000) 2048 83 / 95, 4096 122 / 105, 8192 212 / 200; V = 16 at 50 % (166 000) 4096 139 / 123, 8192 235 / 232; V = 8 at 70 %
+    (199 000) 2048 99 / 126, 4096 151 / 140, 8192 265 / 267.  Called one by one the separate launches keep the host
+    busy for 65 to 70 us and these 35 to 45, so where the device's times are level or a little apart the one launch is ahead: 512 features, V = 8 at
+    90 %, 1024 tokens 42 / 45 replayed, 65 / 45 called, at 80 % 2048 tokens 58 / 58, 65 / 59.  Beyond one workgroup per CU a nearly empty last round
+    costs a whole one: 8192 tokens 135 / 105 (V = 16 at 90 %) and 192 / 174 (99 000 vectors), 6144 143 / 138 (66 000) and 160 / 163 (99 000); 512 features,
+    7168 tokens 108 / 94 (29 000) and 128 / 119 (59 000).  The lines were drawn for a launch 3 us slower and are on its safe side now: between them
+    and where the two are level the separate launches run although the one is ahead (33 000 vectors 1024 and 6144 tokens 52 / 47 and 116 / 99, 99 000
+    3072 tokens 99 / 89, 133 000 to 199 000 4096 tokens; 256 features, V = 8 at 90 %, 6144 and 8192 tokens 58 / 54 and 64 / 56)."""
     if vectors > 100000 or tokens < max(TAIL_TOKENS, vectors // 30):
         return False
     per_round = 16 * cus
