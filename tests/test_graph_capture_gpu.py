@@ -121,3 +121,35 @@ def test_encoder_layer_in_a_graph(built_library, monkeypatch, batch, seq, one_la
         torch.cuda.synchronize()
         assert torch.equal(out, want)
         _between_replays()
+
+
+@pytest.mark.parametrize("mlp", [256, 512])
+def test_encoder_in_a_graph(built_library, mlp):
+    """The lookup and its assertion, the folded layers (512) and the two layers one after the other (256), recorded once and replayed on other
+    tokens and other weights, which every pass packs and multiplies anew."""
+    from sspmm_amd.attention import SparseAttentionEncoder
+    model = SparseAttentionEncoder(50, 256, 8, 0.8, 96, mlp, 64, vec_length=8, layers=2, seed=2).cuda().half().eval()
+    g = torch.Generator("cuda").manual_seed(mlp)
+    sets = [(torch.randint(0, 50, (3, 96), device="cuda", generator=g), torch.randn(256, mlp, device="cuda", generator=g).half() * 0.05) for _ in range(3)]
+    tokens, s, weight = sets[0][0].clone(), torch.cuda.Stream(), model.blocks[1].linear2.weight
+    with torch.no_grad():
+        wants = []
+        for t, w in sets:
+            weight.copy_(w)
+            wants.append(model(t).clone())
+        assert not torch.equal(wants[0], wants[1])
+        s.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(s):
+            model(tokens)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            out = model(tokens)
+        for (t, w), want in zip(sets + sets[:1], wants + wants[:1]):
+            tokens.copy_(t)
+            weight.copy_(w)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want)
+            _between_replays()
