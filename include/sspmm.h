@@ -495,7 +495,8 @@ int sspmm_block_fold_split_f16(int count, const sspmm_half_t *const *src, const 
 /*
  * sspmm_block_dense_f16 with x' = n W21^T + (W2 b1 + b2) + x from what sspmm_block_fold_f16 leaves, or (split) with
  * n W21^T + n W21rest^T; attn is needed.  The hidden features are never made, so they are not rounded, and do not become
- * infinite beyond what fp16 holds; W21 is what has been rounded (above).
+ * infinite beyond what fp16 holds; W21 is what has been rounded (above).  The Python module takes the split entries where mlp > E
+ * and sspmm_block_dense_f16 elsewhere.
  */
 int sspmm_block_dense_folded_f16(int outer, int inner, int E, const sspmm_half_t *x, int64_t x_outer, int64_t x_inner,
                                  const sspmm_half_t *attn, const sspmm_half_t *wo, const sspmm_half_t *bo,
