@@ -499,11 +499,11 @@ class SparseAttentionEncoder(torch.nn.Module):
         """tokens: int [batch, seq] -> [seq, batch, num_class].  A token that is no row of the embedding's table is an error of the
         device, as in torch.nn.Embedding."""
         scale = self.embed_dim ** 0.5
-        if dense_masks is None:
+        if dense_masks is None and _eager_inference():
             table = self._table(tokens)
-            if table is not None:
-                (batch, seq), pe = tokens.shape, self._positions(tokens.size(1), table)
-                if pe is not None and _eager_inference() and self._norms_apply(table) and self._blocks_apply(table, seq, batch):
+            if table is not None and self._norms_apply(table) and self._blocks_apply(table, tokens.size(1), tokens.size(0)):
+                pe = self._positions(tokens.size(1), table)
+                if pe is not None:
                     return self._fused_blocks(tokens, pe, scale, table)
         out = self.encoder(tokens)
         if dense_masks is None and out.dim() == 3:
