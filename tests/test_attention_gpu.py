@@ -7,7 +7,7 @@ import pytest
 import torch
 
 import sspmm_amd
-from sspmm_amd import synth
+from sspmm_amd import _lib, synth
 from gpu_util import dev, max_rel_err
 
 pytestmark = pytest.mark.gpu
@@ -761,6 +761,36 @@ def test_two_linear_layers_as_two_matrices(built_library, E, mlp, count):
         rows = np.arange(E) != (5 if b is blocks[-1] else -1)
         assert np.array_equal(((matrix + rest) * down)[rows], (w2 @ w1)[rows]) and np.abs(rest).max() > 0
         assert not np.isfinite(matrix[~rows]).any() and (rest[~rows] == 0).all()
+
+
+@pytest.mark.parametrize("E,tokens", [(128, 37), (256, 5000), (512, 9000)])
+def test_folded_entries_without_what_the_rounding_leaves(built_library, E, tokens):
+    """The C entries with the matrix alone: the same matrix, and of weights whose products it holds exactly (halves up to 1.5, 256 hidden features,
+    one in 32 not zero: sums of 8 on average) the result with the remainder, which is zero then, to the order of the fp32 sums."""
+    import ctypes as C
+    from sspmm_amd.attention import block_dense, fold_blocks
+    g = torch.Generator("cuda").manual_seed(E)
+    blk, = _two_layers(E, 256, 1, g)
+    L, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    with torch.no_grad():
+        for m in (blk.linear1, blk.linear2):
+            w = torch.randint(-3, 4, m.weight.shape, device="cuda", generator=g) * 0.5
+            m.weight.copy_(w * (torch.rand(m.weight.shape, device="cuda", generator=g) < 1 / 32))
+        packed, (pair,) = fold_blocks([blk], [blk.out_proj], [E // 4])
+        assert (pair.rest == 0).all()
+        x, attn = torch.randn(tokens, 1, E, device="cuda", generator=g).half(), torch.randn(tokens, 1, E, device="cuda", generator=g).half()
+        want = block_dense(x, attn, blk, blk.layer_norm1, keep_x=True, packed=packed, folded=pair)
+    w21, affine, kept, out = torch.empty_like(pair[0]), torch.empty_like(pair[1]), torch.empty_like(x), torch.empty_like(x)
+    one = lambda t: (C.c_void_p * 1)(t.data_ptr())  # noqa: E731
+    assert L.sspmm_block_fold_f16(0, None, None, None, None, None, 1, E, (C.c_int32 * 1)(256), one(blk.linear1.weight), one(blk.linear1.bias),
+                                  one(blk.linear2.weight), one(blk.linear2.bias), w21.data_ptr(), affine.data_ptr(), stream) == 0
+    assert torch.equal(w21, pair[0]) and torch.equal(affine, pair[1])
+    ln2, ln1 = blk.layer_norm2, blk.layer_norm1
+    assert L.sspmm_block_dense_folded_f16(tokens, 1, E, x.data_ptr(), E, E, attn.data_ptr(), packed[0].data_ptr(), blk.out_proj.bias.data_ptr(),
+                                          ln2.weight.data_ptr(), ln2.bias.data_ptr(), ln2.eps, w21.data_ptr(), affine.data_ptr(), ln1.weight.data_ptr(),
+                                          ln1.bias.data_ptr(), ln1.eps, 0, 0, None, None, kept.data_ptr(), out.data_ptr(), stream) == 0
+    for got, ref in zip((kept, out), want):  # (one step of fp16 where a sum lies next to the middle of two)
+        assert (got.double() - ref.double()).abs().max() <= 2.0 ** -10 * ref.double().abs().max()
 
 
 @pytest.mark.parametrize("E,mlp,tokens", [(128, 256, 333), (256, 1024, 500), (256, 512, 4100), (512, 1024, 40), (512, 512, 4100)])
