@@ -640,8 +640,9 @@ hipError_t launch(const BlockDenseArgs &p, hipStream_t stream) {
 // CU one: 8192 tokens of 128, 256, 512 features 15, 26, 56 us against 18, 30, 73; 10000 tokens 25, 43, 101 against 18, 31, 73.
 // Up to 4096 tokens 16 do the same, and a workgroup's chain of products and LayerNorms is shorter: 2048 tokens 10.0, 17.5, 43 us
 // against 12.3, 20.1, 48 with 32 (without attention 4.6, 7.4, 17 against 5.6, 9.2, 20), 4096 tokens 10.9, 19.3, 46 against 12.6, 21.2,
-// 49; 8192 tokens without attention 7.6, 14.2, 36 against 6.6, 11.1, 25.  (Both linear layers, LayerNorms of two exchanges.)  Folded (one matrix), 256 features,
-// 16 / 32 / 64 tokens: 8192 tokens 21 / 16.5 / 19.7, 32768 75 / 50 / 38.5.
+// 49; 8192 tokens without attention 7.6, 14.2, 36 against 6.6, 11.1, 25.  (Both linear layers, LayerNorms of two exchanges.)  Folded, replayed,
+// 16 / 32 / 64 tokens, 128 features: 4096 tokens 6.7 / 7.6 / 10.3, 8192 9.1 / 8.3 / 10.8, 10000 12.6 / 13.7 / 11.2, 32768 28.5 / 27.3 / 17.3; 256: 12.7 / 13.8 / 18.6,
+// 20.1 / 15.7 / 19.8, 27.7 / 25.5 / 20.3, 68 / 53 / 37.3; 512: 36.6 / 37.2 / 47.5, 65.6 / 43.0 / 48.9, 91.8 / 74.0 / 50.0, 243 / 157 / 115.
 template <int E>
 hipError_t launch_for_width(const BlockDenseArgs &p, hipStream_t stream) {
   if (p.tokens <= 256 * 16) return launch<E, 16>(p, stream);
